@@ -126,13 +126,14 @@ struct ModelImage {
   std::vector<int> adj_off;
   std::vector<int4> adj;
   std::vector<int> bin_cons;          // active indices of binary constraints (plane build order)
+  std::vector<int> tabs;              // active indices of table constraints
   std::vector<u64> rel_dense;         // owned dense rows when the desc has none
   const u64* rel = nullptr;           // [nb][max_dom][rel_words]
   int rel_words = 0;
   std::vector<u64> tsup;
   long long sup_words = 0;
   std::vector<u64> init_dom;          // [n][W]
-  std::vector<int> nbr;               // [n] distinct neighbours over the active constraints
+  std::vector<int> nbr;               // [n] distinct neighbours over the active constraints, then tabs
 };
 
 ModelImage make_image(const cpim_model_desc* d, bool skip_non_binary, bool own_rel = false) {
@@ -216,6 +217,7 @@ ModelImage make_image(const cpim_model_desc* d, bool skip_non_binary, bool own_r
       }
       tsup_off += words;
       bin_ordinal_of_active.push_back(-1);
+      im.tabs.push_back((int)im.con.size());
       im.con.push_back(m);
     }
   }
@@ -283,6 +285,7 @@ ModelImage make_image(const cpim_model_desc* d, bool skip_non_binary, bool own_r
         }
       }
   }
+  im.nbr.insert(im.nbr.end(), im.tabs.begin(), im.tabs.end());
   // level 0
   im.init_dom.assign(nw, 0ull);
   for (int v = 0; v < im.n; ++v)
@@ -358,7 +361,8 @@ struct Arena {
 
 struct DevModel {
   int n = 0, W = 0, dpad = 0, max_dom = 0, num_active = 0;
-  DevAlloc adj_off, adj, con, sup, tsup, cap, nbr;
+  DevAlloc adj_off, adj, con, sup, tsup, cap, nbr;  // nbr: [n], then the table constraints
+  int ntabs = 0;
   DevAlloc lnet_img;  // the network image for LDS (LdsNet), when small enough
   LdsNet lnet{};
   long long bytes = 0;
@@ -373,6 +377,8 @@ struct DevModel {
     d.con = con.as<ConMeta>();
     d.sup = sup.as<u64>();
     d.tsup = tsup.as<u64>();
+    d.tabs = nbr.as<int>() + n;
+    d.ntabs = ntabs;
     return d;
   }
 };
@@ -396,35 +402,41 @@ constexpr long long kLdsNetMax = 128 * 1024;
 long long align16(long long b) { return (b + 15) & ~15ll; }
 
 // The LdsNet image of a network: the arrays of DevNet in one block, planes
-// and tables with value stride dc = max_dom instead of dpad.  Built after the
+// and tables with value stride dc (LdsNet) instead of dpad.  Built after the
 // planes (the plane rows are copied from the device planes); skipped when the
 // image would exceed kLdsNetMax.  The copies are queued on s from `h`,
 // which the caller keeps until s is synchronized.
 struct LdsLayout {
-  long long o_adj, o_con, o_sup, o_tsup, bytes;
+  int dc;
+  long long o_adj, o_con, o_sup, o_tsup, o_tabs, bytes;
 };
 
-LdsLayout lds_layout(const ModelImage& im) {
-  const int n = im.n, W = im.W, dc = std::max(1, im.max_dom);
+LdsLayout lds_layout(const ModelImage& im, bool odd = true) {
+  // an even stride only where the odd one alone keeps the image out of LDS
+  const int n = im.n, W = im.W, dc = odd ? im.max_dom | 1 : im.max_dom;
   const long long npairs = (long long)im.bin_cons.size();
   long long tsup_c = 0;
   for (const ConMeta& m : im.con)
     if (m.kind == 1) tsup_c += (long long)m.arity * dc * m.tw;
   LdsLayout L;
+  L.dc = dc;
   L.o_adj = align16(4ll * (n + 1));
   L.o_con = L.o_adj + align16(16ll * (long long)im.adj.size());
   L.o_sup = L.o_con + align16((long long)sizeof(ConMeta) * (long long)im.con.size());
   const long long sup_words = npairs * 2 * W * dc + 64ll * W;
   L.o_tsup = L.o_sup + align16(8 * sup_words);
-  L.bytes = L.o_tsup + align16(8 * std::max<long long>(1, tsup_c));
+  L.o_tabs = L.o_tsup + align16(8 * std::max<long long>(1, tsup_c));
+  L.bytes = L.o_tabs + align16(4 * (long long)im.tabs.size());
+  if (odd && L.bytes > kLdsNetMax) return lds_layout(im, false);
   return L;
 }
 
 void build_lds_image(const ModelImage& im, DevModel& dm, hipStream_t s, std::vector<char>& h,
                      Arena* arena = nullptr) {
-  const int n = im.n, W = im.W, dpad = im.dpad, dc = std::max(1, im.max_dom);
+  const int n = im.n, W = im.W, dpad = im.dpad;
   const long long npairs = (long long)im.bin_cons.size();
   const LdsLayout L = lds_layout(im);
+  const int dc = L.dc;
   const long long o_adj = L.o_adj, o_con = L.o_con, o_sup = L.o_sup, o_tsup = L.o_tsup, bytes = L.bytes;
   if (bytes > kLdsNetMax) return;
   h.assign((size_t)bytes, 0);
@@ -439,7 +451,7 @@ void build_lds_image(const ModelImage& im, DevModel& dm, hipStream_t s, std::vec
       m.off = m.off / (2ll * W * dpad) * (2ll * W * dc);
     } else {
       for (int q = 0; q < m.arity; ++q)
-        for (int a = 0; a < dc; ++a)
+        for (int a = 0; a < im.max_dom; ++a)
           std::memcpy(ts + toff + ((long long)q * dc + a) * m.tw,
                       im.tsup.data() + m.off + ((long long)q * dpad + a) * m.tw, 8 * (size_t)m.tw);
       m.off = toff;
@@ -447,11 +459,12 @@ void build_lds_image(const ModelImage& im, DevModel& dm, hipStream_t s, std::vec
     }
     con[c] = m;
   }
+  if (!im.tabs.empty()) std::memcpy(h.data() + L.o_tabs, im.tabs.data(), 4 * im.tabs.size());
   dm.lnet_img = dev_array(arena, bytes);
   HIPC(hipMemcpyAsync(dm.lnet_img.p, h.data(), (size_t)bytes, hipMemcpyHostToDevice, s));
   if (npairs > 0)
     HIPC(hipMemcpy2DAsync((char*)dm.lnet_img.p + o_sup, 8 * (size_t)dc, dm.sup.p, 8 * (size_t)dpad,
-                          8 * (size_t)dc, (size_t)(npairs * 2 * W), hipMemcpyDeviceToDevice, s));
+                          8 * (size_t)std::min(dc, dpad), (size_t)(npairs * 2 * W), hipMemcpyDeviceToDevice, s));
   dm.bytes += bytes;
   dm.lnet.src = dm.lnet_img.as<uint4>();
   dm.lnet.bytes = (int)bytes;
@@ -460,6 +473,7 @@ void build_lds_image(const ModelImage& im, DevModel& dm, hipStream_t s, std::vec
   dm.lnet.o_con = (int)o_con;
   dm.lnet.o_sup = (int)o_sup;
   dm.lnet.o_tsup = (int)o_tsup;
+  dm.lnet.o_tabs = (int)L.o_tabs;
 }
 
 // Device bytes build_device_model takes from an arena for im (the same
@@ -505,6 +519,7 @@ void build_device_model(const ModelImage& im, DevModel& dm, hipStream_t s, Arena
   upload(dm.tsup, im.tsup, s, dm.bytes, arena);
   upload(dm.cap, im.cap, s, dm.bytes, arena);
   upload(dm.nbr, im.nbr, s, dm.bytes, arena);
+  dm.ntabs = (int)im.tabs.size();
   dm.sup = dev_array(arena, (long long)sizeof(u64) * im.sup_words);
   dm.bytes += sizeof(u64) * im.sup_words;
   const int nb = (int)im.bin_cons.size();
@@ -1913,13 +1928,12 @@ int cpim_gmodel_solve(cpim_gmodel* m, const cpim_solve_opts* opts, cpim_search_s
         bytes + m->dm.lnet.bytes <= (long long)m->props.max_lds - 2048)
       lnet = m->dm.lnet;
     while (true) {
-      if (bytes <= kLdsBudget) {
-        hipLaunchKernelGGL(k_mac<true>, dim3(1), dim3(threads), (size_t)(bytes + lnet.bytes), m->stream, net,
-                           A, (char*)nullptr, lnet);
-      } else {
-        char* scratch = m->get_scratch(bytes);
-        hipLaunchKernelGGL(k_mac<false>, dim3(1), dim3(threads), 0, m->stream, net, A, scratch, LdsNet{});
-      }
+      const bool lds = bytes <= kLdsBudget;
+      char* scratch = lds ? nullptr : m->get_scratch(bytes);
+      const size_t dyn = lds ? (size_t)(bytes + lnet.bytes) : 0;
+      auto* kernel = lds ? (A.weight ? k_mac<true, true> : k_mac<true, false>)
+                         : (A.weight ? k_mac<false, true> : k_mac<false, false>);
+      hipLaunchKernelGGL(kernel, dim3(1), dim3(threads), dyn, m->stream, net, A, scratch, lds ? lnet : LdsNet{});
       HIPC(hipGetLastError());
       HIPC(hipMemcpyAsync(&s, state.p, sizeof(s), hipMemcpyDeviceToHost, m->stream));
       m->sync();

@@ -676,50 +676,36 @@ __global__ void k_sizes(const u64* dom, int* size, int n, int W) {
 // else in a per-workgroup global scratch region) and runs an AC fixpoint over
 // a variable frontier: every round revises all arcs u <- t for the variables
 // t that changed in the previous round, spread over the waves of the
-// workgroup (one arc at a time per wave, taken from an LDS counter).
-// Assigned variables (asg bitmap) are never revised, as in AC3::enforce
-// (src/AC3.cpp:114); the closure is the same with or without that skip.
+// workgroup.  Assigned variables (asg bitmap) are never revised, as in
+// AC3::enforce (src/AC3.cpp:114); the closure is the same with or without
+// that skip.
 // ===========================================================================
 struct WgMem {
   u64* dom;       // [n * W]
-  int* size;      // [n]
-  unsigned* cur;  // [nvw]
-  unsigned* nxt;  // [nvw]
-  unsigned* asg;  // [nvw]
   int* list;      // [n]
   int* pre;       // [n + 1]
+  int* size;      // [n]
+  unsigned* bm;   // [3][nvw] frontier bitmaps, rotating by round
+  unsigned* asg;  // [nvw]
   const int* aoff;   // adjacency offsets (net.adj_off)
   const int4* adj;   // adjacency entries (net.adj)
 };
 
 struct WgCtl {
-  int arc_ctr;
-  int wipe;
-  int nchanged[2];
-  int m;
-  int total;
-  int k;  // arcs per work item this round
-  int sel_var;
-  int sel_val;
+  // lowest round that emptied a domain, of the running fixpoint (slot: see wg_fixpoint)
+  int wipe_round[2];
   unsigned long long revs;
   u64 red[16];  // one slot per wave for block reductions
-  // MAC control
-  int status;
-  int depth;
-  long long npos;
-  long long nneg;
-  long long nodes_here;
-  int trace_len;
   int ok;
 };
 
 __host__ __device__ inline long long wg_mem_bytes(int n, int W) {
   const long long nvw = (n + 31) / 32;
   long long b = 8ll * n * W;
-  b += 4ll * n;          // size
-  b += 4ll * nvw * 3;    // cur, nxt, asg
   b += 4ll * n;          // list
   b += 4ll * (n + 1);    // pre
+  b += 4ll * n;          // size
+  b += 4ll * nvw * 4;    // bm, asg
   return (b + 15) & ~15ll;
 }
 
@@ -731,230 +717,252 @@ __device__ __forceinline__ WgMem wg_carve(char* base, const DevNet& net) {
   m.adj = net.adj;
   m.dom = (u64*)base;
   char* p = base + 8ll * n * W;
-  m.size = (int*)p;
-  p += 4ll * n;
-  m.cur = (unsigned*)p;
-  p += 4ll * nvw;
-  m.nxt = (unsigned*)p;
-  p += 4ll * nvw;
-  m.asg = (unsigned*)p;
-  p += 4ll * nvw;
   m.list = (int*)p;
   p += 4ll * n;
   m.pre = (int*)p;
+  p += 4ll * (n + 1);
+  m.size = (int*)p;
+  p += 4ll * n;
+  m.bm = (unsigned*)p;
+  p += 12ll * nvw;
+  m.asg = (unsigned*)p;
   return m;
 }
 
 __device__ __forceinline__ bool bit_of(const unsigned* bm, int v) { return (bm[v >> 5] >> (v & 31)) & 1u; }
 
-// Record that v changed in this round: set its bit in the round's next
-// frontier (the swapped pointer, not mem.nxt) and count it once.
-__device__ __forceinline__ void wg_mark(unsigned* nxt, WgCtl* ctl, int v, int slot) {
-  const unsigned bit = 1u << (v & 31);
-  const unsigned old = atomicOr(&nxt[v >> 5], bit);
-  if (!(old & bit)) atomicAdd(&ctl->nchanged[slot], 1);
+__device__ __forceinline__ int ld_wg_int(const int* p) {
+  return __hip_atomic_load(const_cast<int*>(p), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
 }
 
-// AC fixpoint from the seed in mem.cur.  both_dirs_round0: in the first round
-// also revise t <- u for every arc of a seed variable t (constraint seeding,
-// as GModel::EnforceGAC(assigned_var) does).  Returns false on wipe-out.
-// Must be called by every thread of the workgroup.  Work items are runs of
-// up to kWgArcs arcs of one changed variable: the lanes of a wave fetch the
-// arcs' metadata together, then the wave revises kP binary arcs at a time
-// (revise_binary_multi keeps the row loads of all in flight), or one by one
-// for tables and assigned targets.  kP = 4 for the MAC kernels (uneven batch
-// 47 ms against 50 ms at kP = 2); 2 elsewhere, where kP = 4 costs occupancy.
-constexpr int kWgArcs = 8;  // most arcs per work item
+// Word w of a revision tgt <- src of the binary constraint whose planes start
+// at off, by one lane: the values of `need` (word w of D(tgt)) without a
+// support in D(src).
+//
+// A step keeps four row reads in flight.  Source side: the rows of four
+// values of src are ORed, and the values of tgt they cover are settled; a
+// value stays open with the product of four tightnesses, so a few steps
+// settle nearly every supported value, whatever the domains' sizes.  Target
+// side: an open value b is settled by the W words of its own row.  The lane
+// takes source steps first and turns to the target side once at most one
+// target step is left, or after three source steps, if that takes fewer steps
+// than the rest of D(src): a true removal then costs W reads instead of a
+// scan of D(src).
+__device__ __forceinline__ u64 lane_unsupported(const DevNet& net, const u64* dom, long long off, int src,
+                                                int pos_src, int w, u64 need) {
+  const int W = net.W, dpad = net.dpad;
+  const u64* rows = net.sup + off + (long long)(pos_src * W + w) * dpad;
+  const u64* ds = dom + (long long)src * W;
+  u64 x = ld_wg(&ds[0]);
+  int left = __popcll(x);
+  for (int j = 1; j < W; ++j) left += __popcll(ld_wg(&ds[j]));
+  int j = 0, done = 0;
+  while (need && left > 0) {
+    const int ts = (__popcll(need) * W + 3) >> 2;
+    if (left > 4 * ts && (ts <= 1 || done >= 3)) break;
+    u64 r[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      while (x == 0ull && j + 1 < W) x = ld_wg(&ds[++j]);
+      const int a = x ? (int)__builtin_ctzll(x) : 0;
+      r[i] = x ? rows[64 * j + a] : 0ull;
+      x &= x - 1ull;
+    }
+    need &= ~((r[0] | r[1]) | (r[2] | r[3]));
+    left -= 4;
+    ++done;
+  }
+  if (need == 0ull || left <= 0) return need;
+  const u64* own = net.sup + off + (long long)(1 - pos_src) * W * dpad + 64 * w;
+  u64 gone = 0ull;
+  if (W == 1) {
+    const u64 d = ld_wg(&ds[0]);
+    while (need) {
+      u64 r[4], bit[4];
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        bit[i] = need & (0ull - need);
+        r[i] = need ? own[__builtin_ctzll(need)] : ~0ull;
+        need &= need - 1ull;
+      }
+#pragma unroll
+      for (int i = 0; i < 4; ++i) gone |= (r[i] & d) ? 0ull : bit[i];
+    }
+    return gone;
+  }
+  while (need) {
+    const int b = (int)__builtin_ctzll(need);
+    bool ok = false;
+    for (int j0 = 0; j0 < W && !ok; j0 += 4) {
+      u64 r[4];
+#pragma unroll
+      for (int i = 0; i < 4; ++i) r[i] = j0 + i < W ? own[(long long)(j0 + i) * dpad + b] : 0ull;
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+        if (j0 + i < W) ok = ok || (r[i] & ld_wg(&ds[j0 + i])) != 0ull;
+    }
+    if (!ok) gone |= 1ull << b;
+    need &= need - 1ull;
+  }
+  return gone;
+}
 
-template <int kP = 2>
-__device__ __forceinline__ bool wg_fixpoint(const DevNet& net, WgMem mem, WgCtl* ctl, bool both_dirs_round0) {
-  const int n = net.n;
+// Word w of the revision tgt <- src by one lane, applied: the removed values
+// leave D(tgt), tgt joins the next frontier, and the lane that brings its
+// size to 0 records the wipe-out.  Lanes that pass a domain word with no
+// values do nothing.
+__device__ __forceinline__ void lane_revise(const DevNet& net, const WgMem& mem, WgCtl* ctl, unsigned* nxt, int slot,
+                                            int round, long long off, int src, int tgt, int pos_src, int w) {
+  u64* word = mem.dom + (long long)tgt * net.W + w;
+  const u64 du = ld_wg(word);
+  const u64 gone = lane_unsupported(net, mem.dom, off, src, pos_src, w, du);
+  if (gone) {
+    const u64 old = and_wg(word, ~gone);
+    const int r = __popcll(old & gone);
+    if (r) {
+      atomicOr(&nxt[tgt >> 5], 1u << (tgt & 31));
+      if (atomicSub(&mem.size[tgt], r) == r) atomicMin(&ctl->wipe_round[slot], round);
+    }
+  }
+}
+
+// Frontier of a fixpoint's first round: variable `seed`, or every variable
+// (seed < 0); the other two bitmaps and the wipe-out word of `slot` are
+// cleared.  Called by every thread, a __syncthreads() before wg_fixpoint.
+__device__ __forceinline__ void wg_seed(const WgMem& mem, WgCtl* ctl, int n, int slot, int seed) {
+  const int nvw = (n + 31) / 32;
+  for (int i = threadIdx.x; i < 3 * nvw; i += blockDim.x) {
+    unsigned v = 0u;
+    if (i < nvw) {
+      const int k = n - 32 * i;
+      if (seed < 0) v = k >= 32 ? 0xffffffffu : ((1u << k) - 1u);
+      else if (i == seed >> 5) v = 1u << (seed & 31);
+    }
+    mem.bm[i] = v;
+  }
+  if (threadIdx.x == 0) ctl->wipe_round[slot] = INT_MAX;
+}
+
+// AC fixpoint from the seed that wg_seed put in mem.bm (a __syncthreads()
+// lies between).  both_dirs_round0: in the first round also revise t <- u for
+// every arc of a seed variable t (constraint seeding, as
+// GModel::EnforceGAC(assigned_var) does).  Returns false on wipe-out.  Must
+// be called by every thread of the workgroup.
+//
+// A unit of work is 64 / Wp arcs of one changed variable t (Wp = W rounded up
+// to a power of two): lane (k, w) revises word w of the k-th arc's target.
+// Every wave numbers the round's units in registers, from the frontier bitmap
+// and the variables' arc counts (lane = variable), and takes every nwaves-th:
+// no list, no shared counter, and one barrier per round.  Tables follow, one
+// per wave, each revised once however many of its variables changed.
+//
+// What bounds it is the chain of dependent reads of a round (frontier,
+// adjacency, domains, rows) and the barrier, not bandwidth.  With a lane per
+// arc word instead of a wave per one to four arcs, one chain serves 64 / Wp
+// arcs and a row read fetches one row of each instead of 64: 1000 search
+// nodes of n=23 d=23 e=253 take 7.4 ms (28.2 ms before), 256 uneven
+// instances (n 20..200, d 8..128) of 64 nodes each 3.4 ms (33 ms before).
+//
+// The frontier bitmaps rotate: round r reads bitmap r % 3, fills (r + 1) % 3
+// and clears (r + 2) % 3, which no wave reads until the barrier of the next
+// round.  A wipe-out is recorded as the round it happened in, so that a wave
+// that still decides round r is not misled by one already in round r + 1.
+// slot: two wipe-out words used in turn by successive fixpoints, so that
+// wg_seed never resets the word a slow wave still reads.
+__device__ __forceinline__ bool wg_fixpoint(const DevNet& net, const WgMem& mem, WgCtl* ctl, int slot,
+                                            bool both_dirs_round0) {
+  const int n = net.n, W = net.W;
   const int nvw = (n + 31) / 32;
   const int tid = threadIdx.x;
   const int nthreads = blockDim.x;
-  const int wave = tid >> 6;
+  const int wave = uniform_int(tid >> 6), nwaves = nthreads >> 6;
   const int lane = lane_id();
-  unsigned* cur = mem.cur;
-  unsigned* nxt = mem.nxt;
-  if (tid == 0) ctl->wipe = 0;
-  unsigned long long revs = 0;
+  int lw = 0;
+  while ((1 << lw) < W) ++lw;
+  const int w = lane & ((1 << lw) - 1), la = lane >> lw, per = 64 >> lw;
+  const long long pair_words = 2ll * W * net.dpad;
+  int revs = 0;
   bool result = true;
+  int c0 = 0, c1 = nvw, c2 = 2 * nvw;
   for (int round = 0;; ++round) {
-    const int slot = round & 1;
-    if (wave == 0) {
-      // item size: at most kWgArcs arcs, small enough for about two items
-      // per wave when the round has few arcs
-      int arcs = 0;
-      for (int v0 = 0; v0 < n; v0 += 64) {
-        const int v = v0 + lane;
-        if (v < n && bit_of(cur, v)) arcs += mem.aoff[v + 1] - mem.aoff[v];
-      }
-      (void)wave_scan_dpp(arcs, &arcs);
-      const int nwaves = nthreads >> 6;
-      const int K = uniform_int(max(1, min(kWgArcs, (arcs + 2 * nwaves - 1) / (2 * nwaves))));
-      int base = 0, ibase = 0;
-      for (int v0 = 0; v0 < n; v0 += 64) {
-        const int v = v0 + lane;
-        const bool f = v < n && bit_of(cur, v);
-        const u64 mask = __ballot(f);
-        const int rank = mbcnt(mask);
-        const int items = f ? (mem.aoff[v + 1] - mem.aoff[v] + K - 1) / K : 0;
-        int round_items = 0;
-        const int inc = wave_scan_dpp(items, &round_items);
-        if (f) {
-          mem.list[base + rank] = v;
-          mem.pre[base + rank] = ibase + inc - items;
-        }
-        base += __popcll(mask);
-        ibase += round_items;
-      }
-      if (lane == 0) {
-        mem.pre[base] = ibase;
-        ctl->m = base;
-        ctl->total = ibase;
-        ctl->k = K;
-        ctl->arc_ctr = 0;
-        ctl->nchanged[slot] = 0;
-      }
-    } else {
-      for (int i = tid - 64; i < nvw; i += nthreads - 64) nxt[i] = 0u;
-    }
-    if (nthreads == 64)
-      for (int i = lane; i < nvw; i += 64) nxt[i] = 0u;
-    __syncthreads();
-    const int total = uniform_int(ctl->total);
-    const int m = uniform_int(ctl->m);
-    const int K = uniform_int(ctl->k);
+    const unsigned* cur = mem.bm + c0;
+    unsigned* nxt = mem.bm + c1;
+    for (int i = tid; i < nvw; i += nthreads) mem.bm[c2 + i] = 0u;
     const bool both = both_dirs_round0 && round == 0;
-    while (true) {
-      int idx = 0;
-      if (lane == 0) idx = atomicAdd(&ctl->arc_ctr, 1);
-      idx = uniform_int(__shfl(idx, 0, 64));
-      if (idx >= total) break;
-      if (uniform_int(ctl->wipe)) break;
-      int lo = 0, hi = m - 1;
-      while (lo < hi) {
-        const int mid = (lo + hi + 1) >> 1;
-        if (mem.pre[mid] <= idx) lo = mid;
-        else hi = mid - 1;
+    int mine = wave;  // this wave's next unit, counted from the block of variables below
+    bool stop = false;
+    for (int v0 = 0; v0 < n && !stop; v0 += 64) {
+      const int v = v0 + lane;
+      const bool f = v < n && bit_of(cur, v);
+      int a0 = 0, deg = 0;
+      if (f) {
+        a0 = mem.aoff[v];
+        deg = mem.aoff[v + 1] - a0;
       }
-      const int t = uniform_int(mem.list[lo]);
-      const int s0 = mem.aoff[t] + (idx - uniform_int(mem.pre[lo])) * K;
-      const int cnt = uniform_int(min(s0 + K, mem.aoff[t + 1]) - s0);
-      int4 e = make_int4(0, 0, 0, 0);
-      if (lane < cnt) e = mem.adj[s0 + lane];
-      for (int i = 0; i < cnt; ++i) {
-        const int c = __builtin_amdgcn_readlane(e.x, i);
-        const int u = __builtin_amdgcn_readlane(e.y, i);
-        bool wiped = false;
-        // up to kP binary arcs with live targets: revised together
-        if (u >= 0 && !both) {
-          int np = 1;
-          while (np < kP && i + np < cnt) {
-            const int un = __builtin_amdgcn_readlane(e.y, i + np);
-            if (un < 0 || uniform_int((int)bit_of(mem.asg, un))) break;
-            ++np;
-          }
-          if (np >= 2 && !uniform_int((int)bit_of(mem.asg, u))) {
-            if (kP >= 4 && np >= 4) {
-              long long o[4];
-              int uu[4], pt[4], r[4];
-              bool w[4];
-#pragma unroll
-              for (int p = 0; p < 4; ++p) {
-                o[p] = (long long)__builtin_amdgcn_readlane(e.w, i + p) * 2 * net.W * net.dpad;
-                uu[p] = __builtin_amdgcn_readlane(e.y, i + p);
-                pt[p] = __builtin_amdgcn_readlane(e.z, i + p);
-              }
-              revise_binary_multi<4>(net, mem.dom, mem.size, t, o, uu, pt, r, w);
-              revs += 4;
-#pragma unroll
-              for (int p = 0; p < 4; ++p) {
-                if (r[p] && lane == 0) wg_mark(nxt, ctl, uu[p], slot);
-                if (w[p] && lane == 0) ctl->wipe = 1;
-              }
-              i += 3;
-              continue;
-            }
-            long long o[2];
-            int uu[2], pt[2], r[2];
-            bool w[2];
-#pragma unroll
-            for (int p = 0; p < 2; ++p) {
-              o[p] = (long long)__builtin_amdgcn_readlane(e.w, i + p) * 2 * net.W * net.dpad;
-              uu[p] = __builtin_amdgcn_readlane(e.y, i + p);
-              pt[p] = __builtin_amdgcn_readlane(e.z, i + p);
-            }
-            revise_binary_multi<2>(net, mem.dom, mem.size, t, o, uu, pt, r, w);
-            revs += 2;
-#pragma unroll
-            for (int p = 0; p < 2; ++p) {
-              if (r[p] && lane == 0) wg_mark(nxt, ctl, uu[p], slot);
-              if (w[p] && lane == 0) ctl->wipe = 1;
-            }
-            ++i;
-            continue;
+      const int units = (deg + per - 1) >> (6 - lw);
+      int total = 0;
+      const int inc = wave_scan_dpp(units, &total);
+      for (; mine < total; mine += nwaves) {
+        if (uniform_int(ld_wg_int(&ctl->wipe_round[slot])) <= round) {
+          stop = true;
+          break;
+        }
+        const int l = (int)__builtin_ctzll(__ballot(inc > mine));
+        const int t = v0 + l;
+        const int k = ((mine - __builtin_amdgcn_readlane(inc - units, l)) << (6 - lw)) + la;
+        const int arc = __builtin_amdgcn_readlane(a0, l) + k;
+        const int dt = __builtin_amdgcn_readlane(deg, l);
+        if (k < dt && w < W) {
+          const int4 e = mem.adj[arc];
+          const int u = e.y;
+          if (u >= 0) {  // binary
+            const long long off = e.w * pair_words;
+            if (!bit_of(mem.asg, u)) lane_revise(net, mem, ctl, nxt, slot, round, off, t, u, e.z, w);
+            if (both && !bit_of(mem.asg, t)) lane_revise(net, mem, ctl, nxt, slot, round, off, u, t, 1 - e.z, w);
           }
         }
-        if (u >= 0) {  // binary
-          const int pos_t = __builtin_amdgcn_readlane(e.z, i);
-          const long long o = (long long)__builtin_amdgcn_readlane(e.w, i) * 2 * net.W * net.dpad;
-          if (!bit_of(mem.asg, u)) {
-            const int r = revise_binary_at(net, mem.dom, mem.size, o, u, t, pos_t, &wiped);
-            ++revs;
-            if (r && lane == 0) wg_mark(nxt, ctl, u, slot);
-            if (wiped && lane == 0) ctl->wipe = 1;
-          }
-          if (both && !bit_of(mem.asg, t)) {
-            const int r = revise_binary_at(net, mem.dom, mem.size, o, t, u, 1 - pos_t, &wiped);
-            ++revs;
-            if (r && lane == 0) wg_mark(nxt, ctl, t, slot);
-            if (wiped && lane == 0) ctl->wipe = 1;
-          }
-        } else {
-          revise_table(net, mem.dom, mem.size, c, both ? -1 : t, mem.asg,
-                       [&](int v, int) {
-                         if (lane == 0) wg_mark(nxt, ctl, v, slot);
-                       },
-                       &wiped);
-          ++revs;
-          if (wiped && lane == 0) ctl->wipe = 1;
-        }
+        revs += min(per, dt - (k - la));
       }
+      mine -= total;
+    }
+    for (int i = nwaves - 1 - wave; i < net.ntabs; i += nwaves) {
+      const int c = uniform_int(net.tabs[i]);
+      const ConMeta* mp = net.con + c;
+      const int y = lane < mp->arity ? mp->scope[lane] : -1;
+      const u64 changed = __ballot(y >= 0 && bit_of(cur, y));
+      if (changed == 0ull) continue;
+      if (uniform_int(ld_wg_int(&ctl->wipe_round[slot])) <= round) break;
+      // one changed variable: its own values keep their supports
+      int skip = -1;
+      if (!both && (changed & (changed - 1ull)) == 0ull) skip = __builtin_amdgcn_readlane(y, (int)__builtin_ctzll(changed));
+      bool wiped = false;
+      revise_table(net, mem.dom, mem.size, c, skip, mem.asg,
+                   [&](int v, int) {
+                     if (lane == 0) atomicOr(&nxt[v >> 5], 1u << (v & 31));
+                   },
+                   &wiped);
+      ++revs;
+      if (wiped && lane == 0) atomicMin(&ctl->wipe_round[slot], round);
     }
     __syncthreads();
-    if (uniform_int(ctl->wipe)) {
+    if (uniform_int(ld_wg_int(&ctl->wipe_round[slot])) <= round) {
       result = false;
       break;
     }
-    if (uniform_int(ctl->nchanged[slot]) == 0) break;
-    unsigned* tmp = cur;
-    cur = nxt;
-    nxt = tmp;
+    bool any = false;
+    for (int i = 0; i < nvw; i += 64) any = any || __ballot(i + lane < nvw && nxt[i + lane] != 0u) != 0ull;
+    if (!any) break;
+    const int c = c0;
+    c0 = c1;
+    c1 = c2;
+    c2 = c;
   }
-  if (lane == 0 && revs) atomicAdd(&ctl->revs, revs);
-  __syncthreads();
+  if (lane == 0 && revs) atomicAdd(&ctl->revs, (unsigned long long)revs);
   return result;
 }
 
 __device__ __forceinline__ void wg_clear_bitmap(unsigned* bm, int nvw) {
   for (int i = threadIdx.x; i < nvw; i += blockDim.x) bm[i] = 0u;
-}
-
-__device__ __forceinline__ void wg_fill_bitmap(unsigned* bm, int n) {
-  const int nvw = (n + 31) / 32;
-  for (int i = threadIdx.x; i < nvw; i += blockDim.x) {
-    const int k = n - 32 * i;
-    bm[i] = k >= 32 ? 0xffffffffu : ((1u << k) - 1u);
-  }
-}
-
-__device__ __forceinline__ void wg_recount(WgMem mem, int n, int W) {
-  for (int v = threadIdx.x; v < n; v += blockDim.x) {
-    int s = 0;
-    for (int w = 0; w < W; ++w) s += __popcll(mem.dom[(long long)v * W + w]);
-    mem.size[v] = s;
-  }
 }
 
 __device__ __forceinline__ void wg_copy_words(u64* dst, const u64* src, long long count) {
@@ -985,13 +993,6 @@ __device__ __forceinline__ u64 wg_reduce_sum_u64(WgCtl* ctl, u64 v) {
   return (u64)uniform_ll((long long)r);
 }
 
-__device__ __forceinline__ u64 wg_dom_hash(WgCtl* ctl, const u64* dom, int n, int W) {
-  u64 h = 0;
-  for (long long i = threadIdx.x; i < (long long)n * W; i += blockDim.x)
-    h += mix64(dom[i] + (u64)i * 0x9E3779B97F4A7C15ull);
-  return wg_reduce_sum_u64(ctl, h);
-}
-
 // ---------------------------------------------------------------------------
 // Block-mode GAC on one level (one workgroup).
 // ---------------------------------------------------------------------------
@@ -1013,19 +1014,12 @@ __global__ void k_block_gac(DevNet net, u64* dom, int* size, int seed_var, char*
   if (threadIdx.x == 0) ctl.revs = 0;
   wg_copy_words(mem.dom, dom, (long long)n * W);
   for (int v = threadIdx.x; v < n; v += blockDim.x) mem.size[v] = size[v];
-  const int nvw = (n + 31) / 32;
-  wg_clear_bitmap(mem.asg, nvw);
-  if (seed_var < 0) {
-    wg_fill_bitmap(mem.cur, n);
-  } else {
-    wg_clear_bitmap(mem.cur, nvw);
-  }
-  __syncthreads();
-  if (seed_var >= 0 && threadIdx.x == 0) mem.cur[seed_var >> 5] |= 1u << (seed_var & 31);
+  wg_clear_bitmap(mem.asg, (n + 31) / 32);
+  wg_seed(mem, &ctl, n, 0, seed_var);
   __syncthreads();
   long long before = 0;
   for (int v = threadIdx.x; v < n; v += blockDim.x) before += mem.size[v];
-  const bool ok = wg_fixpoint(net, mem, &ctl, seed_var >= 0);
+  const bool ok = wg_fixpoint(net, mem, &ctl, 0, seed_var >= 0);
   long long after = 0;
   for (int v = threadIdx.x; v < n; v += blockDim.x) after += mem.size[v];
   const u64 delta = wg_reduce_sum_u64(&ctl, (u64)(before - after));
@@ -1064,17 +1058,17 @@ __global__ void k_singleton_tests(DevNet net, const u64* __restrict__ base_dom,
   wg_copy_words(mem.dom, base_dom, (long long)n * W);
   for (int v = threadIdx.x; v < n; v += blockDim.x) mem.size[v] = base_size[v];
   wg_clear_bitmap(mem.asg, nvw);
-  wg_clear_bitmap(mem.cur, nvw);
+  wg_seed(mem, &ctl, n, 0, x);
   if (threadIdx.x == 0) ctl.revs = 0;
   __syncthreads();
   if (threadIdx.x < W) mem.dom[(long long)x * W + threadIdx.x] = (threadIdx.x == (a >> 6)) ? (1ull << (a & 63)) : 0ull;
   if (threadIdx.x == 0) {
     mem.size[x] = 1;
     mem.asg[x >> 5] |= 1u << (x & 31);
-    mem.cur[x >> 5] |= 1u << (x & 31);
   }
   __syncthreads();
-  const bool ok = wg_fixpoint(net, mem, &ctl, false);
+  const bool ok = wg_fixpoint(net, mem, &ctl, 0, false);
+  __syncthreads();  // every wave's revision count
   if (threadIdx.x == 0) {
     fail[unit] = ok ? 0 : 1;
     if (ctl.revs) atomicAdd(&revs_out[blockIdx.x % kStatSlots], ctl.revs);
@@ -2143,7 +2137,10 @@ struct NodeRec {
 // A copy of a network laid out as it sits in LDS behind the working memory:
 // adjacency offsets, adjacency, constraint metadata, support planes, tables.
 // The value stride of the planes and tables is cut from dpad (64 W) to dc,
-// the largest domain, and the constraint offsets follow that stride.  The
+// the largest domain rounded up to an odd number, and the constraint offsets
+// follow that stride.  Odd, because the lanes of a wave read the same value's
+// rows of different planes: with an even stride of 16 or 32 words they would
+// all meet on the same LDS banks.  The
 // planes are followed by 64 W words of zeros: a target-side revision loads
 // whole 64-value chunks of a row, and the lanes past dc (values that are
 // never live) must still read inside the image.  bytes = 0: no image.
@@ -2151,7 +2148,7 @@ struct LdsNet {
   const uint4* src;  // device copy of the image
   int bytes;         // multiple of 16
   int dc;
-  int o_adj, o_con, o_sup, o_tsup;  // byte offsets in the image
+  int o_adj, o_con, o_sup, o_tsup, o_tabs;  // byte offsets in the image
 };
 
 // Copies the image behind the working memory (at dst) and returns the
@@ -2167,6 +2164,7 @@ __device__ __forceinline__ DevNet wg_load_net(const DevNet& g, const LdsNet& L, 
   ln.con = (const ConMeta*)(dst + L.o_con);
   ln.sup = (const u64*)(dst + L.o_sup);
   ln.tsup = (const u64*)(dst + L.o_tsup);
+  ln.tabs = (const int*)(dst + L.o_tabs);
   return ln;
 }
 
@@ -2195,25 +2193,28 @@ struct MacArgs {
 
 enum { MAC_INIT = 0, MAC_RUNNING = 1, MAC_SAT = 2, MAC_UNSAT = 3, MAC_LIMIT = 4 };
 
-__device__ __forceinline__ void wg_trace(const DevNet& net, WgMem mem, WgCtl* ctl, const MacArgs& A, int positive,
-                         int var, int val, bool ok) {
+// Records node number *len of the search (wave 0; the domains must not change
+// until the workgroup's next barrier).
+__device__ __forceinline__ void wg_trace(const DevNet& net, const WgMem& mem, const MacArgs& A, int* len, int positive,
+                                         int var, int val, bool ok) {
   if (!A.trace) return;
-  const int tl = uniform_int(ctl->trace_len);
-  if (tl < A.trace_cap) {
-    const u64 h = ok ? wg_dom_hash(ctl, mem.dom, net.n, net.W) : 0ull;
-    if (threadIdx.x == 0) {
-      NodeRec r;
-      r.positive = positive;
-      r.var = var;
-      r.value = val;
-      r.consistent = ok ? 1 : 0;
-      r.dom_hash = h;
-      A.trace[tl] = r;
-    }
+  const int tl = *len;
+  *len = tl + 1;
+  if (tl >= A.trace_cap || threadIdx.x >= 64) return;
+  u64 h = 0ull;
+  if (ok) {
+    for (int i = lane_id(); i < net.n * net.W; i += 64) h += mix64(mem.dom[i] + (u64)i * 0x9E3779B97F4A7C15ull);
+    h = wave_sum64_dpp(h);
   }
-  __syncthreads();
-  if (threadIdx.x == 0) ctl->trace_len = tl + 1;
-  __syncthreads();
+  if (threadIdx.x == 0) {
+    NodeRec r;
+    r.positive = positive;
+    r.var = var;
+    r.value = val;
+    r.consistent = ok ? 1 : 0;
+    r.dom_hash = h;
+    A.trace[tl] = r;
+  }
 }
 
 // ---------------------------------------------------------------------------
@@ -2224,8 +2225,8 @@ __device__ __forceinline__ void wg_trace(const DevNet& net, WgMem mem, WgCtl* ct
 // constraint's weight is raised (AC3.cpp:122-126): the input of the dom/wdeg
 // ordering.
 //
-// The queue (ring of n + 1), the queued flags and the variable stamps use the
-// workgroup's arc-list arrays (pre, nxt, list), which this schedule does not
+// The queue (ring of n + 1), the queued flags and the variable stamps use
+// pre, the second frontier bitmap and list, which this schedule does not
 // otherwise need.  Variable stamps restart at 0 on each call, as in the
 // reference.  Constraint stamps stay in global memory as absolute times: a
 // call starts at time base = *clock, reads a stamp s as s - base when
@@ -2249,7 +2250,7 @@ __device__ __forceinline__ bool wave_ac3(const DevNet& net, WgMem mem, const Mac
   const int nvw = (n + 31) / 32;
   const int qcap = n + 1;
   int* q = mem.pre;
-  unsigned* inq = mem.nxt;
+  unsigned* inq = mem.bm + nvw;
   int* sv = mem.list;
   long long base = 0;
   if (lane == 0) base = *A.clock;
@@ -2389,116 +2390,139 @@ __device__ __forceinline__ int wg_select_wdeg(const DevNet& net, WgMem mem, WgCt
   return (int)wg_reduce_min_u64(ctl, best == m ? (u64)bv : ~0ull);
 }
 
-__device__ __forceinline__ void wg_mac_run(const DevNet& net, WgMem mem, WgCtl* ctl, const MacArgs& A) {
+// Loads one level of the trail into the working memory, less value skip_val
+// of variable skip_var (skip_var < 0: nothing), and counts the sizes.
+__device__ __forceinline__ void wg_load_level(const WgMem& mem, const u64* level, int n, int W, int skip_var,
+                                              int skip_val) {
+  for (int v = threadIdx.x; v < n; v += blockDim.x) {
+    int size = 0;
+    for (int w = 0; w < W; ++w) {
+      u64 d = level[(long long)v * W + w];
+      if (v == skip_var && w == (skip_val >> 6)) d &= ~(1ull << (skip_val & 63));
+      mem.dom[(long long)v * W + w] = d;
+      size += __popcll(d);
+    }
+    mem.size[v] = size;
+  }
+}
+
+// The search.  Its control lives in registers, identical in every thread
+// (every value below is wave-uniform); LDS holds the domains, the frontier
+// and the decision stack.  One loop with one fixpoint in it: `phase` says
+// what the fixpoint propagates (the root, a decision x = a, a refutation
+// x != a).  A decision costs two barriers and a refutation one, beside the
+// fixpoint's own.  kWdeg: dom/wdeg ordering, fixpoints in AC3's order.
+template <bool kWdeg>
+__device__ __forceinline__ void wg_mac_run(const DevNet& net, const WgMem& mem, WgCtl* ctl, const MacArgs& A) {
+  enum { ROOT, POSITIVE, NEGATIVE };
   const int n = net.n, W = net.W;
   const int nvw = (n + 31) / 32;
+  const int tid = threadIdx.x, nthreads = blockDim.x, lane = lane_id();
   const long long nw = (long long)n * W;
-  // Search control lives in registers, identical in every thread (all values
-  // below are wave-uniform); LDS only carries what thread 0 publishes.
-  int status = A.state->status;
-  int depth = A.state->depth;
-  long long npos = A.state->npos;
-  long long nneg = A.state->nneg;
-  long long nsol = A.state->nsol;
+  int status = uniform_int(A.state->status);
+  int depth = uniform_int(A.state->depth);
+  long long npos = uniform_ll(A.state->npos);
+  long long nneg = uniform_ll(A.state->nneg);
+  long long nsol = uniform_ll(A.state->nsol);
+  int trace_len = uniform_int(A.state->trace_len);
   long long nodes_here = 0;
-  if (threadIdx.x == 0) {
-    ctl->trace_len = A.state->trace_len;
-    ctl->revs = 0;
-  }
-  status = uniform_int(status);
-  depth = uniform_int(depth);
-  npos = uniform_ll(npos);
-  nneg = uniform_ll(nneg);
-  nsol = uniform_ll(nsol);
-  __syncthreads();
+  // the stack in use: AC3's queue and stamps take list and pre under dom/wdeg
+  int2* stk = kWdeg ? A.stack : (int2*)mem.list;
+  int slot = 0, phase = ROOT, x = -1, a = 0;
+  bool select = false;  // the domains are consistent: take the next decision
+  if (tid == 0) ctl->revs = 0;
+  wg_clear_bitmap(mem.asg, nvw);
   if (status == MAC_INIT) {
-    wg_copy_words(mem.dom, A.trail, nw);
-    wg_clear_bitmap(mem.asg, nvw);
-    __syncthreads();
-    wg_recount(mem, n, W);
-    wg_fill_bitmap(mem.cur, n);
-    __syncthreads();
-    const bool ok = A.weight ? wg_ac3(net, mem, ctl, A, -1) : wg_fixpoint<4>(net, mem, ctl, false);
-    if (ok) wg_copy_words(A.trail, mem.dom, nw);
-    if (A.root_out) wg_copy_words(A.root_out, mem.dom, nw);
-    status = ok ? MAC_RUNNING : MAC_UNSAT;
-    depth = 0;
-    __syncthreads();
+    wg_load_level(mem, A.trail, n, W, -1, 0);
+    wg_seed(mem, ctl, n, slot, -1);
+    status = MAC_RUNNING;
   } else if (status == MAC_RUNNING) {
-    wg_copy_words(mem.dom, A.trail + depth * nw, nw);
-    wg_clear_bitmap(mem.asg, nvw);
-    __syncthreads();
-    wg_recount(mem, n, W);
-    if (threadIdx.x == 0)
-      for (int i = 0; i < depth; ++i) mem.asg[A.stack[i].x >> 5] |= 1u << (A.stack[i].x & 31);
+    wg_load_level(mem, A.trail + depth * nw, n, W, -1, 0);
+    if (!kWdeg)
+      for (int i = tid; i < depth; i += nthreads) stk[i] = A.stack[i];
+    select = true;
+  }
+  __syncthreads();
+  if (select) {
+    for (int i = tid; i < depth; i += nthreads) {
+      const int v = A.stack[i].x;
+      atomicOr(&mem.asg[v >> 5], 1u << (v & 31));
+    }
     __syncthreads();
   }
   while (status == MAC_RUNNING) {
-    const bool over_nodes = A.node_limit > 0 && npos + nneg >= A.node_limit;
-    const bool over_time = A.deadline && uniform_ll((long long)wall_clock64()) > (long long)A.deadline;
-    if (over_nodes || over_time || (A.step_budget > 0 && nodes_here >= A.step_budget)) {
-      // suspend (step budget) or stop (limits) at a consistent state of depth `depth`
-      wg_copy_words(A.trail + depth * nw, mem.dom, nw);
-      if (over_nodes || over_time) status = MAC_LIMIT;
-      __syncthreads();
-      break;
-    }
-    // select: min key over undecided variables, lowest id on ties.  dom-min:
-    // key = |D|; dom/deg: |D| / neighbours (integer), -1 without neighbours,
-    // biased by one so that the packed key stays unsigned.
-    int x;
-    if (A.weight) {
-      x = wg_select_wdeg(net, mem, ctl, A);
-    } else {
-      u64 key = ~0ull;
-      for (int v = threadIdx.x; v < n; v += blockDim.x)
-        if (!bit_of(mem.asg, v)) {
-          unsigned hi = (unsigned)mem.size[v];
-          if (A.nbr) {
-            const int g = A.nbr[v];
-            hi = g == 0 ? 0u : (unsigned)(mem.size[v] / g) + 1u;
+    if (select) {
+      const bool over_nodes = A.node_limit > 0 && npos + nneg >= A.node_limit;
+      const bool over_time = A.deadline && uniform_ll((long long)wall_clock64()) > (long long)A.deadline;
+      if (over_nodes || over_time || (A.step_budget > 0 && nodes_here >= A.step_budget)) {
+        // suspend (step budget) or stop (limits) at a consistent state of depth `depth`
+        wg_copy_words(A.trail + depth * nw, mem.dom, nw);
+        if (over_nodes || over_time) status = MAC_LIMIT;
+        break;
+      }
+      // select: min key over undecided variables, lowest id on ties.  dom-min:
+      // key = |D|; dom/deg: |D| / neighbours (integer), -1 without neighbours,
+      // biased by one so that the packed key stays unsigned.  Every wave
+      // finds it by itself.
+      if (kWdeg) {
+        x = wg_select_wdeg(net, mem, ctl, A);
+      } else {
+        u64 key = ~0ull;
+        for (int v = lane; v < n; v += 64)
+          if (!bit_of(mem.asg, v)) {
+            unsigned hi = (unsigned)mem.size[v];
+            if (A.nbr) {
+              const int g = A.nbr[v];
+              hi = g == 0 ? 0u : (unsigned)(mem.size[v] / g) + 1u;
+            }
+            const u64 k = ((u64)hi << 32) | (unsigned)v;
+            key = k < key ? k : key;
           }
-          const u64 k = ((u64)hi << 32) | (unsigned)v;
-          key = k < key ? k : key;
-        }
-      key = wg_reduce_min_u64(ctl, key);
-      x = (int)(key & 0xffffffffu);
-    }
-    // min value of x (every thread scans the same LDS words)
-    int a = -1;
-    for (int w = 0; w < W && a < 0; ++w) {
-      const u64 dw = mem.dom[(long long)x * W + w];
-      if (dw) a = w * 64 + (int)__builtin_ctzll(dw);
-    }
-    a = uniform_int(a);
-    if (a < 0) {
-      // x has an empty domain that no revision reached (no constraints, an
-      // empty initial domain): the search ends without a solution, with no
-      // node recorded, as the oracle's restatement does
-      status = MAC_UNSAT;
+        x = uniform_int((int)(wave_min64_dpp(key) & 0xffffffffu));
+      }
+      // min value of x (every thread scans the same words)
+      a = -1;
+      for (int w = 0; w < W && a < 0; ++w) {
+        const u64 dw = mem.dom[(long long)x * W + w];
+        if (dw) a = w * 64 + (int)__builtin_ctzll(dw);
+      }
+      a = uniform_int(a);
+      if (a < 0) {
+        // x has an empty domain that no revision reached (no constraints, an
+        // empty initial domain): the search ends without a solution, with no
+        // node recorded, as the oracle's restatement does
+        status = MAC_UNSAT;
+        break;
+      }
+      wg_copy_words(A.trail + depth * nw, mem.dom, nw);
       __syncthreads();
-      break;
+      if (tid < W) mem.dom[(long long)x * W + tid] = (tid == (a >> 6)) ? (1ull << (a & 63)) : 0ull;
+      wg_seed(mem, ctl, n, slot, x);
+      if (tid == 0) {
+        A.stack[depth] = make_int2(x, a);
+        if (!kWdeg) stk[depth] = make_int2(x, a);
+        mem.size[x] = 1;
+        mem.asg[x >> 5] |= 1u << (x & 31);
+      }
+      ++depth;
+      ++npos;
+      ++nodes_here;
+      phase = POSITIVE;
+      __syncthreads();
     }
-    wg_copy_words(A.trail + depth * nw, mem.dom, nw);
-    __syncthreads();
-    if (threadIdx.x < W) mem.dom[(long long)x * W + threadIdx.x] = (threadIdx.x == (a >> 6)) ? (1ull << (a & 63)) : 0ull;
-    wg_clear_bitmap(mem.cur, nvw);
-    __syncthreads();
-    if (threadIdx.x == 0) {
-      A.stack[depth] = make_int2(x, a);
-      mem.size[x] = 1;
-      mem.asg[x >> 5] |= 1u << (x & 31);
-      mem.cur[x >> 5] |= 1u << (x & 31);
+    bool ok = kWdeg ? wg_ac3(net, mem, ctl, A, phase == ROOT ? -1 : x) : wg_fixpoint(net, mem, ctl, slot, false);
+    slot ^= 1;
+    select = true;
+    if (phase == ROOT) {
+      if (ok) wg_copy_words(A.trail, mem.dom, nw);
+      if (A.root_out) wg_copy_words(A.root_out, mem.dom, nw);
+      if (!ok) status = MAC_UNSAT;
+      continue;
     }
-    ++depth;
-    ++npos;
-    ++nodes_here;
-    __syncthreads();
-    bool ok = A.weight ? wg_ac3(net, mem, ctl, A, x) : wg_fixpoint<4>(net, mem, ctl, false);
-    wg_trace(net, mem, ctl, A, 1, x, a, ok);
-    if (ok && depth == n) {
+    wg_trace(net, mem, A, &trace_len, phase == POSITIVE ? 1 : 0, x, a, ok);
+    if (phase == POSITIVE && ok && depth == n) {
       if (A.solution && nsol < (A.sol_cap > 0 ? A.sol_cap : 1))
-        for (int v = threadIdx.x; v < n; v += blockDim.x) {
+        for (int v = tid; v < n; v += nthreads) {
           int sv = -1;
           for (int w = 0; w < W && sv < 0; ++w) {
             const u64 dw = mem.dom[(long long)v * W + w];
@@ -2509,69 +2533,66 @@ __device__ __forceinline__ void wg_mac_run(const DevNet& net, WgMem mem, WgCtl* 
       ++nsol;
       if (A.max_solutions <= 1 || nsol >= A.max_solutions) {
         status = MAC_SAT;
-        __syncthreads();
         break;
       }
       ok = false;  // enumeration: go on as after a failed node
       __syncthreads();
     }
-    while (!ok && depth > 0) {
-      --depth;
-      const int2 d = A.stack[depth];
-      const int dx = uniform_int(d.x), dv = uniform_int(d.y);
-      wg_copy_words(mem.dom, A.trail + depth * nw, nw);
-      __syncthreads();
-      wg_recount(mem, n, W);
-      __syncthreads();
-      if (threadIdx.x == 0) {
-        mem.asg[dx >> 5] &= ~(1u << (dx & 31));
-        mem.dom[(long long)dx * W + (dv >> 6)] &= ~(1ull << (dv & 63));
-        mem.size[dx] -= 1;
+    if (ok) continue;
+    // undo decisions until a refutation leaves its variable a value
+    select = false;
+    phase = NEGATIVE;
+    while (true) {
+      if (depth == 0) {
+        status = MAC_UNSAT;
+        break;
       }
+      --depth;
+      const int2 d = stk[depth];
+      x = uniform_int(d.x);
+      a = uniform_int(d.y);
+      const u64* level = A.trail + depth * nw;
+      wg_load_level(mem, level, n, W, x, a);
+      if (tid == 0) mem.asg[x >> 5] &= ~(1u << (x & 31));
       ++nneg;
       ++nodes_here;
-      wg_clear_bitmap(mem.cur, nvw);
-      __syncthreads();
-      if (uniform_int(mem.size[dx]) == 0) {
-        ok = false;
-      } else {
-        if (threadIdx.x == 0) mem.cur[dx >> 5] |= 1u << (dx & 31);
-        __syncthreads();
-        ok = A.weight ? wg_ac3(net, mem, ctl, A, dx) : wg_fixpoint<4>(net, mem, ctl, false);
+      u64 rest = 0ull;
+      for (int w = 0; w < W; ++w) {
+        const u64 dw = level[(long long)x * W + w];
+        rest |= w == (a >> 6) ? dw & ~(1ull << (a & 63)) : dw;
       }
-      wg_trace(net, mem, ctl, A, 0, dx, dv, ok);
+      if ((u64)uniform_ll((long long)rest) != 0ull) break;
+      wg_trace(net, mem, A, &trace_len, 0, x, a, false);
     }
-    if (!ok) {
-      status = MAC_UNSAT;
-      __syncthreads();
-      break;
-    }
+    if (status != MAC_RUNNING) break;
+    wg_seed(mem, ctl, n, slot, x);
+    __syncthreads();
   }
   __syncthreads();
-  if (threadIdx.x == 0) {
+  if (tid == 0) {
     A.state->status = status;
     A.state->depth = depth;
     A.state->npos = npos;
     A.state->nneg = nneg;
     A.state->nsol = nsol;
     A.state->revisions += (long long)ctl->revs;
-    A.state->trace_len = ctl->trace_len;
+    A.state->trace_len = trace_len;
     A.state->steps += 1;
   }
 }
 
 // lnet.bytes > 0 (kLds only): the network image is copied into LDS behind
 // the working memory and the search reads the network from there.
-template <bool kLds>
+template <bool kLds, bool kWdeg>
 __global__ void k_mac(DevNet net, MacArgs args, char* scratch, LdsNet lnet) {
   extern __shared__ __align__(16) char smem[];
   __shared__ WgCtl ctl;
   if (kLds && lnet.bytes > 0) {
     const DevNet ln = wg_load_net(net, lnet, smem + wg_mem_bytes(net.n, net.W));
-    wg_mac_run(ln, wg_carve(smem, ln), &ctl, args);
+    wg_mac_run<kWdeg>(ln, wg_carve(smem, ln), &ctl, args);
   } else {
     char* base = kLds ? smem : scratch;
-    wg_mac_run(net, wg_carve(base, net), &ctl, args);
+    wg_mac_run<kWdeg>(net, wg_carve(base, net), &ctl, args);
   }
 }
 
@@ -2623,11 +2644,11 @@ __global__ void k_mac_units(const UnitDesc* __restrict__ units, int count, unsig
     const int where = uniform_int(d.use_lds);
     if (where == 2) {
       const DevNet ln = wg_load_net(d.net, d.lnet, smem + wg_mem_bytes(d.net.n, d.net.W));
-      wg_mac_run(ln, wg_carve(smem, ln), &ctl, d.args);
+      wg_mac_run<false>(ln, wg_carve(smem, ln), &ctl, d.args);
     } else if (where == 1) {
-      wg_mac_run(d.net, wg_carve(smem, d.net), &ctl, d.args);
+      wg_mac_run<false>(d.net, wg_carve(smem, d.net), &ctl, d.args);
     } else {
-      wg_mac_run(d.net, wg_carve(scratch + d.scratch_off, d.net), &ctl, d.args);
+      wg_mac_run<false>(d.net, wg_carve(scratch + d.scratch_off, d.net), &ctl, d.args);
     }
     if (threadIdx.x == 0) states_out[u] = *d.args.state;
     if (only >= 0) break;

@@ -1,0 +1,92 @@
+"""The workgroup fixpoint's work split, at its edges (needs an MI355X).
+
+A wave revises 64 / Wp arcs of one changed variable at a time (Wp = words per
+domain rounded up to a power of two), numbers the units of 64 variables at a
+time, and switches from the source's rows to the target's own rows part-way.
+The sizes sit on both sides of each of these limits: 63 to 65 and 130
+variables, degrees below, at and above 64 / Wp, domains of 1 to 16 words with
+full and nearly empty last words, loose and tight relations, tables in between.
+All results are exact: domains, outcomes and node sequences equal the oracle's.
+"""
+import numpy as np
+import pytest
+
+import oracle
+from cpim_amd import GModelAdapter, GModelOptions, workload
+from cpim_amd.model import domains_to_sets, from_tuples
+
+pytestmark = pytest.mark.gpu
+
+# n, d, e, tightness
+SHAPES = [
+    (2, 1, 1, 0.0), (3, 2, 3, 0.3), (20, 63, 60, 0.86), (63, 64, 300, 0.87), (64, 8, 900, 0.28),
+    (65, 33, 70, 0.80), (66, 16, 2145, 0.12), (130, 20, 5000, 0.15), (40, 65, 400, 0.90), (34, 128, 560, 0.93),
+    (33, 129, 300, 0.95), (20, 200, 190, 0.96), (18, 257, 150, 0.975), (12, 320, 60, 0.98), (9, 600, 30, 0.992),
+    (7, 1024, 20, 0.995),
+]
+
+
+def networks(n, d, e, t, seed):
+    return workload.random_binary(n, d, e, t, workload.instance_seed(31, seed), preremove=0.15 if d > 3 else 0.0)
+
+
+@pytest.mark.parametrize("seed", [0, 1])
+@pytest.mark.parametrize("n,d,e,t", SHAPES)
+def test_block_fixpoint_equals_oracle(gpu, n, d, e, t, seed):
+    desc = networks(n, d, e, t, seed)
+    ok, dom, _ = oracle.Oracle(desc).root_ac()
+    with GModelAdapter.Build(desc) as m:
+        st = m.EnforceGAC_Block()
+        assert st.inconsistent == (not ok)
+        if not ok:
+            return
+        assert (m.ReadDomains(0) == dom).all()
+        # one more value gone from one variable: propagation from its arcs alone
+        v = n // 2
+        vals = domains_to_sets(dom, desc.dom_size)[v]
+        cut = dom.copy()
+        cut[v, vals[0] // 64] &= ~np.uint64(1 << (vals[0] % 64))
+        m.WriteDomains(0, cut)
+        st = m.EnforceGAC_Block(v)
+        ok2, dom2, _ = oracle.Oracle(desc.with_init_dom(cut)).root_ac()
+        assert st.inconsistent == (not ok2)
+        if ok2:
+            assert (m.ReadDomains(0) == dom2).all()
+
+
+@pytest.mark.parametrize("n,d,e,t", SHAPES)
+def test_workgroup_singleton_tests_equal_oracle(gpu, n, d, e, t):
+    desc = networks(n, d, e, t, 2)
+    o = oracle.Oracle(desc)
+    ok, dom, _ = o.root_ac()
+    if not ok:
+        pytest.skip("the root is inconsistent")
+    tests = np.array([(v, a) for v, vals in enumerate(domains_to_sets(dom, desc.dom_size)) for a in vals], np.int32)
+    tests = tests[np.linspace(0, len(tests) - 1, min(len(tests), 200)).astype(int)]
+    want, _ = o.singleton_tests(tests)
+    with GModelAdapter.Build(desc) as m:
+        assert not m.EnforceGAC_Block().inconsistent
+        got, _ = m.SingletonTests(tests, mode="workgroup")
+    assert (got == want).all()
+
+
+@pytest.mark.parametrize("tables", [0, 3])
+@pytest.mark.parametrize("n,d,rho", [(20, 5, 0.5), (64, 10, 0.2), (70, 30, 0.15), (30, 70, 0.3), (25, 140, 0.3)])
+def test_search_equals_oracle(gpu, n, d, rho, tables):
+    e = int(round(rho * n * (n - 1) / 2))
+    base = workload.random_binary(n, d, e, 0.95 * workload.phase_transition_tightness(n, d, rho),
+                                  workload.instance_seed(32, n))
+    scopes, lists = [list(s) for s in base.scopes()], list(base.tuple_lists())
+    rng = np.random.default_rng(n)
+    for k in range(tables):  # tables between the binary constraints
+        at = int(rng.integers(0, len(scopes) + 1))
+        scopes.insert(at, rng.choice(n, 3, replace=False).tolist())
+        lists.insert(at, workload.random_table(1000 * n + k, 3, d, min(600, d ** 3 // 2)))
+    desc = from_tuples(base.dom_size, scopes, lists)
+    want = oracle.Oracle(desc, oracle.AC3 if tables else oracle.AC3BIT).mac(node_limit=300, trace_cap=1000)
+    with GModelAdapter.Build(desc, GModelOptions(skip_non_binary=False)) as m:
+        st, sol, trace = m.Solve(node_limit=300, trace_capacity=1000)
+    assert (st.num_solutions, st.num_positive, st.num_negative) == (want.num_sol, want.num_positive, want.num_negative)
+    assert trace == want.trace
+    if want.num_sol:
+        assert (np.asarray(sol) == want.solution).all()
