@@ -11,7 +11,7 @@
 //   tsup [c][pos][a][tw]        table constraints: bitset over tuple indices of the
 //                               tuples whose pos-th value is a.
 //   adj  [adj_off[v]..adj_off[v+1])  CSR of the constraints of v in constraint order:
-//                               {c, other var (binary) or -1 (table), pos of v,
+//                               {c, other var (binary) or -1 (table), pos of v | v << 4,
 //                                binary: plane pair index p (planes at sup + p*2*W*dpad),
 //                                table: -1}
 #pragma once
@@ -45,7 +45,12 @@ struct DevNet {
   const u64* tsup;
   const int* tabs;  // the table constraints
   int ntabs;
+  int cap;          // largest domain
 };
+
+// Position of the variable in the constraint's scope, and the variable itself.
+__device__ __forceinline__ int adj_pos(const int4& e) { return e.z & 15; }
+__device__ __forceinline__ int adj_var(const int4& e) { return e.z >> 4; }
 
 // ---------------------------------------------------------------------------
 // Wave helpers (wave64)
@@ -418,6 +423,78 @@ __device__ __forceinline__ int revise_binary(const DevNet& net, u64* dom, int* s
 // position has a support.
 // ---------------------------------------------------------------------------
 
+// Small tables: one-word domains of at most 16 values, at most 4 positions and
+// 512 tuples (8 words).  Lane (h, p, w) = (lane / 32, lane / 8 % 4, lane % 8)
+// takes word w of the rows of values 8 h .. 8 h + 7 of position p: eight row
+// words in flight, each read once.  The live rows are ORed in the lane, the
+// halves h and then the positions are combined across the wave (permlane
+// swaps and one row rotation), which leaves valid word w in every lane; the
+// lane then tests its eight row words against it.  ~110 vector instructions
+// and two memory round trips for all positions.
+struct SmallTable {
+  int y;   // variable of position p, -1 for lanes past the arity
+  int tw;
+  const u64* rows;  // word w of the row of value 8 h (lanes past arity or tw: any valid word)
+};
+
+__device__ __forceinline__ bool small_table(const DevNet& net, int arity, int tw) {
+  return net.W == 1 && net.cap <= 16 && arity <= 4 && tw <= 8;
+}
+
+__device__ __forceinline__ SmallTable load_small_table(const DevNet& net, int c) {
+  const int lane = lane_id();
+  const int h = lane >> 5, p = (lane >> 3) & 3, w = lane & 7;
+  const ConMeta* mp = net.con + c;
+  SmallTable t;
+  t.tw = mp->tw;
+  t.y = p < mp->arity ? mp->scope[p] : -1;
+  t.rows = net.tsup + mp->off + (t.y >= 0 && w < t.tw ? (p * net.dpad + 8 * h) * t.tw + w : 0);
+  return t;
+}
+
+typedef unsigned v2u __attribute__((ext_vector_type(2)));
+
+// x combined with the lane 32 (16) away: lanes of both halves (both rows of a
+// pair) get the same two values, a first.
+__device__ __forceinline__ v2u swap32(unsigned x) { return __builtin_amdgcn_permlane32_swap(x, x, false, false); }
+__device__ __forceinline__ v2u swap16(unsigned x) { return __builtin_amdgcn_permlane16_swap(x, x, false, false); }
+
+// The values of each position (of domain dp, in every lane of the position)
+// that some valid tuple carries, among them dead values; in every lane of the
+// position.
+__device__ __forceinline__ unsigned small_table_keep(const SmallTable& t, u64 dp) {
+  const int lane = lane_id();
+  const unsigned xs = (lane & 7) < t.tw ? (unsigned)dp >> ((lane >> 5) * 8) : 0u;
+  u64 r[8];
+#pragma unroll
+  for (int k = 0; k < 8; ++k) r[k] = t.rows[k * t.tw];
+  unsigned lo = 0u, hi = 0u;
+#pragma unroll
+  for (int k = 0; k < 8; ++k) {
+    const unsigned m = (unsigned)__builtin_amdgcn_sbfe((int)xs, k, 1);
+    lo |= (unsigned)r[k] & m;
+    hi |= (unsigned)(r[k] >> 32) & m;
+  }
+  v2u a = swap32(lo), b = swap32(hi);
+  lo = a.x | a.y;
+  hi = b.x | b.y;
+  if (t.y < 0) lo = hi = ~0u;
+  lo &= dpp_u32<0x128>(lo);  // positions 0, 1 and 2, 3: 8 lanes apart
+  hi &= dpp_u32<0x128>(hi);
+  a = swap16(lo);
+  b = swap16(hi);
+  lo = a.x & a.y;
+  hi = b.x & b.y;
+  unsigned keep = 0u;
+#pragma unroll
+  for (int k = 0; k < 8; ++k) keep |= (((unsigned)r[k] & lo) | ((unsigned)(r[k] >> 32) & hi)) ? 1u << k : 0u;
+  keep |= dpp_u32<0xB1>(keep);   // lane ^ 1
+  keep |= dpp_u32<0x4E>(keep);   // lane ^ 2
+  keep |= dpp_u32<0x141>(keep);  // the other four lanes of the eight
+  a = swap32(keep);
+  return a.x | (a.y << 8);
+}
+
 template <typename OnRemoved, bool kCoherent = false>
 __device__ __forceinline__ void revise_table(const DevNet& net, u64* dom, int* size, int c,
                                              int skip_var, const unsigned* asg,
@@ -500,7 +577,19 @@ __device__ __forceinline__ void revise_table(const DevNet& net, u64* dom, int* s
       on_removed(y, removed);
     }
   };
-  if (W == 1 && tw <= 8) {
+  if (small_table(net, arity, tw)) {
+    const SmallTable t = load_small_table(net, c);
+    const u64 dp = t.y >= 0 ? ld_dom<kCoherent>(&dom[t.y]) : 0ull;
+    const unsigned gone_l = (unsigned)dp & ~small_table_keep(t, dp);
+    const u64 lost = __ballot(gone_l != 0u);
+    for (int q = 0; lost && q < arity; ++q) {
+      const unsigned gone = (unsigned)__builtin_amdgcn_readlane((int)gone_l, 8 * q);
+      const int v = __builtin_amdgcn_readlane(t.y, 8 * q);
+      if (gone == 0u || !revised(v)) continue;
+      const u64 dv = readlane64(dp, 8 * q);
+      apply(v, lane == 0 ? dv : 0ull, lane == 0 ? dv & ~(u64)gone : 0ull);
+    }
+  } else if (W == 1 && tw <= 8) {
     // One-word domains, at most 512 tuples: every position at once.  Lane
     // (q, w) = (lane / Tp, lane % Tp) ORs word w of the rows of position q's
     // live values, four loads in flight per step; the AND over positions

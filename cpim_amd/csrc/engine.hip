@@ -266,7 +266,7 @@ ModelImage make_image(const cpim_model_desc* d, bool skip_non_binary, bool own_r
       const int other = m.kind == 0 ? m.scope[1 - i] : -1;
       // binary: index of the constraint's plane pair (sup offset / (2 W dpad))
       const int pair = m.kind == 0 ? (int)(m.off / (2ll * im.W * im.dpad)) : -1;
-      im.adj[pos[v]++] = make_int4(c, other, i, pair);
+      im.adj[pos[v]++] = make_int4(c, other, i | v << 4, pair);
     }
   }
   // neighbour counts (Network::get_neighbor, src/Network.cpp:467-474)
@@ -379,6 +379,7 @@ struct DevModel {
     d.tsup = tsup.as<u64>();
     d.tabs = nbr.as<int>() + n;
     d.ntabs = ntabs;
+    d.cap = max_dom;
     return d;
   }
 };
@@ -425,7 +426,8 @@ LdsLayout lds_layout(const ModelImage& im, bool odd = true) {
   L.o_sup = L.o_con + align16((long long)sizeof(ConMeta) * (long long)im.con.size());
   const long long sup_words = npairs * 2 * W * dc + 64ll * W;
   L.o_tsup = L.o_sup + align16(8 * sup_words);
-  L.o_tabs = L.o_tsup + align16(8 * std::max<long long>(1, tsup_c));
+  // small tables read 16 rows a position, past the last one's end by up to 16 x 8 words
+  L.o_tabs = L.o_tsup + align16(8 * std::max<long long>(1, tsup_c + (tsup_c ? 16 * 8 : 0)));
   L.bytes = L.o_tabs + align16(4 * (long long)im.tabs.size());
   if (odd && L.bytes > kLdsNetMax) return lds_layout(im, false);
   return L;

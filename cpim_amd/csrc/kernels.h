@@ -735,48 +735,61 @@ __device__ __forceinline__ int ld_wg_int(const int* p) {
   return __hip_atomic_load(const_cast<int*>(p), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
 }
 
-// Word w of a revision tgt <- src of the binary constraint whose planes start
-// at off, by one lane: the values of `need` (word w of D(tgt)) without a
-// support in D(src).
+// Values of `need` (word w of D(u)) without a support in D(t), one arc word
+// per lane, with one source t for the whole wave; lanes without an arc pass
+// need = 0.  rows: word w of the rows of t's values over D(u); own: the rows
+// of the values of word w of D(u) over D(t), word j at own + j dpad.
 //
-// A step keeps four row reads in flight.  Source side: the rows of four
-// values of src are ORed, and the values of tgt they cover are settled; a
-// value stays open with the product of four tightnesses, so a few steps
-// settle nearly every supported value, whatever the domains' sizes.  Target
-// side: an open value b is settled by the W words of its own row.  The lane
-// takes source steps first and turns to the target side once at most one
-// target step is left, or after three source steps, if that takes fewer steps
-// than the rest of D(src): a true removal then costs W reads instead of a
-// scan of D(src).
-__device__ __forceinline__ u64 lane_unsupported(const DevNet& net, const u64* dom, long long off, int src,
-                                                int pos_src, int w, u64 need) {
+// Source side: the rows of kStep values of t are ORed at a time, and the
+// values of u they cover are settled; a value stays open with the product of
+// kStep tightnesses, so one or two steps settle nearly every supported value
+// whatever the domains' sizes.  The values of t are wave-uniform: scalar
+// instructions pick them, and a lane spends one address and one load on each.
+// Target side: an open value is settled by the W words of its own row.  The
+// wave turns to it when more than two source steps are left and no lane has
+// more than a few open values, so that a true removal costs W reads instead
+// of a scan of D(t).
+template <int kStep = 4>
+__device__ __forceinline__ u64 wave_unsupported(const DevNet& net, const u64* dt, const u64* rows, const u64* own,
+                                                u64 need) {
   const int W = net.W, dpad = net.dpad;
-  const u64* rows = net.sup + off + (long long)(pos_src * W + w) * dpad;
-  const u64* ds = dom + (long long)src * W;
-  u64 x = ld_wg(&ds[0]);
-  int left = __popcll(x);
-  for (int j = 1; j < W; ++j) left += __popcll(ld_wg(&ds[j]));
-  int j = 0, done = 0;
-  while (need && left > 0) {
-    const int ts = (__popcll(need) * W + 3) >> 2;
-    if (left > 4 * ts && (ts <= 1 || done >= 3)) break;
-    u64 r[4];
+  int left = 0;
+  for (int j = 0; j < W; ++j) left += __popcll((u64)uniform_ll((long long)ld_wg(&dt[j])));
+  const int few = W == 1 ? 4 : 2;
+  bool target = false;
+  for (int j = 0; j < W && !target; ++j) {
+    u64 x = (u64)uniform_ll((long long)ld_wg(&dt[j]));
+    const u64* rj = rows + 64 * j;
+    while (x) {
+      // the next kStep values (the first of them again once the word is
+      // exhausted), picked by scalar instructions outside the lanes' branch
+      int a[kStep];
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      while (x == 0ull && j + 1 < W) x = ld_wg(&ds[++j]);
-      const int a = x ? (int)__builtin_ctzll(x) : 0;
-      r[i] = x ? rows[64 * j + a] : 0ull;
-      x &= x - 1ull;
+      for (int i = 0; i < kStep; ++i) {
+        a[i] = uniform_int(x ? (int)__builtin_ctzll(x) : a[0]);
+        x &= x - 1ull;
+      }
+      if (need) {
+        u64 r[kStep];
+#pragma unroll
+        for (int i = 0; i < kStep; ++i) r[i] = rj[a[i]];
+        u64 o = 0ull;
+#pragma unroll
+        for (int i = 0; i < kStep; ++i) o |= r[i];
+        need &= ~o;
+      }
+      left -= kStep;
+      if (__ballot(need != 0ull) == 0ull) return 0ull;
+      if (left > 2 * kStep && __ballot(__popcll(need) > few) == 0ull) {
+        target = true;
+        break;
+      }
     }
-    need &= ~((r[0] | r[1]) | (r[2] | r[3]));
-    left -= 4;
-    ++done;
   }
-  if (need == 0ull || left <= 0) return need;
-  const u64* own = net.sup + off + (long long)(1 - pos_src) * W * dpad + 64 * w;
+  if (!target) return need;
   u64 gone = 0ull;
   if (W == 1) {
-    const u64 d = ld_wg(&ds[0]);
+    const u64 d = (u64)uniform_ll((long long)ld_wg(&dt[0]));
     while (need) {
       u64 r[4], bit[4];
 #pragma unroll
@@ -799,7 +812,7 @@ __device__ __forceinline__ u64 lane_unsupported(const DevNet& net, const u64* do
       for (int i = 0; i < 4; ++i) r[i] = j0 + i < W ? own[(long long)(j0 + i) * dpad + b] : 0ull;
 #pragma unroll
       for (int i = 0; i < 4; ++i)
-        if (j0 + i < W) ok = ok || (r[i] & ld_wg(&ds[j0 + i])) != 0ull;
+        if (j0 + i < W) ok = ok || (r[i] & ld_wg(&dt[j0 + i])) != 0ull;
     }
     if (!ok) gone |= 1ull << b;
     need &= need - 1ull;
@@ -807,22 +820,15 @@ __device__ __forceinline__ u64 lane_unsupported(const DevNet& net, const u64* do
   return gone;
 }
 
-// Word w of the revision tgt <- src by one lane, applied: the removed values
-// leave D(tgt), tgt joins the next frontier, and the lane that brings its
-// size to 0 records the wipe-out.  Lanes that pass a domain word with no
-// values do nothing.
-__device__ __forceinline__ void lane_revise(const DevNet& net, const WgMem& mem, WgCtl* ctl, unsigned* nxt, int slot,
-                                            int round, long long off, int src, int tgt, int pos_src, int w) {
-  u64* word = mem.dom + (long long)tgt * net.W + w;
-  const u64 du = ld_wg(word);
-  const u64 gone = lane_unsupported(net, mem.dom, off, src, pos_src, w, du);
-  if (gone) {
-    const u64 old = and_wg(word, ~gone);
-    const int r = __popcll(old & gone);
-    if (r) {
-      atomicOr(&nxt[tgt >> 5], 1u << (tgt & 31));
-      if (atomicSub(&mem.size[tgt], r) == r) atomicMin(&ctl->wipe_round[slot], round);
-    }
+// Takes `gone` out of a domain word of variable u: u joins the next frontier,
+// and the lane that brings its size to 0 records the wipe-out.
+__device__ __forceinline__ void lane_remove(const WgMem& mem, WgCtl* ctl, unsigned* nxt, int slot, int round, int u,
+                                            u64* word, u64 gone) {
+  const u64 old = and_wg(word, ~gone);
+  const int r = __popcll(old & gone);
+  if (r) {
+    atomicOr(&nxt[u >> 5], 1u << (u & 31));
+    if (atomicSub(&mem.size[u], r) == r) atomicMin(&ctl->wipe_round[slot], round);
   }
 }
 
@@ -841,6 +847,58 @@ __device__ __forceinline__ void wg_seed(const WgMem& mem, WgCtl* ctl, int n, int
     mem.bm[i] = v;
   }
   if (threadIdx.x == 0) ctl->wipe_round[slot] = INT_MAX;
+}
+
+// One round over every arc in adjacency order, a lane per arc, for networks
+// whose image is in LDS and whose domains hold at most 32 values (one 32-bit
+// word).  Lane i of the workgroup keeps its first arc's entry (e0) in
+// registers over the whole fixpoint; the row words of the source's values are
+// read in order, eight at a time, and masked by its domain.  A round is a
+// chain of four LDS round trips (frontier bit and domains, rows, removal)
+// however many variables changed, which is what bounds small networks; up to
+// kFlatArcsPerThread arcs per lane, beyond which reading every entry costs
+// more than numbering the changed variables' arcs.
+constexpr int kFlatArcsPerThread = 4;
+
+__device__ __forceinline__ void wg_round_flat(const DevNet& net, const WgMem& mem, WgCtl* ctl, const unsigned* cur,
+                                              unsigned* nxt, int slot, int round, int narcs, const int4& e0,
+                                              int& revs) {
+  const int tid = threadIdx.x, nthreads = blockDim.x;
+  const int i1 = narcs - (tid & 63);  // the wave's last pass covers it
+  for (int i0 = uniform_int(tid & ~63); i0 < narcs; i0 += nthreads) {
+    int4 e = e0;
+    if (i0 >= nthreads) e = i0 < i1 ? mem.adj[i0 + (tid & 63)] : make_int4(0, -1, 0, 0);
+    const int t = adj_var(e), u = e.y;
+    const int uu = u >= 0 ? u : 0;
+    const unsigned bt = cur[t >> 5], au = mem.asg[uu >> 5];
+    const unsigned dt = (unsigned)ld_wg(&mem.dom[t]), du = (unsigned)ld_wg(&mem.dom[uu]);
+    const bool act = u >= 0 && ((bt >> (t & 31)) & 1u) && !((au >> (uu & 31)) & 1u);
+    const u64 active = __ballot(act);
+    if (active == 0ull) continue;
+    const unsigned x = act ? dt : 0u;
+    unsigned need = act ? du : 0u;
+    // lanes without an arc read plane 0
+    const u64* rows = net.sup + (act ? (2 * e.w + adj_pos(e)) * net.dpad : 0);
+    for (int a0 = 0; a0 < net.cap; a0 += 8) {
+      const unsigned xs = x >> a0;
+      if (__ballot((xs & 0xffu) != 0u) == 0ull) continue;
+      unsigned o = 0u;
+#pragma unroll
+      for (int k = 0; k < 8; ++k) o |= (unsigned)rows[a0 + k] & (unsigned)__builtin_amdgcn_sbfe((int)xs, k, 1);
+      need &= ~o;
+      if (__ballot(need != 0u && (xs >> 8) != 0u) == 0ull) break;
+    }
+    if (need) {
+      const unsigned old = (unsigned)and_wg(&mem.dom[u], ~(u64)need);
+      const unsigned lost = old & need;
+      if (lost) {
+        atomicOr(&nxt[u >> 5], 1u << (u & 31));
+        atomicSub(&mem.size[u], __popc(lost));
+        if (lost == old) atomicMin(&ctl->wipe_round[slot], round);
+      }
+    }
+    revs += __popcll(active);
+  }
 }
 
 // AC fixpoint from the seed that wg_seed put in mem.bm (a __syncthreads()
@@ -867,8 +925,11 @@ __device__ __forceinline__ void wg_seed(const WgMem& mem, WgCtl* ctl, int n, int
 // and clears (r + 2) % 3, which no wave reads until the barrier of the next
 // round.  A wipe-out is recorded as the round it happened in, so that a wave
 // that still decides round r is not misled by one already in round r + 1.
+// kImage: the network is in LDS (wg_load_net), where small domains take
+// wg_round_flat instead of numbered units.
 // slot: two wipe-out words used in turn by successive fixpoints, so that
 // wg_seed never resets the word a slow wave still reads.
+template <bool kImage>
 __device__ __forceinline__ bool wg_fixpoint(const DevNet& net, const WgMem& mem, WgCtl* ctl, int slot,
                                             bool both_dirs_round0) {
   const int n = net.n, W = net.W;
@@ -881,57 +942,112 @@ __device__ __forceinline__ bool wg_fixpoint(const DevNet& net, const WgMem& mem,
   while ((1 << lw) < W) ++lw;
   const int w = lane & ((1 << lw) - 1), la = lane >> lw, per = 64 >> lw;
   const long long pair_words = 2ll * W * net.dpad;
+  bool flat = false;
+  int narcs = 0;
+  int4 e0 = make_int4(0, -1, 0, 0);
+  if constexpr (kImage) {
+    narcs = uniform_int(mem.aoff[n]);
+    flat = W == 1 && net.cap <= 32 && narcs <= kFlatArcsPerThread * nthreads;
+    if (flat && tid < narcs) e0 = mem.adj[tid];
+  }
   int revs = 0;
   bool result = true;
   int c0 = 0, c1 = nvw, c2 = 2 * nvw;
+  // this wave's first table, its lanes' part kept over the rounds
+  const int itab = nwaves - 1 - wave;
+  SmallTable tab0{};
+  if (itab < net.ntabs) tab0 = load_small_table(net, uniform_int(net.tabs[itab]));
   for (int round = 0;; ++round) {
     const unsigned* cur = mem.bm + c0;
     unsigned* nxt = mem.bm + c1;
     for (int i = tid; i < nvw; i += nthreads) mem.bm[c2 + i] = 0u;
     const bool both = both_dirs_round0 && round == 0;
+    if (flat) wg_round_flat(net, mem, ctl, cur, nxt, slot, round, narcs, e0, revs);
     int mine = wave;  // this wave's next unit, counted from the block of variables below
-    bool stop = false;
+    bool stop = flat;
     for (int v0 = 0; v0 < n && !stop; v0 += 64) {
       const int v = v0 + lane;
-      const bool f = v < n && bit_of(cur, v);
       int a0 = 0, deg = 0;
-      if (f) {
+      if (v < n) {
         a0 = mem.aoff[v];
-        deg = mem.aoff[v + 1] - a0;
+        deg = bit_of(cur, v) ? mem.aoff[v + 1] - a0 : 0;
       }
       const int units = (deg + per - 1) >> (6 - lw);
       int total = 0;
       const int inc = wave_scan_dpp(units, &total);
-      for (; mine < total; mine += nwaves) {
-        if (uniform_int(ld_wg_int(&ctl->wipe_round[slot])) <= round) {
+      for (;; mine += nwaves) {
+        const int q = uniform_int(mine);
+        if (q >= total) break;
+        const int wr = ld_wg_int(&ctl->wipe_round[slot]);
+        const int l = (int)__builtin_ctzll(__ballot(inc > q));
+        const int t = v0 + l;
+        const int k0 = (q - __builtin_amdgcn_readlane(inc - units, l)) << (6 - lw);
+        const int cnt = min(per, __builtin_amdgcn_readlane(deg, l) - k0);
+        const int arc = __builtin_amdgcn_readlane(a0, l) + k0 + la;
+        const u64* dt = mem.dom + (long long)t * W;
+        int u = -1;
+        u64 need = 0ull;
+        u64* word = nullptr;
+        const u64* pair = net.sup;
+        int pos_t = 0;
+        if (la < cnt && w < W) {
+          const int4 e = mem.adj[arc];
+          u = e.y;
+          pos_t = adj_pos(e);
+          pair += e.w * pair_words;
+          if (u >= 0) {  // binary
+            word = mem.dom + (long long)u * W + w;
+            if (!bit_of(mem.asg, u)) need = ld_wg(word);
+          }
+        }
+        if (uniform_int(wr) <= round) {
           stop = true;
           break;
         }
-        const int l = (int)__builtin_ctzll(__ballot(inc > mine));
-        const int t = v0 + l;
-        const int k = ((mine - __builtin_amdgcn_readlane(inc - units, l)) << (6 - lw)) + la;
-        const int arc = __builtin_amdgcn_readlane(a0, l) + k;
-        const int dt = __builtin_amdgcn_readlane(deg, l);
-        if (k < dt && w < W) {
-          const int4 e = mem.adj[arc];
-          const int u = e.y;
-          if (u >= 0) {  // binary
-            const long long off = e.w * pair_words;
-            if (!bit_of(mem.asg, u)) lane_revise(net, mem, ctl, nxt, slot, round, off, t, u, e.z, w);
-            if (both && !bit_of(mem.asg, t)) lane_revise(net, mem, ctl, nxt, slot, round, off, u, t, 1 - e.z, w);
+        const u64 gone = wave_unsupported(net, dt, pair + (long long)(pos_t * W + w) * net.dpad,
+                                          pair + (long long)(1 - pos_t) * W * net.dpad + 64 * w, need);
+        if (gone) lane_remove(mem, ctl, nxt, slot, round, u, word, gone);
+        revs += cnt;
+        if (both && !bit_of(mem.asg, t)) {
+          // t <- u for the same arcs, one after the other (first round only):
+          // source u, target t, whose words the lanes 0..W-1 hold
+          for (int i = 0; i < cnt; ++i) {
+            const int ui = uniform_int(mem.adj[arc - la + i].y);
+            if (ui < 0) continue;
+            const int pi = 1 - uniform_int(adj_pos(mem.adj[arc - la + i]));
+            const u64* pp = net.sup + uniform_int(mem.adj[arc - la + i].w) * pair_words;
+            u64* tw = mem.dom + (long long)t * W + lane;
+            const u64 g = wave_unsupported(net, mem.dom + (long long)ui * W,
+                                           pp + (long long)(pi * W + (lane < W ? lane : 0)) * net.dpad,
+                                           pp + (long long)(1 - pi) * W * net.dpad + 64 * (lane < W ? lane : 0),
+                                           lane < W ? ld_wg(tw) : 0ull);
+            if (g) lane_remove(mem, ctl, nxt, slot, round, t, tw, g);
           }
+          revs += cnt;
         }
-        revs += min(per, dt - (k - la));
       }
       mine -= total;
     }
-    for (int i = nwaves - 1 - wave; i < net.ntabs; i += nwaves) {
+    for (int i = itab; i < net.ntabs; i += nwaves) {
       const int c = uniform_int(net.tabs[i]);
-      const ConMeta* mp = net.con + c;
-      const int y = lane < mp->arity ? mp->scope[lane] : -1;
-      const u64 changed = __ballot(y >= 0 && bit_of(cur, y));
+      if (i != itab) tab0 = load_small_table(net, c);
+      const bool small = uniform_int(small_table(net, net.con[c].arity, tab0.tw)) != 0;
+      int y = tab0.y;
+      if (!small) y = lane < net.con[c].arity ? net.con[c].scope[lane] : -1;
+      const int yy = y >= 0 ? y : 0;
+      const bool mine_changed = y >= 0 && bit_of(cur, yy);
+      const bool assigned = bit_of(mem.asg, yy);
+      const u64 dp = small ? ld_wg(&mem.dom[yy]) : 0ull;
+      const u64 changed = __ballot(mine_changed);
       if (changed == 0ull) continue;
-      if (uniform_int(ld_wg_int(&ctl->wipe_round[slot])) <= round) break;
+      ++revs;
+      if (small) {
+        // lane 8 p removes for position p
+        const unsigned gone = (unsigned)dp & ~small_table_keep(tab0, dp);
+        if (gone && y >= 0 && !assigned && lane < 32 && (lane & 7) == 0)
+          lane_remove(mem, ctl, nxt, slot, round, y, &mem.dom[y], (u64)gone);
+        continue;
+      }
       // one changed variable: its own values keep their supports
       int skip = -1;
       if (!both && (changed & (changed - 1ull)) == 0ull) skip = __builtin_amdgcn_readlane(y, (int)__builtin_ctzll(changed));
@@ -941,17 +1057,17 @@ __device__ __forceinline__ bool wg_fixpoint(const DevNet& net, const WgMem& mem,
                      if (lane == 0) atomicOr(&nxt[v >> 5], 1u << (v & 31));
                    },
                    &wiped);
-      ++revs;
       if (wiped && lane == 0) atomicMin(&ctl->wipe_round[slot], round);
     }
     __syncthreads();
-    if (uniform_int(ld_wg_int(&ctl->wipe_round[slot])) <= round) {
+    const int wr = ld_wg_int(&ctl->wipe_round[slot]);
+    unsigned any = 0u;
+    for (int i = lane; i < nvw; i += 64) any |= nxt[i];
+    if (uniform_int(wr) <= round) {
       result = false;
       break;
     }
-    bool any = false;
-    for (int i = 0; i < nvw; i += 64) any = any || __ballot(i + lane < nvw && nxt[i + lane] != 0u) != 0ull;
-    if (!any) break;
+    if (__ballot(any != 0u) == 0ull) break;
     const int c = c0;
     c0 = c1;
     c1 = c2;
@@ -1019,7 +1135,7 @@ __global__ void k_block_gac(DevNet net, u64* dom, int* size, int seed_var, char*
   __syncthreads();
   long long before = 0;
   for (int v = threadIdx.x; v < n; v += blockDim.x) before += mem.size[v];
-  const bool ok = wg_fixpoint(net, mem, &ctl, 0, seed_var >= 0);
+  const bool ok = wg_fixpoint<false>(net, mem, &ctl, 0, seed_var >= 0);
   long long after = 0;
   for (int v = threadIdx.x; v < n; v += blockDim.x) after += mem.size[v];
   const u64 delta = wg_reduce_sum_u64(&ctl, (u64)(before - after));
@@ -1067,7 +1183,7 @@ __global__ void k_singleton_tests(DevNet net, const u64* __restrict__ base_dom,
     mem.asg[x >> 5] |= 1u << (x & 31);
   }
   __syncthreads();
-  const bool ok = wg_fixpoint(net, mem, &ctl, 0, false);
+  const bool ok = wg_fixpoint<false>(net, mem, &ctl, 0, false);
   __syncthreads();  // every wave's revision count
   if (threadIdx.x == 0) {
     fail[unit] = ok ? 0 : 1;
@@ -1356,7 +1472,7 @@ __global__ void k_sliced_tests(DevNet net, const u64* __restrict__ base_dom,
       if (lane < cnt) e = net.adj[s0 + lane];
       for (int i = 0; i < cnt; ++i) {
         const int u = __builtin_amdgcn_readlane(e.y, i);
-        const int pos_t = __builtin_amdgcn_readlane(e.z, i);
+        const int pos_t = __builtin_amdgcn_readlane(adj_pos(e), i);
         const long long o = (long long)__builtin_amdgcn_readlane(e.w, i) * 2 * W * dpad;
         const u64* plane_u = net.sup + o + (long long)(1 - pos_t) * W * dpad;
         const bool tu = uniform_int((int)bit_of(touched, u));
@@ -2042,7 +2158,7 @@ __global__ void __launch_bounds__(kWideMaxThreads, kWideWavesPerSimd) k_sliced_w
         if (j >= deg) break;
         const int4 e = net.adj[a0 + j];
         const int u = uniform_int(e.y);
-        const int pos_t = uniform_int(e.z);
+        const int pos_t = uniform_int(adj_pos(e));
         const long long o = (long long)uniform_int(e.w) * 2 * W * dpad;
         const u64* plane_u = net.sup + o + (long long)(1 - pos_t) * W * dpad;
         const bool tu = uniform_int((int)bit_of(touched, u));
@@ -2412,7 +2528,7 @@ __device__ __forceinline__ void wg_load_level(const WgMem& mem, const u64* level
 // what the fixpoint propagates (the root, a decision x = a, a refutation
 // x != a).  A decision costs two barriers and a refutation one, beside the
 // fixpoint's own.  kWdeg: dom/wdeg ordering, fixpoints in AC3's order.
-template <bool kWdeg>
+template <bool kWdeg, bool kImage>
 __device__ __forceinline__ void wg_mac_run(const DevNet& net, const WgMem& mem, WgCtl* ctl, const MacArgs& A) {
   enum { ROOT, POSITIVE, NEGATIVE };
   const int n = net.n, W = net.W;
@@ -2510,7 +2626,7 @@ __device__ __forceinline__ void wg_mac_run(const DevNet& net, const WgMem& mem, 
       phase = POSITIVE;
       __syncthreads();
     }
-    bool ok = kWdeg ? wg_ac3(net, mem, ctl, A, phase == ROOT ? -1 : x) : wg_fixpoint(net, mem, ctl, slot, false);
+    bool ok = kWdeg ? wg_ac3(net, mem, ctl, A, phase == ROOT ? -1 : x) : wg_fixpoint<kImage>(net, mem, ctl, slot, false);
     slot ^= 1;
     select = true;
     if (phase == ROOT) {
@@ -2589,10 +2705,10 @@ __global__ void k_mac(DevNet net, MacArgs args, char* scratch, LdsNet lnet) {
   __shared__ WgCtl ctl;
   if (kLds && lnet.bytes > 0) {
     const DevNet ln = wg_load_net(net, lnet, smem + wg_mem_bytes(net.n, net.W));
-    wg_mac_run<kWdeg>(ln, wg_carve(smem, ln), &ctl, args);
+    wg_mac_run<kWdeg, true>(ln, wg_carve(smem, ln), &ctl, args);
   } else {
     char* base = kLds ? smem : scratch;
-    wg_mac_run<kWdeg>(net, wg_carve(base, net), &ctl, args);
+    wg_mac_run<kWdeg, false>(net, wg_carve(base, net), &ctl, args);
   }
 }
 
@@ -2644,11 +2760,11 @@ __global__ void k_mac_units(const UnitDesc* __restrict__ units, int count, unsig
     const int where = uniform_int(d.use_lds);
     if (where == 2) {
       const DevNet ln = wg_load_net(d.net, d.lnet, smem + wg_mem_bytes(d.net.n, d.net.W));
-      wg_mac_run<false>(ln, wg_carve(smem, ln), &ctl, d.args);
+      wg_mac_run<false, true>(ln, wg_carve(smem, ln), &ctl, d.args);
     } else if (where == 1) {
-      wg_mac_run<false>(d.net, wg_carve(smem, d.net), &ctl, d.args);
+      wg_mac_run<false, false>(d.net, wg_carve(smem, d.net), &ctl, d.args);
     } else {
-      wg_mac_run<false>(d.net, wg_carve(scratch + d.scratch_off, d.net), &ctl, d.args);
+      wg_mac_run<false, false>(d.net, wg_carve(scratch + d.scratch_off, d.net), &ctl, d.args);
     }
     if (threadIdx.x == 0) states_out[u] = *d.args.state;
     if (only >= 0) break;

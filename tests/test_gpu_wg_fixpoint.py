@@ -90,3 +90,52 @@ def test_search_equals_oracle(gpu, n, d, rho, tables):
     assert trace == want.trace
     if want.num_sol:
         assert (np.asarray(sol) == want.solution).all()
+
+
+@pytest.mark.parametrize("n,d,e,t", [
+    # 1 to 4 arcs a lane at 1024 threads, and past it (4096 arcs); 31 to 33 values
+    (80, 2, 500, 0.01), (80, 2, 1030, 0.005), (80, 2, 2047, 0.003), (80, 2, 2049, 0.003),
+    (23, 31, 200, 0.30), (23, 32, 200, 0.31), (23, 33, 200, 0.31), (12, 8, 40, 0.45), (3, 1, 3, 0.0),
+])
+def test_lds_search_equals_oracle(gpu, n, d, e, t):
+    desc = workload.random_binary(n, d, e, t, workload.instance_seed(33, n * 100 + d))
+    want = oracle.Oracle(desc).mac(node_limit=400, trace_cap=1000)
+    with GModelAdapter.Build(desc) as m:
+        st, _, trace = m.Solve(node_limit=400, trace_capacity=1000)
+    assert (st.num_solutions, st.num_positive, st.num_negative) == (want.num_sol, want.num_positive, want.num_negative)
+    assert trace == want.trace
+
+
+@pytest.mark.parametrize("d,arity,tuples", [
+    (16, 3, 512), (16, 3, 513), (17, 3, 512), (16, 4, 500), (16, 5, 300), (15, 3, 449), (8, 4, 448), (9, 2, 40),
+    (4, 3, 1), (2, 4, 5), (5, 3, 64), (5, 3, 65), (1, 3, 1),
+])
+def test_small_tables_equal_oracle(gpu, d, arity, tuples):
+    # the one-pass revision of small tables and the forms beyond its limits
+    # (16 values, 4 positions, 512 tuples), in every engine that revises tables
+    n = 12
+    rng = np.random.default_rng(1000 * d + tuples)
+    scopes = [rng.choice(n, max(2, arity - (k & 1)), replace=False).tolist() for k in range(7)]
+    lists = [workload.random_table(77 * d + k, len(s), d, min(tuples, max(1, d ** len(s) * 3 // 4)))
+             for k, s in enumerate(scopes)]
+    base = workload.random_binary(n, d, 12, 0.15 if d > 2 else 0.0, workload.instance_seed(34, d))
+    desc = from_tuples(base.dom_size, [list(s) for s in base.scopes()] + scopes, list(base.tuple_lists()) + lists)
+    o = oracle.Oracle(desc, oracle.AC3)
+    ok, dom, _ = o.root_ac()
+    want = oracle.Oracle(desc, oracle.AC3).mac(node_limit=200, trace_cap=600)
+    opts = GModelOptions(skip_non_binary=False)
+    for run in ("EnforceGAC_Block", "EnforceGAC", "EnforceGAC_Persistent"):
+        with GModelAdapter.Build(desc, opts) as m:
+            st = getattr(m, run)(False) if run != "EnforceGAC_Block" else m.EnforceGAC_Block()
+            assert st.inconsistent == (not ok), run
+            assert not ok or (m.ReadDomains(0) == dom).all(), run
+    with GModelAdapter.Build(desc, opts) as m:
+        st, _, trace = m.Solve(node_limit=200, trace_capacity=600)
+        assert (st.num_solutions, st.num_positive, st.num_negative) == \
+            (want.num_sol, want.num_positive, want.num_negative)
+        assert trace == want.trace
+    with GModelAdapter.Build(desc, opts) as m:
+        sok, sdom, _ = oracle.Oracle(desc, oracle.AC3).sac1()
+        st = m.EnforceSAC(mode="workgroup")
+        assert st.consistent == sok
+        assert not sok or (m.ReadDomains(0) == sdom).all()
