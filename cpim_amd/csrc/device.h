@@ -46,6 +46,7 @@ struct DevNet {
   const int* tabs;  // the table constraints
   int ntabs;
   int cap;          // largest domain
+  int simple;       // 1: no two binary constraints have the same scope
 };
 
 // Position of the variable in the constraint's scope, and the variable itself.

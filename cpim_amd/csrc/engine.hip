@@ -127,6 +127,7 @@ struct ModelImage {
   std::vector<int4> adj;
   std::vector<int> bin_cons;          // active indices of binary constraints (plane build order)
   std::vector<int> tabs;              // active indices of table constraints
+  bool simple = true;                 // no two binary constraints have the same scope
   std::vector<u64> rel_dense;         // owned dense rows when the desc has none
   const u64* rel = nullptr;           // [nb][max_dom][rel_words]
   int rel_words = 0;
@@ -272,10 +273,15 @@ ModelImage make_image(const cpim_model_desc* d, bool skip_non_binary, bool own_r
   // neighbour counts (Network::get_neighbor, src/Network.cpp:467-474)
   im.nbr.assign(im.n, 0);
   {
-    std::vector<int> seen(im.n, -1);
+    std::vector<int> seen(im.n, -1), paired(im.n, -1);
     for (int v = 0; v < im.n; ++v)
       for (int k = im.adj_off[v]; k < im.adj_off[v + 1]; ++k) {
         const auto& m = im.con[im.adj[k].x];
+        if (m.kind == 0) {
+          const int y = im.adj[k].y;
+          if (paired[y] == v) im.simple = false;
+          paired[y] = v;
+        }
         for (int i = 0; i < m.arity; ++i) {
           const int y = m.scope[i];
           if (y != v && seen[y] != v) {
@@ -363,6 +369,7 @@ struct DevModel {
   int n = 0, W = 0, dpad = 0, max_dom = 0, num_active = 0;
   DevAlloc adj_off, adj, con, sup, tsup, cap, nbr;  // nbr: [n], then the table constraints
   int ntabs = 0;
+  bool simple = false;
   DevAlloc lnet_img;  // the network image for LDS (LdsNet), when small enough
   LdsNet lnet{};
   long long bytes = 0;
@@ -380,6 +387,7 @@ struct DevModel {
     d.tabs = nbr.as<int>() + n;
     d.ntabs = ntabs;
     d.cap = max_dom;
+    d.simple = simple ? 1 : 0;
     return d;
   }
 };
@@ -522,6 +530,7 @@ void build_device_model(const ModelImage& im, DevModel& dm, hipStream_t s, Arena
   upload(dm.cap, im.cap, s, dm.bytes, arena);
   upload(dm.nbr, im.nbr, s, dm.bytes, arena);
   dm.ntabs = (int)im.tabs.size();
+  dm.simple = im.simple;
   dm.sup = dev_array(arena, (long long)sizeof(u64) * im.sup_words);
   dm.bytes += sizeof(u64) * im.sup_words;
   const int nb = (int)im.bin_cons.size();

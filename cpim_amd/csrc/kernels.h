@@ -820,6 +820,70 @@ __device__ __forceinline__ u64 wave_unsupported(const DevNet& net, const u64* dt
   return gone;
 }
 
+// wave_unsupported with a source per lane: the values of `need` (word w of
+// D(tgt)) without a support in D(src), for the constraint whose planes start
+// at off.  The lane takes source steps of four rows and turns to the target
+// side (four row reads a step) once at most one such step is left, or after
+// three source steps, if that takes fewer steps than the rest of D(src).
+__device__ __forceinline__ u64 lane_unsupported(const DevNet& net, const u64* dom, long long off, int src,
+                                                int pos_src, int w, u64 need) {
+  const int W = net.W, dpad = net.dpad;
+  const u64* rows = net.sup + off + (long long)(pos_src * W + w) * dpad;
+  const u64* ds = dom + (long long)src * W;
+  u64 x = ld_wg(&ds[0]);
+  int left = __popcll(x);
+  for (int j = 1; j < W; ++j) left += __popcll(ld_wg(&ds[j]));
+  int j = 0, done = 0;
+  while (need && left > 0) {
+    const int ts = (__popcll(need) * W + 3) >> 2;
+    if (left > 4 * ts && (ts <= 1 || done >= 3)) break;
+    u64 r[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      while (x == 0ull && j + 1 < W) x = ld_wg(&ds[++j]);
+      const int a = x ? (int)__builtin_ctzll(x) : 0;
+      r[i] = x ? rows[64 * j + a] : 0ull;
+      x &= x - 1ull;
+    }
+    need &= ~((r[0] | r[1]) | (r[2] | r[3]));
+    left -= 4;
+    ++done;
+  }
+  if (need == 0ull || left <= 0) return need;
+  const u64* own = net.sup + off + (long long)(1 - pos_src) * W * dpad + 64 * w;
+  u64 gone = 0ull;
+  if (W == 1) {
+    const u64 d = ld_wg(&ds[0]);
+    while (need) {
+      u64 r[4], bit[4];
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        bit[i] = need & (0ull - need);
+        r[i] = need ? own[__builtin_ctzll(need)] : ~0ull;
+        need &= need - 1ull;
+      }
+#pragma unroll
+      for (int i = 0; i < 4; ++i) gone |= (r[i] & d) ? 0ull : bit[i];
+    }
+    return gone;
+  }
+  while (need) {
+    const int b = (int)__builtin_ctzll(need);
+    bool ok = false;
+    for (int j0 = 0; j0 < W && !ok; j0 += 4) {
+      u64 r[4];
+#pragma unroll
+      for (int i = 0; i < 4; ++i) r[i] = j0 + i < W ? own[(long long)(j0 + i) * dpad + b] : 0ull;
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+        if (j0 + i < W) ok = ok || (r[i] & ld_wg(&ds[j0 + i])) != 0ull;
+    }
+    if (!ok) gone |= 1ull << b;
+    need &= need - 1ull;
+  }
+  return gone;
+}
+
 // Takes `gone` out of a domain word of variable u: u joins the next frontier,
 // and the lane that brings its size to 0 records the wipe-out.
 __device__ __forceinline__ void lane_remove(const WgMem& mem, WgCtl* ctl, unsigned* nxt, int slot, int round, int u,
@@ -2351,6 +2415,15 @@ __device__ __forceinline__ void wg_trace(const DevNet& net, const WgMem& mem, co
 // Lane 0 does every load and store of the control state and broadcasts what
 // it read, so the same code is correct whether the arrays are in LDS or in
 // global scratch; control values are wave-uniform.
+//
+// Networks without parallel binary constraints (net.simple) revise up to 64
+// of x's constraints at once.  The other variables of those constraints are
+// distinct and D(x) is fixed until a revision takes values of x, so the
+// revisions are independent and are all computed from the state before the
+// first; they are then committed in list order (queue positions and stamps
+// from the lanes' ranks) up to the first that takes values of x, which runs
+// by itself, or the first wipe-out, whose constraint gains the weight.  One
+// after another they cost about 1.5 us each, a chain of dependent reads.
 // seed: one variable, or -1 for all variables in id order.
 // ---------------------------------------------------------------------------
 __device__ __forceinline__ int lane0_load(const int* p) {
@@ -2404,12 +2477,104 @@ __device__ __forceinline__ bool wave_ac3(const DevNet& net, WgMem mem, const Mac
   if (seed >= 0) insert(seed);
   bool ok = true;
   unsigned long long nrev = 0;
+  const int W = net.W;
+  int lw = 0;
+  while ((1 << lw) < W) ++lw;
+  const int w = lane & ((1 << lw) - 1), la = lane >> lw, per = 64 >> lw;
+  const long long pair_words = 2ll * W * net.dpad;
+  // pred in some lane of this lane's arc, as a mask with one bit per arc (bit 0 of its lanes)
+  auto arcs_with = [&](bool pred) -> u64 {
+    u64 m = __ballot(pred);
+    for (int d = (1 << lw) >> 1; d > 0; d >>= 1) m |= m >> d;
+    u64 first = 1ull;
+    for (int d = 1 << lw; d < 64; d <<= 1) first |= first << d;
+    return m & first;
+  };
   while (ok && front != rear) {
     const int x = lane0_load(&q[front]);
     front = front + 1 == qcap ? 0 : front + 1;
     if (lane == 0) inq[x >> 5] &= ~(1u << (x & 31));
-    const int k1 = mem.aoff[x + 1];
-    for (int k = mem.aoff[x]; k < k1; ++k) {
+    const int k1 = uniform_int(mem.aoff[x + 1]);
+    const bool asgx = uniform_int((int)bit_of(mem.asg, x)) != 0;
+    for (int k = uniform_int(mem.aoff[x]); k < k1; ++k) {
+      if (net.simple) {
+        // the constraints k .. k + per - 1 at once, from the state before the
+        // first of them: exact up to the first one that takes values of x
+        // (the later ones then see another D(x)), the first table and the
+        // first wipe-out
+        const bool in = k + la < k1 && la < per && w < W;
+        const int4 e = in ? mem.adj[k + la] : make_int4(0, -1, 0, 0);
+        const bool table = in && e.y < 0;
+        const int y = in && !table ? e.y : x;
+        const int px = adj_pos(e);
+        const long long sc = in ? A.stamp_tab[e.x] : 0ll;
+        const int stc = sc > base ? (int)(sc - base) : 0;
+        const int svx = ld_wg_int(&sv[x]), svy = ld_wg_int(&sv[y]);
+        u64* ydom = mem.dom + (long long)y * W + w;
+        const u64 dy = in && !table ? ld_wg(ydom) : 0ull;
+        const bool act = in && !table && svx > stc;
+        const bool yrev = act && !bit_of(mem.asg, y);
+        const u64* pair = net.sup + (in && !table ? e.w * pair_words : 0ll);
+        const u64 need = yrev ? dy : 0ull;
+        const u64 gone = wave_unsupported(net, mem.dom + (long long)x * W, pair + (long long)(px * W + w) * net.dpad,
+                                          pair + (long long)(1 - px) * W * net.dpad + 64 * w, need);
+        const int bit0 = la << lw;
+        const u64 lose = arcs_with(gone != 0ull);
+        const u64 wipe = lose & ~arcs_with((need & ~gone) != 0ull);
+        const bool mine_lose = (lose >> bit0) & 1ull;
+        // x <- y: when y changed since the constraint's stamp, or lost values
+        // just now; those had no support in D(x), so the old D(y) decides the same
+        const bool xrev = act && !asgx && (svy > stc || (px == 1 && mine_lose && !((wipe >> bit0) & 1ull)));
+        u64 xgone = 0ull;
+        if (xrev)
+          xgone = lane_unsupported(net, mem.dom, (long long)(pair - net.sup), y, 1 - px, w,
+                                   ld_wg(&mem.dom[(long long)x * W + w]));
+        const u64 xlose = arcs_with(xgone != 0ull), tabs = arcs_with(table);
+        const u64 acts = arcs_with(act);
+        // lanes of the arcs that can be committed
+        const u64 halt = xlose | tabs;
+        const int stop = min((int)(halt ? __builtin_ctzll(halt) : 64), (int)(wipe ? __builtin_ctzll(wipe) : 64));
+        const bool wiped = wipe && stop == (int)__builtin_ctzll(wipe) && !((halt >> (stop & 63)) & 1ull);
+        const u64 before = stop >= 64 ? ~0ull : (1ull << stop) - 1ull;
+        const u64 done = acts & before, ins = lose & before;
+        const bool commit = act && ((before >> bit0) & 1ull);
+        if ((commit || (wiped && bit0 == stop)) && gone) {
+          (void)and_wg(ydom, ~gone);
+          atomicSub(&mem.size[y], __popcll(gone));
+        }
+        nrev += __popcll(arcs_with(yrev && (commit || (wiped && bit0 == stop))));
+        nrev += __popcll(arcs_with(xrev && commit));
+        const u64 below = (1ull << bit0) - 1ull;
+        const int t0 = t + __popcll(done & below) + __popcll(ins & below);
+        if (commit && w == 0) {
+          A.stamp_tab[e.x] = base + t0 + (mine_lose ? 2 : 1);
+          if (mine_lose) __hip_atomic_store(&sv[y], t0 + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+        }
+        const bool queued = (ld_wg_int((const int*)&inq[y >> 5]) >> (y & 31)) & 1;
+        const u64 add = arcs_with(commit && mine_lose && !queued);
+        if (commit && mine_lose && !queued && w == 0) {
+          int at = rear + __popcll(add & below);
+          at = at >= qcap ? at - qcap : at;
+          __hip_atomic_store(&q[at], y, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+          atomicOr(&inq[y >> 5], 1u << (y & 31));
+        }
+        rear += __popcll(add);
+        rear = rear >= qcap ? rear - qcap : rear;
+        t += __popcll(done) + __popcll(ins);
+        __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "workgroup");
+        if (wiped) {
+          const int cw = __builtin_amdgcn_readlane(e.x, stop);
+          if (lane == 0) A.weight[cw] += 1.0f;
+          ok = false;
+          break;
+        }
+        k += stop >= 64 ? per : (stop >> lw);
+        if (stop >= 64 || k >= k1) {
+          --k;
+          continue;
+        }
+        // constraint k takes values of x, or is a table: by itself
+      }
       const int c = uniform_int(mem.adj[k].x);
       long long sc = 0;
       if (lane == 0) sc = A.stamp_tab[c];

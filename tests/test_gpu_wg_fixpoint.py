@@ -139,3 +139,42 @@ def test_small_tables_equal_oracle(gpu, d, arity, tuples):
         st = m.EnforceSAC(mode="workgroup")
         assert st.consistent == sok
         assert not sok or (m.ReadDomains(0) == sdom).all()
+
+
+@pytest.mark.parametrize("kind", ["binary", "tables", "parallel"])
+@pytest.mark.parametrize("n,d,rho", [
+    # degrees below and above 64 / Wp constraints, domains of 1 to 5 words
+    (25, 6, 0.5), (90, 8, 0.9), (40, 20, 0.3), (25, 70, 0.5), (40, 100, 0.95), (20, 150, 0.5), (24, 300, 0.95),
+])
+def test_wdeg_search_and_weights_equal_oracle(gpu, n, d, rho, kind):
+    # dom/wdeg: fixpoints in AC3's order, many constraints of a variable at a
+    # time; tables and parallel constraints take them one after another
+    e = int(round(rho * n * (n - 1) / 2))
+    desc = workload.random_binary(n, d, e, 0.97 * workload.phase_transition_tightness(n, d, rho),
+                                  workload.instance_seed(35, n))
+    if kind != "binary":
+        scopes, lists = [list(s) for s in desc.scopes()], list(desc.tuple_lists())
+        rng = np.random.default_rng(n)
+        for k in range(4):
+            at = int(rng.integers(0, len(scopes) + 1))
+            if kind == "tables":
+                scope = rng.choice(n, 3, replace=False).tolist()
+                tup = workload.random_table(500 * n + k, 3, d, min(900, d ** 3 // 2))
+            else:  # a second constraint on an existing pair, half of them the other way round
+                c = int(rng.integers(0, len(scopes)))
+                scope, tup = scopes[c][::-1] if k & 1 else scopes[c], lists[c][:, ::-1] if k & 1 else lists[c]
+                tup = np.ascontiguousarray(tup[rng.random(len(tup)) < 0.9])
+            scopes.insert(at, list(scope))
+            lists.insert(at, tup)
+        desc = from_tuples(desc.dom_size, scopes, lists)
+    algo = oracle.AC3 if kind == "tables" else oracle.AC3BIT
+    with oracle.var_heuristic(2):
+        o = oracle.Oracle(desc, algo)
+        want = o.mac(node_limit=120, trace_cap=600)
+        weights = o.weights().copy()
+    with GModelAdapter.Build(desc, GModelOptions(skip_non_binary=False)) as m:
+        st, _, trace = m.Solve(node_limit=120, trace_capacity=600, heuristic="dom/wdeg")
+        assert trace == want.trace
+        assert (st.num_solutions, st.num_positive, st.num_negative) == \
+            (want.num_sol, want.num_positive, want.num_negative)
+        assert (m.Weights() == weights).all()
