@@ -2692,7 +2692,7 @@ __device__ __forceinline__ void wg_load_level(const WgMem& mem, const u64* level
 // and the decision stack.  One loop with one fixpoint in it: `phase` says
 // what the fixpoint propagates (the root, a decision x = a, a refutation
 // x != a).  A decision costs two barriers and a refutation one, beside the
-// fixpoint's own.  kWdeg: dom/wdeg ordering, fixpoints in AC3's order.
+// fixpoint's own.  kWdeg: dom/wdeg ordering, wipe-outs repeated in AC3's order.
 template <bool kWdeg, bool kImage>
 __device__ __forceinline__ void wg_mac_run(const DevNet& net, const WgMem& mem, WgCtl* ctl, const MacArgs& A) {
   enum { ROOT, POSITIVE, NEGATIVE };
@@ -2791,7 +2791,21 @@ __device__ __forceinline__ void wg_mac_run(const DevNet& net, const WgMem& mem, 
       phase = POSITIVE;
       __syncthreads();
     }
-    bool ok = kWdeg ? wg_ac3(net, mem, ctl, A, phase == ROOT ? -1 : x) : wg_fixpoint<kImage>(net, mem, ctl, slot, false);
+    bool ok = wg_fixpoint<kImage>(net, mem, ctl, slot, false);
+    if (kWdeg && !ok) {
+      // a wipe-out raises the weight of the constraint that AC3's order
+      // empties a domain with first: propagate again, in that order, from the
+      // domains before.  (Without a wipe-out the closure is the same in any
+      // order and no weight changes.)
+      const u64* level = A.trail + (phase == POSITIVE ? depth - 1 : depth) * nw;
+      wg_load_level(mem, level, n, W, phase == NEGATIVE ? x : -1, a);
+      __syncthreads();
+      if (phase == POSITIVE) {
+        if (tid < W) mem.dom[(long long)x * W + tid] = (tid == (a >> 6)) ? (1ull << (a & 63)) : 0ull;
+        if (tid == 0) mem.size[x] = 1;
+      }
+      ok = wg_ac3(net, mem, ctl, A, phase == ROOT ? -1 : x);
+    }
     slot ^= 1;
     select = true;
     if (phase == ROOT) {
