@@ -1696,10 +1696,30 @@ void run_singleton_sliced(cpim_gmodel* m, const int2* tests_host, long long coun
 void run_singleton_plain(cpim_gmodel* m, const int2* tests, long long count, unsigned char* fail_host,
                          cpim_sac_stats* st);
 
-// CPIM_SAC_BATCHED picks the bit-sliced kernel when the network allows it.
+// CPIM_SAC_BATCHED: one workgroup per test for networks with tables and for
+// passes with little work, the bit-sliced kernels otherwise.  The estimate is
+// the arc words of the tests' first two rounds: the deg arcs of the tested
+// variable, then those of its deg neighbours, at most all.  A bit-sliced
+// group walks its changed variables one after another, 5 us and more each,
+// with one group per variable: passes that do not fill the chip wait on that
+// chain, where one workgroup per test has a test's rounds only.  Measured,
+// workgroup against sliced, per pass: n=60 d=37 e=500 (0.6M arc words) 0.03
+// against 0.11 ms, at tightness 0.655 (cascades) 0.18 against 1.79 ms; n=120
+// d=50 e=3570 (21M) 0.24 against 0.68 ms; n=100 d=100 e=1500 (18M) 0.35
+// against 0.36 ms; n=200 d=64 e=4000 (20M) 0.34 against 0.41 ms; n=200 d=128
+// e=3000 (46M) 0.96 against 0.41 ms; n=300 d=200 e=6000 (384M) 8.3 against
+// 1.3 ms.
+constexpr long long kWorkgroupArcWords = 22ll << 20;
+
+bool few_arc_words(const cpim_gmodel* m, long long tests) {
+  const double arcs = (double)m->im.adj.size(), deg = arcs / m->dm.n;
+  return (double)tests * std::min(arcs, deg * (deg + 1.0)) * m->dm.W <= (double)kWorkgroupArcWords;
+}
+
 void run_singleton_device(cpim_gmodel* m, int mode, const int2* tests, long long count, unsigned char* fail_out,
                           cpim_sac_stats* st, SacScratch& S) {
-  if (mode == CPIM_SAC_BATCHED) mode = sliced_eligible(m) ? CPIM_SAC_SLICED : CPIM_SAC_WORKGROUP;
+  if (mode == CPIM_SAC_BATCHED)
+    mode = sliced_eligible(m) && !(fits_lds(m) && few_arc_words(m, count)) ? CPIM_SAC_SLICED : CPIM_SAC_WORKGROUP;
   if (mode == CPIM_SAC_SLICED) {
     if (!sliced_eligible(m))
       fail(CPIM_ERR_UNSUPPORTED, "bit-sliced singleton tests need a binary network whose work lists fit in LDS");

@@ -239,8 +239,8 @@ typedef struct cpim_sac_stats {
 int cpim_tune_set(const char* name, int64_t value);
 int cpim_tune_get(const char* name, int64_t* value);
 
-#define CPIM_SAC_BATCHED 0   /* every singleton test of a pass on the device: SLICED when the network
-                                allows it (binary constraints only), else WORKGROUP */
+#define CPIM_SAC_BATCHED 0   /* every singleton test of a pass on the device: SLICED for large passes
+                                over binary networks, else WORKGROUP */
 #define CPIM_SAC_PLAIN 1     /* one host-driven fixpoint per singleton test */
 #define CPIM_SAC_WORKGROUP 2 /* one workgroup per singleton test, domain copy in LDS */
 #define CPIM_SAC_SLICED 3    /* 64 singleton tests per workgroup, bit-sliced; CPIM_ERR_UNSUPPORTED

@@ -178,3 +178,16 @@ def test_wdeg_search_and_weights_equal_oracle(gpu, n, d, rho, kind):
         assert (st.num_solutions, st.num_positive, st.num_negative) == \
             (want.num_sol, want.num_positive, want.num_negative)
         assert (m.Weights() == weights).all()
+
+
+@pytest.mark.parametrize("n,d,e,t", [(60, 37, 500, 0.62), (100, 100, 1650, 0.55), (100, 100, 1690, 0.55)])
+def test_sac_pass_same_on_both_sides_of_the_kernel_choice(gpu, n, d, e, t):
+    # little work goes to one workgroup per test, more to the bit-sliced
+    # kernels (23,068,672 arc words: e = 1673 at n = d = 100)
+    desc = workload.random_binary(n, d, e, t, workload.instance_seed(36, e), preremove=0.0)
+    with GModelAdapter.Build(desc) as m:
+        assert not m.EnforceGAC_Auto().inconsistent
+        tests = np.array([(v, a) for v, vals in enumerate(domains_to_sets(m.ReadDomains(0), desc.dom_size))
+                          for a in vals], np.int32)
+        got = {mode: m.SingletonTests(tests, mode=mode)[0] for mode in ("auto", "sliced", "workgroup")}
+    assert (got["auto"] == got["sliced"]).all() and (got["auto"] == got["workgroup"]).all()
