@@ -620,14 +620,15 @@ struct cpim_gmodel {
   int assigned_size = 0;
   DevAlloc dom;    // [max_depth][n][W]
   DevAlloc size;   // [max_depth][n]
-  DevAlloc front;  // 3 x nfw
+  DevAlloc front;  // three bitmaps of variables (grid rounds), or one of constraints (asynchronous)
   DevAlloc ctl;    // GacCtl
   GacCtl* ctl_host = nullptr;  // pinned copy of the control block (host rounds)
   DevAlloc block_out;
   DevAlloc async_ctl;
   DevAlloc scratch;  // workgroup-engine scratch when a copy does not fit in LDS
   long long scratch_bytes = 0;
-  int nfw = 0;
+  int nfw = 0;     // words of a bitmap of the constraints
+  int nvw = 0;     // words of a bitmap of the variables
   std::vector<int2> assigned;  // d_assigned mirror: (var, value) per level
   DevProps props;
   SacScratch sac;
@@ -775,12 +776,13 @@ int cpim_gmodel_create(const cpim_model_desc* desc, const cpim_gmodel_options* o
                        m->level_size(0), n, m->dm.W);
     HIPC(hipGetLastError());
     m->nfw = std::max(1, (m->dm.num_active + 31) / 32);
-    m->front = DevAlloc(sizeof(unsigned) * 3ll * m->nfw);
+    m->nvw = (n + 31) / 32;
+    m->front = DevAlloc(sizeof(unsigned) * std::max<long long>(m->nfw, 3ll * m->nvw));
     m->ctl = DevAlloc(sizeof(GacCtl));
     m->block_out = DevAlloc(sizeof(BlockGacOut));
     m->assigned.assign(m->max_depth, make_int2(-1, -1));
     m->dm.bytes += sizeof(u64) * lw * m->max_depth + sizeof(int) * (long long)n * m->max_depth +
-                   sizeof(unsigned) * 3ll * m->nfw + sizeof(GacCtl);
+                   sizeof(unsigned) * std::max<long long>(m->nfw, 3ll * m->nvw) + sizeof(GacCtl);
     m->sync();
     *out = m.release();
   });
@@ -837,65 +839,48 @@ unsigned long long fixpoint_budget_ticks(const cpim_gmodel* m) {
                 : (unsigned long long)(khz * kAsyncBudgetMs);
 }
 
-// Workgroups per CU of the persistent fixpoint (kPersistentThreads each): one
-// workgroup of 16 waves per CU is what the kernel's ~105 VGPRs allow, and it
-// keeps the barrier at one arrival per CU.
-constexpr int kPersistentBlocksPerCu = 1;
-
-// Parts per frontier word of a grid round: the smallest power of two (at
-// most 32) that gives about `per_wave` work units per wave of `waves`.  One
-// word-domain networks revise kPairBatch constraints per wave step, so one
-// unit of several constraints per wave suffices there; otherwise four units
-// of fewer constraints.
-int frontier_parts(int nfw, long long waves, int W) {
-  const long long per_wave = W == 1 ? 1 : 4;
-  int parts = 1;
-  while (parts < 32 && (long long)nfw * parts < per_wave * waves) parts *= 2;
-  return parts;
-}
-
 unsigned long long slot_sum(const unsigned long long (&v)[kStatSlots]) {
   unsigned long long t = 0;
   for (unsigned long long x : v) t += x;
   return t;
 }
 
-// Start of a frontier fixpoint: control block and frontiers cleared, the
-// first frontier seeded with every constraint (assigned_var < 0) or with the
-// constraints of assigned_var.
-void gac_start(cpim_gmodel* m, int assigned_var, unsigned* F, GacCtl* ctl) {
-  const long long words = 3ll * m->nfw;
-  const int blocks = (int)std::max<long long>(1, std::min<long long>((words + 255) / 256, 1024));
-  hipLaunchKernelGGL(k_gac_init, dim3(blocks), dim3(256), 0, m->stream, ctl, F, m->nfw, m->dm.num_active,
-                     assigned_var < 0 ? 1 : 0);
-  if (assigned_var >= 0)
-    hipLaunchKernelGGL(k_seed_var, dim3(1), dim3(256), 0, m->stream, F, m->dm.adj_off.as<int>(),
-                       m->dm.adj.as<int4>(), assigned_var);
+// Start of a grid fixpoint: control block and changed bitmaps cleared.
+void gac_start(cpim_gmodel* m, unsigned* F, GacCtl* ctl) {
+  const int blocks = (int)std::max<long long>(1, std::min<long long>((3ll * m->nvw + 255) / 256, 1024));
+  hipLaunchKernelGGL(k_gac_init, dim3(blocks), dim3(256), 0, m->stream, ctl, F, m->nvw);
   HIPC(hipGetLastError());
 }
 
-// The persistent fixpoint kernel on the current level, after gac_start.
-// Every workgroup must be resident for the grid barrier: at most the
-// occupancy limit per CU (and at most kPersistentBlocksPerCu) on every CU.
-// If some were not resident, the barrier's bounded wait turns that into the
-// time-budget error the caller reports (ctl->err).
-void persistent_launch(cpim_gmodel* m, unsigned* F, GacCtl* ctl) {
+// Lanes of a grid round: one per word of every arc, words rounded up to a
+// power of two.
+long long grid_lanes(const cpim_gmodel* m) {
+  long long wp = 1;
+  while (wp < m->dm.W) wp *= 2;
+  return (long long)m->im.adj.size() * wp;
+}
+
+// Largest round copy of the persistent fixpoint in LDS: one workgroup per CU.
+constexpr long long kPersistentLdsMax = 128 * 1024;
+
+// The persistent fixpoint kernel on the current level, after gac_start: a
+// lane per arc word, at most one 1024-thread workgroup per CU.  Every
+// workgroup must be resident for the grid barrier; if some were not, the
+// barrier's bounded wait turns that into the time-budget error the caller
+// reports (ctl->err).
+void persistent_launch(cpim_gmodel* m, int assigned_var, unsigned* F, GacCtl* ctl) {
   const int L = m->current_level;
-  const int threads = kPersistentThreads;
-  int per_cu = 0;
-  HIPC(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, k_gac_persistent, threads, 0));
-  per_cu = std::max(1, std::min(per_cu, kPersistentBlocksPerCu));
-  const int waves_per_block = threads / 64;
-  const int nfw = m->nfw;
-  const int parts = frontier_parts(nfw, (long long)per_cu * waves_per_block * m->props.cus, m->dm.W);
-  const long long units = (long long)nfw * parts;
-  const int grid = (int)std::max<long long>(
-      1, std::min<long long>((units + waves_per_block - 1) / waves_per_block, (long long)per_cu * m->props.cus));
+  const long long lanes = grid_lanes(m);
+  const long long lds = persistent_lds_bytes(m->dm.n, m->dm.W);
+  const bool staged = lds <= std::min<long long>(kPersistentLdsMax, m->props.max_lds - 1024);
+  const long long want = (std::max(lanes, 64ll * m->dm.ntabs) + kPersistentThreads - 1) / kPersistentThreads;
+  const int grid = (int)std::max<long long>(1, std::min<long long>(want, m->props.cus));
   const long long max_rounds = (long long)m->dm.n * m->dm.max_dom + 2;
   const int mr = (int)std::min<long long>(max_rounds, INT_MAX);
   const unsigned long long max_ticks = fixpoint_budget_ticks(m);
-  hipLaunchKernelGGL(k_gac_persistent, dim3(grid), dim3(threads), 0, m->stream, m->dm.net(), m->level_dom(L),
-                     m->level_size(L), F, nfw, ctl, mr, parts, max_ticks);
+  hipLaunchKernelGGL(staged ? k_gac_persistent<true> : k_gac_persistent<false>, dim3(grid), dim3(kPersistentThreads),
+                     staged ? (size_t)lds : 0, m->stream, m->dm.net(), m->level_dom(L), m->level_size(L), F, m->nvw,
+                     ctl, mr, assigned_var, (int)m->im.adj.size(), max_ticks);
   HIPC(hipGetLastError());
 }
 
@@ -914,16 +899,15 @@ void gac_grid(cpim_gmodel* m, int assigned_var, bool persistent, cpim_gac_stats*
   int* size = m->level_size(L);
   unsigned* F = m->front.as<unsigned>();
   GacCtl* ctl = m->ctl.as<GacCtl>();
-  const int nfw = m->nfw;
   if (!m->ctl_host) HIPC(hipHostMalloc((void**)&m->ctl_host, sizeof(GacCtl), hipHostMallocDefault));
   m->gac_events();
   double kms = 0.0;
   HIPC(hipEventRecord(m->gev[0], m->stream));
-  gac_start(m, assigned_var, F, ctl);
+  gac_start(m, F, ctl);
   int rounds = 0;
   GacCtl res{};
   if (persistent) {
-    persistent_launch(m, F, ctl);
+    persistent_launch(m, assigned_var, F, ctl);
     HIPC(hipEventRecord(m->gev[1], m->stream));
     HIPC(hipMemcpyAsync(m->ctl_host, ctl, sizeof(res), hipMemcpyDeviceToHost, m->stream));
     m->sync();
@@ -932,19 +916,16 @@ void gac_grid(cpim_gmodel* m, int assigned_var, bool persistent, cpim_gac_stats*
     if (res.err) fail(CPIM_ERR_RUNTIME, "persistent fixpoint exceeded its time budget at a grid barrier");
     rounds = res.rounds;
   } else {
-    // about four work units per resident wave (32 per CU)
     DevNet net = m->dm.net();
     const int threads = 256;
     const long long max_rounds = (long long)m->dm.n * m->dm.max_dom + 2;
-    const int parts = frontier_parts(nfw, 32ll * m->props.cus, m->dm.W);
-    const int waves_per_block = threads / 64;
-    const long long units = (long long)nfw * parts;
-    const int grid = (int)std::max<long long>(1, std::min<long long>((units + waves_per_block - 1) / waves_per_block,
-                                                                      8ll * m->props.cus));
+    const long long lanes = grid_lanes(m);
+    const int grid = (int)std::max<long long>(
+        1, std::min<long long>((std::max(lanes, 64ll * m->dm.ntabs) + threads - 1) / threads, 8ll * m->props.cus));
     for (int r = 0; r < max_rounds; ++r) {
       if (r > 0) HIPC(hipEventRecord(m->gev[0], m->stream));
-      hipLaunchKernelGGL(k_gac_round, dim3(grid), dim3(threads), 0, m->stream, net, dom, size, F, nfw,
-                         ctl, r, parts);
+      hipLaunchKernelGGL(k_gac_round, dim3(grid), dim3(threads), 0, m->stream, net, dom, size, F, m->nvw,
+                         ctl, r, assigned_var, (int)m->im.adj.size());
       HIPC(hipGetLastError());
       HIPC(hipEventRecord(m->gev[1], m->stream));
       HIPC(hipMemcpyAsync(m->ctl_host, ctl, sizeof(res), hipMemcpyDeviceToHost, m->stream));

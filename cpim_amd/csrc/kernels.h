@@ -51,12 +51,159 @@ __global__ void k_build_planes(const u64* __restrict__ rel, int nb, int max_dom,
   }
 }
 
+// Domain word seen by a lane: agent scope (other XCDs' completed updates), or
+// workgroup scope (LDS, or global memory that nobody writes meanwhile or whose
+// stale words only keep too much).
+template <bool kCoherent>
+__device__ __forceinline__ u64 ld_view(const u64* p) {
+  if constexpr (kCoherent) return __hip_atomic_load(const_cast<u64*>(p), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  else return ld_wg(p);
+}
+
+// Open values of some lanes, settled by the whole wave: for each lane with
+// todo, the 64 lanes take the values of its word one each and read the words
+// of their rows (own: index in sup of the row words of the word's first value)
+// against D(src), one word after the other while some value is open: the
+// first word of a row is a coalesced 512-byte read and settles most values.
+// kSettle arc words at a time.  Returns, in the lanes with todo, the values of
+// `need` without a support; `need` unchanged in the others.
+constexpr int kSettle = 8;
+
+template <bool kCoherent>
+__device__ __forceinline__ u64 wave_settle(const DevNet& net, const u64* dom, long long own, int src, u64 need,
+                                           u64 todo) {
+  const int W = net.W, lane = lane_id();
+  while (todo) {
+    int l[kSettle];
+    u64 open[kSettle];
+#pragma unroll
+    for (int p = 0; p < kSettle; ++p) {
+      l[p] = uniform_int(todo ? (int)__builtin_ctzll(todo) : l[0]);
+      open[p] = todo ? readlane64(need, l[p]) : 0ull;
+      todo &= todo - 1ull;
+    }
+    for (int j = 0; j < W; ++j) {
+      u64 r[kSettle], d[kSettle], any = 0ull;
+#pragma unroll
+      for (int p = 0; p < kSettle; ++p) {
+        const u64* row = net.sup + (long long)readlane64((u64)own, l[p]) + (long long)j * net.dpad;
+        r[p] = (open[p] >> lane) & 1ull ? row[lane] : 0ull;
+        d[p] = ld_view<kCoherent>(&dom[(long long)__builtin_amdgcn_readlane(src, l[p]) * W + j]);
+      }
+#pragma unroll
+      for (int p = 0; p < kSettle; ++p) {
+        open[p] &= ~__ballot((r[p] & d[p]) != 0ull);
+        any |= open[p];
+      }
+      if (any == 0ull) break;
+    }
+#pragma unroll
+    for (int p = kSettle - 1; p >= 0; --p)
+      if (lane == l[p]) need = open[p];
+  }
+  return need;
+}
+
+// The values of `need` (word w of D(tgt)) without a support in D(src), for the
+// constraint whose planes start at off: one arc word per lane, each with its
+// own source; lanes without an arc pass need = 0.  Called by whole waves.
+// Source side: the rows of four values of src at a time are ORed, and the
+// values of tgt they cover are settled; a value stays open with the product of
+// four tightnesses, so a few such steps settle nearly every value of a loose
+// relation.  Target side: an open value is settled by the W words of its own
+// row, by the lane, four reads a step.  Lanes that tight relations leave with
+// more than 12 steps per four words of a domain (never one-word domains) are
+// settled by the wave, one after the other (wave_settle; kTight: the search
+// kernels leave that path out, whose networks are loose enough to be found a
+// solution in, and which lose 10% to its registers).
+template <bool kCoherent, bool kTight>
+__device__ __forceinline__ u64 arcs_unsupported(const DevNet& net, const u64* dom, long long off, int src, int pos_src,
+                                                int w, u64 need) {
+  const int W = net.W, dpad = net.dpad;
+  const long long own = off + (long long)(1 - pos_src) * W * dpad + 64 * w;
+  const u64* ds = dom + (long long)src * W;
+  bool wave = false;
+  if (need) {
+    const u64* rows = net.sup + off + (long long)(pos_src * W + w) * dpad;
+    u64 x = ld_view<kCoherent>(&ds[0]);
+    int left = __popcll(x);
+    for (int j = 1; j < W; ++j) left += __popcll(ld_view<kCoherent>(&ds[j]));
+    int j = 0, done = 0, ts = 0;
+    while (need && left > 0) {
+      ts = (__popcll(need) * W + 3) >> 2;
+      if (left > 4 * ts && (ts <= 1 || done >= 3)) break;
+      if (kTight && done >= 2 && min(left, 4 * ts) > 48 * ((W + 3) >> 2)) {
+        wave = true;
+        break;
+      }
+      u64 r[4];
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        while (x == 0ull && j + 1 < W) x = ld_view<kCoherent>(&ds[++j]);
+        const int a = x ? (int)__builtin_ctzll(x) : 0;
+        r[i] = x ? rows[64 * j + a] : 0ull;
+        x &= x - 1ull;
+      }
+      need &= ~((r[0] | r[1]) | (r[2] | r[3]));
+      left -= 4;
+      ++done;
+    }
+    if (!wave && left > 0) {  // the target side, by the lane
+      const u64* mine = net.sup + own;
+      u64 open = need;
+      if (W == 1) {
+        const u64 d = ld_view<kCoherent>(&ds[0]);
+        while (open) {
+          u64 r[4], bit[4];
+#pragma unroll
+          for (int i = 0; i < 4; ++i) {
+            bit[i] = open & (0ull - open);
+            r[i] = open ? mine[__builtin_ctzll(open)] : 0ull;
+            open &= open - 1ull;
+          }
+#pragma unroll
+          for (int i = 0; i < 4; ++i)
+            if (r[i] & d) need &= ~bit[i];
+        }
+      }
+      while (open) {
+        const int b = (int)__builtin_ctzll(open);
+        bool ok = false;
+        for (int j0 = 0; j0 < W && !ok; j0 += 4) {
+          u64 r[4];
+#pragma unroll
+          for (int i = 0; i < 4; ++i) r[i] = j0 + i < W ? mine[(long long)(j0 + i) * dpad + b] : 0ull;
+#pragma unroll
+          for (int i = 0; i < 4; ++i)
+            if (j0 + i < W) ok = ok || (r[i] & ld_view<kCoherent>(&ds[j0 + i])) != 0ull;
+        }
+        if (ok) need &= ~(1ull << b);
+        open &= open - 1ull;
+      }
+    }
+  }
+  if (!kTight) return need;
+  const u64 todo = __ballot(wave);
+  return todo ? wave_settle<kCoherent>(net, dom, own, src, need, todo) : need;
+}
+
 // ===========================================================================
-// Grid engine: rounds over a bitmap frontier of constraints.
-// Three frontier buffers rotate: in round r, F[r%3] is read, F[(r+1)%3]
-// collects the next frontier, F[(r+2)%3] (read in round r-1) is cleared.
-// Termination uses epochs that only grow (last_push_round, wipe_round), so
-// every block takes the same decision after a barrier without any reset.
+// Grid engine: rounds over a bitmap of the variables that changed.
+// In round r a lane takes one word of one arc u <- t of the adjacency list,
+// if t changed in round r - 1.  Three bitmaps rotate: F[r % 3] is read,
+// F[(r + 1) % 3] collects the round's changes, F[(r + 2) % 3] (read in round
+// r - 1) is cleared.  last_push_round only grows and wipe_round is only
+// lowered to the running round, so every block takes the same decision after
+// a barrier.
+//
+// A round is bound by its chain of dependent reads (changed bit, domains,
+// rows, removal), a full one by the rows' bandwidth.  The earlier rounds kept
+// a frontier of constraints, each revised in both directions by a wave that
+// read 64 rows of either side, and every removal marked all constraints of its
+// variable.  Kernel time, before and after (host-driven rounds): n=2000 d=64
+// e=40000, one round without removals 24.8 -> 12.5 us; its cascade at t=0.886
+// (10 rounds, 6,485 removals) 225 -> 151 us, persistent 269 -> 162 us; n=500
+// d=250 e=20000 t=0.963 (5 rounds) 293 -> 188 us, persistent 346 -> 195 us.
 // ===========================================================================
 // Statistics counters are spread over kStatSlots addresses (by block), and
 // the grid rounds add one workgroup total per round: device-scope atomics on
@@ -65,17 +212,13 @@ __global__ void k_build_planes(const u64* __restrict__ rel, int nb, int max_dom,
 constexpr int kStatSlots = 256;
 
 struct GacCtl {
-  unsigned scanner[3];
-  int last_push_round;  // highest round that enqueued a constraint
+  int last_push_round;  // highest round that changed a domain (host-driven rounds)
   int wipe_round;       // lowest round that emptied a domain
   int rounds;           // rounds executed (written at the end)
   int converged;
-  int pad;
-  // grid barrier of the persistent kernel: arrivals in this generation, the
-  // generation, and the error flag set by a block whose wait ran out of time
   unsigned long long bar_ticket;  // grid barrier arrivals so far (only grows)
-  int err;
-  int pad2;
+  int err;              // set by a block whose barrier wait ran out of time
+  int pad;
   unsigned long long deletions[kStatSlots];
   unsigned long long revisions[kStatSlots];
 };
@@ -84,52 +227,90 @@ __device__ __forceinline__ int ld_agent(const int* p) {
   return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
-__device__ __forceinline__ void push_var(const DevNet& net, int v, unsigned* B, GacCtl* ctl, int r) {
-  const int lane = lane_id();
-  const int b0 = net.adj_off[v], b1 = net.adj_off[v + 1];
-  for (int i = b0 + lane; i < b1; i += 64) {
-    const int c = net.adj[i].x;
-    atomicOr(&B[c >> 5], 1u << (c & 31));
-  }
-  // the epoch only grows: skip the atomic once another wave has raised it
-  if (lane == 0 && ld_agent(&ctl->last_push_round) < r) atomicMax(&ctl->last_push_round, r);
-}
-
-template <bool kCoherent = false>
-__device__ __forceinline__ void grid_process_constraint(const DevNet& net, u64* dom, int* size,
-                                                        int c, unsigned* B, GacCtl* ctl, int r,
-                                                        unsigned long long& revs,
-                                                        unsigned long long& dels) {
-  const ConMeta* mp = net.con + c;
-  bool wiped = false;
-  if (mp->kind == 0) {
-    const int x = mp->scope[0], y = mp->scope[1];
-    int rx = revise_binary<kCoherent>(net, dom, size, c, x, y, 1, &wiped);
-    ++revs;
-    if (wiped) atomicMin(&ctl->wipe_round, r);
-    if (rx) {
-      dels += rx;
-      push_var(net, x, B, ctl, r);
-    }
-    int ry = revise_binary<kCoherent>(net, dom, size, c, y, x, 0, &wiped);
-    ++revs;
-    if (wiped) atomicMin(&ctl->wipe_round, r);
-    if (ry) {
-      dels += ry;
-      push_var(net, y, B, ctl, r);
-    }
+// One word of one arc per lane (lanes with act false do nothing).  view: the
+// domains as the lane reads them (global memory, or the round's copy in LDS);
+// removals go to dom.  W = 1: the word returned by the AND tells the wipe-out,
+// so the size update needs no answer.
+template <bool kCoherent>
+__device__ __forceinline__ void grid_arc(const DevNet& net, const u64* view, u64* dom, int* size, unsigned* nxt,
+                                         GacCtl* ctl, int r, const int4& e, int w, bool act, int& dels) {
+  const int W = net.W, u = e.y;
+  const u64 need = act ? ld_view<kCoherent>(&view[(long long)u * W + w]) : 0ull;
+  const u64 gone = arcs_unsupported<kCoherent, true>(net, view, act ? e.w * (2ll * W * net.dpad) : 0ll, adj_var(e), adj_pos(e),
+                                               act ? w : 0, need);
+  if (gone == 0ull) return;
+  const u64 old = atomicAnd(&dom[(long long)u * W + w], ~gone);
+  const int lost = __popcll(old & gone);
+  if (lost == 0) return;
+  dels += lost;
+  atomicOr(&nxt[u >> 5], 1u << (u & 31));
+  bool wiped;
+  if (W == 1) {
+    wiped = (old & ~gone) == 0ull;
+    (void)__hip_atomic_fetch_add(&size[u], -lost, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
   } else {
-    auto on_removed = [&](int v, int k) {
-      dels += k;
-      push_var(net, v, B, ctl, r);
+    wiped = atomicSub(&size[u], lost) == lost;
+  }
+  if (wiped) atomicMin(&ctl->wipe_round, r);
+}
+
+// The arcs and tables of round r that this grid's waves take.  cur: the
+// variables that changed (round 0: seed < 0 takes every arc and table, else
+// those on variable `seed`, in both directions); e0: the arc of this lane's
+// first turn, kept in registers by the persistent kernel (kept true).  With
+// several words a wave's arcs lie nwaves apart in the list, so that the arcs
+// of one variable (a late round's few changes) fall to as many waves: what
+// they settle together, wave_settle does one after the other.  One-word arcs
+// stay in list order, 64 neighbours to a wave (a 10-round cascade of 80,000
+// arcs 162 us against 187 us spread).
+template <bool kCoherent>
+__device__ __forceinline__ void grid_round(const DevNet& net, const u64* view, u64* dom, int* size,
+                                           const unsigned* cur, unsigned* nxt, GacCtl* ctl, int r, int seed,
+                                           bool kept, const int4& e0, int narcs, int& revs, int& dels) {
+  const int W = net.W, lane = lane_id();
+  int lw = 0;
+  while ((1 << lw) < W) ++lw;
+  const int w = lane & ((1 << lw) - 1);
+  const int nwaves = (int)(((long long)gridDim.x * blockDim.x) >> 6);
+  const int gw = uniform_int((int)(((long long)blockIdx.x * blockDim.x + threadIdx.x) >> 6));
+  auto changed = [&](int v) -> bool {
+    const unsigned* p = &cur[v >> 5];
+    const unsigned word = kCoherent ? (unsigned)ld_agent((const int*)p) : *p;
+    return (word >> (v & 31)) & 1u;
+  };
+  // whole waves: lanes past the end take no arc
+  const int4 none = make_int4(0, -1, 0, 0);
+  const long long per_pass = (long long)nwaves << (6 - lw);
+  for (long long base = 0; base < narcs; base += per_pass) {
+    const long long i = base + (W > 1 ? (long long)(lane >> lw) * nwaves + gw : (long long)gw * 64 + lane);
+    const int4 e = kept && base == 0 ? e0 : (i < narcs ? net.adj[i] : none);
+    const int t = adj_var(e), u = e.y;
+    const bool act = u >= 0 && w < W && (r > 0 ? changed(t) : (seed < 0 || t == seed || u == seed));
+    const u64 m = __ballot(act && w == 0);
+    if (__ballot(act) == 0ull) continue;
+    revs += __popcll(m);
+    grid_arc<kCoherent>(net, view, dom, size, nxt, ctl, r, e, w, act, dels);
+  }
+  // tables, one per wave, the last waves of the grid first
+  for (int k = nwaves - 1 - gw; k < net.ntabs; k += nwaves) {
+    const int c = uniform_int(net.tabs[k]);
+    const ConMeta* mp = net.con + c;
+    const int y = lane < mp->arity ? mp->scope[lane] : -1;
+    if (__ballot(y >= 0 && (r > 0 ? changed(y) : (seed < 0 || y == seed))) == 0ull) continue;
+    bool wiped = false;
+    auto on_removed = [&](int v, int n) {
+      if (lane == 0) {
+        dels += n;
+        atomicOr(&nxt[v >> 5], 1u << (v & 31));
+      }
     };
-    revise_table<decltype(on_removed), kCoherent>(net, dom, size, c, -1, nullptr, on_removed, &wiped);
+    revise_table<decltype(on_removed), true>(net, dom, size, c, -1, nullptr, on_removed, &wiped);
     ++revs;
-    if (wiped) atomicMin(&ctl->wipe_round, r);
+    if (wiped && lane == 0) atomicMin(&ctl->wipe_round, r);
   }
 }
 
-// Binary constraints over one-word domains (W = 1), up to kPairBatch at a
+// Binary constraints over one-word domains (W = 1), up to kAsyncPairBatch at a
 // time, by one wave.  Both arcs of a constraint c = (x, y) are revised from
 // the same D(x) and D(y): value a of x keeps iff row a of plane 0 meets D(y),
 // value b of y keeps iff row b of plane 1 meets D(x).  With W = 1 the rows of
@@ -143,17 +324,15 @@ __device__ __forceinline__ void grid_process_constraint(const DevNet& net, u64* 
 // for a one-word domain the returned word gives the exact removals and the
 // wipe-out (a non-empty word this AND empties), so the size update needs no
 // returned value.
-constexpr int kPairBatch = 4;
-// The asynchronous fixpoint takes eight: its waves are few (two per CU) and
+// Eight at a time: the asynchronous fixpoint's waves are few (two per CU) and
 // bound by the latency of their own loads, so more rows in flight per wave
-// pay (3.6-3.75 ms against 3.85-4.1 ms on the C2 cascade), where the round
-// kernels lose occupancy at eight.
+// pay (3.6-3.75 ms against 3.85-4.1 ms at four on the C2 cascade).
 constexpr int kAsyncPairBatch = 8;
 
 // The revisions of one batch; returns the mask of lanes whose variable (in
 // myv) lost values, the values removed in the batch, and whether some domain
 // was emptied by it.
-template <bool kCoherent, int P = kPairBatch>
+template <bool kCoherent, int P = kAsyncPairBatch>
 __device__ __forceinline__ u64 revise_pairs_w1(const DevNet& net, u64* dom, int* size, const int (&cs)[P],
                                                int k, int& myv, int& removed_total, bool& wiped_any) {
   const int lane = lane_id();
@@ -204,94 +383,14 @@ __device__ __forceinline__ u64 revise_pairs_w1(const DevNet& net, u64* dom, int*
   return __ballot(removed_l > 0);
 }
 
-template <bool kCoherent>
-__device__ __forceinline__ void grid_pairs_w1(const DevNet& net, u64* dom, int* size, const int (&cs)[kPairBatch],
-                                              int k, unsigned* B, GacCtl* ctl, int r,
-                                              unsigned long long& revs, unsigned long long& dels) {
-  int myv = -1, removed = 0;
-  bool wiped = false;
-  u64 changed = revise_pairs_w1<kCoherent>(net, dom, size, cs, k, myv, removed, wiped);
-  revs += 2 * k;
-  dels += removed;
-  if (wiped && lane_id() == 0) atomicMin(&ctl->wipe_round, r);
-  while (changed) {
-    const int l = (int)__builtin_ctzll(changed);
-    changed &= changed - 1ull;
-    push_var(net, __builtin_amdgcn_readlane(myv, l), B, ctl, r);
-  }
-}
-
-// Work units are (frontier word, part) pairs: part p of word w covers the
-// constraint bits [p * 32 / parts, (p + 1) * 32 / parts) of A[w], so a round
-// over few words still spreads over many waves; waves take units in a fixed
-// stride.  kCoherent: domains and frontier words are read with agent-scope
-// loads (rounds of one launch, written by other XCDs since the last barrier).
-// With one-word domains, binary constraints go kPairBatch at a time through
-// grid_pairs_w1.
-// revs / dels: the calling wave's statistics, accumulated.
-template <bool kCoherent = false>
-__device__ __forceinline__ void grid_round(const DevNet& net, u64* dom, int* size, unsigned* F,
-                                           int nfw, GacCtl* ctl, int r, int parts,
-                                           unsigned long long& revs, unsigned long long& dels) {
-  unsigned* A = F + (long long)(r % 3) * nfw;
-  unsigned* B = F + (long long)((r + 1) % 3) * nfw;
-  unsigned* Cl = F + (long long)((r + 2) % 3) * nfw;
-  if (blockIdx.x == 0 && threadIdx.x == 0) atomicExch(&ctl->scanner[(r + 1) % 3], 0u);
-  for (long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x; i < nfw;
-       i += (long long)gridDim.x * blockDim.x) {
-    if (kCoherent) __hip_atomic_store(&Cl[i], 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    else Cl[i] = 0u;
-  }
-  const long long units = (long long)nfw * parts;
-  const int pbits = 32 / parts;
-  // static stride over the units: one counter for tens of thousands of units
-  // would serialize on its atomic
-  const long long nwaves_grid = (long long)gridDim.x * (blockDim.x >> 6);
-  for (long long ui = (long long)blockIdx.x * (blockDim.x >> 6) + (threadIdx.x >> 6); ui < units;
-       ui += nwaves_grid) {
-    if (ld_agent(&ctl->wipe_round) <= r) break;
-    const int wi = (int)(ui / parts);
-    const int part = ui - wi * parts;
-    const unsigned pmask = pbits == 32 ? ~0u : (((1u << pbits) - 1u) << (part * pbits));
-    const unsigned aw = kCoherent ? (unsigned)ld_agent((const int*)&A[wi]) : A[wi];
-    unsigned bits = (unsigned)uniform_int((int)(aw & pmask));
-    if (net.W == 1) {
-      while (bits) {
-        int cs[kPairBatch] = {0, 0, 0, 0};
-        int k = 0;
-        while (bits && k < kPairBatch) {
-          const int b = __ffs(bits) - 1;
-          bits &= bits - 1u;
-          const int c = wi * 32 + b;
-          if (net.con[c].kind != 0) {
-            grid_process_constraint<kCoherent>(net, dom, size, c, B, ctl, r, revs, dels);
-            continue;
-          }
-#pragma unroll
-          for (int p = 0; p < kPairBatch; ++p)
-            if (p == k) cs[p] = c;
-          ++k;
-        }
-        if (k) grid_pairs_w1<kCoherent>(net, dom, size, cs, k, B, ctl, r, revs, dels);
-      }
-      continue;
-    }
-    while (bits) {
-      const int b = __ffs(bits) - 1;
-      bits &= bits - 1u;
-      grid_process_constraint<kCoherent>(net, dom, size, wi * 32 + b, B, ctl, r, revs, dels);
-    }
-  }
-}
-
-// Adds the waves' statistics to the grid's totals: one workgroup total per
-// call, on the workgroup's slot.  blk: two LDS words, zero on entry.  Every
-// thread of the workgroup calls it.
-__device__ __forceinline__ void flush_grid_stats(GacCtl* ctl, unsigned long long* blk, unsigned long long revs,
-                                                 unsigned long long dels) {
-  if (lane_id() == 0 && (revs | dels)) {
-    atomicAdd(&blk[0], revs);
-    atomicAdd(&blk[1], dels);
+// Adds the lanes' removals and the waves' revisions to the grid's totals: one
+// workgroup total per call, on the workgroup's slot.  blk: two LDS words, zero
+// on entry.  Every thread of the workgroup calls it.
+__device__ __forceinline__ void flush_grid_stats(GacCtl* ctl, unsigned long long* blk, int revs, int dels) {
+  const u64 wave_dels = wave_sum64_dpp((u64)dels);
+  if (lane_id() == 0 && (wave_dels | (u64)revs)) {
+    atomicAdd(&blk[0], (unsigned long long)revs);
+    atomicAdd(&blk[1], wave_dels);
   }
   __syncthreads();
   if (threadIdx.x == 0 && (blk[0] | blk[1])) {
@@ -300,17 +399,24 @@ __device__ __forceinline__ void flush_grid_stats(GacCtl* ctl, unsigned long long
   }
 }
 
-// One round per launch (host-driven fixpoint).
-__global__ void k_gac_round(DevNet net, u64* dom, int* size, unsigned* F, int nfw, GacCtl* ctl,
-                            int r, int parts) {
+// One round per launch (host-driven fixpoint).  A launch queued behind the
+// round that ended the fixpoint does nothing.
+__global__ void k_gac_round(DevNet net, u64* dom, int* size, unsigned* F, int nvw, GacCtl* ctl, int r, int seed,
+                            int narcs) {
   __shared__ unsigned long long blk[2];
+  if (r > 0 && (ctl->last_push_round < r - 1 || ctl->wipe_round < r)) return;
   if (threadIdx.x == 0) {
     blk[0] = 0ull;
     blk[1] = 0ull;
   }
   __syncthreads();
-  unsigned long long revs = 0, dels = 0;
-  grid_round(net, dom, size, F, nfw, ctl, r, parts, revs, dels);
+  for (long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x; i < nvw; i += (long long)gridDim.x * blockDim.x)
+    F[(long long)((r + 2) % 3) * nvw + i] = 0u;
+  int revs = 0, dels = 0;
+  grid_round<false>(net, dom, dom, size, F + (long long)(r % 3) * nvw, F + (long long)((r + 1) % 3) * nvw, ctl, r, seed,
+                    false, make_int4(0, -1, 0, 0), narcs, revs, dels);
+  // the epoch only grows: skip the atomic once another wave has raised it
+  if (__ballot(dels > 0) && lane_id() == 0 && ld_agent(&ctl->last_push_round) < r) atomicMax(&ctl->last_push_round, r);
   flush_grid_stats(ctl, blk, revs, dels);
 }
 
@@ -325,18 +431,16 @@ __global__ void k_gac_round(DevNet net, u64* dom, int* size, unsigned* F, int nf
 // Every wait is bounded: a waiter whose device wall clock passes the launch's
 // budget, or that sees the error flag another block raised, stops waiting and
 // its block leaves, so the launch always ends (an error, never a hang), even
-// if the workgroups were not all resident.  The decision taken after the
-// barrier (next round, wipe-out, fixpoint, error) is made by thread 0 and
-// broadcast through LDS; every wave reads it back as a wave-uniform value
+// if the workgroups were not all resident.  Thread 0 broadcasts the outcome
+// through LDS; every wave reads it back as a wave-uniform value
 // (readfirstlane), so the round loop leaves through a scalar branch.
-// The round decision uses epochs that only grow (last_push_round,
-// wipe_round): a block that already runs round r + 1 can raise them, but
-// never so that a slower block would decide differently for round r.
+// The round decision is taken at the start of the next round from what the
+// barrier made visible: wipe_round < r (a block already in round r can only
+// set it to r), and no bit in the bitmap of round r - 1's changes (nobody
+// writes it before the next barrier).
 // ===========================================================================
-enum : int { kRoundNext = 0, kRoundWipe = 1, kRoundFixpoint = 2, kRoundError = 3 };
-
 // Every write a round makes that another workgroup reads in a later round
-// (domain words, sizes, frontier bits, epochs, the cleared frontier) is an
+// (domain words, sizes, changed bits, wipe_round, the cleared bitmap) is an
 // agent-scope atomic, and every such read is an agent-scope atomic load, so
 // the data never waits in a cache that another XCD cannot see.  Before the
 // barrier each wave therefore only waits until its own memory operations have
@@ -352,9 +456,9 @@ __device__ __forceinline__ void wait_memory_ops() {
   __builtin_amdgcn_s_waitcnt(0x0F70);
 }
 
-__device__ __forceinline__ int grid_barrier_decide(GacCtl* ctl, unsigned nblocks, int r,
-                                                   unsigned long long t0, unsigned long long max_ticks,
-                                                   int* s_decision) {
+// Returns false when the launch's budget ran out here or elsewhere.
+__device__ __forceinline__ bool grid_barrier(GacCtl* ctl, unsigned nblocks, unsigned long long t0,
+                                             unsigned long long max_ticks, int* s_ok) {
   wait_memory_ops();
   __syncthreads();
   if (threadIdx.x == 0) {
@@ -363,38 +467,44 @@ __device__ __forceinline__ int grid_barrier_decide(GacCtl* ctl, unsigned nblocks
     // count reaches the end of this ticket's round
     const unsigned long long ticket = atomicAdd(&ctl->bar_ticket, 1ull);
     const unsigned long long target = (ticket / nblocks + 1) * nblocks;
-    int st = kRoundNext;
+    int ok = 1;
     while (__hip_atomic_load(&ctl->bar_ticket, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) < target) {
-      if (__hip_atomic_load(&ctl->err, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) {
-        st = kRoundError;
+      if (ld_agent(&ctl->err)) {
+        ok = 0;
         break;
       }
       if (wall_clock64() - t0 > max_ticks) {
         atomicExch(&ctl->err, 1);
-        st = kRoundError;
+        ok = 0;
         break;
       }
       __builtin_amdgcn_s_sleep(1);
     }
-    if (st == kRoundNext && __hip_atomic_load(&ctl->err, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT))
-      st = kRoundError;
-    if (st == kRoundNext) {
-      const int wr = ld_agent(&ctl->wipe_round);
-      const int lp = ld_agent(&ctl->last_push_round);
-      st = wr <= r ? kRoundWipe : (lp < r ? kRoundFixpoint : kRoundNext);
-    }
-    *s_decision = st;
+    *s_ok = ok;
   }
   __syncthreads();
-  return uniform_int(*s_decision);
+  return uniform_int(*s_ok) != 0;
 }
 
 constexpr int kPersistentThreads = 1024;
 
-__global__ void __launch_bounds__(kPersistentThreads) k_gac_persistent(DevNet net, u64* dom, int* size, unsigned* F, int nfw,
-                                                        GacCtl* ctl, int max_rounds, int parts,
-                                                        unsigned long long max_ticks) {
-  __shared__ int s_decision;
+// LDS bytes of a round's copy of the domains and of the changed bitmap.
+__host__ __device__ inline long long persistent_lds_bytes(int n, int W) {
+  return 8ll * n * W + 4ll * ((n + 31) / 32);
+}
+
+// kStaged: each round starts with a copy of the domains and of the changed
+// bitmap into LDS (one trip to memory for both, coalesced), and every lane
+// reads them there; otherwise the lanes read them from memory.  A round is
+// then that copy, the rows, the removals and the barrier: a chain of four to
+// six memory round trips, which is what bounds a cascade's many small rounds.
+// The first arc of each lane stays in registers over the rounds.
+template <bool kStaged>
+__global__ void __launch_bounds__(kPersistentThreads) k_gac_persistent(DevNet net, u64* dom, int* size, unsigned* F,
+                                                                       int nvw, GacCtl* ctl, int max_rounds, int seed,
+                                                                       int narcs, unsigned long long max_ticks) {
+  extern __shared__ __align__(16) char smem[];
+  __shared__ int s_ok;
   __shared__ unsigned long long blk[2];
   if (threadIdx.x == 0) {
     blk[0] = 0ull;
@@ -402,55 +512,70 @@ __global__ void __launch_bounds__(kPersistentThreads) k_gac_persistent(DevNet ne
   }
   __syncthreads();
   const unsigned long long t0 = wall_clock64();
-  int r = 0;
-  int decision = kRoundNext;
-  unsigned long long revs = 0, dels = 0;  // the wave's, over every round
-  for (; r < max_rounds; ++r) {
-    grid_round<true>(net, dom, size, F, nfw, ctl, r, parts, revs, dels);
-    decision = grid_barrier_decide(ctl, gridDim.x, r, t0, max_ticks, &s_decision);
-    if (decision != kRoundNext) break;
+  const int tid = threadIdx.x, lane = lane_id();
+  const long long words = (long long)net.n * net.W;
+  u64* sdom = (u64*)smem;
+  unsigned* scur = (unsigned*)(smem + 8 * words);
+  int lw = 0;
+  while ((1 << lw) < net.W) ++lw;
+  const long long i0 = (long long)blockIdx.x * blockDim.x + tid;
+  const long long arc0 = net.W > 1 ? (long long)(lane >> lw) * ((gridDim.x * blockDim.x) >> 6) + (i0 >> 6) : i0;
+  const int4 e0 = arc0 < narcs ? net.adj[arc0] : make_int4(0, -1, 0, 0);
+  int r = 0, revs = 0, dels = 0;  // the wave's revisions and the lane's removals, over every round
+  enum { NEXT, WIPE, FIXPOINT, ERROR } decision = NEXT;
+  if (kStaged) {
+    for (long long i = tid; i < words; i += blockDim.x) sdom[i] = ld_view<true>(&dom[i]);
+    __syncthreads();
+  }
+  while (true) {
+    unsigned* cur = F + (long long)(r % 3) * nvw;
+    unsigned* nxt = F + (long long)((r + 1) % 3) * nvw;
+    for (long long i = i0; i < nvw; i += (long long)gridDim.x * blockDim.x)
+      __hip_atomic_store(&F[(long long)((r + 2) % 3) * nvw + i], 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    if (kStaged) grid_round<false>(net, sdom, dom, size, scur, nxt, ctl, r, seed, true, e0, narcs, revs, dels);
+    else grid_round<true>(net, dom, dom, size, cur, nxt, ctl, r, seed, true, e0, narcs, revs, dels);
+    if (!grid_barrier(ctl, gridDim.x, t0, max_ticks, &s_ok)) {
+      decision = ERROR;
+      break;
+    }
+    ++r;
+    const int wr = ld_agent(&ctl->wipe_round);
+    if (kStaged) {
+      for (long long i = tid; i < words; i += blockDim.x) sdom[i] = ld_view<true>(&dom[i]);
+      for (int i = tid; i < nvw; i += blockDim.x) scur[i] = (unsigned)ld_agent((const int*)&nxt[i]);
+      __syncthreads();
+    }
+    unsigned bits = 0u;
+    for (int i = lane; i < nvw; i += 64) bits |= kStaged ? scur[i] : (unsigned)ld_agent((const int*)&nxt[i]);
+    const bool any = __ballot(bits != 0u) != 0ull;
+    if (uniform_int(wr) < r) decision = WIPE;
+    else if (!any) decision = FIXPOINT;
+    if (decision != NEXT || r >= max_rounds) break;
   }
   flush_grid_stats(ctl, blk, revs, dels);
-  if (blockIdx.x == 0 && threadIdx.x == 0) {
-    ctl->rounds = r < max_rounds ? r + 1 : max_rounds;
-    ctl->converged = decision == kRoundFixpoint ? 1 : 0;
+  if (blockIdx.x == 0 && tid == 0) {
+    ctl->rounds = r;
+    ctl->converged = decision == FIXPOINT ? 1 : 0;
   }
 }
 
-// Start of a host-driven fixpoint in one launch: the control block, the three
-// frontier buffers cleared, and with seed_all every constraint in the first.
-__global__ void k_gac_init(GacCtl* ctl, unsigned* F, int nfw, int ncons, int seed_all) {
+// Start of a grid fixpoint: the control block and the three bitmaps cleared.
+__global__ void k_gac_init(GacCtl* ctl, unsigned* F, int nvw) {
   const long long i0 = (long long)blockIdx.x * blockDim.x + threadIdx.x;
   if (i0 == 0) {
-    for (int k = 0; k < 3; ++k) ctl->scanner[k] = 0u;
     ctl->last_push_round = -1;
     ctl->wipe_round = INT_MAX;
     ctl->rounds = 0;
     ctl->converged = 0;
-    ctl->pad = 0;
     ctl->bar_ticket = 0ull;
     ctl->err = 0;
-    ctl->pad2 = 0;
+    ctl->pad = 0;
   }
   for (long long i = i0; i < kStatSlots; i += (long long)gridDim.x * blockDim.x) {
     ctl->deletions[i] = 0ull;
     ctl->revisions[i] = 0ull;
   }
-  for (long long i = i0; i < 3ll * nfw; i += (long long)gridDim.x * blockDim.x) {
-    unsigned v = 0u;
-    if (seed_all && i < nfw) {
-      const int k = ncons - (int)(i * 32);
-      v = k >= 32 ? 0xffffffffu : (k <= 0 ? 0u : ((1u << k) - 1u));
-    }
-    F[i] = v;
-  }
-}
-
-__global__ void k_seed_var(unsigned* F, const int* adj_off, const int4* adj, int var) {
-  for (int i = adj_off[var] + threadIdx.x; i < adj_off[var + 1]; i += blockDim.x) {
-    const int c = adj[i].x;
-    atomicOr(&F[c >> 5], 1u << (c & 31));
-  }
+  for (long long i = i0; i < 3ll * nvw; i += (long long)gridDim.x * blockDim.x) F[i] = 0u;
 }
 
 // ===========================================================================
@@ -740,23 +865,24 @@ __device__ __forceinline__ int ld_wg_int(const int* p) {
 // need = 0.  rows: word w of the rows of t's values over D(u); own: the rows
 // of the values of word w of D(u) over D(t), word j at own + j dpad.
 //
-// Source side: the rows of kStep values of t are ORed at a time, and the
-// values of u they cover are settled; a value stays open with the product of
-// kStep tightnesses, so one or two steps settle nearly every supported value
-// whatever the domains' sizes.  The values of t are wave-uniform: scalar
-// instructions pick them, and a lane spends one address and one load on each.
-// Target side: an open value is settled by the W words of its own row.  The
-// wave turns to it when more than two source steps are left and no lane has
-// more than a few open values, so that a true removal costs W reads instead
-// of a scan of D(t).
-template <int kStep = 4>
-__device__ __forceinline__ u64 wave_unsupported(const DevNet& net, const u64* dt, const u64* rows, const u64* own,
-                                                u64 need) {
+// As arcs_unsupported, but the values of t are wave-uniform: scalar
+// instructions pick them, four rows a step (eight cost bandwidth on networks
+// read from memory: 256 uneven instances 4.3 ms against 2.7 ms), and a lane
+// spends one address and one load on each.  With more than two source steps
+// left, the wave turns to the target side once no lane has more than a few
+// open values, or (several words) after three steps if settling the others one
+// after the other takes fewer steps than the rest of D(t).
+template <bool kTight>
+__device__ __forceinline__ u64 wave_unsupported(const DevNet& net, const u64* dom, int t, const u64* rows,
+                                                const u64* own, u64 need) {
+  constexpr int kStep = 4;
   const int W = net.W, dpad = net.dpad;
+  const u64* dt = dom + (long long)t * W;
   int left = 0;
   for (int j = 0; j < W; ++j) left += __popcll((u64)uniform_ll((long long)ld_wg(&dt[j])));
   const int few = W == 1 ? 4 : 2;
   bool target = false;
+  int done = 0;
   for (int j = 0; j < W && !target; ++j) {
     u64 x = (u64)uniform_ll((long long)ld_wg(&dt[j]));
     const u64* rj = rows + 64 * j;
@@ -779,15 +905,31 @@ __device__ __forceinline__ u64 wave_unsupported(const DevNet& net, const u64* dt
         need &= ~o;
       }
       left -= kStep;
+      ++done;
       if (__ballot(need != 0ull) == 0ull) return 0ull;
-      if (left > 2 * kStep && __ballot(__popcll(need) > few) == 0ull) {
-        target = true;
-        break;
+      if (left > 2 * kStep) {
+        const u64 many = __ballot(__popcll(need) > few);
+        if (many == 0ull ||
+            (kTight && W > 1 && done >= 3 && (__popcll(many) + kSettle - 1) / kSettle * 2 * kStep < left)) {
+          target = true;
+          break;
+        }
       }
     }
   }
   if (!target) return need;
-  u64 gone = 0ull;
+  u64 settled = 0ull;  // values that the wave settled as unsupported
+  if (kTight && W > 1) {
+    const u64 many = __ballot(__popcll(need) > few);
+    if (many) {
+      const u64 left_open = wave_settle<false>(net, dom, (long long)(own - net.sup), t, need, many);
+      if (__popcll(need) > few) {
+        settled = left_open;
+        need = 0ull;
+      }
+    }
+  }
+  u64 gone = settled;
   if (W == 1) {
     const u64 d = (u64)uniform_ll((long long)ld_wg(&dt[0]));
     while (need) {
@@ -813,70 +955,6 @@ __device__ __forceinline__ u64 wave_unsupported(const DevNet& net, const u64* dt
 #pragma unroll
       for (int i = 0; i < 4; ++i)
         if (j0 + i < W) ok = ok || (r[i] & ld_wg(&dt[j0 + i])) != 0ull;
-    }
-    if (!ok) gone |= 1ull << b;
-    need &= need - 1ull;
-  }
-  return gone;
-}
-
-// wave_unsupported with a source per lane: the values of `need` (word w of
-// D(tgt)) without a support in D(src), for the constraint whose planes start
-// at off.  The lane takes source steps of four rows and turns to the target
-// side (four row reads a step) once at most one such step is left, or after
-// three source steps, if that takes fewer steps than the rest of D(src).
-__device__ __forceinline__ u64 lane_unsupported(const DevNet& net, const u64* dom, long long off, int src,
-                                                int pos_src, int w, u64 need) {
-  const int W = net.W, dpad = net.dpad;
-  const u64* rows = net.sup + off + (long long)(pos_src * W + w) * dpad;
-  const u64* ds = dom + (long long)src * W;
-  u64 x = ld_wg(&ds[0]);
-  int left = __popcll(x);
-  for (int j = 1; j < W; ++j) left += __popcll(ld_wg(&ds[j]));
-  int j = 0, done = 0;
-  while (need && left > 0) {
-    const int ts = (__popcll(need) * W + 3) >> 2;
-    if (left > 4 * ts && (ts <= 1 || done >= 3)) break;
-    u64 r[4];
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      while (x == 0ull && j + 1 < W) x = ld_wg(&ds[++j]);
-      const int a = x ? (int)__builtin_ctzll(x) : 0;
-      r[i] = x ? rows[64 * j + a] : 0ull;
-      x &= x - 1ull;
-    }
-    need &= ~((r[0] | r[1]) | (r[2] | r[3]));
-    left -= 4;
-    ++done;
-  }
-  if (need == 0ull || left <= 0) return need;
-  const u64* own = net.sup + off + (long long)(1 - pos_src) * W * dpad + 64 * w;
-  u64 gone = 0ull;
-  if (W == 1) {
-    const u64 d = ld_wg(&ds[0]);
-    while (need) {
-      u64 r[4], bit[4];
-#pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        bit[i] = need & (0ull - need);
-        r[i] = need ? own[__builtin_ctzll(need)] : ~0ull;
-        need &= need - 1ull;
-      }
-#pragma unroll
-      for (int i = 0; i < 4; ++i) gone |= (r[i] & d) ? 0ull : bit[i];
-    }
-    return gone;
-  }
-  while (need) {
-    const int b = (int)__builtin_ctzll(need);
-    bool ok = false;
-    for (int j0 = 0; j0 < W && !ok; j0 += 4) {
-      u64 r[4];
-#pragma unroll
-      for (int i = 0; i < 4; ++i) r[i] = j0 + i < W ? own[(long long)(j0 + i) * dpad + b] : 0ull;
-#pragma unroll
-      for (int i = 0; i < 4; ++i)
-        if (j0 + i < W) ok = ok || (r[i] & ld_wg(&ds[j0 + i])) != 0ull;
     }
     if (!ok) gone |= 1ull << b;
     need &= need - 1ull;
@@ -993,7 +1071,7 @@ __device__ __forceinline__ void wg_round_flat(const DevNet& net, const WgMem& me
 // wg_round_flat instead of numbered units.
 // slot: two wipe-out words used in turn by successive fixpoints, so that
 // wg_seed never resets the word a slow wave still reads.
-template <bool kImage>
+template <bool kImage, bool kTight>
 __device__ __forceinline__ bool wg_fixpoint(const DevNet& net, const WgMem& mem, WgCtl* ctl, int slot,
                                             bool both_dirs_round0) {
   const int n = net.n, W = net.W;
@@ -1048,7 +1126,6 @@ __device__ __forceinline__ bool wg_fixpoint(const DevNet& net, const WgMem& mem,
         const int k0 = (q - __builtin_amdgcn_readlane(inc - units, l)) << (6 - lw);
         const int cnt = min(per, __builtin_amdgcn_readlane(deg, l) - k0);
         const int arc = __builtin_amdgcn_readlane(a0, l) + k0 + la;
-        const u64* dt = mem.dom + (long long)t * W;
         int u = -1;
         u64 need = 0ull;
         u64* word = nullptr;
@@ -1068,8 +1145,8 @@ __device__ __forceinline__ bool wg_fixpoint(const DevNet& net, const WgMem& mem,
           stop = true;
           break;
         }
-        const u64 gone = wave_unsupported(net, dt, pair + (long long)(pos_t * W + w) * net.dpad,
-                                          pair + (long long)(1 - pos_t) * W * net.dpad + 64 * w, need);
+        const u64 gone = wave_unsupported<kTight>(net, mem.dom, t, pair + (long long)(pos_t * W + w) * net.dpad,
+                                                  pair + (long long)(1 - pos_t) * W * net.dpad + 64 * w, need);
         if (gone) lane_remove(mem, ctl, nxt, slot, round, u, word, gone);
         revs += cnt;
         if (both && !bit_of(mem.asg, t)) {
@@ -1079,12 +1156,12 @@ __device__ __forceinline__ bool wg_fixpoint(const DevNet& net, const WgMem& mem,
             const int ui = uniform_int(mem.adj[arc - la + i].y);
             if (ui < 0) continue;
             const int pi = 1 - uniform_int(adj_pos(mem.adj[arc - la + i]));
-            const u64* pp = net.sup + uniform_int(mem.adj[arc - la + i].w) * pair_words;
             u64* tw = mem.dom + (long long)t * W + lane;
-            const u64 g = wave_unsupported(net, mem.dom + (long long)ui * W,
-                                           pp + (long long)(pi * W + (lane < W ? lane : 0)) * net.dpad,
-                                           pp + (long long)(1 - pi) * W * net.dpad + 64 * (lane < W ? lane : 0),
-                                           lane < W ? ld_wg(tw) : 0ull);
+            const u64* pp = net.sup + uniform_int(mem.adj[arc - la + i].w) * pair_words;
+            const int wl = lane < W ? lane : 0;
+            const u64 g = wave_unsupported<kTight>(net, mem.dom, ui, pp + (long long)(pi * W + wl) * net.dpad,
+                                                   pp + (long long)(1 - pi) * W * net.dpad + 64 * wl,
+                                                   lane < W ? ld_wg(tw) : 0ull);
             if (g) lane_remove(mem, ctl, nxt, slot, round, t, tw, g);
           }
           revs += cnt;
@@ -1199,7 +1276,7 @@ __global__ void k_block_gac(DevNet net, u64* dom, int* size, int seed_var, char*
   __syncthreads();
   long long before = 0;
   for (int v = threadIdx.x; v < n; v += blockDim.x) before += mem.size[v];
-  const bool ok = wg_fixpoint<false>(net, mem, &ctl, 0, seed_var >= 0);
+  const bool ok = wg_fixpoint<false, true>(net, mem, &ctl, 0, seed_var >= 0);
   long long after = 0;
   for (int v = threadIdx.x; v < n; v += blockDim.x) after += mem.size[v];
   const u64 delta = wg_reduce_sum_u64(&ctl, (u64)(before - after));
@@ -1247,7 +1324,7 @@ __global__ void k_singleton_tests(DevNet net, const u64* __restrict__ base_dom,
     mem.asg[x >> 5] |= 1u << (x & 31);
   }
   __syncthreads();
-  const bool ok = wg_fixpoint<false>(net, mem, &ctl, 0, false);
+  const bool ok = wg_fixpoint<false, true>(net, mem, &ctl, 0, false);
   __syncthreads();  // every wave's revision count
   if (threadIdx.x == 0) {
     fail[unit] = ok ? 0 : 1;
@@ -2514,10 +2591,10 @@ __device__ __forceinline__ bool wave_ac3(const DevNet& net, WgMem mem, const Mac
         const u64 dy = in && !table ? ld_wg(ydom) : 0ull;
         const bool act = in && !table && svx > stc;
         const bool yrev = act && !bit_of(mem.asg, y);
-        const u64* pair = net.sup + (in && !table ? e.w * pair_words : 0ll);
+        const long long off = in && !table ? e.w * pair_words : 0ll;
         const u64 need = yrev ? dy : 0ull;
-        const u64 gone = wave_unsupported(net, mem.dom + (long long)x * W, pair + (long long)(px * W + w) * net.dpad,
-                                          pair + (long long)(1 - px) * W * net.dpad + 64 * w, need);
+        const u64 gone = wave_unsupported<false>(net, mem.dom, x, net.sup + off + (long long)(px * W + w) * net.dpad,
+                                                 net.sup + off + (long long)(1 - px) * W * net.dpad + 64 * w, need);
         const int bit0 = la << lw;
         const u64 lose = arcs_with(gone != 0ull);
         const u64 wipe = lose & ~arcs_with((need & ~gone) != 0ull);
@@ -2525,10 +2602,8 @@ __device__ __forceinline__ bool wave_ac3(const DevNet& net, WgMem mem, const Mac
         // x <- y: when y changed since the constraint's stamp, or lost values
         // just now; those had no support in D(x), so the old D(y) decides the same
         const bool xrev = act && !asgx && (svy > stc || (px == 1 && mine_lose && !((wipe >> bit0) & 1ull)));
-        u64 xgone = 0ull;
-        if (xrev)
-          xgone = lane_unsupported(net, mem.dom, (long long)(pair - net.sup), y, 1 - px, w,
-                                   ld_wg(&mem.dom[(long long)x * W + w]));
+        const u64 xgone = arcs_unsupported<false, false>(net, mem.dom, off, y, 1 - px, in ? w : 0,
+                                           xrev ? ld_wg(&mem.dom[(long long)x * W + w]) : 0ull);
         const u64 xlose = arcs_with(xgone != 0ull), tabs = arcs_with(table);
         const u64 acts = arcs_with(act);
         // lanes of the arcs that can be committed
@@ -2791,7 +2866,7 @@ __device__ __forceinline__ void wg_mac_run(const DevNet& net, const WgMem& mem, 
       phase = POSITIVE;
       __syncthreads();
     }
-    bool ok = wg_fixpoint<kImage>(net, mem, ctl, slot, false);
+    bool ok = wg_fixpoint<kImage, false>(net, mem, ctl, slot, false);
     if (kWdeg && !ok) {
       // a wipe-out raises the weight of the constraint that AC3's order
       // empties a domain with first: propagate again, in that order, from the

@@ -191,3 +191,44 @@ def test_sac_pass_same_on_both_sides_of_the_kernel_choice(gpu, n, d, e, t):
                           for a in vals], np.int32)
         got = {mode: m.SingletonTests(tests, mode=mode)[0] for mode in ("auto", "sliced", "workgroup")}
     assert (got["auto"] == got["sliced"]).all() and (got["auto"] == got["workgroup"]).all()
+
+
+GRID_SHAPES = SHAPES + [
+    (1030, 1000, 60, 0.993),   # domains above 128 KB: the persistent rounds read them from memory
+    (1030, 1000, 40, 0.5),
+    (2000, 8, 140000, 0.02),   # more arcs than the persistent grid has lanes
+    (300, 250, 4000, 0.96), (300, 130, 4000, 0.93),
+]
+
+
+@pytest.mark.parametrize("mode", ["plain", "persistent"])
+@pytest.mark.parametrize("n,d,e,t", GRID_SHAPES)
+def test_grid_rounds_equal_oracle(gpu, n, d, e, t, mode):
+    # a lane per arc word: tight relations settled by the wave, and a seed of
+    # one variable (its constraints in both directions in the first round)
+    desc = networks(n, d, e, t, 3)
+    ok, dom, _ = oracle.Oracle(desc).root_ac()
+    with GModelAdapter.Build(desc) as m:
+        run = (lambda v: m.EnforceGAC(False, v)) if mode == "plain" else (lambda v: m.EnforceGAC_Persistent(False, v))
+        before = m.ReadDomains(0)
+        st = run(-1)
+        assert st.inconsistent == (not ok)
+        if not ok:
+            return
+        got = m.ReadDomains(0)
+        assert (got == dom).all() and st.converged
+        assert st.deletions == int(np.bitwise_count(before).sum()) - int(np.bitwise_count(dom).sum())
+        sizes = np.bitwise_count(dom).sum(axis=1)
+        for v in range(0, n, max(1, n // 50)):
+            assert m.GetDomainSize(v, 0) == sizes[v]
+        v = n // 2
+        a = int(domains_to_sets(dom, desc.dom_size)[v][0])
+        cut = dom.copy()
+        cut[v] = 0
+        cut[v, a // 64] = np.uint64(1 << (a % 64))
+        m.WriteDomains(0, cut)
+        st = run(v)
+        ok2, dom2, _ = oracle.Oracle(desc.with_init_dom(cut)).root_ac()
+        assert st.inconsistent == (not ok2)
+        if ok2:
+            assert (m.ReadDomains(0) == dom2).all()
