@@ -608,12 +608,56 @@ struct SacScratch {
 };
 
 // ---------------------------------------------------------------------------
+// Host boxes: pinned memory that kernels answer in (HostBox in kernels.h), one
+// per model from its first call on.  Pinning takes tens of microseconds, so
+// models that come and go hand their boxes on through a pool of at most
+// kBoxPool; every box returns to it, or is freed, with its model.
+// ---------------------------------------------------------------------------
+namespace {
+
+constexpr long long kBoxDataBytes = 64 * 1024;
+constexpr size_t kBoxPool = 8;
+std::mutex g_box_mu;
+std::vector<HostBox*> g_boxes;
+
+HostBox* take_box() {
+  {
+    std::lock_guard<std::mutex> lock(g_box_mu);
+    if (!g_boxes.empty()) {
+      HostBox* b = g_boxes.back();
+      g_boxes.pop_back();
+      return b;
+    }
+  }
+  void* p = nullptr;
+  HIPC(hipHostMalloc(&p, sizeof(HostBox) + kBoxDataBytes, hipHostMallocPortable | hipHostMallocMapped | hipHostMallocCoherent));
+  HostBox* b = static_cast<HostBox*>(p);
+  b->seq = 0;
+  return b;
+}
+
+void give_box(HostBox* b) {
+  if (!b) return;
+  {
+    std::lock_guard<std::mutex> lock(g_box_mu);
+    if (g_boxes.size() < kBoxPool) {
+      g_boxes.push_back(b);
+      return;
+    }
+  }
+  (void)hipHostFree(b);
+}
+
+}  // namespace
+
+// ---------------------------------------------------------------------------
 // GModel
 // ---------------------------------------------------------------------------
 struct cpim_gmodel {
   int device = 0;
   hipStream_t stream = nullptr;
   ModelImage im;  // host layout (rel pointer not kept beyond build)
+  Arena arena;    // the device arrays below, in one allocation
   DevModel dm;
   int max_depth = 0;
   int current_level = 0;
@@ -622,8 +666,8 @@ struct cpim_gmodel {
   DevAlloc size;   // [max_depth][n]
   DevAlloc front;  // three bitmaps of variables (grid rounds), or one of constraints (asynchronous)
   DevAlloc ctl;    // GacCtl
-  GacCtl* ctl_host = nullptr;  // pinned copy of the control block (host rounds)
-  DevAlloc block_out;
+  bool ctl_ready = false;      // ctl and front are in their first state (k_gac_init, grid_finish)
+  mutable HostBox* box_ = nullptr;  // answers of the model's kernels
   DevAlloc async_ctl;
   DevAlloc scratch;  // workgroup-engine scratch when a copy does not fit in LDS
   long long scratch_bytes = 0;
@@ -656,6 +700,47 @@ struct cpim_gmodel {
     HIPC(hipStreamSynchronize(stream));  // `ones` and `one` are host stack memory
   }
 
+  // The box and the number of the next call that answers in it.
+  HostBox* box() const {
+    if (!box_) box_ = take_box();
+    return box_;
+  }
+  unsigned long long next_seq() const { return box()->seq + 1; }
+
+  // Waits for call `seq` (its kernel is the last work queued on the stream):
+  // the kernel's answer arrives a few microseconds before the runtime reports
+  // the stream idle.  The stream is asked now and then, so that a launch that
+  // failed ends the wait with its error.
+  void wait_box(unsigned long long seq) const {
+    const unsigned long long* at = &box_->seq;
+    for (unsigned i = 1;; ++i) {
+      if (__atomic_load_n(at, __ATOMIC_ACQUIRE) == seq) return;
+      __builtin_ia32_pause();
+      if ((i & 4095u) == 0u) {
+        const hipError_t e = hipStreamQuery(stream);
+        if (e == hipErrorNotReady) {
+          (void)hipGetLastError();
+          continue;
+        }
+        HIPC(e);
+        if (__atomic_load_n(at, __ATOMIC_ACQUIRE) == seq) return;
+        fail(CPIM_ERR_RUNTIME, "a kernel ended without its answer");
+      }
+    }
+  }
+  double ticks_ms(unsigned long long ticks) const { return (double)ticks / (double)std::max<long long>(props.wall_khz, 1); }
+
+  // One k_level_op on a level, and its answer.
+  int level_op(int op, int level, int var, int value) const {
+    HostBox* b = box();
+    const unsigned long long seq = next_seq();
+    hipLaunchKernelGGL(k_level_op, dim3(1), dim3(256), 0, stream, op, level_dom(level), level_size(level), dm.n, dm.W,
+                       dm.max_dom, var, value, &b->scalar, &b->seq, seq);
+    HIPC(hipGetLastError());
+    wait_box(seq);
+    return b->scalar;
+  }
+
   void gac_events() {
     for (hipEvent_t& e : gev)
       if (!e) HIPC(hipEventCreate(&e));
@@ -679,6 +764,7 @@ struct cpim_gmodel {
     return scratch.as<char>();
   }
   void sync() { HIPC(hipStreamSynchronize(stream)); }
+  bool level_in_box() const { return 8 * level_words() <= kBoxDataBytes; }
 };
 
 extern "C" {
@@ -762,27 +848,30 @@ int cpim_gmodel_create(const cpim_model_desc* desc, const cpim_gmodel_options* o
     m->props = props_of(o.device_id);
     HIPC(hipStreamCreateWithFlags(&m->stream, hipStreamNonBlocking));
     m->im = std::move(im);
-    build_device_model(m->im, m->dm, m->stream);
+    const int n = m->im.n;
+    m->max_depth = n + 1;
+    m->nfw = std::max(1, (m->im.num_active + 31) / 32);
+    m->nvw = (n + 31) / 32;
+    const long long lw = (long long)n * m->im.W;
+    const long long dom_bytes = (long long)sizeof(u64) * lw * m->max_depth;
+    const long long size_bytes = (long long)sizeof(int) * n * m->max_depth;
+    const long long front_bytes = (long long)sizeof(unsigned) * std::max<long long>(m->nfw, 3ll * m->nvw);
+    m->arena.reserve(model_arena_bytes(m->im) + Arena::round(dom_bytes) + Arena::round(size_bytes) +
+                     Arena::round(front_bytes) + Arena::round((long long)sizeof(GacCtl)));
+    build_device_model(m->im, m->dm, m->stream, &m->arena);
     m->im.rel = nullptr;
     m->im.rel_dense.clear();
     m->im.rel_dense.shrink_to_fit();
-    const int n = m->dm.n;
-    m->max_depth = n + 1;
-    const long long lw = m->level_words();
-    m->dom = DevAlloc(sizeof(u64) * lw * m->max_depth);
-    m->size = DevAlloc(sizeof(int) * (long long)n * m->max_depth);
+    m->dom = m->arena.take(dom_bytes);
+    m->size = m->arena.take(size_bytes);
+    m->front = m->arena.take(front_bytes);
+    m->ctl = m->arena.take((long long)sizeof(GacCtl));
     HIPC(hipMemcpyAsync(m->dom.p, m->im.init_dom.data(), sizeof(u64) * lw, hipMemcpyHostToDevice, m->stream));
     hipLaunchKernelGGL(k_sizes, dim3((n + 255) / 256), dim3(256), 0, m->stream, m->level_dom(0),
                        m->level_size(0), n, m->dm.W);
     HIPC(hipGetLastError());
-    m->nfw = std::max(1, (m->dm.num_active + 31) / 32);
-    m->nvw = (n + 31) / 32;
-    m->front = DevAlloc(sizeof(unsigned) * std::max<long long>(m->nfw, 3ll * m->nvw));
-    m->ctl = DevAlloc(sizeof(GacCtl));
-    m->block_out = DevAlloc(sizeof(BlockGacOut));
     m->assigned.assign(m->max_depth, make_int2(-1, -1));
-    m->dm.bytes += sizeof(u64) * lw * m->max_depth + sizeof(int) * (long long)n * m->max_depth +
-                   sizeof(unsigned) * std::max<long long>(m->nfw, 3ll * m->nvw) + sizeof(GacCtl);
+    m->dm.bytes += dom_bytes + size_bytes + front_bytes + (long long)sizeof(GacCtl);
     m->sync();
     *out = m.release();
   });
@@ -794,7 +883,7 @@ int cpim_gmodel_destroy(cpim_gmodel* m) {
     DeviceGuard g(m->device);
     if (m->stream) (void)hipStreamSynchronize(m->stream);
     hipStream_t s = m->stream;
-    if (m->ctl_host) (void)hipHostFree(m->ctl_host);
+    give_box(m->box_);
     for (hipEvent_t e : m->gev)
       if (e) (void)hipEventDestroy(e);
     delete m;
@@ -845,7 +934,7 @@ unsigned long long slot_sum(const unsigned long long (&v)[kStatSlots]) {
   return t;
 }
 
-// Start of a grid fixpoint: control block and changed bitmaps cleared.
+// Control block and changed bitmaps cleared.
 void gac_start(cpim_gmodel* m, unsigned* F, GacCtl* ctl) {
   const int blocks = (int)std::max<long long>(1, std::min<long long>((3ll * m->nvw + 255) / 256, 1024));
   hipLaunchKernelGGL(k_gac_init, dim3(blocks), dim3(256), 0, m->stream, ctl, F, m->nvw);
@@ -863,12 +952,13 @@ long long grid_lanes(const cpim_gmodel* m) {
 // Largest round copy of the persistent fixpoint in LDS: one workgroup per CU.
 constexpr long long kPersistentLdsMax = 128 * 1024;
 
-// The persistent fixpoint kernel on the current level, after gac_start: a
-// lane per arc word, at most one 1024-thread workgroup per CU.  Every
-// workgroup must be resident for the grid barrier; if some were not, the
+// The persistent fixpoint kernel on the current level, with ctl and F in their
+// first state: a lane per arc word, at most one 1024-thread workgroup per CU.
+// Every workgroup must be resident for the grid barrier; if some were not, the
 // barrier's bounded wait turns that into the time-budget error the caller
-// reports (ctl->err).
-void persistent_launch(cpim_gmodel* m, int assigned_var, unsigned* F, GacCtl* ctl) {
+// reports (out->err).
+void persistent_launch(cpim_gmodel* m, int assigned_var, unsigned* F, GacCtl* ctl, GacResult* out,
+                       unsigned long long* seq_at, unsigned long long seq) {
   const int L = m->current_level;
   const long long lanes = grid_lanes(m);
   const long long lds = persistent_lds_bytes(m->dm.n, m->dm.W);
@@ -880,67 +970,79 @@ void persistent_launch(cpim_gmodel* m, int assigned_var, unsigned* F, GacCtl* ct
   const unsigned long long max_ticks = fixpoint_budget_ticks(m);
   hipLaunchKernelGGL(staged ? k_gac_persistent<true> : k_gac_persistent<false>, dim3(grid), dim3(kPersistentThreads),
                      staged ? (size_t)lds : 0, m->stream, m->dm.net(), m->level_dom(L), m->level_size(L), F, m->nvw,
-                     ctl, mr, assigned_var, (int)m->im.adj.size(), max_ticks);
+                     ctl, mr, assigned_var, (int)m->im.adj.size(), max_ticks, out, seq_at, seq);
   HIPC(hipGetLastError());
 }
 
-void fill_gac_stats(const GacCtl& res, int rounds, double kms, cpim_gac_stats* st) {
+void fill_gac_stats(const GacResult& res, int rounds, bool converged, double kms, cpim_gac_stats* st) {
   st->iterations = rounds;
-  st->deletions = (int32_t)slot_sum(res.deletions);
+  st->deletions = (int32_t)res.deletions;
   st->inconsistent = res.wipe_round != INT_MAX;
-  st->converged = st->inconsistent ? 0 : res.converged;
-  st->revisions = (int64_t)slot_sum(res.revisions);
+  st->converged = st->inconsistent ? 0 : converged;
+  st->revisions = (int64_t)res.revisions;
   st->kernel_ms = kms;
 }
 
+// Rounds of a host-driven fixpoint queued before the host looks at their
+// outcome: one, then two, four, ... up to this many.  A look costs about 10 us,
+// a launch that finds the fixpoint over about 2 us.
+constexpr int kRoundsAhead = 8;
+
 void gac_grid(cpim_gmodel* m, int assigned_var, bool persistent, cpim_gac_stats* st) {
   const int L = m->current_level;
-  u64* dom = m->level_dom(L);
-  int* size = m->level_size(L);
   unsigned* F = m->front.as<unsigned>();
   GacCtl* ctl = m->ctl.as<GacCtl>();
-  if (!m->ctl_host) HIPC(hipHostMalloc((void**)&m->ctl_host, sizeof(GacCtl), hipHostMallocDefault));
-  m->gac_events();
+  HostBox* box = m->box();
+  if (!m->ctl_ready) gac_start(m, F, ctl);
+  m->ctl_ready = false;  // until this fixpoint has put it back
+  unsigned long long seq = m->next_seq();
   double kms = 0.0;
-  HIPC(hipEventRecord(m->gev[0], m->stream));
-  gac_start(m, F, ctl);
   int rounds = 0;
-  GacCtl res{};
+  GacResult res{};
+  bool converged = false;
   if (persistent) {
-    persistent_launch(m, assigned_var, F, ctl);
-    HIPC(hipEventRecord(m->gev[1], m->stream));
-    HIPC(hipMemcpyAsync(m->ctl_host, ctl, sizeof(res), hipMemcpyDeviceToHost, m->stream));
-    m->sync();
-    kms = m->gac_elapsed_ms();
-    res = *m->ctl_host;
+    persistent_launch(m, assigned_var, F, ctl, &box->gac, &box->seq, seq);
+    m->wait_box(seq);
+    res = box->gac;
+    kms = m->ticks_ms(res.ticks);
     if (res.err) fail(CPIM_ERR_RUNTIME, "persistent fixpoint exceeded its time budget at a grid barrier");
     rounds = res.rounds;
+    converged = res.converged != 0;
   } else {
-    DevNet net = m->dm.net();
-    const int threads = 256;
+    const DevNet net = m->dm.net();
     const long long max_rounds = (long long)m->dm.n * m->dm.max_dom + 2;
-    const long long lanes = grid_lanes(m);
+    const long long lanes = std::max(grid_lanes(m), 64ll * m->dm.ntabs);
     const int grid = (int)std::max<long long>(
-        1, std::min<long long>((std::max(lanes, 64ll * m->dm.ntabs) + threads - 1) / threads, 8ll * m->props.cus));
-    for (int r = 0; r < max_rounds; ++r) {
-      if (r > 0) HIPC(hipEventRecord(m->gev[0], m->stream));
-      hipLaunchKernelGGL(k_gac_round, dim3(grid), dim3(threads), 0, m->stream, net, dom, size, F, m->nvw,
-                         ctl, r, assigned_var, (int)m->im.adj.size());
-      HIPC(hipGetLastError());
-      HIPC(hipEventRecord(m->gev[1], m->stream));
-      HIPC(hipMemcpyAsync(m->ctl_host, ctl, sizeof(res), hipMemcpyDeviceToHost, m->stream));
-      m->sync();
-      kms += m->gac_elapsed_ms();
-      res = *m->ctl_host;
-      rounds = r + 1;
-      if (res.wipe_round <= r) break;
-      if (res.last_push_round < r) {
-        res.converged = 1;
-        break;
+        1, std::min<long long>((lanes + kRoundThreads - 1) / kRoundThreads, 2ll * m->props.cus));
+    // each round of a batch answers in a result of its own
+    GacResult* answers = reinterpret_cast<GacResult*>(box->data);
+    bool over = false;
+    for (int r0 = 0, ahead = 1; r0 < max_rounds && !over; r0 += ahead, ahead = std::min(2 * ahead, kRoundsAhead)) {
+      const int k = (int)std::min<long long>(ahead, max_rounds - r0);
+      for (int i = 0; i < k; ++i, ++seq) {
+        answers[i].rounds = 0;  // stays 0 if the fixpoint was over before
+        hipLaunchKernelGGL(k_gac_round, dim3(grid), dim3(kRoundThreads), 0, m->stream, net, m->level_dom(L),
+                           m->level_size(L), F, m->nvw, ctl, r0 + i, assigned_var, (int)m->im.adj.size(), &answers[i],
+                           &box->seq, seq);
+        HIPC(hipGetLastError());
+      }
+      m->wait_box(seq - 1);
+      for (int i = 0; i < k && !over; ++i) {
+        if (answers[i].rounds == 0) continue;
+        res = answers[i];
+        kms += m->ticks_ms(res.ticks);
+        rounds = res.rounds;
+        converged = res.last_push_round < rounds - 1;
+        over = converged || res.wipe_round < rounds;
       }
     }
+    if (!over) {  // rounds bounded by the number of values: not reached
+      m->sync();
+      gac_start(m, F, ctl);
+    }
   }
-  fill_gac_stats(res, rounds, kms, st);
+  m->ctl_ready = true;
+  fill_gac_stats(res, rounds, converged, kms, st);
 }
 
 void gac_async(cpim_gmodel* m, int assigned_var, cpim_gac_stats* st) {
@@ -949,6 +1051,7 @@ void gac_async(cpim_gmodel* m, int assigned_var, cpim_gac_stats* st) {
   int* size = m->level_size(L);
   unsigned* F = m->front.as<unsigned>();
   const int nfw = m->nfw;
+  m->ctl_ready = false;  // the frontier of constraints goes where the changed bitmaps lie
   if (!m->async_ctl.p) m->async_ctl = DevAlloc(sizeof(AsyncCtl));
   AsyncCtl* ctl = m->async_ctl.as<AsyncCtl>();
   m->gac_events();
@@ -987,28 +1090,19 @@ void gac_block(cpim_gmodel* m, int assigned_var, cpim_gac_stats* st) {
   DevNet net = m->dm.net();
   const long long bytes = wg_mem_bytes(m->dm.n, m->dm.W);
   const int threads = 1024;
-  BlockGacOut* out = m->block_out.as<BlockGacOut>();
-  m->gac_events();
-  HIPC(hipEventRecord(m->gev[0], m->stream));
+  HostBox* box = m->box();
+  const unsigned long long seq = m->next_seq();
   if (bytes <= kLdsBudget) {
     hipLaunchKernelGGL(k_block_gac<true>, dim3(1), dim3(threads), (size_t)bytes, m->stream, net,
-                       m->level_dom(L), m->level_size(L), assigned_var, (char*)nullptr, out);
+                       m->level_dom(L), m->level_size(L), assigned_var, (char*)nullptr, &box->gac, &box->seq, seq);
   } else {
     char* scratch = m->get_scratch(bytes);
     hipLaunchKernelGGL(k_block_gac<false>, dim3(1), dim3(threads), 0, m->stream, net, m->level_dom(L),
-                       m->level_size(L), assigned_var, scratch, out);
+                       m->level_size(L), assigned_var, scratch, &box->gac, &box->seq, seq);
   }
   HIPC(hipGetLastError());
-  HIPC(hipEventRecord(m->gev[1], m->stream));
-  BlockGacOut res{};
-  HIPC(hipMemcpyAsync(&res, out, sizeof(res), hipMemcpyDeviceToHost, m->stream));
-  m->sync();
-  st->kernel_ms = m->gac_elapsed_ms();
-  st->iterations = 1;
-  st->deletions = (int32_t)res.deletions;
-  st->inconsistent = !res.consistent;
-  st->converged = res.consistent;
-  st->revisions = (int64_t)res.revisions;
+  m->wait_box(seq);
+  fill_gac_stats(box->gac, 1, box->gac.converged != 0, m->ticks_ms(box->gac.ticks), st);
 }
 
 int auto_gac_mode(const cpim_gmodel* m, int assigned_var) {
@@ -1048,19 +1142,45 @@ void check_level(const cpim_gmodel* m, int level, const char* fn) {
     fail(CPIM_ERR_RUNTIME, std::string("[GModel::") + fn + "] Invalid level: " + std::to_string(level));
 }
 
-std::vector<u64> read_var(const cpim_gmodel* m, int var, int level) {
-  std::vector<u64> w(m->dm.W);
-  HIPC(hipMemcpyAsync(w.data(), m->level_dom(level) + (long long)var * m->dm.W, sizeof(u64) * m->dm.W,
-                      hipMemcpyDeviceToHost, m->stream));
-  HIPC(hipStreamSynchronize(m->stream));
-  return w;
+// Host copy of one level.  Levels that fit the box come through it with one
+// launch (larger ones through the runtime's copies).
+void read_level(const cpim_gmodel* m, int level, u64* out) {
+  const size_t bytes = sizeof(u64) * (size_t)m->level_words();
+  if (!m->level_in_box()) {
+    HIPC(hipMemcpyAsync(out, m->level_dom(level), bytes, hipMemcpyDeviceToHost, m->stream));
+    HIPC(hipStreamSynchronize(m->stream));
+    return;
+  }
+  HostBox* box = m->box();
+  const unsigned long long seq = m->next_seq();
+  hipLaunchKernelGGL(k_level_get, dim3(1), dim3(1024), 0, m->stream, m->level_dom(level), box->data,
+                     (int)m->level_words(), &box->seq, seq);
+  HIPC(hipGetLastError());
+  m->wait_box(seq);
+  std::memcpy(out, box->data, bytes);
 }
 
-int read_size(const cpim_gmodel* m, int var, int level) {
-  int s = 0;
-  HIPC(hipMemcpyAsync(&s, m->level_size(level) + var, sizeof(int), hipMemcpyDeviceToHost, m->stream));
-  HIPC(hipStreamSynchronize(m->stream));
-  return s;
+// Sets one level to the words that fill(words) writes, sizes included.
+template <typename Fill>
+void write_level(cpim_gmodel* m, int level, Fill&& fill) {
+  const int n = m->dm.n, W = m->dm.W;
+  if (!m->level_in_box()) {
+    std::vector<u64> w((size_t)m->level_words());
+    fill(w.data());
+    HIPC(hipMemcpyAsync(m->level_dom(level), w.data(), sizeof(u64) * w.size(), hipMemcpyHostToDevice, m->stream));
+    hipLaunchKernelGGL(k_sizes, dim3((n + 255) / 256), dim3(256), 0, m->stream, m->level_dom(level),
+                       m->level_size(level), n, W);
+    HIPC(hipGetLastError());
+    m->sync();
+    return;
+  }
+  HostBox* box = m->box();
+  const unsigned long long seq = m->next_seq();
+  fill(reinterpret_cast<u64*>(box->data));
+  hipLaunchKernelGGL(k_level_put, dim3(1), dim3(1024), 0, m->stream, reinterpret_cast<const u64*>(box->data),
+                     m->level_dom(level), m->level_size(level), n, W, &box->seq, seq);
+  HIPC(hipGetLastError());
+  m->wait_box(seq);
 }
 
 }  // namespace
@@ -1084,11 +1204,19 @@ int cpim_gmodel_create_new_level(cpim_gmodel* m, int32_t* new_level) {
       fail(CPIM_ERR_RUNTIME, "[GModel::CreateNewLevel] Max depth reached: " + std::to_string(m->max_depth));
     DeviceGuard g(m->device);
     const int L = ++m->current_level;
-    HIPC(hipMemcpyAsync(m->level_dom(L), m->level_dom(L - 1), sizeof(u64) * m->level_words(),
-                        hipMemcpyDeviceToDevice, m->stream));
-    HIPC(hipMemcpyAsync(m->level_size(L), m->level_size(L - 1), sizeof(int) * m->dm.n,
-                        hipMemcpyDeviceToDevice, m->stream));
-    m->sync();
+    if (m->level_in_box()) {
+      const unsigned long long seq = m->next_seq();
+      hipLaunchKernelGGL(k_level_copy, dim3(1), dim3(1024), 0, m->stream, m->level_dom(L - 1), m->level_dom(L),
+                         m->level_size(L - 1), m->level_size(L), m->dm.n, m->dm.W, &m->box()->seq, seq);
+      HIPC(hipGetLastError());
+      m->wait_box(seq);
+    } else {
+      HIPC(hipMemcpyAsync(m->level_dom(L), m->level_dom(L - 1), sizeof(u64) * m->level_words(),
+                          hipMemcpyDeviceToDevice, m->stream));
+      HIPC(hipMemcpyAsync(m->level_size(L), m->level_size(L - 1), sizeof(int) * m->dm.n, hipMemcpyDeviceToDevice,
+                          m->stream));
+      m->sync();
+    }
     *new_level = L;
   });
 }
@@ -1121,13 +1249,7 @@ int cpim_gmodel_assign_value(cpim_gmodel* m, int32_t var, int32_t value, int32_t
     if (value < 0 || value >= m->dm.max_dom)
       fail(CPIM_ERR_RUNTIME, "[GModel::AssignValue] Invalid value: " + std::to_string(value));
     DeviceGuard g(m->device);
-    std::vector<u64> w(m->dm.W, 0ull);
-    w[value >> 6] = 1ull << (value & 63);
-    const int one = 1;
-    HIPC(hipMemcpyAsync(m->level_dom(level) + (long long)var * m->dm.W, w.data(), sizeof(u64) * m->dm.W,
-                        hipMemcpyHostToDevice, m->stream));
-    HIPC(hipMemcpyAsync(m->level_size(level) + var, &one, sizeof(int), hipMemcpyHostToDevice, m->stream));
-    m->sync();
+    m->level_op(kOpAssign, level, var, value);
     m->assigned[level] = make_int2(var, value);
     m->assigned_size = std::max(m->assigned_size, level + 1);
     *ok = 1;
@@ -1142,17 +1264,7 @@ int cpim_gmodel_remove_value(cpim_gmodel* m, int32_t var, int32_t value, int32_t
     *ok = 0;
     if (value < 0 || value >= m->dm.max_dom) return;
     DeviceGuard g(m->device);
-    std::vector<u64> w = read_var(m, var, level);
-    const u64 bit = 1ull << (value & 63);
-    if (!(w[value >> 6] & bit)) return;
-    w[value >> 6] &= ~bit;
-    int s = 0;
-    for (u64 x : w) s += __builtin_popcountll(x);
-    HIPC(hipMemcpyAsync(m->level_dom(level) + (long long)var * m->dm.W + (value >> 6), &w[value >> 6],
-                        sizeof(u64), hipMemcpyHostToDevice, m->stream));
-    HIPC(hipMemcpyAsync(m->level_size(level) + var, &s, sizeof(int), hipMemcpyHostToDevice, m->stream));
-    m->sync();
-    *ok = s > 0;
+    *ok = m->level_op(kOpRemove, level, var, value) > 0;
   });
 }
 
@@ -1162,7 +1274,7 @@ int cpim_gmodel_domain_size(const cpim_gmodel* m, int32_t var, int32_t level, in
     check_var(m, var, "GetDomainSize");
     check_level(m, level, "GetDomainSize");
     DeviceGuard g(m->device);
-    *size = read_size(m, var, level);
+    *size = m->level_op(kOpSize, level, var, 0);
   });
 }
 
@@ -1171,16 +1283,7 @@ int cpim_gmodel_min_domain_var(const cpim_gmodel* m, int32_t level, int32_t* var
     REQUIRE(m && var, "null argument");
     check_level(m, level, "GetMinDomainVar");
     DeviceGuard g(m->device);
-    std::vector<int> s(m->dm.n);
-    HIPC(hipMemcpyAsync(s.data(), m->level_size(level), sizeof(int) * m->dm.n, hipMemcpyDeviceToHost, m->stream));
-    HIPC(hipStreamSynchronize(m->stream));
-    int best = -1, best_size = m->dm.max_dom + 1;
-    for (int v = 0; v < m->dm.n; ++v)
-      if (s[v] > 1 && s[v] < best_size) {
-        best_size = s[v];
-        best = v;
-      }
-    *var = best;
+    *var = m->level_op(kOpMinVar, level, 0, 0);
   });
 }
 
@@ -1190,7 +1293,7 @@ int cpim_gmodel_is_assigned(const cpim_gmodel* m, int32_t var, int32_t level, in
     check_var(m, var, "IsAssigned");
     check_level(m, level, "IsAssigned");
     DeviceGuard g(m->device);
-    *res = read_size(m, var, level) == 1;
+    *res = m->level_op(kOpSize, level, var, 0) == 1;
   });
 }
 
@@ -1199,23 +1302,8 @@ int cpim_gmodel_is_fully_assigned(const cpim_gmodel* m, int32_t level, int32_t* 
     REQUIRE(m && res, "null argument");
     check_level(m, level, "IsFullyAssigned");
     DeviceGuard g(m->device);
-    std::vector<int> s(m->dm.n);
-    HIPC(hipMemcpyAsync(s.data(), m->level_size(level), sizeof(int) * m->dm.n, hipMemcpyDeviceToHost, m->stream));
-    HIPC(hipStreamSynchronize(m->stream));
-    *res = std::all_of(s.begin(), s.end(), [](int x) { return x == 1; });
+    *res = m->level_op(kOpAll, level, 0, 0);
   });
-}
-
-static int first_from(const std::vector<u64>& w, int start, int max_dom) {
-  for (int a = start; a < 64 * (int)w.size(); ++a) {
-    const u64 word = w[a >> 6] >> (a & 63);
-    if (word) {
-      const int v = a + (int)__builtin_ctzll(word);
-      return v < max_dom ? v : -1;
-    }
-    a |= 63;
-  }
-  return -1;
 }
 
 int cpim_gmodel_assigned_value(const cpim_gmodel* m, int32_t var, int32_t level, int32_t* value) {
@@ -1224,11 +1312,7 @@ int cpim_gmodel_assigned_value(const cpim_gmodel* m, int32_t var, int32_t level,
     check_var(m, var, "GetAssignedValue");
     check_level(m, level, "GetAssignedValue");
     DeviceGuard g(m->device);
-    if (read_size(m, var, level) != 1) {
-      *value = -1;
-      return;
-    }
-    *value = first_from(read_var(m, var, level), 0, m->dm.max_dom);
+    *value = m->level_op(kOpAssigned, level, var, 0);
   });
 }
 
@@ -1238,7 +1322,7 @@ int cpim_gmodel_first_value(const cpim_gmodel* m, int32_t var, int32_t level, in
     check_var(m, var, "GetFirstValue");
     check_level(m, level, "GetFirstValue");
     DeviceGuard g(m->device);
-    *value = first_from(read_var(m, var, level), 0, m->dm.max_dom);
+    *value = m->level_op(kOpFirst, level, var, 0);
   });
 }
 
@@ -1252,7 +1336,7 @@ int cpim_gmodel_next_value(const cpim_gmodel* m, int32_t var, int32_t value, int
       return;
     }
     DeviceGuard g(m->device);
-    *next = first_from(read_var(m, var, level), value + 1, m->dm.max_dom);
+    *next = m->level_op(kOpFirst, level, var, value + 1);
   });
 }
 
@@ -1261,9 +1345,7 @@ int cpim_gmodel_read_domains(const cpim_gmodel* m, int32_t level, uint64_t* out)
     REQUIRE(m && out, "null argument");
     check_level(m, level, "ReadDomains");
     DeviceGuard g(m->device);
-    HIPC(hipMemcpyAsync(out, m->level_dom(level), sizeof(u64) * m->level_words(), hipMemcpyDeviceToHost,
-                        m->stream));
-    HIPC(hipStreamSynchronize(m->stream));
+    read_level(m, level, reinterpret_cast<u64*>(out));
   });
 }
 
@@ -1294,18 +1376,14 @@ int cpim_gmodel_write_domains(cpim_gmodel* m, int32_t level, const uint64_t* in)
     DeviceGuard g(m->device);
     // mask to the domain capacities so that sizes stay exact
     const u64* inw = reinterpret_cast<const u64*>(in);
-    std::vector<u64> w(inw, inw + m->level_words());
-    for (int v = 0; v < m->dm.n; ++v)
-      for (int j = 0; j < m->dm.W; ++j) {
-        const int k = m->im.cap[v] - 64 * j;
-        const u64 mask = k >= 64 ? ~0ull : (k <= 0 ? 0ull : ((1ull << k) - 1ull));
-        w[(long long)v * m->dm.W + j] &= mask;
-      }
-    HIPC(hipMemcpyAsync(m->level_dom(level), w.data(), sizeof(u64) * w.size(), hipMemcpyHostToDevice, m->stream));
-    hipLaunchKernelGGL(k_sizes, dim3((m->dm.n + 255) / 256), dim3(256), 0, m->stream, m->level_dom(level),
-                       m->level_size(level), m->dm.n, m->dm.W);
-    HIPC(hipGetLastError());
-    m->sync();
+    write_level(m, level, [&](u64* w) {
+      for (int v = 0; v < m->dm.n; ++v)
+        for (int j = 0; j < m->dm.W; ++j) {
+          const int k = m->im.cap[v] - 64 * j;
+          const u64 mask = k >= 64 ? ~0ull : (k <= 0 ? 0ull : ((1ull << k) - 1ull));
+          w[(long long)v * m->dm.W + j] = inw[(long long)v * m->dm.W + j] & mask;
+        }
+    });
   });
 }
 
@@ -1758,13 +1836,6 @@ std::vector<int2> all_tests(cpim_gmodel* m, const std::vector<u64>& dom) {
   return t;
 }
 
-std::vector<u64> read_level(cpim_gmodel* m, int level) {
-  std::vector<u64> d(m->level_words());
-  HIPC(hipMemcpyAsync(d.data(), m->level_dom(level), sizeof(u64) * d.size(), hipMemcpyDeviceToHost, m->stream));
-  m->sync();
-  return d;
-}
-
 }  // namespace
 
 extern "C" {
@@ -1828,7 +1899,8 @@ int cpim_gmodel_enforce_sac(cpim_gmodel* m, int32_t mode, cpim_sac_stats* st) {
     }
     SacScratch& S = m->sac;
     while (true) {
-      std::vector<u64> dom = read_level(m, L);
+      std::vector<u64> dom((size_t)m->level_words());
+      read_level(m, L, dom.data());
       std::vector<int2> tests = all_tests(m, dom);
       std::vector<unsigned char> fl(tests.size(), 0);
       run_singleton_device(m, mode, tests.data(), (long long)tests.size(), fl.data(), st, S);
@@ -1849,11 +1921,7 @@ int cpim_gmodel_enforce_sac(cpim_gmodel* m, int32_t mode, cpim_sac_stats* st) {
         for (int w = 0; w < m->dm.W; ++w) any |= dom[(long long)v * m->dm.W + w];
         empty = any == 0;
       }
-      HIPC(hipMemcpyAsync(m->level_dom(L), dom.data(), sizeof(u64) * dom.size(), hipMemcpyHostToDevice, m->stream));
-      hipLaunchKernelGGL(k_sizes, dim3((m->dm.n + 255) / 256), dim3(256), 0, m->stream, m->level_dom(L),
-                         m->level_size(L), m->dm.n, m->dm.W);
-      HIPC(hipGetLastError());
-      m->sync();
+      write_level(m, L, [&](u64* w) { std::memcpy(w, dom.data(), sizeof(u64) * dom.size()); });
       if (empty) {
         st->consistent = 0;
         return;

@@ -205,6 +205,62 @@ __device__ __forceinline__ u64 arcs_unsupported(const DevNet& net, const u64* do
 // (10 rounds, 6,485 removals) 225 -> 151 us, persistent 269 -> 162 us; n=500
 // d=250 e=20000 t=0.963 (5 rounds) 293 -> 188 us, persistent 346 -> 195 us.
 // ===========================================================================
+// Outcome of a fixpoint (or of one of its host-driven rounds).
+struct GacResult {
+  int rounds;           // rounds executed (persistent, one workgroup)
+  int converged;
+  int err;              // the launch's time budget ran out
+  int last_push_round;  // as in GacCtl
+  int wipe_round;       // INT_MAX: no wipe-out
+  int pad;
+  unsigned long long deletions, revisions;
+  unsigned long long ticks;  // device clock ticks of the launch
+};
+
+// Pinned host memory a kernel answers in, so that a call costs one launch and
+// no copies: the kernel stores its result there (system-scope stores, which go
+// through to host memory), waits until they have completed, and stores the
+// call's number in `seq`, on which the host waits.
+struct HostBox {
+  unsigned long long seq;
+  int scalar;
+  int pad;
+  GacResult gac;
+  alignas(64) unsigned long long data[1];  // kBoxDataBytes
+};
+
+__device__ __forceinline__ void box_store(unsigned long long* p, unsigned long long v) {
+  __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+}
+__device__ __forceinline__ void box_store(int* p, int v) {
+  __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+}
+
+__device__ __forceinline__ void wait_memory_ops() {
+  // vmcnt(0); expcnt and lgkmcnt left at their maxima (no wait)
+  __builtin_amdgcn_s_waitcnt(0x0F70);
+}
+
+// Ends a call: every thread of the (single or last) workgroup calls it.
+__device__ __forceinline__ void box_publish(unsigned long long* seq_at, unsigned long long seq) {
+  wait_memory_ops();
+  __syncthreads();
+  if (threadIdx.x == 0 && seq_at) box_store(seq_at, seq);
+}
+
+__device__ __forceinline__ void store_result(GacResult* out, int rounds, int converged, int err, int lp, int wipe,
+                                             unsigned long long dels, unsigned long long revs,
+                                             unsigned long long ticks) {
+  box_store(&out->rounds, rounds);
+  box_store(&out->converged, converged);
+  box_store(&out->err, err);
+  box_store(&out->last_push_round, lp);
+  box_store(&out->wipe_round, wipe);
+  box_store(&out->deletions, dels);
+  box_store(&out->revisions, revs);
+  box_store(&out->ticks, ticks);
+}
+
 // Statistics counters are spread over kStatSlots addresses (by block), and
 // the grid rounds add one workgroup total per round: device-scope atomics on
 // one address serialize, and one from every wave of an 8,192-wave round on
@@ -214,11 +270,10 @@ constexpr int kStatSlots = 256;
 struct GacCtl {
   int last_push_round;  // highest round that changed a domain (host-driven rounds)
   int wipe_round;       // lowest round that emptied a domain
-  int rounds;           // rounds executed (written at the end)
-  int converged;
   unsigned long long bar_ticket;  // grid barrier arrivals so far (only grows)
   int err;              // set by a block whose barrier wait ran out of time
-  int pad;
+  unsigned done;        // blocks that finished
+  unsigned long long start;  // device clock at the start of the launch
   unsigned long long deletions[kStatSlots];
   unsigned long long revisions[kStatSlots];
 };
@@ -383,31 +438,93 @@ __device__ __forceinline__ u64 revise_pairs_w1(const DevNet& net, u64* dom, int*
   return __ballot(removed_l > 0);
 }
 
-// Adds the lanes' removals and the waves' revisions to the grid's totals: one
-// workgroup total per call, on the workgroup's slot.  blk: two LDS words, zero
-// on entry.  Every thread of the workgroup calls it.
-__device__ __forceinline__ void flush_grid_stats(GacCtl* ctl, unsigned long long* blk, int revs, int dels) {
+// LDS of grid_finish.
+struct GridEnd {
+  unsigned long long tot[2];
+  int last;
+};
+
+// End of a grid kernel.  Adds the lanes' removals and the waves' revisions to
+// the grid's totals, one workgroup total on the workgroup's slot; the last
+// workgroup to finish sums the slots, stores the outcome and, when `final` of
+// the epochs says that the fixpoint is over, puts the control block and the
+// bitmaps back to their first state, so that the next fixpoint starts without
+// a launch to clear them.  e->tot: zero on entry.  Every thread calls it.
+template <typename Final>
+__device__ __forceinline__ void grid_finish(GacCtl* ctl, unsigned* F, int nvw, GridEnd* e, int revs, int dels, int rounds,
+                                            int converged, unsigned long long start, Final final, GacResult* out,
+                                            unsigned long long* seq_at, unsigned long long seq) {
+  const int tid = threadIdx.x, lane = lane_id();
   const u64 wave_dels = wave_sum64_dpp((u64)dels);
-  if (lane_id() == 0 && (wave_dels | (u64)revs)) {
-    atomicAdd(&blk[0], (unsigned long long)revs);
-    atomicAdd(&blk[1], wave_dels);
+  if (lane == 0 && (wave_dels | (u64)revs)) {
+    atomicAdd(&e->tot[0], (unsigned long long)revs);
+    atomicAdd(&e->tot[1], wave_dels);
+  }
+  wait_memory_ops();
+  __syncthreads();
+  if (tid == 0) {
+    if (e->tot[0] | e->tot[1]) {
+      atomicAdd(&ctl->revisions[blockIdx.x % kStatSlots], e->tot[0]);
+      atomicAdd(&ctl->deletions[blockIdx.x % kStatSlots], e->tot[1]);
+    }
+    e->tot[0] = 0ull;
+    e->tot[1] = 0ull;
+    wait_memory_ops();
+    const unsigned ticket = atomicAdd(&ctl->done, 1u);
+    e->last = (ticket + 1u) % gridDim.x == 0u ? 1 : 0;
   }
   __syncthreads();
-  if (threadIdx.x == 0 && (blk[0] | blk[1])) {
-    atomicAdd(&ctl->revisions[blockIdx.x % kStatSlots], blk[0]);
-    atomicAdd(&ctl->deletions[blockIdx.x % kStatSlots], blk[1]);
+  if (uniform_int(e->last) == 0) return;
+  u64 r = 0ull, d = 0ull;
+  for (int i = tid; i < kStatSlots; i += blockDim.x) {
+    r += ld_view<true>((const u64*)&ctl->revisions[i]);
+    d += ld_view<true>((const u64*)&ctl->deletions[i]);
   }
+  r = wave_sum64_dpp(r);
+  d = wave_sum64_dpp(d);
+  if (lane == 0) {
+    atomicAdd(&e->tot[0], r);
+    atomicAdd(&e->tot[1], d);
+  }
+  const int lp = uniform_int(ld_agent(&ctl->last_push_round)), wr = uniform_int(ld_agent(&ctl->wipe_round));
+  const int err = uniform_int(ld_agent(&ctl->err));
+  __syncthreads();
+  if (tid == 0)
+    store_result(out, rounds, converged, err, lp, wr, e->tot[1], e->tot[0],
+                 wall_clock64() - (start ? start : ld_view<true>((const u64*)&ctl->start)));
+  if (!err && final(lp, wr)) {
+    for (int i = tid; i < kStatSlots; i += blockDim.x) {
+      ctl->deletions[i] = 0ull;
+      ctl->revisions[i] = 0ull;
+    }
+    for (int i = tid; i < 3 * nvw; i += blockDim.x) F[i] = 0u;
+    if (tid == 0) {
+      ctl->last_push_round = -1;
+      ctl->wipe_round = INT_MAX;
+      ctl->bar_ticket = 0ull;
+      ctl->done = 0u;
+    }
+  }
+  box_publish(seq_at, seq);
 }
 
+constexpr int kRoundThreads = 1024;
+
 // One round per launch (host-driven fixpoint).  A launch queued behind the
-// round that ended the fixpoint does nothing.
-__global__ void k_gac_round(DevNet net, u64* dom, int* size, unsigned* F, int nvw, GacCtl* ctl, int r, int seed,
-                            int narcs) {
-  __shared__ unsigned long long blk[2];
-  if (r > 0 && (ctl->last_push_round < r - 1 || ctl->wipe_round < r)) return;
+// round that ended the fixpoint only answers.
+__global__ void __launch_bounds__(kRoundThreads) k_gac_round(DevNet net, u64* dom, int* size, unsigned* F, int nvw,
+                                                             GacCtl* ctl, int r, int seed, int narcs, GacResult* out,
+                                                             unsigned long long* seq_at, unsigned long long seq) {
+  __shared__ GridEnd end;
+  if (r > 0 && (ctl->last_push_round < r - 1 || ctl->wipe_round < r)) {
+    if (blockIdx.x == 0 && threadIdx.x == 0) box_store(seq_at, seq);
+    return;
+  }
   if (threadIdx.x == 0) {
-    blk[0] = 0ull;
-    blk[1] = 0ull;
+    end.tot[0] = 0ull;
+    end.tot[1] = 0ull;
+    if (blockIdx.x == 0)
+      __hip_atomic_store(&ctl->start, (unsigned long long)wall_clock64(), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
   }
   __syncthreads();
   for (long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x; i < nvw; i += (long long)gridDim.x * blockDim.x)
@@ -417,7 +534,8 @@ __global__ void k_gac_round(DevNet net, u64* dom, int* size, unsigned* F, int nv
                     false, make_int4(0, -1, 0, 0), narcs, revs, dels);
   // the epoch only grows: skip the atomic once another wave has raised it
   if (__ballot(dels > 0) && lane_id() == 0 && ld_agent(&ctl->last_push_round) < r) atomicMax(&ctl->last_push_round, r);
-  flush_grid_stats(ctl, blk, revs, dels);
+  grid_finish(ctl, F, nvw, &end, revs, dels, r + 1, 0, 0ull, [&](int lp, int wr) { return lp < r || wr <= r; }, out,
+              seq_at, seq);
 }
 
 // ===========================================================================
@@ -451,11 +569,6 @@ __global__ void k_gac_round(DevNet net, u64* dom, int* size, unsigned* F, int nv
 // cascade took 1.41 ms, fence-free 1.06 ms.)  The
 // asynchronous fixpoint relies on the same coherence of agent-scope
 // accesses, with no barrier at all.
-__device__ __forceinline__ void wait_memory_ops() {
-  // vmcnt(0); expcnt and lgkmcnt left at their maxima (no wait)
-  __builtin_amdgcn_s_waitcnt(0x0F70);
-}
-
 // Returns false when the launch's budget ran out here or elsewhere.
 __device__ __forceinline__ bool grid_barrier(GacCtl* ctl, unsigned nblocks, unsigned long long t0,
                                              unsigned long long max_ticks, int* s_ok) {
@@ -502,13 +615,15 @@ __host__ __device__ inline long long persistent_lds_bytes(int n, int W) {
 template <bool kStaged>
 __global__ void __launch_bounds__(kPersistentThreads) k_gac_persistent(DevNet net, u64* dom, int* size, unsigned* F,
                                                                        int nvw, GacCtl* ctl, int max_rounds, int seed,
-                                                                       int narcs, unsigned long long max_ticks) {
+                                                                       int narcs, unsigned long long max_ticks,
+                                                                       GacResult* out, unsigned long long* seq_at,
+                                                                       unsigned long long seq) {
   extern __shared__ __align__(16) char smem[];
   __shared__ int s_ok;
-  __shared__ unsigned long long blk[2];
+  __shared__ GridEnd end;
   if (threadIdx.x == 0) {
-    blk[0] = 0ull;
-    blk[1] = 0ull;
+    end.tot[0] = 0ull;
+    end.tot[1] = 0ull;
   }
   __syncthreads();
   const unsigned long long t0 = wall_clock64();
@@ -552,24 +667,21 @@ __global__ void __launch_bounds__(kPersistentThreads) k_gac_persistent(DevNet ne
     else if (!any) decision = FIXPOINT;
     if (decision != NEXT || r >= max_rounds) break;
   }
-  flush_grid_stats(ctl, blk, revs, dels);
-  if (blockIdx.x == 0 && tid == 0) {
-    ctl->rounds = r;
-    ctl->converged = decision == FIXPOINT ? 1 : 0;
-  }
+  grid_finish(ctl, F, nvw, &end, revs, dels, r, decision == FIXPOINT ? 1 : 0, t0, [](int, int) { return true; }, out,
+              seq_at, seq);
 }
 
-// Start of a grid fixpoint: the control block and the three bitmaps cleared.
+// First state of a grid fixpoint's control block and bitmaps (kept from one
+// fixpoint to the next by grid_finish, but for one that ended in an error).
 __global__ void k_gac_init(GacCtl* ctl, unsigned* F, int nvw) {
   const long long i0 = (long long)blockIdx.x * blockDim.x + threadIdx.x;
   if (i0 == 0) {
     ctl->last_push_round = -1;
     ctl->wipe_round = INT_MAX;
-    ctl->rounds = 0;
-    ctl->converged = 0;
     ctl->bar_ticket = 0ull;
     ctl->err = 0;
-    ctl->pad = 0;
+    ctl->done = 0u;
+    ctl->start = 0ull;
   }
   for (long long i = i0; i < kStatSlots; i += (long long)gridDim.x * blockDim.x) {
     ctl->deletions[i] = 0ull;
@@ -1253,16 +1365,10 @@ __device__ __forceinline__ u64 wg_reduce_sum_u64(WgCtl* ctl, u64 v) {
 // ---------------------------------------------------------------------------
 // Block-mode GAC on one level (one workgroup).
 // ---------------------------------------------------------------------------
-struct BlockGacOut {
-  int consistent;
-  int rounds;
-  unsigned long long revisions;
-  long long deletions;
-};
-
 template <bool kLds>
 __global__ void k_block_gac(DevNet net, u64* dom, int* size, int seed_var, char* scratch,
-                            BlockGacOut* out) {
+                            GacResult* out, unsigned long long* seq_at, unsigned long long seq) {
+  const unsigned long long t0 = wall_clock64();
   extern __shared__ __align__(16) char smem[];
   __shared__ WgCtl ctl;
   const int n = net.n, W = net.W;
@@ -1282,11 +1388,102 @@ __global__ void k_block_gac(DevNet net, u64* dom, int* size, int seed_var, char*
   const u64 delta = wg_reduce_sum_u64(&ctl, (u64)(before - after));
   wg_copy_words(dom, mem.dom, (long long)n * W);
   for (int v = threadIdx.x; v < n; v += blockDim.x) size[v] = mem.size[v];
-  if (threadIdx.x == 0) {
-    out->consistent = ok;
-    out->revisions = ctl.revs;
-    out->deletions = (long long)delta;
+  if (threadIdx.x == 0)
+    store_result(out, 1, ok ? 1 : 0, 0, 0, ok ? INT_MAX : 0, delta, ctl.revs, wall_clock64() - t0);
+  box_publish(seq_at, seq);
+}
+
+// ---------------------------------------------------------------------------
+// Level operations, one workgroup each, answering in the host box: one launch
+// a call (a call took a copy each way through the runtime's staging memory,
+// three kernels and a stream synchronization).
+// ---------------------------------------------------------------------------
+__global__ void k_level_put(const u64* src, u64* dom, int* size, int n, int W, unsigned long long* seq_at,
+                            unsigned long long seq) {
+  for (int v = threadIdx.x; v < n; v += blockDim.x) {
+    int s = 0;
+    for (int w = 0; w < W; ++w) {
+      const u64 d = __hip_atomic_load(const_cast<u64*>(&src[(long long)v * W + w]), __ATOMIC_RELAXED,
+                                      __HIP_MEMORY_SCOPE_SYSTEM);
+      dom[(long long)v * W + w] = d;
+      s += __popcll(d);
+    }
+    size[v] = s;
   }
+  box_publish(seq_at, seq);
+}
+
+__global__ void k_level_get(const u64* dom, unsigned long long* dst, int words, unsigned long long* seq_at,
+                            unsigned long long seq) {
+  for (int i = threadIdx.x; i < words; i += blockDim.x) box_store(&dst[i], dom[i]);
+  box_publish(seq_at, seq);
+}
+
+__global__ void k_level_copy(const u64* src, u64* dst, const int* src_size, int* dst_size, int n, int W,
+                             unsigned long long* seq_at, unsigned long long seq) {
+  for (int i = threadIdx.x; i < n * W; i += blockDim.x) dst[i] = src[i];
+  for (int i = threadIdx.x; i < n; i += blockDim.x) dst_size[i] = src_size[i];
+  box_publish(seq_at, seq);
+}
+
+enum LevelOp {
+  kOpAssign,    // D(var) = {value}
+  kOpRemove,    // D(var) -= {value}; answers the new size, -1 if the value was not there
+  kOpSize,      // |D(var)|
+  kOpFirst,     // smallest value >= value of D(var), -1 if none
+  kOpAssigned,  // the value of an assigned variable, -1 otherwise
+  kOpMinVar,    // variable with the smallest |D| > 1, the lowest id on ties; -1 if none
+  kOpAll        // 1: every variable is assigned
+};
+
+__global__ void __launch_bounds__(256) k_level_op(int op, u64* dom, int* size, int n, int W, int max_dom, int var,
+                                                  int value, int* answer, unsigned long long* seq_at,
+                                                  unsigned long long seq) {
+  __shared__ u64 red[4];
+  const int tid = threadIdx.x;
+  u64* d = dom + (long long)var * W;
+  int res = 0;
+  if (op == kOpMinVar || op == kOpAll) {
+    u64 key = ~0ull;
+    for (int v = tid; v < n; v += 256) {
+      const int s = size[v];
+      const u64 k = op == kOpAll ? (u64)(s == 1) : (s > 1 ? ((u64)(unsigned)s << 32) | (unsigned)v : ~0ull);
+      key = k < key ? k : key;
+    }
+    key = wave_min64_dpp(key);
+    if (lane_id() == 0) red[tid >> 6] = key;
+    __syncthreads();
+    for (int i = 0; i < 4; ++i) key = red[i] < key ? red[i] : key;
+    res = op == kOpAll ? (int)(key & 1ull) : (key == ~0ull ? -1 : (int)(unsigned)key);
+  } else if (tid == 0) {
+    if (op == kOpAssign) {
+      for (int w = 0; w < W; ++w) d[w] = w == (value >> 6) ? 1ull << (value & 63) : 0ull;
+      size[var] = 1;
+    } else if (op == kOpRemove) {
+      const u64 bit = 1ull << (value & 63);
+      res = -1;
+      if (d[value >> 6] & bit) {
+        d[value >> 6] &= ~bit;
+        res = 0;
+        for (int w = 0; w < W; ++w) res += __popcll(d[w]);
+        size[var] = res;
+      }
+    } else if (op == kOpSize) {
+      res = size[var];
+    } else {
+      const int start = op == kOpAssigned ? 0 : value;
+      res = -1;
+      if (op == kOpFirst || size[var] == 1)
+        for (int w = start >> 6; w < W && res < 0; ++w) {
+          u64 x = d[w];
+          if (w == start >> 6) x &= ~0ull << (start & 63);
+          if (x) res = 64 * w + (int)__builtin_ctzll(x);
+        }
+      if (res >= max_dom) res = -1;
+    }
+  }
+  if (tid == 0) box_store(answer, res);
+  box_publish(seq_at, seq);
 }
 
 // ---------------------------------------------------------------------------

@@ -149,7 +149,7 @@ class GModel:
                         st.revisions, st.kernel_ms)
 
     def EnforceGAC(self, verbose: bool = True, assigned_var: int = -1) -> GacStats:
-        """Host-driven rounds (one launch + sync per round), like the reference."""
+        """Host-driven rounds (one launch per round), like the reference."""
         st = self._gac(assigned_var, N.CPIM_GAC_PLAIN)
         if verbose:
             print(f"[GAC-Bitmap] iterations={st.iterations} deletions={st.deletions} "

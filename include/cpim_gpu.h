@@ -139,9 +139,9 @@ int cpim_gmodel_get_info(const cpim_gmodel* model, cpim_gmodel_info* out);
 
 /* GacStats (include/GModel.cuh:17-21).  deletions is the popcount delta of
  * the level (never double counted).  revisions counts executed arc revisions.
- * kernel_ms is the device time of the fixpoint's kernels, measured with HIP
- * events on the model's stream (summed over the rounds of host-driven rounds,
- * so the host round trips between them are not in it). */
+ * kernel_ms is the device time of the fixpoint's kernels by the device clock
+ * (asynchronous mode: HIP events), summed over the rounds of host-driven
+ * rounds, so the host round trips between them are not in it. */
 typedef struct cpim_gac_stats {
   int32_t iterations;
   int32_t deletions;
@@ -151,7 +151,8 @@ typedef struct cpim_gac_stats {
   double kernel_ms;
 } cpim_gac_stats;
 
-#define CPIM_GAC_PLAIN 0      /* host-driven rounds, one launch + sync per round */
+#define CPIM_GAC_PLAIN 0      /* host-driven rounds, one launch per round; the host looks at the outcome
+                                 after 1, 2, 4 and then every 8 rounds */
 #define CPIM_GAC_PERSISTENT 1 /* all rounds in one launch of co-resident workgroups, a grid
                                  barrier between rounds; every barrier wait is bounded by the
                                  fixpoint_budget_us knob (CPIM_ERR_RUNTIME when it runs out) */
