@@ -679,25 +679,21 @@ struct cpim_gmodel {
   hipEvent_t gev[2] = {nullptr, nullptr};  // kernel timing of the fixpoint entry points
   // dom/wdeg bookkeeping of the network (Tabular::weight, Network.cpp:303):
   // weights start at 1 with the model and persist across solves, as the
-  // reference's constraint weights do; the stamps and clock order AC3's
-  // revisions across calls
-  DevAlloc wdeg_weight, wdeg_stamp, wdeg_clock;
+  // reference's constraint weights do; the stamps order AC3's revisions
+  // within a call (in LDS where they fit)
+  DevAlloc wdeg_weight, wdeg_stamp;
 
-  // the weights, stamps and clock, allocated and set to their first values on
-  // first use or on reset
+  // the weights (and room for the stamps), allocated on first use, and the
+  // weights set to 1, on first use or on reset
   void wdeg_init() {
     const int nc = std::max(1, dm.num_active);
     if (!wdeg_weight.p) {
       wdeg_weight = DevAlloc(sizeof(float) * nc);
-      wdeg_stamp = DevAlloc(sizeof(long long) * nc);
-      wdeg_clock = DevAlloc(sizeof(long long));
+      wdeg_stamp = DevAlloc(sizeof(int) * nc);
     }
     const std::vector<float> ones(nc, 1.0f);
-    const long long one = 1;
     HIPC(hipMemcpyAsync(wdeg_weight.p, ones.data(), sizeof(float) * nc, hipMemcpyHostToDevice, stream));
-    HIPC(hipMemsetAsync(wdeg_stamp.p, 0, sizeof(long long) * nc, stream));
-    HIPC(hipMemcpyAsync(wdeg_clock.p, &one, sizeof(one), hipMemcpyHostToDevice, stream));
-    HIPC(hipStreamSynchronize(stream));  // `ones` and `one` are host stack memory
+    HIPC(hipStreamSynchronize(stream));  // `ones` is host stack memory
   }
 
   // The box and the number of the next call that answers in it.
@@ -1987,8 +1983,7 @@ int cpim_gmodel_solve(cpim_gmodel* m, const cpim_solve_opts* opts, cpim_search_s
     if (o.var_heuristic == CPIM_VARH_DOM_WDEG) {
       if (!m->wdeg_weight.p) m->wdeg_init();
       A.weight = m->wdeg_weight.as<float>();
-      A.stamp_tab = m->wdeg_stamp.as<long long>();
-      A.clock = m->wdeg_clock.as<long long>();
+      A.stamp_tab = m->wdeg_stamp.as<int>();
     }
     DevNet net = m->dm.net();
     const long long bytes = wg_mem_bytes(n, m->dm.W);
@@ -2007,13 +2002,17 @@ int cpim_gmodel_solve(cpim_gmodel* m, const cpim_solve_opts* opts, cpim_search_s
     if (knob("mac_lds_net") == 0 && m->dm.lnet.bytes > 0 &&
         bytes + m->dm.lnet.bytes <= (long long)m->props.max_lds - 2048)
       lnet = m->dm.lnet;
+    const bool lds = bytes <= kLdsBudget;
+    long long dyn = lds ? bytes + lnet.bytes : 0;
+    if (A.weight && dyn + 16 + 4ll * m->dm.num_active <= (long long)m->props.max_lds - 2048) {
+      A.stamp_off = (int)std::max(16ll, dyn);  // 0 means memory
+      dyn = A.stamp_off + 4ll * m->dm.num_active;
+    }
     while (true) {
-      const bool lds = bytes <= kLdsBudget;
       char* scratch = lds ? nullptr : m->get_scratch(bytes);
-      const size_t dyn = lds ? (size_t)(bytes + lnet.bytes) : 0;
       auto* kernel = lds ? (A.weight ? k_mac<true, true> : k_mac<true, false>)
                          : (A.weight ? k_mac<false, true> : k_mac<false, false>);
-      hipLaunchKernelGGL(kernel, dim3(1), dim3(threads), dyn, m->stream, net, A, scratch, lds ? lnet : LdsNet{});
+      hipLaunchKernelGGL(kernel, dim3(1), dim3(threads), (size_t)dyn, m->stream, net, A, scratch, lds ? lnet : LdsNet{});
       HIPC(hipGetLastError());
       HIPC(hipMemcpyAsync(&s, state.p, sizeof(s), hipMemcpyDeviceToHost, m->stream));
       m->sync();

@@ -924,6 +924,7 @@ struct WgMem {
   int* size;      // [n]
   unsigned* bm;   // [3][nvw] frontier bitmaps, rotating by round
   unsigned* asg;  // [nvw]
+  int* stamp;     // [ncons] constraint stamps (dom/wdeg), NULL otherwise
   const int* aoff;   // adjacency offsets (net.adj_off)
   const int4* adj;   // adjacency entries (net.adj)
 };
@@ -950,6 +951,7 @@ __device__ __forceinline__ WgMem wg_carve(char* base, const DevNet& net) {
   const int n = net.n, W = net.W;
   const int nvw = (n + 31) / 32;
   WgMem m;
+  m.stamp = nullptr;
   m.aoff = net.adj_off;
   m.adj = net.adj;
   m.dom = (u64*)base;
@@ -2638,11 +2640,11 @@ struct MacArgs {
   u64 deadline;           // wall_clock64 ticks (0 = none)
   u64* root_out;          // [n][W] root-fixpoint domains, or NULL
   const int* nbr;         // [n] neighbour counts: dom/deg ordering; NULL = dom-min
-  // dom/wdeg ordering (all NULL otherwise); fixpoints then follow AC3's
-  // schedule so that the weights grow as the reference's do
+  // dom/wdeg ordering (all NULL otherwise); wipe-outs are then repeated in
+  // AC3's schedule so that the weights grow as the reference's do
   float* weight;          // [ncons] constraint weights, start at 1
-  long long* stamp_tab;   // [ncons] constraint stamps (absolute times), start at 0
-  long long* clock;       // [1] stamp clock, starts at 1
+  int* stamp_tab;         // [ncons] constraint stamps, where they do not go in LDS
+  int stamp_off;          // byte offset of the constraint stamps in dynamic LDS, 0 = stamp_tab
 };
 
 enum { MAC_INIT = 0, MAC_RUNNING = 1, MAC_SAT = 2, MAC_UNSAT = 3, MAC_LIMIT = 4 };
@@ -2681,11 +2683,8 @@ __device__ __forceinline__ void wg_trace(const DevNet& net, const WgMem& mem, co
 //
 // The queue (ring of n + 1), the queued flags and the variable stamps use
 // pre, the second frontier bitmap and list, which this schedule does not
-// otherwise need.  Variable stamps restart at 0 on each call, as in the
-// reference.  Constraint stamps stay in global memory as absolute times: a
-// call starts at time base = *clock, reads a stamp s as s - base when
-// s > base and as 0 otherwise (the reference's reset to 0, without touching
-// every constraint), and leaves *clock past its last stamp.
+// otherwise need.  Variable and constraint stamps restart at 0 on each call,
+// as in the reference; the constraint stamps lie in LDS where they fit.
 // Lane 0 does every load and store of the control state and broadcasts what
 // it read, so the same code is correct whether the arrays are in LDS or in
 // global scratch; control values are wave-uniform.
@@ -2695,15 +2694,28 @@ __device__ __forceinline__ void wg_trace(const DevNet& net, const WgMem& mem, co
 // distinct and D(x) is fixed until a revision takes values of x, so the
 // revisions are independent and are all computed from the state before the
 // first; they are then committed in list order (queue positions and stamps
-// from the lanes' ranks) up to the first that takes values of x, which runs
-// by itself, or the first wipe-out, whose constraint gains the weight.  One
-// after another they cost about 1.5 us each, a chain of dependent reads.
-// seed: one variable, or -1 for all variables in id order.
+// from the lanes' ranks) up to the first that takes values of x, or the first
+// wipe-out, whose constraint gains the weight.  One after another they cost
+// about 3.5 us each, a chain of dependent reads; a batch costs about 3.2 us.
+// 100 nodes of 100 variables (domains of 50, 742 constraints) took 11.1 ms
+// with the constraint that takes values of x revised by itself after its
+// batch, and 7.3 ms with it committed as the batch's last.
 // ---------------------------------------------------------------------------
 __device__ __forceinline__ int lane0_load(const int* p) {
   int v = 0;
   if (lane_id() == 0) v = *p;
   return __builtin_amdgcn_readlane(v, 0);
+}
+
+typedef int v4i __attribute__((ext_vector_type(4)));
+
+// Adjacency entry k of a list that ends at k1; no arc past the end.  (A plain
+// vector: the runtime's int4 class goes through scratch memory when a value is
+// chosen between two.)
+__device__ __forceinline__ v4i load_arc(const int4* adj, int k, int k1) {
+  v4i e = {0, -1, 0, 0};
+  if (k < k1) e = *(const v4i*)(adj + k);
+  return e;
 }
 
 __device__ __forceinline__ bool wave_ac3(const DevNet& net, WgMem mem, const MacArgs& A, int seed,
@@ -2715,9 +2727,6 @@ __device__ __forceinline__ bool wave_ac3(const DevNet& net, WgMem mem, const Mac
   int* q = mem.pre;
   unsigned* inq = mem.bm + nvw;
   int* sv = mem.list;
-  long long base = 0;
-  if (lane == 0) base = *A.clock;
-  base = (long long)readlane64((u64)base, 0);
   int front = 0, rear = 0, t = 0;
   if (seed >= 0) {
     for (int v = lane; v < n; v += 64) sv[v] = 0;
@@ -2756,33 +2765,48 @@ __device__ __forceinline__ bool wave_ac3(const DevNet& net, WgMem mem, const Mac
   while ((1 << lw) < W) ++lw;
   const int w = lane & ((1 << lw) - 1), la = lane >> lw, per = 64 >> lw;
   const long long pair_words = 2ll * W * net.dpad;
-  // pred in some lane of this lane's arc, as a mask with one bit per arc (bit 0 of its lanes)
+  // pred in some lane of an arc, as a mask with one bit per arc (bit 0 of its lanes)
+  u64 arc_bits = 1ull;
+  for (int d = 1 << lw; d < 64; d <<= 1) arc_bits |= arc_bits << d;
   auto arcs_with = [&](bool pred) -> u64 {
     u64 m = __ballot(pred);
     for (int d = (1 << lw) >> 1; d > 0; d >>= 1) m |= m >> d;
-    u64 first = 1ull;
-    for (int d = 1 << lw; d < 64; d <<= 1) first |= first << d;
-    return m & first;
+    return m & arc_bits;
   };
+  int next_x = -1, next_k0 = 0, next_k1 = 0;
+  v4i next_e = {0, -1, 0, 0};
   while (ok && front != rear) {
     const int x = lane0_load(&q[front]);
     front = front + 1 == qcap ? 0 : front + 1;
     if (lane == 0) inq[x >> 5] &= ~(1u << (x & 31));
-    const int k1 = uniform_int(mem.aoff[x + 1]);
+    // x's constraints; those of the next variable in the queue, if there is
+    // one, are read ahead
+    const bool read_ahead = x == next_x;
+    const int k0 = read_ahead ? next_k0 : uniform_int(mem.aoff[x]);
+    const int k1 = read_ahead ? next_k1 : uniform_int(mem.aoff[x + 1]);
+    v4i first_e = next_e;
+    if (!read_ahead) first_e = load_arc(mem.adj, k0 + la, k1);
+    next_x = -1;
+    if (net.simple && front != rear) {
+      next_x = lane0_load(&q[front]);
+      next_k0 = uniform_int(mem.aoff[next_x]);
+      next_k1 = uniform_int(mem.aoff[next_x + 1]);
+      next_e = load_arc(mem.adj, next_k0 + la, next_k1);
+    }
     const bool asgx = uniform_int((int)bit_of(mem.asg, x)) != 0;
-    for (int k = uniform_int(mem.aoff[x]); k < k1; ++k) {
+    for (int k = k0; k < k1; ++k) {
       if (net.simple) {
         // the constraints k .. k + per - 1 at once, from the state before the
-        // first of them: exact up to the first one that takes values of x
-        // (the later ones then see another D(x)), the first table and the
-        // first wipe-out
+        // first of them: exact up to and with the first one that takes values
+        // of x (the later ones then see another D(x)), before the first table,
+        // and up to the first wipe-out
         const bool in = k + la < k1 && la < per && w < W;
-        const int4 e = in ? mem.adj[k + la] : make_int4(0, -1, 0, 0);
+        v4i e = first_e;
+        if (k != k0) e = load_arc(mem.adj, k + la, k1);
         const bool table = in && e.y < 0;
         const int y = in && !table ? e.y : x;
-        const int px = adj_pos(e);
-        const long long sc = in ? A.stamp_tab[e.x] : 0ll;
-        const int stc = sc > base ? (int)(sc - base) : 0;
+        const int px = (e.z & 15);
+        const int stc = in ? ld_wg_int(&mem.stamp[e.x]) : 0;
         const int svx = ld_wg_int(&sv[x]), svy = ld_wg_int(&sv[y]);
         u64* ydom = mem.dom + (long long)y * W + w;
         const u64 dy = in && !table ? ld_wg(ydom) : 0ull;
@@ -2794,64 +2818,80 @@ __device__ __forceinline__ bool wave_ac3(const DevNet& net, WgMem mem, const Mac
                                                  net.sup + off + (long long)(1 - px) * W * net.dpad + 64 * w, need);
         const int bit0 = la << lw;
         const u64 lose = arcs_with(gone != 0ull);
-        const u64 wipe = lose & ~arcs_with((need & ~gone) != 0ull);
+        const u64 wipe_y = lose & ~arcs_with((need & ~gone) != 0ull);
         const bool mine_lose = (lose >> bit0) & 1ull;
         // x <- y: when y changed since the constraint's stamp, or lost values
-        // just now; those had no support in D(x), so the old D(y) decides the same
-        const bool xrev = act && !asgx && (svy > stc || (px == 1 && mine_lose && !((wipe >> bit0) & 1ull)));
-        const u64 xgone = arcs_unsupported<false, false>(net, mem.dom, off, y, 1 - px, in ? w : 0,
-                                           xrev ? ld_wg(&mem.dom[(long long)x * W + w]) : 0ull);
-        const u64 xlose = arcs_with(xgone != 0ull), tabs = arcs_with(table);
-        const u64 acts = arcs_with(act);
-        // lanes of the arcs that can be committed
-        const u64 halt = xlose | tabs;
-        const int stop = min((int)(halt ? __builtin_ctzll(halt) : 64), (int)(wipe ? __builtin_ctzll(wipe) : 64));
-        const bool wiped = wipe && stop == (int)__builtin_ctzll(wipe) && !((halt >> (stop & 63)) & 1ull);
-        const u64 before = stop >= 64 ? ~0ull : (1ull << stop) - 1ull;
+        // just now.  Neither direction sees the other's removals: a value
+        // removed for want of a support supported nothing there.
+        const bool xrev = act && !asgx && (svy > stc || (px == 1 && mine_lose && !((wipe_y >> bit0) & 1ull)));
+        const u64 dx = xrev ? ld_wg(&mem.dom[(long long)x * W + w]) : 0ull;
+        const u64 xgone = arcs_unsupported<false, false>(net, mem.dom, off, y, 1 - px, in ? w : 0, dx);
+        const u64 xlose = arcs_with(xgone != 0ull), tabs = arcs_with(table), acts = arcs_with(act);
+        const u64 wipe = wipe_y | (xlose & ~arcs_with((dx & ~xgone) != 0ull));
+        const u64 halt = xlose | tabs | wipe;
+        const int stop = halt ? (int)__builtin_ctzll(halt) : 64;  // bit of the arc that ends the batch
+        const u64 at = stop < 64 ? 1ull << stop : 0ull;
+        const bool wiped = (wipe & at) != 0ull, last = !wiped && (xlose & at) != 0ull;
+        // the arcs before it are committed, and that arc itself but for a table
+        const u64 before = stop >= 64 ? ~0ull : (at - 1ull) | (tabs & at ? 0ull : at);
         const u64 done = acts & before, ins = lose & before;
         const bool commit = act && ((before >> bit0) & 1ull);
-        if ((commit || (wiped && bit0 == stop)) && gone) {
+        const bool mine_last = last && bit0 == stop;
+        if (commit && gone) {
           (void)and_wg(ydom, ~gone);
           atomicSub(&mem.size[y], __popcll(gone));
         }
-        nrev += __popcll(arcs_with(yrev && (commit || (wiped && bit0 == stop))));
-        nrev += __popcll(arcs_with(xrev && commit));
-        const u64 below = (1ull << bit0) - 1ull;
-        const int t0 = t + __popcll(done & below) + __popcll(ins & below);
-        if (commit && w == 0) {
-          A.stamp_tab[e.x] = base + t0 + (mine_lose ? 2 : 1);
-          if (mine_lose) __hip_atomic_store(&sv[y], t0 + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+        if (mine_last && xgone) {
+          (void)and_wg(&mem.dom[(long long)x * W + w], ~xgone);
+          atomicSub(&mem.size[x], __popcll(xgone));
         }
-        const bool queued = (ld_wg_int((const int*)&inq[y >> 5]) >> (y & 31)) & 1;
-        const u64 add = arcs_with(commit && mine_lose && !queued);
-        if (commit && mine_lose && !queued && w == 0) {
-          int at = rear + __popcll(add & below);
-          at = at >= qcap ? at - qcap : at;
-          __hip_atomic_store(&q[at], y, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
-          atomicOr(&inq[y >> 5], 1u << (y & 31));
-        }
-        rear += __popcll(add);
-        rear = rear >= qcap ? rear - qcap : rear;
-        t += __popcll(done) + __popcll(ins);
-        __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "workgroup");
+        // (a wipe-out ends its constraint with the first of the two revisions)
+        const bool counted = commit && !(wiped && bit0 == stop);
+        nrev += __popcll(arcs_with(yrev && counted)) + __popcll(arcs_with(xrev && counted)) + (wiped ? 1 : 0);
         if (wiped) {
           const int cw = __builtin_amdgcn_readlane(e.x, stop);
           if (lane == 0) A.weight[cw] += 1.0f;
           ok = false;
           break;
         }
-        k += stop >= 64 ? per : (stop >> lw);
-        if (stop >= 64 || k >= k1) {
+        // times: an arc's removals, then its stamp; of the last arc, the first
+        // position's variable first
+        const u64 below = (1ull << bit0) - 1ull;
+        const int t0 = t + __popcll(done & below) + __popcll(ins & below);
+        const int y_late = mine_last && px == 0 ? 1 : 0, x_late = mine_last && px == 1 && mine_lose ? 1 : 0;
+        if (commit && w == 0) {
+          __hip_atomic_store(&mem.stamp[e.x], t0 + 1 + (mine_lose ? 1 : 0) + (mine_last ? 1 : 0), __ATOMIC_RELAXED,
+                             __HIP_MEMORY_SCOPE_WORKGROUP);
+          if (mine_lose) __hip_atomic_store(&sv[y], t0 + 1 + y_late, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+          if (mine_last) __hip_atomic_store(&sv[x], t0 + 1 + x_late, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+        }
+        const bool queued = (ld_wg_int((const int*)&inq[y >> 5]) >> (y & 31)) & 1;
+        const bool xqueued = (ld_wg_int((const int*)&inq[x >> 5]) >> (x & 31)) & 1;
+        const u64 add = arcs_with(commit && mine_lose && !queued);
+        const int xadd = last && !xqueued ? 1 : 0;
+        auto put = [&](int rank, int v) {
+          int pos = rear + rank;
+          pos = pos >= qcap ? pos - qcap : pos;
+          __hip_atomic_store(&q[pos], v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+          atomicOr(&inq[v >> 5], 1u << (v & 31));
+        };
+        const int rank = __popcll(add & below);
+        if (commit && mine_lose && !queued && w == 0) put(rank + (y_late && xadd ? 1 : 0), y);
+        if (mine_last && xadd && w == 0) put(rank + (x_late && ((add >> bit0) & 1ull) ? 1 : 0), x);
+        const int adds = __popcll(add) + (int)uniform_int(xadd);
+        rear += adds;
+        rear = rear >= qcap ? rear - qcap : rear;
+        t += __popcll(done) + __popcll(ins) + (last ? 1 : 0);
+        __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "workgroup");
+        k += stop >= 64 ? per : (stop >> lw) + (last ? 1 : 0);
+        if (stop >= 64 || last || k >= k1) {
           --k;
           continue;
         }
-        // constraint k takes values of x, or is a table: by itself
+        // constraint k is a table: by itself
       }
       const int c = uniform_int(mem.adj[k].x);
-      long long sc = 0;
-      if (lane == 0) sc = A.stamp_tab[c];
-      sc = (long long)readlane64((u64)sc, 0);
-      const int stc = sc > base ? (int)(sc - base) : 0;
+      const int stc = lane0_load(&mem.stamp[c]);
       if (!(lane0_load(&sv[x]) > stc)) continue;
       const ConMeta* mp = net.con + c;
       const int arity = mp->arity;
@@ -2883,10 +2923,9 @@ __device__ __forceinline__ bool wave_ac3(const DevNet& net, WgMem mem, const Mac
       }
       if (!ok) break;
       ++t;
-      if (lane == 0) A.stamp_tab[c] = base + t;
+      if (lane == 0) mem.stamp[c] = t;
     }
   }
-  if (lane == 0) *A.clock = base + t + 1;
   *revs += nrev;
   return ok;
 }
@@ -2894,6 +2933,7 @@ __device__ __forceinline__ bool wave_ac3(const DevNet& net, WgMem mem, const Mac
 // AC3-scheduled fixpoint for the whole workgroup: wave 0 runs it, the other
 // waves wait at the barrier.
 __device__ __forceinline__ bool wg_ac3(const DevNet& net, WgMem mem, WgCtl* ctl, const MacArgs& A, int seed) {
+  for (int i = threadIdx.x; i < net.ncons; i += blockDim.x) mem.stamp[i] = 0;
   __syncthreads();
   if (threadIdx.x < 64) {
     unsigned long long revs = 0;
@@ -2912,16 +2952,19 @@ __device__ __forceinline__ bool wg_ac3(const DevNet& net, WgMem mem, WgCtl* ctl,
 // undecided variable; key = -1 when |D(x)| = 1 or x_w = 0, else |D(x)| / x_w
 // in double (IEEE division, as on the host); the lowest id among the smallest
 // keys.  Non-negative doubles order as their bit patterns, -1 maps to 0.
-__device__ __forceinline__ int wg_select_wdeg(const DevNet& net, WgMem mem, WgCtl* ctl, const MacArgs& A) {
-  const int n = net.n;
+// A row of 16 lanes sums the weights of one variable's constraints (whole
+// numbers, so the sum is exact in any order).
+__device__ __forceinline__ int wg_select_wdeg(const DevNet& net, const WgMem& mem, WgCtl* ctl, const MacArgs& A) {
+  const int n = net.n, row = threadIdx.x >> 4, rows = blockDim.x >> 4, l = threadIdx.x & 15;
   u64 best = ~0ull;
   int bv = n;
-  for (int v = threadIdx.x; v < n; v += blockDim.x) {
-    if (bit_of(mem.asg, v)) continue;
-    double xw = 0.0;
-    const int k1 = mem.aoff[v + 1];
-    for (int k = mem.aoff[v]; k < k1; ++k) {
+  for (int v = row; v < n; v += rows) {
+    const bool open = !bit_of(mem.asg, v);
+    u64 sum = 0ull;
+    const int k1 = open ? mem.aoff[v + 1] : 0;
+    for (int k = open ? mem.aoff[v] + l : 0; k < k1; k += 16) {
       const int4 e = mem.adj[k];
+      const float weight = A.weight[e.x];
       int cnt = 0;
       if (e.y >= 0) {
         cnt = 1 + (bit_of(mem.asg, e.y) ? 0 : 1);
@@ -2929,8 +2972,14 @@ __device__ __forceinline__ int wg_select_wdeg(const DevNet& net, WgMem mem, WgCt
         const ConMeta* mp = net.con + e.x;
         for (int i = 0; i < mp->arity; ++i) cnt += bit_of(mem.asg, mp->scope[i]) ? 0 : 1;
       }
-      if (cnt > 1) xw += (double)A.weight[e.x];
+      if (cnt > 1) sum += (u64)weight;
     }
+    sum += dpp_ror_u64_1(sum);
+    sum += dpp_ror_u64_2(sum);
+    sum += dpp_ror_u64_4(sum);
+    sum += dpp_ror_u64_8(sum);
+    if (!open) continue;
+    const double xw = (double)sum;
     const int sz = mem.size[v];
     const double key = (sz == 1 || xw == 0.0) ? -1.0 : (double)sz / xw;
     const u64 k = key < 0.0 ? 0ull : (u64)__double_as_longlong(key);
@@ -3154,12 +3203,17 @@ template <bool kLds, bool kWdeg>
 __global__ void k_mac(DevNet net, MacArgs args, char* scratch, LdsNet lnet) {
   extern __shared__ __align__(16) char smem[];
   __shared__ WgCtl ctl;
+  int* stamp = nullptr;
+  if (kWdeg) stamp = args.stamp_off ? (int*)(smem + args.stamp_off) : args.stamp_tab;
   if (kLds && lnet.bytes > 0) {
     const DevNet ln = wg_load_net(net, lnet, smem + wg_mem_bytes(net.n, net.W));
-    wg_mac_run<kWdeg, true>(ln, wg_carve(smem, ln), &ctl, args);
+    WgMem mem = wg_carve(smem, ln);
+    mem.stamp = stamp;
+    wg_mac_run<kWdeg, true>(ln, mem, &ctl, args);
   } else {
-    char* base = kLds ? smem : scratch;
-    wg_mac_run<kWdeg, false>(net, wg_carve(base, net), &ctl, args);
+    WgMem mem = wg_carve(kLds ? smem : scratch, net);
+    mem.stamp = stamp;
+    wg_mac_run<kWdeg, false>(net, mem, &ctl, args);
   }
 }
 
