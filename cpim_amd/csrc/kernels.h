@@ -1285,9 +1285,10 @@ __device__ __forceinline__ bool wg_fixpoint(const DevNet& net, const WgMem& mem,
     }
     for (int i = itab; i < net.ntabs; i += nwaves) {
       const int c = uniform_int(net.tabs[i]);
-      if (i != itab) tab0 = load_small_table(net, c);
-      const bool small = uniform_int(small_table(net, net.con[c].arity, tab0.tw)) != 0;
-      int y = tab0.y;
+      SmallTable tab = tab0;
+      if (i != itab) tab = load_small_table(net, c);
+      const bool small = uniform_int(small_table(net, net.con[c].arity, tab.tw)) != 0;
+      int y = tab.y;
       if (!small) y = lane < net.con[c].arity ? net.con[c].scope[lane] : -1;
       const int yy = y >= 0 ? y : 0;
       const bool mine_changed = y >= 0 && bit_of(cur, yy);
@@ -1298,7 +1299,7 @@ __device__ __forceinline__ bool wg_fixpoint(const DevNet& net, const WgMem& mem,
       ++revs;
       if (small) {
         // lane 8 p removes for position p
-        const unsigned gone = (unsigned)dp & ~small_table_keep(tab0, dp);
+        const unsigned gone = (unsigned)dp & ~small_table_keep(tab, dp);
         if (gone && y >= 0 && !assigned && lane < 32 && (lane & 7) == 0)
           lane_remove(mem, ctl, nxt, slot, round, y, &mem.dom[y], (u64)gone);
         continue;

@@ -232,3 +232,32 @@ def test_grid_rounds_equal_oracle(gpu, n, d, e, t, mode):
         assert st.inconsistent == (not ok2)
         if ok2:
             assert (m.ReadDomains(0) == dom2).all()
+
+
+@pytest.mark.parametrize("tables", [4, 5, 16, 17, 40])
+def test_many_small_tables_equal_oracle(gpu, tables):
+    """More tables than the workgroup has waves (4 in a singleton test, 16 in
+    the others): a wave takes several, over several rounds."""
+    n, d = 24, 16
+    base = workload.random_binary(n, d, 60, 0.35, workload.instance_seed(37, 1))
+    scopes, lists = [list(s) for s in base.scopes()], list(base.tuple_lists())
+    rng = np.random.default_rng(40)
+    for k in range(tables):
+        at = int(rng.integers(0, len(scopes) + 1))
+        scopes.insert(at, rng.choice(n, 3, replace=False).tolist())
+        lists.insert(at, workload.random_table(24000 + k, 3, d, 500))
+    desc = from_tuples(base.dom_size, scopes, lists)
+    o = oracle.Oracle(desc, oracle.AC3)
+    want = o.mac(node_limit=300, trace_cap=1000)
+    with GModelAdapter.Build(desc, GModelOptions(skip_non_binary=False)) as m:
+        st, _, trace = m.Solve(node_limit=300, trace_capacity=1000)
+        assert (st.num_positive, st.num_negative) == (want.num_positive, want.num_negative)
+        assert trace == want.trace
+        ok, dom, _ = oracle.Oracle(desc, oracle.AC3).root_ac()
+        assert m.EnforceGAC_Block().inconsistent == (not ok)
+        if ok:
+            assert (m.ReadDomains(0) == dom).all()
+            tests = np.array([(v, a) for v, vals in enumerate(domains_to_sets(dom, desc.dom_size)) for a in vals],
+                             np.int32)
+            got, _ = m.SingletonTests(tests, mode="workgroup")
+            assert (got == oracle.Oracle(desc, oracle.AC3).singleton_tests(tests)[0]).all()
