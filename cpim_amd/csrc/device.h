@@ -194,6 +194,17 @@ __device__ __forceinline__ u64 wave_min64_dpp(u64 v) {
   return readlane_rows_min(v);
 }
 
+__device__ __forceinline__ unsigned wave_min32_dpp(unsigned v) {
+  v = min(v, dpp_u32<0x121>(v));
+  v = min(v, dpp_u32<0x122>(v));
+  v = min(v, dpp_u32<0x124>(v));
+  v = min(v, dpp_u32<0x128>(v));
+  unsigned r = (unsigned)__builtin_amdgcn_readlane((int)v, 0);
+#pragma unroll
+  for (int l = 16; l < 64; l += 16) r = min(r, (unsigned)__builtin_amdgcn_readlane((int)v, l));
+  return r;
+}
+
 __device__ __forceinline__ u64 wave_sum64_dpp(u64 v) {
   v += dpp_ror_u64_1(v);
   v += dpp_ror_u64_2(v);
@@ -460,15 +471,17 @@ typedef unsigned v2u __attribute__((ext_vector_type(2)));
 __device__ __forceinline__ v2u swap32(unsigned x) { return __builtin_amdgcn_permlane32_swap(x, x, false, false); }
 __device__ __forceinline__ v2u swap16(unsigned x) { return __builtin_amdgcn_permlane16_swap(x, x, false, false); }
 
-// The values of each position (of domain dp, in every lane of the position)
-// that some valid tuple carries, among them dead values; in every lane of the
-// position.
-__device__ __forceinline__ unsigned small_table_keep(const SmallTable& t, u64 dp) {
-  const int lane = lane_id();
-  const unsigned xs = (lane & 7) < t.tw ? (unsigned)dp >> ((lane >> 5) * 8) : 0u;
-  u64 r[8];
+__device__ __forceinline__ void small_table_rows(const SmallTable& t, u64 (&r)[8]) {
 #pragma unroll
   for (int k = 0; k < 8; ++k) r[k] = t.rows[k * t.tw];
+}
+
+// The values of each position (of domain dp, in every lane of the position)
+// that some valid tuple carries, among them dead values; in every lane of the
+// position.  r: small_table_rows.
+__device__ __forceinline__ unsigned small_table_keep(int y, int tw, const u64 (&r)[8], unsigned dp) {
+  const int lane = lane_id();
+  const unsigned xs = (lane & 7) < tw ? dp >> ((lane >> 5) * 8) : 0u;
   unsigned lo = 0u, hi = 0u;
 #pragma unroll
   for (int k = 0; k < 8; ++k) {
@@ -479,7 +492,7 @@ __device__ __forceinline__ unsigned small_table_keep(const SmallTable& t, u64 dp
   v2u a = swap32(lo), b = swap32(hi);
   lo = a.x | a.y;
   hi = b.x | b.y;
-  if (t.y < 0) lo = hi = ~0u;
+  if (y < 0) lo = hi = ~0u;
   lo &= dpp_u32<0x128>(lo);  // positions 0, 1 and 2, 3: 8 lanes apart
   hi &= dpp_u32<0x128>(hi);
   a = swap16(lo);
@@ -581,7 +594,9 @@ __device__ __forceinline__ void revise_table(const DevNet& net, u64* dom, int* s
   if (small_table(net, arity, tw)) {
     const SmallTable t = load_small_table(net, c);
     const u64 dp = t.y >= 0 ? ld_dom<kCoherent>(&dom[t.y]) : 0ull;
-    const unsigned gone_l = (unsigned)dp & ~small_table_keep(t, dp);
+    u64 r[8];
+    small_table_rows(t, r);
+    const unsigned gone_l = (unsigned)dp & ~small_table_keep(t.y, t.tw, r, (unsigned)dp);
     const u64 lost = __ballot(gone_l != 0u);
     for (int q = 0; lost && q < arity; ++q) {
       const unsigned gone = (unsigned)__builtin_amdgcn_readlane((int)gone_l, 8 * q);

@@ -484,6 +484,18 @@ void build_lds_image(const ModelImage& im, DevModel& dm, hipStream_t s, std::vec
   dm.lnet.o_sup = (int)o_sup;
   dm.lnet.o_tsup = (int)o_tsup;
   dm.lnet.o_tabs = (int)L.o_tabs;
+  // wg_fixpoint_flat: a lane per variable, kFlatArcs arcs a lane (one if a
+  // domain has more than 16 values), a wave per table
+  const int arcs = (int)im.adj.size(), tabs = (int)im.tabs.size();
+  auto waves = [](int lanes) { return 64 * ((lanes + 63) / 64); };
+  const int per_lane = im.max_dom <= 16 ? kFlatArcs : 1;
+  const int least = std::max(waves(n), std::max(64, waves((arcs + per_lane - 1) / per_lane)) + 64 * tabs);
+  bool small = W == 1 && im.max_dom <= 32 && tabs <= kFlatTables && least <= 1024;
+  for (const ConMeta& m : im.con) small = small && (m.kind == 0 || (im.max_dom <= 16 && m.arity <= 4 && m.tw <= 8));
+  if (small) {
+    dm.lnet.flat_min = least;
+    dm.lnet.flat_threads = std::min(1024, std::max(least, waves(arcs) + 64 * tabs));
+  }
 }
 
 // Device bytes build_device_model takes from an arena for im (the same
@@ -1987,7 +1999,6 @@ int cpim_gmodel_solve(cpim_gmodel* m, const cpim_solve_opts* opts, cpim_search_s
     }
     DevNet net = m->dm.net();
     const long long bytes = wg_mem_bytes(n, m->dm.W);
-    const int threads = 1024;
     hipEvent_t e0, e1;
     HIPC(hipEventCreate(&e0));
     HIPC(hipEventCreate(&e1));
@@ -2003,6 +2014,7 @@ int cpim_gmodel_solve(cpim_gmodel* m, const cpim_solve_opts* opts, cpim_search_s
         bytes + m->dm.lnet.bytes <= (long long)m->props.max_lds - 2048)
       lnet = m->dm.lnet;
     const bool lds = bytes <= kLdsBudget;
+    const int threads = lds && lnet.flat_min && !A.weight ? lnet.flat_threads : 1024;
     long long dyn = lds ? bytes + lnet.bytes : 0;
     if (A.weight && dyn + 16 + 4ll * m->dm.num_active <= (long long)m->props.max_lds - 2048) {
       A.stamp_off = (int)std::max(16ll, dyn);  // 0 means memory

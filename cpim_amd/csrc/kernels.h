@@ -932,6 +932,7 @@ struct WgMem {
 struct WgCtl {
   // lowest round that emptied a domain, of the running fixpoint (slot: see wg_fixpoint)
   int wipe_round[2];
+  int2 flat[3];  // wg_fixpoint_flat: a round removed values, emptied a domain
   unsigned long long revs;
   u64 red[16];  // one slot per wave for block reductions
   int ok;
@@ -1105,58 +1106,6 @@ __device__ __forceinline__ void wg_seed(const WgMem& mem, WgCtl* ctl, int n, int
   if (threadIdx.x == 0) ctl->wipe_round[slot] = INT_MAX;
 }
 
-// One round over every arc in adjacency order, a lane per arc, for networks
-// whose image is in LDS and whose domains hold at most 32 values (one 32-bit
-// word).  Lane i of the workgroup keeps its first arc's entry (e0) in
-// registers over the whole fixpoint; the row words of the source's values are
-// read in order, eight at a time, and masked by its domain.  A round is a
-// chain of four LDS round trips (frontier bit and domains, rows, removal)
-// however many variables changed, which is what bounds small networks; up to
-// kFlatArcsPerThread arcs per lane, beyond which reading every entry costs
-// more than numbering the changed variables' arcs.
-constexpr int kFlatArcsPerThread = 4;
-
-__device__ __forceinline__ void wg_round_flat(const DevNet& net, const WgMem& mem, WgCtl* ctl, const unsigned* cur,
-                                              unsigned* nxt, int slot, int round, int narcs, const int4& e0,
-                                              int& revs) {
-  const int tid = threadIdx.x, nthreads = blockDim.x;
-  const int i1 = narcs - (tid & 63);  // the wave's last pass covers it
-  for (int i0 = uniform_int(tid & ~63); i0 < narcs; i0 += nthreads) {
-    int4 e = e0;
-    if (i0 >= nthreads) e = i0 < i1 ? mem.adj[i0 + (tid & 63)] : make_int4(0, -1, 0, 0);
-    const int t = adj_var(e), u = e.y;
-    const int uu = u >= 0 ? u : 0;
-    const unsigned bt = cur[t >> 5], au = mem.asg[uu >> 5];
-    const unsigned dt = (unsigned)ld_wg(&mem.dom[t]), du = (unsigned)ld_wg(&mem.dom[uu]);
-    const bool act = u >= 0 && ((bt >> (t & 31)) & 1u) && !((au >> (uu & 31)) & 1u);
-    const u64 active = __ballot(act);
-    if (active == 0ull) continue;
-    const unsigned x = act ? dt : 0u;
-    unsigned need = act ? du : 0u;
-    // lanes without an arc read plane 0
-    const u64* rows = net.sup + (act ? (2 * e.w + adj_pos(e)) * net.dpad : 0);
-    for (int a0 = 0; a0 < net.cap; a0 += 8) {
-      const unsigned xs = x >> a0;
-      if (__ballot((xs & 0xffu) != 0u) == 0ull) continue;
-      unsigned o = 0u;
-#pragma unroll
-      for (int k = 0; k < 8; ++k) o |= (unsigned)rows[a0 + k] & (unsigned)__builtin_amdgcn_sbfe((int)xs, k, 1);
-      need &= ~o;
-      if (__ballot(need != 0u && (xs >> 8) != 0u) == 0ull) break;
-    }
-    if (need) {
-      const unsigned old = (unsigned)and_wg(&mem.dom[u], ~(u64)need);
-      const unsigned lost = old & need;
-      if (lost) {
-        atomicOr(&nxt[u >> 5], 1u << (u & 31));
-        atomicSub(&mem.size[u], __popc(lost));
-        if (lost == old) atomicMin(&ctl->wipe_round[slot], round);
-      }
-    }
-    revs += __popcll(active);
-  }
-}
-
 // AC fixpoint from the seed that wg_seed put in mem.bm (a __syncthreads()
 // lies between).  both_dirs_round0: in the first round also revise t <- u for
 // every arc of a seed variable t (constraint seeding, as
@@ -1181,11 +1130,9 @@ __device__ __forceinline__ void wg_round_flat(const DevNet& net, const WgMem& me
 // and clears (r + 2) % 3, which no wave reads until the barrier of the next
 // round.  A wipe-out is recorded as the round it happened in, so that a wave
 // that still decides round r is not misled by one already in round r + 1.
-// kImage: the network is in LDS (wg_load_net), where small domains take
-// wg_round_flat instead of numbered units.
 // slot: two wipe-out words used in turn by successive fixpoints, so that
 // wg_seed never resets the word a slow wave still reads.
-template <bool kImage, bool kTight>
+template <bool kTight>
 __device__ __forceinline__ bool wg_fixpoint(const DevNet& net, const WgMem& mem, WgCtl* ctl, int slot,
                                             bool both_dirs_round0) {
   const int n = net.n, W = net.W;
@@ -1198,14 +1145,6 @@ __device__ __forceinline__ bool wg_fixpoint(const DevNet& net, const WgMem& mem,
   while ((1 << lw) < W) ++lw;
   const int w = lane & ((1 << lw) - 1), la = lane >> lw, per = 64 >> lw;
   const long long pair_words = 2ll * W * net.dpad;
-  bool flat = false;
-  int narcs = 0;
-  int4 e0 = make_int4(0, -1, 0, 0);
-  if constexpr (kImage) {
-    narcs = uniform_int(mem.aoff[n]);
-    flat = W == 1 && net.cap <= 32 && narcs <= kFlatArcsPerThread * nthreads;
-    if (flat && tid < narcs) e0 = mem.adj[tid];
-  }
   int revs = 0;
   bool result = true;
   int c0 = 0, c1 = nvw, c2 = 2 * nvw;
@@ -1218,9 +1157,8 @@ __device__ __forceinline__ bool wg_fixpoint(const DevNet& net, const WgMem& mem,
     unsigned* nxt = mem.bm + c1;
     for (int i = tid; i < nvw; i += nthreads) mem.bm[c2 + i] = 0u;
     const bool both = both_dirs_round0 && round == 0;
-    if (flat) wg_round_flat(net, mem, ctl, cur, nxt, slot, round, narcs, e0, revs);
     int mine = wave;  // this wave's next unit, counted from the block of variables below
-    bool stop = flat;
+    bool stop = false;
     for (int v0 = 0; v0 < n && !stop; v0 += 64) {
       const int v = v0 + lane;
       int a0 = 0, deg = 0;
@@ -1299,7 +1237,9 @@ __device__ __forceinline__ bool wg_fixpoint(const DevNet& net, const WgMem& mem,
       ++revs;
       if (small) {
         // lane 8 p removes for position p
-        const unsigned gone = (unsigned)dp & ~small_table_keep(tab, dp);
+        u64 rows[8];
+        small_table_rows(tab, rows);
+        const unsigned gone = (unsigned)dp & ~small_table_keep(tab.y, tab.tw, rows, (unsigned)dp);
         if (gone && y >= 0 && !assigned && lane < 32 && (lane & 7) == 0)
           lane_remove(mem, ctl, nxt, slot, round, y, &mem.dom[y], (u64)gone);
         continue;
@@ -1331,6 +1271,193 @@ __device__ __forceinline__ bool wg_fixpoint(const DevNet& net, const WgMem& mem,
   }
   if (lane == 0 && revs) atomicAdd(&ctl->revs, (unsigned long long)revs);
   return result;
+}
+
+// The same fixpoint for a search on a small network: domains of at most 32
+// values (one 32-bit word), kFlatArcs arcs a lane (one if a domain has more
+// than 16 values) and small tables only, one per wave.  Every lane keeps its
+// arcs' support rows in registers over the whole search (32 rows of 32 bits,
+// or 4 x 16 rows of 16 bits), a table's wave the rows of its table, so a round
+// reads nothing but domains.  An arc is revised when its source's domain is
+// not the one it last saw, so no frontier is kept; the first round revises
+// the arcs of the seed only, whose domain the caller passes, so the caller's
+// store of it needs no barrier before.
+//
+// What bounds it is a round's chain of three LDS round trips (domains,
+// removal, flags), some 60 dependent instructions and the barrier; waves
+// beyond those that the arcs and tables fill only add to the instructions
+// each SIMD issues, hence LdsNet::flat_threads.  1000 search nodes of n=23
+// d=23 e=253 take 3.3 ms; 5.8 ms with frontier bitmaps, the rows read from LDS
+// every round and 1024 threads.
+constexpr int kFlatArcs = 4;     // arcs per lane, of domains of at most 16 values
+constexpr int kFlatTables = 16;  // one per wave
+
+typedef short v2s __attribute__((ext_vector_type(2)));
+
+struct FlatNet {
+  int tu[kFlatArcs];  // source | target << 16, -1: no binary arc
+  // rows of the source's values over the target: one a word (wide), or values
+  // i and i + 8 in the halves of word i of the arc's eight; a table's wave:
+  // the words of its eight rows
+  unsigned rows[8 * kFlatArcs];
+  int arcs;    // arcs of the wave's lanes, wave-uniform (a table's wave has none)
+  bool wide;
+  bool table;  // the wave has a table
+  int y, tw;   // of the table: SmallTable
+};
+
+// The domains of its arcs' sources (0: of its table position's variable) that
+// a lane last revised them for: D as it is, after a fixpoint.
+struct FlatSeen {
+  unsigned arc[kFlatArcs];
+};
+
+__device__ __forceinline__ FlatNet wg_load_flat(const DevNet& net, const WgMem& mem) {
+  FlatNet f;
+  const int tid = threadIdx.x;
+  const int lanes = blockDim.x - 64 * net.ntabs;  // that take arcs
+  const int narcs = uniform_int(mem.aoff[net.n]);
+  const int first = uniform_int(tid & ~63);
+  f.table = first >= lanes;
+  f.arcs = !f.table && first < narcs ? (narcs - first + lanes - 1) / lanes : 0;
+  f.wide = net.cap > 16;
+#pragma unroll
+  for (int k = 0; k < kFlatArcs; ++k) {
+    const int i = k * lanes + tid;
+    int4 e = make_int4(0, -1, 0, 0);
+    if (!f.table && i < narcs) e = mem.adj[i];
+    f.tu[k] = e.y >= 0 ? adj_var(e) | (e.y << 16) : -1;
+    // lanes without an arc take the rows of plane 0; rows past the source's
+    // domain, of other planes or of the padding behind the last, are masked
+    // by it
+    const u64* row = net.sup + (e.y >= 0 ? (2 * e.w + adj_pos(e)) * net.dpad : 0);
+    if (!f.wide) {
+#pragma unroll
+      for (int v = 0; v < 8; ++v) f.rows[8 * k + v] = ((unsigned)row[v] & 0xffffu) | ((unsigned)row[v + 8] << 16);
+    } else if (k == 0) {
+#pragma unroll
+      for (int v = 0; v < 8 * kFlatArcs; ++v) f.rows[v] = (unsigned)row[v];
+    }
+  }
+  f.y = -1;
+  f.tw = 0;
+  if (f.table) {
+    const SmallTable t = load_small_table(net, uniform_int(net.tabs[(first - lanes) >> 6]));
+    f.y = t.y;
+    f.tw = t.tw;
+    u64 r[8];
+    small_table_rows(t, r);
+#pragma unroll
+    for (int v = 0; v < 8; ++v) {
+      f.rows[2 * v] = (unsigned)r[v];
+      f.rows[2 * v + 1] = (unsigned)(r[v] >> 32);
+    }
+  }
+  return f;
+}
+
+// Every domain as it is now, before the fixpoint of a refutation (the
+// domains must not change before the next barrier).
+__device__ __forceinline__ void wg_flat_see(const WgMem& mem, const FlatNet& f, FlatSeen& seen) {
+#pragma unroll
+  for (int k = 0; k < kFlatArcs; ++k)
+    if (k < f.arcs) seen.arc[k] = (unsigned)ld_wg(&mem.dom[f.tu[k] >= 0 ? f.tu[k] & 0xffff : 0]);
+  if (f.table) seen.arc[0] = (unsigned)ld_wg(&mem.dom[f.y >= 0 ? f.y : 0]);
+}
+
+// seed < 0: every arc and table.  seed_dom: D(seed); seed_assigned: the seed
+// is a decision (its asg bit need not be visible yet).  turn: the flags of the
+// round (kept over the fixpoints of a search).
+__device__ __forceinline__ bool wg_fixpoint_flat(const WgMem& mem, WgCtl* ctl, const FlatNet& f, FlatSeen& seen,
+                                                 int seed, unsigned seed_dom, bool seed_assigned, int& turn,
+                                                 int& revs) {
+  const int lane = lane_id();
+  unsigned skip = 0u;  // bit k: arc k (0: the table position) has no target, or an assigned one
+#pragma unroll
+  for (int k = 0; k < kFlatArcs; ++k)
+    if (k < f.arcs) {
+      const int u = f.tu[k] >> 16;
+      const int uu = u >= 0 ? u : 0;
+      if (u < 0 || bit_of(mem.asg, uu) || (seed_assigned && u == seed)) skip |= 1u << k;
+    }
+  const int y = f.y >= 0 ? f.y : 0;
+  if (f.table && (f.y < 0 || bit_of(mem.asg, y) || (seed_assigned && y == seed))) skip = 1u;
+  bool first = true;
+  while (true) {
+    const int next = turn == 2 ? 0 : turn + 1;
+    if (threadIdx.x == 0) ctl->flat[next] = make_int2(0, 0);
+    const bool seeded = first && seed >= 0, all = first && seed < 0;
+    bool changed = false, wiped = false;
+    auto remove = [&](int u, unsigned gone) {
+      const unsigned old = (unsigned)and_wg(&mem.dom[u], ~(u64)gone);
+      const unsigned lost = old & gone;
+      if (lost) {
+        atomicSub(&mem.size[u], __popc(lost));
+        changed = true;
+        wiped = wiped || lost == old;
+      }
+    };
+#pragma unroll
+    for (int k = 0; k < kFlatArcs; ++k)
+      if (k < f.arcs) {
+        const int u = f.tu[k] >> 16, t = u >= 0 ? f.tu[k] & 0xffff : 0;
+        const unsigned dt = (unsigned)ld_wg(&mem.dom[t]);
+        const unsigned du = (unsigned)ld_wg(&mem.dom[u >= 0 ? u : 0]);
+        // (the first round leaves the other arcs what they have seen: their
+        // sources may be losing values already)
+        const unsigned d = !seeded ? dt : t == seed ? seed_dom : seen.arc[k];
+        const bool act = (seeded ? t == seed : all || d != seen.arc[k]) && !((skip >> k) & 1u);
+        seen.arc[k] = d;
+        const u64 active = __ballot(act);
+        if (active) {
+          unsigned o = 0u;
+          if (!f.wide) {
+            const unsigned x = (d & 0xffu) | ((d & 0xff00u) << 8);
+            const v2s xs = __builtin_bit_cast(v2s, x);
+#pragma unroll
+            for (int v = 0; v < 8; ++v) {
+              const v2s m = (v2s)(xs << (short)(15 - v)) >> (short)15;
+              o |= f.rows[8 * k + v] & __builtin_bit_cast(unsigned, m);
+            }
+            o = (o | (o >> 16)) & 0xffffu;
+          } else if (k == 0) {
+#pragma unroll
+            for (int b = 0; b < kFlatArcs; ++b) {
+              if (__ballot(act && ((d >> (8 * b)) & 0xffu) != 0u) == 0ull) continue;
+#pragma unroll
+              for (int v = 8 * b; v < 8 * b + 8; ++v)
+                o |= f.rows[v] & (unsigned)__builtin_amdgcn_sbfe((int)d, v, 1);
+            }
+          }
+          const unsigned gone = act ? du & ~o : 0u;
+          if (gone) remove(u, gone);
+          revs += __popcll(active);
+        }
+      }
+    if (f.table) {
+      const unsigned now = (unsigned)ld_wg(&mem.dom[y]);
+      const unsigned dp = seeded && y == seed ? seed_dom : now;
+      const bool act = f.y >= 0 && (seeded ? y == seed : all || dp != seen.arc[0]);
+      if (__ballot(act)) {
+        ++revs;
+        u64 r[8];
+#pragma unroll
+        for (int v = 0; v < 8; ++v) r[v] = ((u64)f.rows[2 * v + 1] << 32) | f.rows[2 * v];
+        const unsigned keep = small_table_keep(f.y, f.tw, r, dp);
+        seen.arc[0] = skip ? dp : dp & keep;  // its own removals take no tuple
+        const unsigned gone = dp & ~keep;
+        if (gone && !skip && lane < 32 && (lane & 7) == 0) remove(y, gone);  // lane 8 p: position p
+      }
+    }
+    if (changed) __hip_atomic_store(&ctl->flat[turn].x, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+    if (wiped) __hip_atomic_store(&ctl->flat[turn].y, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+    __syncthreads();
+    const u64 flags = (u64)uniform_ll((long long)ld_wg((const u64*)&ctl->flat[turn]));
+    turn = next;
+    first = false;
+    if (flags >> 32) return false;
+    if (flags == 0ull) return true;
+  }
 }
 
 __device__ __forceinline__ void wg_clear_bitmap(unsigned* bm, int nvw) {
@@ -1385,7 +1512,7 @@ __global__ void k_block_gac(DevNet net, u64* dom, int* size, int seed_var, char*
   __syncthreads();
   long long before = 0;
   for (int v = threadIdx.x; v < n; v += blockDim.x) before += mem.size[v];
-  const bool ok = wg_fixpoint<false, true>(net, mem, &ctl, 0, seed_var >= 0);
+  const bool ok = wg_fixpoint<true>(net, mem, &ctl, 0, seed_var >= 0);
   long long after = 0;
   for (int v = threadIdx.x; v < n; v += blockDim.x) after += mem.size[v];
   const u64 delta = wg_reduce_sum_u64(&ctl, (u64)(before - after));
@@ -1524,7 +1651,7 @@ __global__ void k_singleton_tests(DevNet net, const u64* __restrict__ base_dom,
     mem.asg[x >> 5] |= 1u << (x & 31);
   }
   __syncthreads();
-  const bool ok = wg_fixpoint<false, true>(net, mem, &ctl, 0, false);
+  const bool ok = wg_fixpoint<true>(net, mem, &ctl, 0, false);
   __syncthreads();  // every wave's revision count
   if (threadIdx.x == 0) {
     fail[unit] = ok ? 0 : 1;
@@ -2606,6 +2733,9 @@ struct LdsNet {
   int bytes;         // multiple of 16
   int dc;
   int o_adj, o_con, o_sup, o_tsup, o_tabs;  // byte offsets in the image
+  // wg_fixpoint_flat: the smallest workgroup that can run it (0: none can) and
+  // the largest that its arcs and tables fill
+  int flat_min, flat_threads;
 };
 
 // Copies the image behind the working memory (at dst) and returns the
@@ -3013,9 +3143,12 @@ __device__ __forceinline__ void wg_load_level(const WgMem& mem, const u64* level
 // (every value below is wave-uniform); LDS holds the domains, the frontier
 // and the decision stack.  One loop with one fixpoint in it: `phase` says
 // what the fixpoint propagates (the root, a decision x = a, a refutation
-// x != a).  A decision costs two barriers and a refutation one, beside the
-// fixpoint's own.  kWdeg: dom/wdeg ordering, wipe-outs repeated in AC3's order.
-template <bool kWdeg, bool kImage>
+// x != a).  A decision costs two barriers (one with kFlat) and a refutation
+// one, beside the fixpoint's own.  kWdeg: dom/wdeg ordering, wipe-outs
+// repeated in AC3's order.  kFlat: wg_fixpoint_flat propagates, and a
+// refutation that follows its decision takes the domains from registers (dom
+// and dom/deg only).
+template <bool kWdeg, bool kFlat>
 __device__ __forceinline__ void wg_mac_run(const DevNet& net, const WgMem& mem, WgCtl* ctl, const MacArgs& A) {
   enum { ROOT, POSITIVE, NEGATIVE };
   const int n = net.n, W = net.W;
@@ -3033,11 +3166,19 @@ __device__ __forceinline__ void wg_mac_run(const DevNet& net, const WgMem& mem, 
   int2* stk = kWdeg ? A.stack : (int2*)mem.list;
   int slot = 0, phase = ROOT, x = -1, a = 0;
   bool select = false;  // the domains are consistent: take the next decision
-  if (tid == 0) ctl->revs = 0;
+  FlatNet flat{};
+  FlatSeen seen{};
+  int turn = 0, flat_revs = 0;
+  unsigned saved = 0u, dx = 0u;  // before the last decision: D(tid), D(x)
+  if constexpr (kFlat) flat = wg_load_flat(net, mem);
+  if (tid == 0) {
+    ctl->revs = 0;
+    if (kFlat) ctl->flat[0] = make_int2(0, 0);
+  }
   wg_clear_bitmap(mem.asg, nvw);
   if (status == MAC_INIT) {
     wg_load_level(mem, A.trail, n, W, -1, 0);
-    wg_seed(mem, ctl, n, slot, -1);
+    if (!kFlat) wg_seed(mem, ctl, n, slot, -1);
     status = MAC_RUNNING;
   } else if (status == MAC_RUNNING) {
     wg_load_level(mem, A.trail + depth * nw, n, W, -1, 0);
@@ -3047,6 +3188,7 @@ __device__ __forceinline__ void wg_mac_run(const DevNet& net, const WgMem& mem, 
   }
   __syncthreads();
   if (select) {
+    if constexpr (kFlat) wg_flat_see(mem, flat, seen);
     for (int i = tid; i < depth; i += nthreads) {
       const int v = A.stack[i].x;
       atomicOr(&mem.asg[v >> 5], 1u << (v & 31));
@@ -3069,6 +3211,24 @@ __device__ __forceinline__ void wg_mac_run(const DevNet& net, const WgMem& mem, 
       // finds it by itself.
       if (kWdeg) {
         x = wg_select_wdeg(net, mem, ctl, A);
+      } else if constexpr (kFlat) {
+        unsigned key = ~0u, dv = 0u;
+        for (int v = lane; v < n; v += 64) {
+          const unsigned d = (unsigned)ld_wg(&mem.dom[v]);
+          unsigned hi = (unsigned)__popc(d);
+          if (A.nbr) {
+            const int g = A.nbr[v];
+            hi = g == 0 ? 0u : hi / (unsigned)g + 1u;
+          }
+          const unsigned k = (hi << 16) | (unsigned)v;
+          if (!bit_of(mem.asg, v) && k < key) {
+            key = k;
+            dv = d;
+          }
+        }
+        const unsigned least = wave_min32_dpp(key);
+        x = (int)(least & 0xffffu);
+        dx = (unsigned)__builtin_amdgcn_readlane((int)dv, x & 63);
       } else {
         u64 key = ~0ull;
         for (int v = lane; v < n; v += 64)
@@ -3085,11 +3245,15 @@ __device__ __forceinline__ void wg_mac_run(const DevNet& net, const WgMem& mem, 
       }
       // min value of x (every thread scans the same words)
       a = -1;
-      for (int w = 0; w < W && a < 0; ++w) {
-        const u64 dw = mem.dom[(long long)x * W + w];
-        if (dw) a = w * 64 + (int)__builtin_ctzll(dw);
+      if constexpr (kFlat) {
+        if (dx) a = (int)__builtin_ctz(dx);
+      } else {
+        for (int w = 0; w < W && a < 0; ++w) {
+          const u64 dw = mem.dom[(long long)x * W + w];
+          if (dw) a = w * 64 + (int)__builtin_ctzll(dw);
+        }
+        a = uniform_int(a);
       }
-      a = uniform_int(a);
       if (a < 0) {
         // x has an empty domain that no revision reached (no constraints, an
         // empty initial domain): the search ends without a solution, with no
@@ -3097,10 +3261,18 @@ __device__ __forceinline__ void wg_mac_run(const DevNet& net, const WgMem& mem, 
         status = MAC_UNSAT;
         break;
       }
-      wg_copy_words(A.trail + depth * nw, mem.dom, nw);
+      if constexpr (kFlat) {
+        if (tid < n) {
+          const u64 d = ld_wg(&mem.dom[tid]);
+          saved = (unsigned)d;
+          A.trail[depth * nw + tid] = d;
+        }
+      } else {
+        wg_copy_words(A.trail + depth * nw, mem.dom, nw);
+      }
       __syncthreads();
       if (tid < W) mem.dom[(long long)x * W + tid] = (tid == (a >> 6)) ? (1ull << (a & 63)) : 0ull;
-      wg_seed(mem, ctl, n, slot, x);
+      if (!kFlat) wg_seed(mem, ctl, n, slot, x);
       if (tid == 0) {
         A.stack[depth] = make_int2(x, a);
         if (!kWdeg) stk[depth] = make_int2(x, a);
@@ -3111,9 +3283,16 @@ __device__ __forceinline__ void wg_mac_run(const DevNet& net, const WgMem& mem, 
       ++npos;
       ++nodes_here;
       phase = POSITIVE;
-      __syncthreads();
+      if (!kFlat) __syncthreads();
     }
-    bool ok = wg_fixpoint<kImage, false>(net, mem, ctl, slot, false);
+    bool ok;
+    if constexpr (kFlat) {
+      const unsigned bit = 1u << (a & 31);
+      ok = wg_fixpoint_flat(mem, ctl, flat, seen, phase == ROOT ? -1 : x, phase == POSITIVE ? bit : dx & ~bit,
+                            phase == POSITIVE, turn, flat_revs);
+    } else {
+      ok = wg_fixpoint<false>(net, mem, ctl, slot, false);
+    }
     if (kWdeg && !ok) {
       // a wipe-out raises the weight of the constraint that AC3's order
       // empties a domain with first: propagate again, in that order, from the
@@ -3158,7 +3337,7 @@ __device__ __forceinline__ void wg_mac_run(const DevNet& net, const WgMem& mem, 
     if (ok) continue;
     // undo decisions until a refutation leaves its variable a value
     select = false;
-    phase = NEGATIVE;
+    if (!kFlat) phase = NEGATIVE;
     while (true) {
       if (depth == 0) {
         status = MAC_UNSAT;
@@ -3169,22 +3348,41 @@ __device__ __forceinline__ void wg_mac_run(const DevNet& net, const WgMem& mem, 
       x = uniform_int(d.x);
       a = uniform_int(d.y);
       const u64* level = A.trail + depth * nw;
-      wg_load_level(mem, level, n, W, x, a);
+      u64 rest = 0ull;
+      if constexpr (kFlat) {
+        if (phase != POSITIVE) {
+          saved = tid < n ? (unsigned)level[tid] : 0u;
+          dx = (unsigned)uniform_int((int)level[x]);
+        }
+        phase = NEGATIVE;
+        rest = dx & ~(1u << (a & 31));
+        if (tid < n) {
+          const unsigned d = tid == x ? (unsigned)rest : saved;
+          mem.dom[tid] = d;
+          mem.size[tid] = __popc(d);
+        }
+      } else {
+        wg_load_level(mem, level, n, W, x, a);
+        for (int w = 0; w < W; ++w) {
+          const u64 dw = level[(long long)x * W + w];
+          rest |= w == (a >> 6) ? dw & ~(1ull << (a & 63)) : dw;
+        }
+      }
       if (tid == 0) mem.asg[x >> 5] &= ~(1u << (x & 31));
       ++nneg;
       ++nodes_here;
-      u64 rest = 0ull;
-      for (int w = 0; w < W; ++w) {
-        const u64 dw = level[(long long)x * W + w];
-        rest |= w == (a >> 6) ? dw & ~(1ull << (a & 63)) : dw;
-      }
       if ((u64)uniform_ll((long long)rest) != 0ull) break;
       wg_trace(net, mem, A, &trace_len, 0, x, a, false);
     }
     if (status != MAC_RUNNING) break;
-    wg_seed(mem, ctl, n, slot, x);
+    if (!kFlat) wg_seed(mem, ctl, n, slot, x);
     __syncthreads();
+    if constexpr (kFlat) {
+      wg_flat_see(mem, flat, seen);
+      __syncthreads();
+    }
   }
+  if (kFlat && lane == 0 && flat_revs) atomicAdd(&ctl->revs, (unsigned long long)flat_revs);
   __syncthreads();
   if (tid == 0) {
     A.state->status = status;
@@ -3210,7 +3408,8 @@ __global__ void k_mac(DevNet net, MacArgs args, char* scratch, LdsNet lnet) {
     const DevNet ln = wg_load_net(net, lnet, smem + wg_mem_bytes(net.n, net.W));
     WgMem mem = wg_carve(smem, ln);
     mem.stamp = stamp;
-    wg_mac_run<kWdeg, true>(ln, mem, &ctl, args);
+    if (!kWdeg && lnet.flat_min && lnet.flat_min <= (int)blockDim.x) wg_mac_run<false, true>(ln, mem, &ctl, args);
+    else wg_mac_run<kWdeg, false>(ln, mem, &ctl, args);
   } else {
     WgMem mem = wg_carve(kLds ? smem : scratch, net);
     mem.stamp = stamp;
@@ -3266,7 +3465,10 @@ __global__ void k_mac_units(const UnitDesc* __restrict__ units, int count, unsig
     const int where = uniform_int(d.use_lds);
     if (where == 2) {
       const DevNet ln = wg_load_net(d.net, d.lnet, smem + wg_mem_bytes(d.net.n, d.net.W));
-      wg_mac_run<false, true>(ln, wg_carve(smem, ln), &ctl, d.args);
+      if (uniform_int(d.lnet.flat_min && d.lnet.flat_min <= (int)blockDim.x))
+        wg_mac_run<false, true>(ln, wg_carve(smem, ln), &ctl, d.args);
+      else
+        wg_mac_run<false, false>(ln, wg_carve(smem, ln), &ctl, d.args);
     } else if (where == 1) {
       wg_mac_run<false, false>(d.net, wg_carve(smem, d.net), &ctl, d.args);
     } else {

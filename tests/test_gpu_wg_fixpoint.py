@@ -12,7 +12,7 @@ import numpy as np
 import pytest
 
 import oracle
-from cpim_amd import GModelAdapter, GModelOptions, workload
+from cpim_amd import GModelAdapter, GModelOptions, Server, workload
 from cpim_amd.model import domains_to_sets, from_tuples
 
 pytestmark = pytest.mark.gpu
@@ -104,6 +104,40 @@ def test_lds_search_equals_oracle(gpu, n, d, e, t):
         st, _, trace = m.Solve(node_limit=400, trace_capacity=1000)
     assert (st.num_solutions, st.num_positive, st.num_negative) == (want.num_sol, want.num_positive, want.num_negative)
     assert trace == want.trace
+
+
+@pytest.mark.parametrize("n,d,e,t,tables", [
+    # one and two arcs a lane beside tables, one arc a lane above 16 values;
+    # 16 tables and one too many; as many variables as lanes
+    (30, 16, 100, 0.35, 4), (30, 16, 240, 0.22, 2), (30, 17, 100, 0.35, 0), (24, 16, 60, 0.35, 16),
+    (24, 16, 60, 0.35, 17), (64, 4, 64, 0.3, 1), (65, 4, 64, 0.3, 0), (200, 3, 230, 0.2, 0), (5, 16, 0, 0.0, 2),
+])
+def test_small_network_searches_equal_oracle(gpu, n, d, e, t, tables):
+    """Solve in one go, and on a server in steps of seven nodes (each resumes
+    from the stored state)."""
+    base = workload.random_binary(n, d, e, t, workload.instance_seed(36, n * 100 + d))
+    scopes, lists = [list(s) for s in base.scopes()], list(base.tuple_lists())
+    rng = np.random.default_rng(n + d)
+    for k in range(tables):  # tables between the binary constraints
+        at = int(rng.integers(0, len(scopes) + 1))
+        scopes.insert(at, rng.choice(n, 3, replace=False).tolist())
+        lists.insert(at, workload.random_table(1000 * n + k, 3, d, min(500, d ** 3 // 2)))
+    desc = from_tuples(base.dom_size, scopes, lists)
+    want = oracle.Oracle(desc, oracle.AC3 if tables else oracle.AC3BIT).mac(node_limit=300, trace_cap=1000)
+    counts = (want.num_sol, want.num_positive, want.num_negative)
+    with GModelAdapter.Build(desc, GModelOptions(skip_non_binary=False)) as m:
+        st, sol, trace = m.Solve(node_limit=300, trace_capacity=1000)
+    assert (st.num_solutions, st.num_positive, st.num_negative) == counts
+    assert trace == want.trace
+    srv = Server(max_slots=1, nodes_per_step=7)
+    rid = srv.submit(desc, node_limit=300)
+    while not srv.poll():
+        srv.step()
+    r = srv.result(rid)
+    srv.close()
+    assert (r["num_positive"], r["num_negative"]) == counts[1:]
+    if want.num_sol:
+        assert (np.asarray(sol) == want.solution).all() and (np.asarray(r["solution"]) == want.solution).all()
 
 
 @pytest.mark.parametrize("d,arity,tuples", [
