@@ -1113,20 +1113,27 @@ void gac_block(cpim_gmodel* m, int assigned_var, cpim_gac_stats* st) {
   fill_gac_stats(box->gac, 1, box->gac.converged != 0, m->ticks_ms(box->gac.ticks), st);
 }
 
-int auto_gac_mode(const cpim_gmodel* m, int assigned_var) {
-  // Small networks: one workgroup with the domains in LDS (one launch, no
-  // grid barrier).  Large ones seeded with every constraint: host-driven
-  // rounds, each spread over the whole grid (few rounds at the benchmark
-  // tightness; 0.21 ms against 0.52 ms asynchronous for one fixpoint of
-  // 80,000 revisions).  Large ones seeded from one variable: the
-  // asynchronous one-launch fixpoint, which has no per-round host sync.
-  if (fits_lds(m) && m->dm.num_active <= 4096) return CPIM_GAC_BLOCK;
-  return assigned_var < 0 ? CPIM_GAC_PLAIN : CPIM_GAC_ASYNC;
+// Constraints times words a domain up to which AUTO takes one workgroup with
+// the domains in LDS, and beyond which the host-driven rounds, each spread
+// over the grid.  Measured (one workgroup against rounds, us; the root of a
+// network whose revisions all find supports / of one that cascades / after
+// one assignment): 300 constraints of 20 values 16/23/25 against 15/38/28;
+// 1000 of 16 values 23/32/31 against 16/38/33; 1000 of 64 values 24/85/32
+// against 16/58/30; 2500 of 16 values 35/57/38 against 16/58/32; 1000 of 200
+// values (4 words) 43/712/36 against 17/189/35.  The asynchronous kernel takes
+// 200 to 750 us after one assignment where the rounds take 31 to 39 (500 to
+// 2000 variables); the persistent kernel is faster still (21 to 34), but needs
+// every workgroup resident at once, which AUTO does not ask of a caller with
+// several streams.
+constexpr long long kAutoBlockWords = 800;
+
+int auto_gac_mode(const cpim_gmodel* m) {
+  return fits_lds(m) && (long long)m->dm.num_active * m->dm.W <= kAutoBlockWords ? CPIM_GAC_BLOCK : CPIM_GAC_PLAIN;
 }
 
 void gac(cpim_gmodel* m, int assigned_var, int mode, cpim_gac_stats* st) {
   std::memset(st, 0, sizeof(*st));
-  if (mode == CPIM_GAC_AUTO) mode = auto_gac_mode(m, assigned_var);
+  if (mode == CPIM_GAC_AUTO) mode = auto_gac_mode(m);
   if (m->dm.num_active == 0) {
     st->converged = 1;
     return;

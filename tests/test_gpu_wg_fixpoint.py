@@ -295,3 +295,28 @@ def test_many_small_tables_equal_oracle(gpu, tables):
                              np.int32)
             got, _ = m.SingletonTests(tests, mode="workgroup")
             assert (got == oracle.Oracle(desc, oracle.AC3).singleton_tests(tests)[0]).all()
+
+
+@pytest.mark.parametrize("n,d,e,t", [
+    # one workgroup up to 800 constraint words, rounds over the grid beyond
+    (60, 9, 799, 0.3), (60, 9, 800, 0.3), (60, 9, 801, 0.3), (60, 70, 400, 0.9), (60, 70, 401, 0.9), (150, 20, 5000, 0.1),
+])
+def test_auto_fixpoint_equals_oracle(gpu, n, d, e, t):
+    desc = networks(n, d, e, t, 3)
+    ok, dom, _ = oracle.Oracle(desc).root_ac()
+    with GModelAdapter.Build(desc) as m:
+        assert m.EnforceGAC_Auto().inconsistent == (not ok)
+        if not ok:
+            return
+        assert (m.ReadDomains(0) == dom).all()
+        for v in (0, n - 1):  # one variable assigned
+            a = domains_to_sets(dom, desc.dom_size)[v][-1]
+            cut = dom.copy()
+            cut[v] = 0
+            cut[v, a // 64] = np.uint64(1 << (a % 64))
+            m.WriteDomains(0, cut)
+            st = m.EnforceGAC_Auto(v)
+            ok2, dom2, _ = oracle.Oracle(desc.with_init_dom(cut)).root_ac()
+            assert st.inconsistent == (not ok2)
+            if ok2:
+                assert (m.ReadDomains(0) == dom2).all()
