@@ -6,7 +6,7 @@ words), e=20000 distinct pairs, every tuple forbidden with p=0.5.  After the
 root GAC fixpoint, one step = one SAC pass = every singleton test (x = a) of
 the current domains (128,000 tests), each a full GAC fixpoint on its own
 domain copy, all in one persistent launch.  The plain path (one host-driven
-fixpoint per test, one launch + sync per round) and the CPU oracle are timed
+fixpoint per test, one launch per round) and the CPU oracle are timed
 on bounded samples of the same tests in the same run.
 
 Prints one JSON line.  roofline.achieved counts the schedule-independent

@@ -400,11 +400,6 @@ __device__ __forceinline__ int kth_value(u64 d_l, int W, int k) {
   return a;
 }
 
-// Offset in sup of the planes of a binary arc's constraint.
-__device__ __forceinline__ long long arc_plane_off(const DevNet& net, const int4& e) {
-  return (long long)e.w * 2 * net.W * net.dpad;
-}
-
 template <bool kCoherent = false>
 __device__ __forceinline__ int revise_binary(const DevNet& net, u64* dom, int* size, int c, int u,
                                              int t, int pos_t, bool* wiped) {

@@ -1123,8 +1123,12 @@ __device__ __forceinline__ void wg_seed(const WgMem& mem, WgCtl* ctl, int n, int
 // adjacency, domains, rows) and the barrier, not bandwidth.  With a lane per
 // arc word instead of a wave per one to four arcs, one chain serves 64 / Wp
 // arcs and a row read fetches one row of each instead of 64: 1000 search
-// nodes of n=23 d=23 e=253 take 7.4 ms (28.2 ms before), 256 uneven
-// instances (n 20..200, d 8..128) of 64 nodes each 3.4 ms (33 ms before).
+// nodes of n=23 d=23 e=253 took 7.4 ms (28.2 ms before; they now take
+// wg_fixpoint_flat), 256 uneven instances (n 20..200, d 8..128) of 64 nodes
+// each 2.7 ms (33 ms before).  The heaviest of those, rounds of some 14,000
+// arc words with the rows in memory, are bound by the cache lines that a
+// wave's row reads touch: neither rows of two values a load nor adjacency
+// entries read ahead gained anything.
 //
 // The frontier bitmaps rotate: round r reads bitmap r % 3, fills (r + 1) % 3
 // and clears (r + 2) % 3, which no wave reads until the barrier of the next
