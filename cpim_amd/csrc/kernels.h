@@ -765,7 +765,7 @@ __device__ __forceinline__ void async_process_constraint(const DevNet& net, u64*
       dels += k;
       push_var_async(net, v, F, ctl, owed);
     };
-    revise_table<decltype(on_removed), true>(net, dom, size, c, -1, nullptr, on_removed, &wiped);
+    revise_table<decltype(on_removed), true, false>(net, dom, size, c, -1, nullptr, on_removed, &wiped);
     ++revs;
     if (wiped && lane_id() == 0) atomicExch(&ctl->wipe, 1);
   }
