@@ -1314,6 +1314,7 @@ struct FlatNet {
 // a lane last revised them for: D as it is, after a fixpoint.
 struct FlatSeen {
   unsigned arc[kFlatArcs];
+  unsigned skip;  // bit k: arc k (0: the table position) has no target, or an assigned one
 };
 
 __device__ __forceinline__ FlatNet wg_load_flat(const DevNet& net, const WgMem& mem) {
@@ -1360,32 +1361,41 @@ __device__ __forceinline__ FlatNet wg_load_flat(const DevNet& net, const WgMem& 
   return f;
 }
 
-// Every domain as it is now, before the fixpoint of a refutation (the
-// domains must not change before the next barrier).
+// Every domain and assigned variable as they are now, before the first
+// fixpoint and that of a refutation (nothing may change before the next
+// barrier).
 __device__ __forceinline__ void wg_flat_see(const WgMem& mem, const FlatNet& f, FlatSeen& seen) {
+  seen.skip = 0u;
 #pragma unroll
   for (int k = 0; k < kFlatArcs; ++k)
-    if (k < f.arcs) seen.arc[k] = (unsigned)ld_wg(&mem.dom[f.tu[k] >= 0 ? f.tu[k] & 0xffff : 0]);
-  if (f.table) seen.arc[0] = (unsigned)ld_wg(&mem.dom[f.y >= 0 ? f.y : 0]);
+    if (k < f.arcs) {
+      const int u = f.tu[k] >> 16, uu = u >= 0 ? u : 0;
+      seen.arc[k] = (unsigned)ld_wg(&mem.dom[u >= 0 ? f.tu[k] & 0xffff : 0]);
+      if (u < 0 || bit_of(mem.asg, uu)) seen.skip |= 1u << k;
+    }
+  if (f.table) {
+    const int y = f.y >= 0 ? f.y : 0;
+    seen.arc[0] = (unsigned)ld_wg(&mem.dom[y]);
+    if (f.y < 0 || bit_of(mem.asg, y)) seen.skip = 1u;
+  }
 }
 
 // seed < 0: every arc and table.  seed_dom: D(seed); seed_assigned: the seed
-// is a decision (its asg bit need not be visible yet).  turn: the flags of the
-// round (kept over the fixpoints of a search).
+// is a decision.  turn: the flags of the round (kept over the fixpoints of a
+// search).  Which targets are assigned is kept with what the lanes have seen:
+// read from LDS at each fixpoint, it cost 2% of a search.
 __device__ __forceinline__ bool wg_fixpoint_flat(const WgMem& mem, WgCtl* ctl, const FlatNet& f, FlatSeen& seen,
                                                  int seed, unsigned seed_dom, bool seed_assigned, int& turn,
                                                  int& revs) {
   const int lane = lane_id();
-  unsigned skip = 0u;  // bit k: arc k (0: the table position) has no target, or an assigned one
-#pragma unroll
-  for (int k = 0; k < kFlatArcs; ++k)
-    if (k < f.arcs) {
-      const int u = f.tu[k] >> 16;
-      const int uu = u >= 0 ? u : 0;
-      if (u < 0 || bit_of(mem.asg, uu) || (seed_assigned && u == seed)) skip |= 1u << k;
-    }
   const int y = f.y >= 0 ? f.y : 0;
-  if (f.table && (f.y < 0 || bit_of(mem.asg, y) || (seed_assigned && y == seed))) skip = 1u;
+  if (seed_assigned) {
+#pragma unroll
+    for (int k = 0; k < kFlatArcs; ++k)
+      if (k < f.arcs && (f.tu[k] >> 16) == seed) seen.skip |= 1u << k;
+    if (f.table && y == seed) seen.skip = 1u;
+  }
+  const unsigned skip = seen.skip;
   bool first = true;
   while (true) {
     const int next = turn == 2 ? 0 : turn + 1;
@@ -3184,6 +3194,10 @@ __device__ __forceinline__ void wg_mac_run(const DevNet& net, const WgMem& mem, 
     wg_load_level(mem, A.trail, n, W, -1, 0);
     if (!kFlat) wg_seed(mem, ctl, n, slot, -1);
     status = MAC_RUNNING;
+    if constexpr (kFlat) {
+      __syncthreads();
+      wg_flat_see(mem, flat, seen);
+    }
   } else if (status == MAC_RUNNING) {
     wg_load_level(mem, A.trail + depth * nw, n, W, -1, 0);
     if (!kWdeg)
@@ -3192,12 +3206,15 @@ __device__ __forceinline__ void wg_mac_run(const DevNet& net, const WgMem& mem, 
   }
   __syncthreads();
   if (select) {
-    if constexpr (kFlat) wg_flat_see(mem, flat, seen);
     for (int i = tid; i < depth; i += nthreads) {
       const int v = A.stack[i].x;
       atomicOr(&mem.asg[v >> 5], 1u << (v & 31));
     }
     __syncthreads();
+    if constexpr (kFlat) {
+      wg_flat_see(mem, flat, seen);
+      __syncthreads();
+    }
   }
   while (status == MAC_RUNNING) {
     if (select) {
