@@ -978,7 +978,7 @@ void persistent_launch(cpim_gmodel* m, int assigned_var, unsigned* F, GacCtl* ct
   const unsigned long long max_ticks = fixpoint_budget_ticks(m);
   hipLaunchKernelGGL(staged ? k_gac_persistent<true> : k_gac_persistent<false>, dim3(grid), dim3(kPersistentThreads),
                      staged ? (size_t)lds : 0, m->stream, m->dm.net(), m->level_dom(L), m->level_size(L), F, m->nvw,
-                     ctl, mr, assigned_var, (int)m->im.adj.size(), max_ticks, out, seq_at, seq);
+                     ctl, mr, assigned_var, assigned_var >= 0 ? 1 : 0, (int)m->im.adj.size(), max_ticks, out, seq_at, seq);
   HIPC(hipGetLastError());
 }
 
@@ -996,7 +996,9 @@ void fill_gac_stats(const GacResult& res, int rounds, bool converged, double kms
 // a launch that finds the fixpoint over about 2 us.
 constexpr int kRoundsAhead = 8;
 
-void gac_grid(cpim_gmodel* m, int assigned_var, bool persistent, cpim_gac_stats* st) {
+// by_variable: a seeded fixpoint keeps a frontier of variables, as the workgroup
+// fixpoint does, instead of one of constraints (host-driven rounds only).
+void gac_grid(cpim_gmodel* m, int assigned_var, bool persistent, cpim_gac_stats* st, bool by_variable = false) {
   const int L = m->current_level;
   unsigned* F = m->front.as<unsigned>();
   GacCtl* ctl = m->ctl.as<GacCtl>();
@@ -1030,8 +1032,9 @@ void gac_grid(cpim_gmodel* m, int assigned_var, bool persistent, cpim_gac_stats*
       for (int i = 0; i < k; ++i, ++seq) {
         answers[i].rounds = 0;  // stays 0 if the fixpoint was over before
         hipLaunchKernelGGL(k_gac_round, dim3(grid), dim3(kRoundThreads), 0, m->stream, net, m->level_dom(L),
-                           m->level_size(L), F, m->nvw, ctl, r0 + i, assigned_var, (int)m->im.adj.size(), &answers[i],
-                           &box->seq, seq);
+                           m->level_size(L), F, m->nvw, ctl, r0 + i, assigned_var,
+                           assigned_var >= 0 && !by_variable ? 1 : 0, (int)m->im.adj.size(), &answers[i], &box->seq,
+                           seq);
         HIPC(hipGetLastError());
       }
       m->wait_box(seq - 1);
@@ -1126,6 +1129,11 @@ void gac_block(cpim_gmodel* m, int assigned_var, cpim_gac_stats* st) {
 // every workgroup resident at once, which AUTO does not ask of a caller with
 // several streams.
 constexpr long long kAutoBlockWords = 800;
+// Constraints up to which a fixpoint that AUTO seeds with one variable keeps a
+// frontier of variables (domains that fit in LDS), and beyond which it keeps
+// one of constraints.  On a level that is not at its closure the two answer
+// differently, so this line stays, whichever kernel runs.
+constexpr int kAutoByVariable = 4096;
 
 int auto_gac_mode(const cpim_gmodel* m) {
   return fits_lds(m) && (long long)m->dm.num_active * m->dm.W <= kAutoBlockWords ? CPIM_GAC_BLOCK : CPIM_GAC_PLAIN;
@@ -1133,13 +1141,14 @@ int auto_gac_mode(const cpim_gmodel* m) {
 
 void gac(cpim_gmodel* m, int assigned_var, int mode, cpim_gac_stats* st) {
   std::memset(st, 0, sizeof(*st));
+  const bool by_variable = mode == CPIM_GAC_AUTO && fits_lds(m) && m->dm.num_active <= kAutoByVariable;
   if (mode == CPIM_GAC_AUTO) mode = auto_gac_mode(m);
   if (m->dm.num_active == 0) {
     st->converged = 1;
     return;
   }
   switch (mode) {
-    case CPIM_GAC_PLAIN: gac_grid(m, assigned_var, false, st); break;
+    case CPIM_GAC_PLAIN: gac_grid(m, assigned_var, false, st, by_variable); break;
     case CPIM_GAC_PERSISTENT: gac_grid(m, assigned_var, true, st); break;
     case CPIM_GAC_BLOCK: gac_block(m, assigned_var, st); break;
     case CPIM_GAC_ASYNC: gac_async(m, assigned_var, st); break;

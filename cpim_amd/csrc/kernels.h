@@ -190,7 +190,10 @@ __device__ __forceinline__ u64 arcs_unsupported(const DevNet& net, const u64* do
 // ===========================================================================
 // Grid engine: rounds over a bitmap of the variables that changed.
 // In round r a lane takes one word of one arc u <- t of the adjacency list,
-// if t changed in round r - 1.  Three bitmaps rotate: F[r % 3] is read,
+// if t changed in round r - 1.  A fixpoint seeded with one variable may start
+// from a level that is not at its closure, and then reaches less than the
+// whole closure: as a frontier of constraints does (`pairs`: u <- t also if u
+// changed), or as one of variables does.  Three bitmaps rotate: F[r % 3] is read,
 // F[(r + 1) % 3] collects the round's changes, F[(r + 2) % 3] (read in round
 // r - 1) is cleared.  last_push_round only grows and wipe_round is only
 // lowered to the running round, so every block takes the same decision after
@@ -311,7 +314,8 @@ __device__ __forceinline__ void grid_arc(const DevNet& net, const u64* view, u64
 
 // The arcs and tables of round r that this grid's waves take.  cur: the
 // variables that changed (round 0: seed < 0 takes every arc and table, else
-// those on variable `seed`, in both directions); e0: the arc of this lane's
+// those on variable `seed`, in both directions); pairs: later rounds take the
+// changed variables' constraints in both directions too; e0: the arc of this lane's
 // first turn, kept in registers by the persistent kernel (kept true).  With
 // several words a wave's arcs lie nwaves apart in the list, so that the arcs
 // of one variable (a late round's few changes) fall to as many waves: what
@@ -321,7 +325,7 @@ __device__ __forceinline__ void grid_arc(const DevNet& net, const u64* view, u64
 template <bool kCoherent>
 __device__ __forceinline__ void grid_round(const DevNet& net, const u64* view, u64* dom, int* size,
                                            const unsigned* cur, unsigned* nxt, GacCtl* ctl, int r, int seed,
-                                           bool kept, const int4& e0, int narcs, int& revs, int& dels) {
+                                           bool pairs, bool kept, const int4& e0, int narcs, int& revs, int& dels) {
   const int W = net.W, lane = lane_id();
   int lw = 0;
   while ((1 << lw) < W) ++lw;
@@ -340,7 +344,8 @@ __device__ __forceinline__ void grid_round(const DevNet& net, const u64* view, u
     const long long i = base + (W > 1 ? (long long)(lane >> lw) * nwaves + gw : (long long)gw * 64 + lane);
     const int4 e = kept && base == 0 ? e0 : (i < narcs ? net.adj[i] : none);
     const int t = adj_var(e), u = e.y;
-    const bool act = u >= 0 && w < W && (r > 0 ? changed(t) : (seed < 0 || t == seed || u == seed));
+    const bool act =
+        u >= 0 && w < W && (r > 0 ? changed(t) || (pairs && changed(u)) : (seed < 0 || t == seed || u == seed));
     const u64 m = __ballot(act && w == 0);
     if (__ballot(act) == 0ull) continue;
     revs += __popcll(m);
@@ -351,7 +356,12 @@ __device__ __forceinline__ void grid_round(const DevNet& net, const u64* view, u
     const int c = uniform_int(net.tabs[k]);
     const ConMeta* mp = net.con + c;
     const int y = lane < mp->arity ? mp->scope[lane] : -1;
-    if (__ballot(y >= 0 && (r > 0 ? changed(y) : (seed < 0 || y == seed))) == 0ull) continue;
+    const u64 some = __ballot(y >= 0 && (r > 0 ? changed(y) : (seed < 0 || y == seed)));
+    if (some == 0ull) continue;
+    // one changed variable of a frontier of variables: its own position stays
+    int skip = -1;
+    if (!pairs && seed >= 0 && r > 0 && (some & (some - 1ull)) == 0ull)
+      skip = __builtin_amdgcn_readlane(y, (int)__builtin_ctzll(some));
     bool wiped = false;
     auto on_removed = [&](int v, int n) {
       if (lane == 0) {
@@ -359,7 +369,7 @@ __device__ __forceinline__ void grid_round(const DevNet& net, const u64* view, u
         atomicOr(&nxt[v >> 5], 1u << (v & 31));
       }
     };
-    revise_table<decltype(on_removed), true>(net, dom, size, c, -1, nullptr, on_removed, &wiped);
+    revise_table<decltype(on_removed), true>(net, dom, size, c, skip, nullptr, on_removed, &wiped);
     ++revs;
     if (wiped && lane == 0) atomicMin(&ctl->wipe_round, r);
   }
@@ -513,8 +523,9 @@ constexpr int kRoundThreads = 1024;
 // One round per launch (host-driven fixpoint).  A launch queued behind the
 // round that ended the fixpoint only answers.
 __global__ void __launch_bounds__(kRoundThreads) k_gac_round(DevNet net, u64* dom, int* size, unsigned* F, int nvw,
-                                                             GacCtl* ctl, int r, int seed, int narcs, GacResult* out,
-                                                             unsigned long long* seq_at, unsigned long long seq) {
+                                                             GacCtl* ctl, int r, int seed, int pairs, int narcs,
+                                                             GacResult* out, unsigned long long* seq_at,
+                                                             unsigned long long seq) {
   __shared__ GridEnd end;
   if (r > 0 && (ctl->last_push_round < r - 1 || ctl->wipe_round < r)) {
     if (blockIdx.x == 0 && threadIdx.x == 0) box_store(seq_at, seq);
@@ -531,7 +542,7 @@ __global__ void __launch_bounds__(kRoundThreads) k_gac_round(DevNet net, u64* do
     F[(long long)((r + 2) % 3) * nvw + i] = 0u;
   int revs = 0, dels = 0;
   grid_round<false>(net, dom, dom, size, F + (long long)(r % 3) * nvw, F + (long long)((r + 1) % 3) * nvw, ctl, r, seed,
-                    false, make_int4(0, -1, 0, 0), narcs, revs, dels);
+                    pairs != 0, false, make_int4(0, -1, 0, 0), narcs, revs, dels);
   // the epoch only grows: skip the atomic once another wave has raised it
   if (__ballot(dels > 0) && lane_id() == 0 && ld_agent(&ctl->last_push_round) < r) atomicMax(&ctl->last_push_round, r);
   grid_finish(ctl, F, nvw, &end, revs, dels, r + 1, 0, 0ull, [&](int lp, int wr) { return lp < r || wr <= r; }, out,
@@ -615,7 +626,8 @@ __host__ __device__ inline long long persistent_lds_bytes(int n, int W) {
 template <bool kStaged>
 __global__ void __launch_bounds__(kPersistentThreads) k_gac_persistent(DevNet net, u64* dom, int* size, unsigned* F,
                                                                        int nvw, GacCtl* ctl, int max_rounds, int seed,
-                                                                       int narcs, unsigned long long max_ticks,
+                                                                       int pairs, int narcs,
+                                                                       unsigned long long max_ticks,
                                                                        GacResult* out, unsigned long long* seq_at,
                                                                        unsigned long long seq) {
   extern __shared__ __align__(16) char smem[];
@@ -647,8 +659,8 @@ __global__ void __launch_bounds__(kPersistentThreads) k_gac_persistent(DevNet ne
     unsigned* nxt = F + (long long)((r + 1) % 3) * nvw;
     for (long long i = i0; i < nvw; i += (long long)gridDim.x * blockDim.x)
       __hip_atomic_store(&F[(long long)((r + 2) % 3) * nvw + i], 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    if (kStaged) grid_round<false>(net, sdom, dom, size, scur, nxt, ctl, r, seed, true, e0, narcs, revs, dels);
-    else grid_round<true>(net, dom, dom, size, cur, nxt, ctl, r, seed, true, e0, narcs, revs, dels);
+    if (kStaged) grid_round<false>(net, sdom, dom, size, scur, nxt, ctl, r, seed, pairs != 0, true, e0, narcs, revs, dels);
+    else grid_round<true>(net, dom, dom, size, cur, nxt, ctl, r, seed, pairs != 0, true, e0, narcs, revs, dels);
     if (!grid_barrier(ctl, gridDim.x, t0, max_ticks, &s_ok)) {
       decision = ERROR;
       break;
