@@ -1252,15 +1252,18 @@ __device__ __forceinline__ bool wg_fixpoint(const DevNet& net, const WgMem& mem,
       if (changed == 0ull) continue;
       ++revs;
       if (small) {
-        // lane 8 p removes for position p
+        // lane 8 p removes for position p, but not for the only changed one
         u64 rows[8];
         small_table_rows(tab, rows);
         const unsigned gone = (unsigned)dp & ~small_table_keep(tab.y, tab.tw, rows, (unsigned)dp);
-        if (gone && y >= 0 && !assigned && lane < 32 && (lane & 7) == 0)
+        const unsigned pos = (unsigned)changed & 0x01010101u;
+        const u64 stays = both || (pos & (pos - 1u)) ? 0ull : pos;
+        if (gone && y >= 0 && !assigned && lane < 32 && (lane & 7) == 0 && !((stays >> lane) & 1ull))
           lane_remove(mem, ctl, nxt, slot, round, y, &mem.dom[y], (u64)gone);
         continue;
       }
-      // one changed variable: its own values keep their supports
+      // one changed variable: its own position is not revised (AC3 does not
+      // either, src/AC3.cpp:106-118; at a closure its values keep their supports)
       int skip = -1;
       if (!both && (changed & (changed - 1ull)) == 0ull) skip = __builtin_amdgcn_readlane(y, (int)__builtin_ctzll(changed));
       bool wiped = false;

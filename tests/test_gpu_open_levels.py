@@ -7,7 +7,7 @@ depends on what it looks at again, and that is part of each mode's answer:
 * host-driven, persistent, allocation-free and asynchronous fixpoints keep a
   frontier of constraints, as GModel::EnforceGAC does (src/GModel.cu:1110-1220):
   every position of a constraint is revised once one of its variables changed;
-* the workgroup fixpoint keeps a frontier of variables, as
+* the workgroup fixpoint and the singleton tests keep a frontier of variables, as
   AC3 does (src/AC3.cpp:99-141): a position is revised once another of the
   constraint's variables changed; a seeded fixpoint revises every position of
   the seed's constraints too.
@@ -96,10 +96,10 @@ MODES = {
     "auto": (None, lambda m, v: m.EnforceGAC_Auto(v)),
 }
 
-# n, d, e, t, tables, tuples: one and two words, with and without tables,
+# n, d, e, t, tables, tuples: one and two words, small tables and larger ones,
 # and 300, 1,000 and 4,200 constraints
 SHAPES = [
-    (60, 8, 90, 0.55, 0, 0), (40, 70, 60, 0.925, 0, 0), (40, 20, 40, 0.72, 14, 400),
+    (60, 8, 90, 0.55, 0, 0), (60, 8, 90, 0.45, 20, 60), (40, 70, 60, 0.925, 0, 0), (40, 20, 40, 0.72, 14, 400),
     (200, 6, 1000, 0.30, 0, 0), (200, 6, 950, 0.26, 60, 70), (600, 6, 4200, 0.27, 0, 0),
 ]
 
@@ -126,3 +126,15 @@ def test_seeded_fixpoint_on_an_open_level(gpu, shape, mode):
                 got = domains_to_sets(m.ReadDomains(0), desc.dom_size)
                 assert [set(g) for g in got] == want, seed
     assert other, "the two frontiers agree on every seed: the shape tests nothing"
+
+
+@pytest.mark.parametrize("shape", [s for s in SHAPES if s[2] < 1000], ids=str)
+def test_workgroup_singleton_tests_on_an_open_level(gpu, shape):
+    n, d, e, t, tables, tuples = shape
+    desc, sets = network(n, d, e, t, tables, 1, tuples)
+    tests = [(v, a) for v, s in enumerate(sets) for a in sorted(s)][::max(1, n * d // 150)]
+    want = [seeded_closure(desc, sets[:v] + [{a}] + sets[v + 1:], v, "assigned") is None for v, a in tests]
+    with GModelAdapter.Build(desc, GModelOptions(skip_non_binary=False)) as m:
+        m.WriteDomains(0, words(sets, m.dom_words))
+        got, _ = m.SingletonTests(np.array(tests, np.int32), mode="workgroup")
+    assert got.astype(bool).tolist() == want
