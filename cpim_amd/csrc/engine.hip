@@ -686,6 +686,19 @@ struct cpim_gmodel {
   int nfw = 0;     // words of a bitmap of the constraints
   int nvw = 0;     // words of a bitmap of the variables
   std::vector<int2> assigned;  // d_assigned mirror: (var, value) per level
+  // per level: at its closure (a fixpoint ended consistent and nothing wrote
+  // since), closed but for the domain of one variable (its id), or open
+  enum : int { kOpen = -2, kClosed = -1 };
+  std::vector<int> closure;
+  void wrote(int level, int var) {
+    int& c = closure[level];
+    c = c == kClosed || c == var ? var : kOpen;
+  }
+  // the fixpoint over every constraint (var < 0) or from var ended
+  void settled(int level, int before, int var, const cpim_gac_stats& st) {
+    const bool all = var < 0 || before == kClosed || before == var;
+    closure[level] = st.converged && !st.inconsistent && all ? kClosed : kOpen;
+  }
   DevProps props;
   SacScratch sac;
   hipEvent_t gev[2] = {nullptr, nullptr};  // kernel timing of the fixpoint entry points
@@ -879,6 +892,7 @@ int cpim_gmodel_create(const cpim_model_desc* desc, const cpim_gmodel_options* o
                        m->level_size(0), n, m->dm.W);
     HIPC(hipGetLastError());
     m->assigned.assign(m->max_depth, make_int2(-1, -1));
+    m->closure.assign(m->max_depth, cpim_gmodel::kOpen);
     m->dm.bytes += dom_bytes + size_bytes + front_bytes + (long long)sizeof(GacCtl);
     m->sync();
     *out = m.release();
@@ -1147,6 +1161,8 @@ void gac(cpim_gmodel* m, int assigned_var, int mode, cpim_gac_stats* st) {
     st->converged = 1;
     return;
   }
+  const int L = m->current_level, before = m->closure[L];
+  m->closure[L] = cpim_gmodel::kOpen;
   switch (mode) {
     case CPIM_GAC_PLAIN: gac_grid(m, assigned_var, false, st, by_variable); break;
     case CPIM_GAC_PERSISTENT: gac_grid(m, assigned_var, true, st); break;
@@ -1154,6 +1170,7 @@ void gac(cpim_gmodel* m, int assigned_var, int mode, cpim_gac_stats* st) {
     case CPIM_GAC_ASYNC: gac_async(m, assigned_var, st); break;
     default: fail(CPIM_ERR_INVALID_ARGUMENT, "unknown GAC mode " + std::to_string(mode));
   }
+  m->settled(L, before, assigned_var, *st);
 }
 
 void check_var(const cpim_gmodel* m, int var, const char* fn) {
@@ -1188,6 +1205,7 @@ void read_level(const cpim_gmodel* m, int level, u64* out) {
 template <typename Fill>
 void write_level(cpim_gmodel* m, int level, Fill&& fill) {
   const int n = m->dm.n, W = m->dm.W;
+  m->closure[level] = cpim_gmodel::kOpen;
   if (!m->level_in_box()) {
     std::vector<u64> w((size_t)m->level_words());
     fill(w.data());
@@ -1228,6 +1246,7 @@ int cpim_gmodel_create_new_level(cpim_gmodel* m, int32_t* new_level) {
       fail(CPIM_ERR_RUNTIME, "[GModel::CreateNewLevel] Max depth reached: " + std::to_string(m->max_depth));
     DeviceGuard g(m->device);
     const int L = ++m->current_level;
+    m->closure[L] = m->closure[L - 1];
     if (m->level_in_box()) {
       const unsigned long long seq = m->next_seq();
       hipLaunchKernelGGL(k_level_copy, dim3(1), dim3(1024), 0, m->stream, m->level_dom(L - 1), m->level_dom(L),
@@ -1273,6 +1292,7 @@ int cpim_gmodel_assign_value(cpim_gmodel* m, int32_t var, int32_t value, int32_t
     if (value < 0 || value >= m->dm.max_dom)
       fail(CPIM_ERR_RUNTIME, "[GModel::AssignValue] Invalid value: " + std::to_string(value));
     DeviceGuard g(m->device);
+    m->wrote(level, var);
     m->level_op(kOpAssign, level, var, value);
     m->assigned[level] = make_int2(var, value);
     m->assigned_size = std::max(m->assigned_size, level + 1);
@@ -1288,6 +1308,7 @@ int cpim_gmodel_remove_value(cpim_gmodel* m, int32_t var, int32_t value, int32_t
     *ok = 0;
     if (value < 0 || value >= m->dm.max_dom) return;
     DeviceGuard g(m->device);
+    m->wrote(level, var);
     *ok = m->level_op(kOpRemove, level, var, value) > 0;
   });
 }
@@ -1801,8 +1822,12 @@ bool few_arc_words(const cpim_gmodel* m, long long tests) {
 
 void run_singleton_device(cpim_gmodel* m, int mode, const int2* tests, long long count, unsigned char* fail_out,
                           cpim_sac_stats* st, SacScratch& S) {
+  // (on an open level the two kernels answer differently: a bit-sliced test
+  // sees what the other tests of its group revise, so it stays the choice there)
+  const bool closed = m->closure[m->current_level] == cpim_gmodel::kClosed;
   if (mode == CPIM_SAC_BATCHED)
-    mode = sliced_eligible(m) && !(fits_lds(m) && few_arc_words(m, count)) ? CPIM_SAC_SLICED : CPIM_SAC_WORKGROUP;
+    mode = sliced_eligible(m) && !(closed && fits_lds(m) && few_arc_words(m, count)) ? CPIM_SAC_SLICED
+                                                                                     : CPIM_SAC_WORKGROUP;
   if (mode == CPIM_SAC_SLICED) {
     if (!sliced_eligible(m))
       fail(CPIM_ERR_UNSUPPORTED, "bit-sliced singleton tests need a binary network whose work lists fit in LDS");
@@ -1821,6 +1846,7 @@ void run_singleton_plain(cpim_gmodel* m, const int2* tests, long long count, uns
   const int L = m->current_level;
   if (L + 1 >= m->max_depth) fail(CPIM_ERR_RUNTIME, "no free level for singleton tests");
   const int T = L + 1;
+  m->closure[T] = cpim_gmodel::kOpen;
   const long long t0 = now_ns();
   std::vector<u64> word(m->dm.W);
   const int one = 1;
@@ -1981,6 +2007,7 @@ int cpim_gmodel_solve(cpim_gmodel* m, const cpim_solve_opts* opts, cpim_search_s
     REQUIRE(m->current_level == 0, "the device solver starts from level 0");
     DeviceGuard g(m->device);
     std::memset(st, 0, sizeof(*st));
+    m->closure[0] = cpim_gmodel::kOpen;  // until the root closure is back
     const int n = m->dm.n;
     const long long t0 = now_ns();
     const long long sol_cap = std::max<long long>(1, o.solution_capacity);
@@ -2090,6 +2117,7 @@ int cpim_gmodel_solve(cpim_gmodel* m, const cpim_solve_opts* opts, cpim_search_s
                        m->dm.W);
     HIPC(hipGetLastError());
     m->sync();
+    if (!(s.status == MAC_UNSAT && s.npos + s.nneg == 0)) m->closure[0] = cpim_gmodel::kClosed;
   });
 }
 

@@ -138,3 +138,18 @@ def test_workgroup_singleton_tests_on_an_open_level(gpu, shape):
         m.WriteDomains(0, words(sets, m.dom_words))
         got, _ = m.SingletonTests(np.array(tests, np.int32), mode="workgroup")
     assert got.astype(bool).tolist() == want
+
+
+@pytest.mark.parametrize("shape", [(60, 8, 90, 0.6), (60, 8, 100, 0.6), (80, 6, 140, 0.5), (50, 30, 90, 0.85)], ids=str)
+def test_auto_singleton_tests_on_an_open_level(gpu, shape):
+    """Binary networks: on an open level a bit-sliced test sees what the other
+    tests of its group revise as well, so which tests fail depends on the
+    kernel, and the automatic choice stays with the bit-sliced one there."""
+    n, d, e, t = shape
+    desc, sets = network(n, d, e, t, 0, 1)
+    tests = np.array([(v, a) for v, s in enumerate(sets) for a in sorted(s)], np.int32)
+    with GModelAdapter.Build(desc) as m:
+        m.WriteDomains(0, words(sets, m.dom_words))
+        got = {mode: m.SingletonTests(tests, mode=mode)[0] for mode in ("auto", "sliced", "workgroup")}
+        assert (got["sliced"] != got["workgroup"]).any(), "the two kernels agree: the shape tests nothing"
+        assert (got["auto"] == got["sliced"]).all()
