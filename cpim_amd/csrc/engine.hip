@@ -645,6 +645,7 @@ HostBox* take_box() {
   HIPC(hipHostMalloc(&p, sizeof(HostBox) + kBoxDataBytes, hipHostMallocPortable | hipHostMallocMapped | hipHostMallocCoherent));
   HostBox* b = static_cast<HostBox*>(p);
   b->seq = 0;
+  b->issued = 0;
   return b;
 }
 
@@ -721,12 +722,14 @@ struct cpim_gmodel {
     HIPC(hipStreamSynchronize(stream));  // `ones` is host stack memory
   }
 
-  // The box and the number of the next call that answers in it.
+  // The box and the number of the next call that answers in it (counted by the
+  // host: a launch that failed may leave earlier ones queued, which still
+  // store their numbers).
   HostBox* box() const {
     if (!box_) box_ = take_box();
     return box_;
   }
-  unsigned long long next_seq() const { return box()->seq + 1; }
+  unsigned long long next_seq() const { return ++box()->issued; }
 
   // Waits for call `seq` (its kernel is the last work queued on the stream):
   // the kernel's answer arrives a few microseconds before the runtime reports
@@ -1043,15 +1046,18 @@ void gac_grid(cpim_gmodel* m, int assigned_var, bool persistent, cpim_gac_stats*
     bool over = false;
     for (int r0 = 0, ahead = 1; r0 < max_rounds && !over; r0 += ahead, ahead = std::min(2 * ahead, kRoundsAhead)) {
       const int k = (int)std::min<long long>(ahead, max_rounds - r0);
-      for (int i = 0; i < k; ++i, ++seq) {
+      for (int i = 0; i < k; ++i) {
+        if (r0 + i > 0) seq = m->next_seq();
         answers[i].rounds = 0;  // stays 0 if the fixpoint was over before
         hipLaunchKernelGGL(k_gac_round, dim3(grid), dim3(kRoundThreads), 0, m->stream, net, m->level_dom(L),
                            m->level_size(L), F, m->nvw, ctl, r0 + i, assigned_var,
                            assigned_var >= 0 && !by_variable ? 1 : 0, (int)m->im.adj.size(), &answers[i], &box->seq,
                            seq);
-        HIPC(hipGetLastError());
+        const hipError_t e = hipGetLastError();
+        if (e != hipSuccess) (void)hipStreamSynchronize(m->stream);  // the rounds queued before answer in the box
+        HIPC(e);
       }
-      m->wait_box(seq - 1);
+      m->wait_box(seq);
       for (int i = 0; i < k && !over; ++i) {
         if (answers[i].rounds == 0) continue;
         res = answers[i];

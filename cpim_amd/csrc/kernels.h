@@ -225,7 +225,8 @@ struct GacResult {
 // through to host memory), waits until they have completed, and stores the
 // call's number in `seq`, on which the host waits.
 struct HostBox {
-  unsigned long long seq;
+  unsigned long long seq;     // the last call answered
+  unsigned long long issued;  // the last call numbered (the host's)
   int scalar;
   int pad;
   GacResult gac;
