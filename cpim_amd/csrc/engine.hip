@@ -5,6 +5,7 @@
 #include <atomic>
 #include <chrono>
 #include <climits>
+#include <cmath>
 #include <cstdio>
 #include <cstdlib>
 #include <cstring>
@@ -128,6 +129,9 @@ struct ModelImage {
   std::vector<int> bin_cons;          // active indices of binary constraints (plane build order)
   std::vector<int> tabs;              // active indices of table constraints
   bool simple = true;                 // no two binary constraints have the same scope
+  int max_deg = 0;                    // most constraints on one variable
+  double reach = 0.0;                 // arcs of a variable and of its neighbours, mean over the values
+  double density = 0.0;               // allowed share of the binary tuples (sample_density)
   std::vector<u64> rel_dense;         // owned dense rows when the desc has none
   const u64* rel = nullptr;           // [nb][max_dom][rel_words]
   int rel_words = 0;
@@ -136,6 +140,24 @@ struct ModelImage {
   std::vector<u64> init_dom;          // [n][W]
   std::vector<int> nbr;               // [n] distinct neighbours over the active constraints, then tabs
 };
+
+// Share of the tuples that the binary constraints allow, from at most 8 rows
+// each of at most 32 constraints.
+double sample_density(const ModelImage& im) {
+  const size_t nb = im.bin_cons.size();
+  long long ones = 0, all = 0;
+  for (size_t i = 0; i < std::min<size_t>(nb, 32); ++i) {
+    const size_t k = i * nb / std::min<size_t>(nb, 32);
+    const ConMeta& m = im.con[im.bin_cons[k]];
+    const int cx = im.cap[m.scope[0]], rows = std::min(cx, 8);
+    for (int j = 0; j < rows; ++j) {
+      const u64* row = im.rel + (k * im.max_dom + (size_t)j * cx / rows) * im.rel_words;
+      for (int w = 0; w < im.W; ++w) ones += __builtin_popcountll(row[w]);
+    }
+    all += (long long)rows * im.cap[m.scope[1]];
+  }
+  return all ? std::min(1.0, (double)ones / (double)all) : 1.0;
+}
 
 ModelImage make_image(const cpim_model_desc* d, bool skip_non_binary, bool own_rel = false) {
   REQUIRE(d != nullptr, "model description is null");
@@ -292,6 +314,17 @@ ModelImage make_image(const cpim_model_desc* d, bool skip_non_binary, bool own_r
       }
   }
   im.nbr.insert(im.nbr.end(), im.tabs.begin(), im.tabs.end());
+  double values = 0.0;
+  for (int v = 0; v < im.n; ++v) {
+    long long arcs = deg[v];
+    for (int k = im.adj_off[v]; k < im.adj_off[v + 1]; ++k)
+      if (im.adj[k].y >= 0) arcs += deg[im.adj[k].y];
+    im.max_deg = std::max(im.max_deg, deg[v]);
+    im.reach += (double)std::min<long long>(arcs, (long long)im.adj.size()) * im.cap[v];
+    values += im.cap[v];
+  }
+  im.reach /= values;
+  im.density = sample_density(im);
   // level 0
   im.init_dom.assign(nw, 0ull);
   for (int v = 0; v < im.n; ++v)
@@ -1806,24 +1839,50 @@ void run_singleton_sliced(cpim_gmodel* m, const int2* tests_host, long long coun
 void run_singleton_plain(cpim_gmodel* m, const int2* tests, long long count, unsigned char* fail_host,
                          cpim_sac_stats* st);
 
-// CPIM_SAC_BATCHED: one workgroup per test for networks with tables and for
-// passes with little work, the bit-sliced kernels otherwise.  The estimate is
-// the arc words of the tests' first two rounds: the deg arcs of the tested
-// variable, then those of its deg neighbours, at most all.  A bit-sliced
-// group walks its changed variables one after another, 5 us and more each,
-// with one group per variable: passes that do not fill the chip wait on that
-// chain, where one workgroup per test has a test's rounds only.  Measured,
-// workgroup against sliced, per pass: n=60 d=37 e=500 (0.6M arc words) 0.03
-// against 0.11 ms, at tightness 0.655 (cascades) 0.18 against 1.79 ms; n=120
-// d=50 e=3570 (21M) 0.24 against 0.68 ms; n=100 d=100 e=1500 (18M) 0.35
-// against 0.36 ms; n=200 d=64 e=4000 (20M) 0.34 against 0.41 ms; n=200 d=128
-// e=3000 (46M) 0.96 against 0.41 ms; n=300 d=200 e=6000 (384M) 8.3 against
-// 1.3 ms.
-constexpr long long kWorkgroupArcWords = 22ll << 20;
-
-bool few_arc_words(const cpim_gmodel* m, long long tests) {
-  const double arcs = (double)m->im.adj.size(), deg = arcs / m->dm.n;
-  return (double)tests * std::min(arcs, deg * (deg + 1.0)) * m->dm.W <= (double)kWorkgroupArcWords;
+// CPIM_SAC_BATCHED: one workgroup per test for networks with tables and where
+// the estimates below say so, the bit-sliced kernels otherwise.  Both estimates
+// are of a pass without cascades, in microseconds:
+//  * workgroups: as many turns of the resident workgroups as the tests take,
+//    each about 18 plus its arc words in two rounds (`reach`);
+//  * bit-sliced: the variables that a group of 64 M tests changes, walked one
+//    after another, about 8 each; where one variable has far more constraints
+//    than the others (a star), the group that tests it walks that many.
+// With cascades a bit-sliced group walks every variable that any of its tests
+// changes, and workgroups win up to some 24 x 2^20 arc words (n=480 d=256 e=4800
+// t=0.887, 215M: 276 against 30 ms; n=300 d=100 e=3000 t=0.826, 26M: 25.5
+// against 33.5 ms).  A variable whose neighbour kept p d values loses a value to
+// it with probability (1 - p)^(p d); 50 values lost to deg neighbours are the
+// line (24 lost at n=300 d=64 e=1000 t=0.80, 965 against 631 us; 73 at t=0.84,
+// 1350 against 4026 us).
+// A long chain (a path, a lattice) takes about as many rounds as it changes
+// variables, and every turn of workgroups pays for all of them: there a group's
+// variables, times the arcs within reach over a path's six, must outnumber the
+// turns.  Measured, workgroups against bit-sliced, us:
+//   n=60 d=37 e=500      88 / 173, cascading 330 / 2899
+//   n=120 d=50 e=3570   309 / 761      n=200 d=64 e=4000   379 / 503
+//   n=100 d=100 e=1500  347 / 421      n=500 d=16 e=3000   171 / 342
+//   n=200 d=64 e=800    182 / 157, cascading 1572 / 5611
+//   n=60 d=300 e=300    427 / 341, cascading 6686 / 26152
+//   n=100 d=128 e=600   215 / 199      n=200 d=128 e=2000  616 / 398
+//   star n=600 d=64     684 / 1309     star n=2000 d=64    6977 / 5211
+//   path n=60 d=37      495 / 355      path n=700 d=64     148098 / 8566
+//   lattice 25x25 d=16  196 / 242      lattice 25x25 d=40  608 / 216
+bool tests_by_workgroup(const cpim_gmodel* m, long long tests) {
+  const long long bytes = wg_mem_bytes(m->dm.n, m->dm.W);
+  if (bytes > kLdsBudget) return false;
+  const double cus = std::max(1, m->props.cus), W = m->dm.W, d = m->dm.max_dom;
+  const double per_cu = (double)std::min<long long>(8, std::max<long long>(1, m->props.max_lds / (bytes + 512)));
+  const double turns = (double)tests / (cus * per_cu);
+  const int M = std::max(1, wide_masks_for(m, tests));
+  const double deg = (double)m->im.adj.size() / m->dm.n;
+  const double vars = std::max(1.0, 64.0 * M / d);
+  const double waves = std::max(1.0, std::ceil((double)tests / (64.0 * M * 2.0 * cus)));
+  const double by_wg = turns * (18.0 + m->im.reach * W / 50.0);
+  const double sliced = waves * (vars * (1.0 + deg) * (7.5 + 0.5 * W) + 2.5 * (m->im.max_deg - deg));
+  const double p = m->im.density;
+  const bool cascades =
+      (double)tests * m->im.reach * W <= (double)(24ll << 20) && d * deg * std::pow(1.0 - p, p * d) >= 50.0;
+  return (cascades || by_wg <= sliced) && 1.6 * turns <= vars * std::max(1.0, m->im.reach / (cascades ? 3.0 : 6.0));
 }
 
 void run_singleton_device(cpim_gmodel* m, int mode, const int2* tests, long long count, unsigned char* fail_out,
@@ -1832,8 +1891,7 @@ void run_singleton_device(cpim_gmodel* m, int mode, const int2* tests, long long
   // sees what the other tests of its group revise, so it stays the choice there)
   const bool closed = m->closure[m->current_level] == cpim_gmodel::kClosed;
   if (mode == CPIM_SAC_BATCHED)
-    mode = sliced_eligible(m) && !(closed && fits_lds(m) && few_arc_words(m, count)) ? CPIM_SAC_SLICED
-                                                                                     : CPIM_SAC_WORKGROUP;
+    mode = sliced_eligible(m) && !(closed && tests_by_workgroup(m, count)) ? CPIM_SAC_SLICED : CPIM_SAC_WORKGROUP;
   if (mode == CPIM_SAC_SLICED) {
     if (!sliced_eligible(m))
       fail(CPIM_ERR_UNSUPPORTED, "bit-sliced singleton tests need a binary network whose work lists fit in LDS");
