@@ -113,9 +113,8 @@ __device__ __forceinline__ u64 wave_settle(const DevNet& net, const u64* dom, lo
 // relation.  Target side: an open value is settled by the W words of its own
 // row, by the lane, four reads a step.  Lanes that tight relations leave with
 // more than 12 steps per four words of a domain (never one-word domains) are
-// settled by the wave, one after the other (wave_settle; kTight: the search
-// kernels leave that path out, whose networks are loose enough to be found a
-// solution in, and which lose 10% to its registers).
+// settled by the wave, one after the other (wave_settle; kTight: the searches
+// take that path only on networks of wide domains and many constraints).
 template <bool kCoherent, bool kTight>
 __device__ __forceinline__ u64 arcs_unsupported(const DevNet& net, const u64* dom, long long off, int src, int pos_src,
                                                 int w, u64 need) {
@@ -3177,8 +3176,8 @@ __device__ __forceinline__ void wg_load_level(const WgMem& mem, const u64* level
 // one, beside the fixpoint's own.  kWdeg: dom/wdeg ordering, wipe-outs
 // repeated in AC3's order.  kFlat: wg_fixpoint_flat propagates, and a
 // refutation that follows its decision takes the domains from registers (dom
-// and dom/deg only).
-template <bool kWdeg, bool kFlat>
+// and dom/deg only).  kTight: tight relations are settled by the wave.
+template <bool kWdeg, bool kFlat, bool kTight>
 __device__ __forceinline__ void wg_mac_run(const DevNet& net, const WgMem& mem, WgCtl* ctl, const MacArgs& A) {
   enum { ROOT, POSITIVE, NEGATIVE };
   const int n = net.n, W = net.W;
@@ -3328,7 +3327,7 @@ __device__ __forceinline__ void wg_mac_run(const DevNet& net, const WgMem& mem, 
       ok = wg_fixpoint_flat(mem, ctl, flat, seen, phase == ROOT ? -1 : x, phase == POSITIVE ? bit : dx & ~bit,
                             phase == POSITIVE, turn, flat_revs);
     } else {
-      ok = wg_fixpoint<false>(net, mem, ctl, slot, false);
+      ok = wg_fixpoint<kTight>(net, mem, ctl, slot, false);
     }
     if (kWdeg && !ok) {
       // a wipe-out raises the weight of the constraint that AC3's order
@@ -3434,8 +3433,9 @@ __device__ __forceinline__ void wg_mac_run(const DevNet& net, const WgMem& mem, 
 }
 
 // lnet.bytes > 0 (kLds only): the network image is copied into LDS behind
-// the working memory and the search reads the network from there.
-template <bool kLds, bool kWdeg>
+// the working memory and the search reads the network from there.  kTight: the
+// network is one for the tight path (tight_search; it has no image).
+template <bool kLds, bool kWdeg, bool kTight>
 __global__ void k_mac(DevNet net, MacArgs args, char* scratch, LdsNet lnet) {
   extern __shared__ __align__(16) char smem[];
   __shared__ WgCtl ctl;
@@ -3445,12 +3445,12 @@ __global__ void k_mac(DevNet net, MacArgs args, char* scratch, LdsNet lnet) {
     const DevNet ln = wg_load_net(net, lnet, smem + wg_mem_bytes(net.n, net.W));
     WgMem mem = wg_carve(smem, ln);
     mem.stamp = stamp;
-    if (!kWdeg && lnet.flat_min && lnet.flat_min <= (int)blockDim.x) wg_mac_run<false, true>(ln, mem, &ctl, args);
-    else wg_mac_run<kWdeg, false>(ln, mem, &ctl, args);
+    if (!kWdeg && lnet.flat_min && lnet.flat_min <= (int)blockDim.x) wg_mac_run<false, true, false>(ln, mem, &ctl, args);
+    else wg_mac_run<kWdeg, false, false>(ln, mem, &ctl, args);
   } else {
     WgMem mem = wg_carve(kLds ? smem : scratch, net);
     mem.stamp = stamp;
-    wg_mac_run<kWdeg, false>(net, mem, &ctl, args);
+    wg_mac_run<kWdeg, false, kTight>(net, mem, &ctl, args);
   }
 }
 
@@ -3465,12 +3465,15 @@ struct UnitDesc {
   long long scratch_off;  // per-unit global scratch when the domain does not fit in LDS
   int use_lds;            // 1: working memory in LDS; 2: network image in LDS as well
   int reset;              // 1: start the search over: level 0 = init, state = MAC_INIT
+  int tight;              // 1: the fixpoints keep the tight path (k_mac_units<true>)
   const u64* init;        // the unit's initial domains, [n][W]
   LdsNet lnet;
 };
 
 // states_out[u] receives a copy of unit u's state when its launch ends, so
-// the host reads every unit's outcome with one copy.
+// the host reads every unit's outcome with one copy.  kTight: launches with a
+// unit for the tight path (the others of it still leave it out).
+template <bool kTight>
 __global__ void k_mac_units(const UnitDesc* __restrict__ units, int count, unsigned* counter,
                             int only, char* scratch, MacState* states_out) {
   extern __shared__ __align__(16) char smem[];
@@ -3503,13 +3506,16 @@ __global__ void k_mac_units(const UnitDesc* __restrict__ units, int count, unsig
     if (where == 2) {
       const DevNet ln = wg_load_net(d.net, d.lnet, smem + wg_mem_bytes(d.net.n, d.net.W));
       if (uniform_int(d.lnet.flat_min && d.lnet.flat_min <= (int)blockDim.x))
-        wg_mac_run<false, true>(ln, wg_carve(smem, ln), &ctl, d.args);
+        wg_mac_run<false, true, false>(ln, wg_carve(smem, ln), &ctl, d.args);
       else
-        wg_mac_run<false, false>(ln, wg_carve(smem, ln), &ctl, d.args);
+        wg_mac_run<false, false, false>(ln, wg_carve(smem, ln), &ctl, d.args);
     } else if (where == 1) {
-      wg_mac_run<false, false>(d.net, wg_carve(smem, d.net), &ctl, d.args);
+      if (kTight && uniform_int(d.tight)) wg_mac_run<false, false, kTight>(d.net, wg_carve(smem, d.net), &ctl, d.args);
+      else wg_mac_run<false, false, false>(d.net, wg_carve(smem, d.net), &ctl, d.args);
     } else {
-      wg_mac_run<false, false>(d.net, wg_carve(scratch + d.scratch_off, d.net), &ctl, d.args);
+      const WgMem mem = wg_carve(scratch + d.scratch_off, d.net);
+      if (kTight && uniform_int(d.tight)) wg_mac_run<false, false, kTight>(d.net, mem, &ctl, d.args);
+      else wg_mac_run<false, false, false>(d.net, mem, &ctl, d.args);
     }
     if (threadIdx.x == 0) states_out[u] = *d.args.state;
     if (only >= 0) break;

@@ -3,7 +3,8 @@ the right one (needs an MI355X)."""
 import numpy as np
 import pytest
 
-from cpim_amd import GModelAdapter, workload
+import oracle
+from cpim_amd import Batch, GModelAdapter, workload
 from cpim_amd.model import ModelDesc, domains_to_sets, words_for
 
 pytestmark = pytest.mark.gpu
@@ -57,3 +58,49 @@ def test_sac_pass_takes_the_faster_kernel(gpu, name, make, faster):
     slower = "sliced" if faster == "workgroup" else "workgroup"
     # the kernels are 2.5 to 9 times apart: half-way between them, by ratio
     assert ms["auto"] < (ms[faster] * ms[slower]) ** 0.5, ms
+
+
+@pytest.mark.parametrize("heuristic", ["dom", "dom/wdeg"])
+@pytest.mark.parametrize("n,d,e,t", [
+    # searches settle tight relations by the wave from 12,288 arc words of
+    # three-word domains on: both sides of that line, and wider domains
+    (80, 150, 1535, 0.93), (80, 150, 1536, 0.93), (50, 1000, 600, 0.97), (300, 250, 3000, 0.963),
+])
+def test_tight_search_equals_oracle(gpu, n, d, e, t, heuristic):
+    desc = workload.random_binary(n, d, e, t, workload.instance_seed(42, e))
+    with oracle.var_heuristic(2 if heuristic == "dom/wdeg" else 0):
+        o = oracle.Oracle(desc)
+        want = o.mac(node_limit=40, trace_cap=200)
+        weights = o.weights().copy()
+    with GModelAdapter.Build(desc) as m:
+        st, _, trace = m.Solve(node_limit=40, trace_capacity=200, heuristic=heuristic)
+        assert (st.num_solutions, st.num_positive, st.num_negative) == \
+            (want.num_sol, want.num_positive, want.num_negative)
+        assert trace == want.trace
+        if heuristic == "dom/wdeg":
+            assert (m.Weights() == weights).all()
+
+
+def test_tight_and_other_units_of_a_batch_equal_oracle(gpu):
+    shapes = [(80, 150, 1536, 0.93), (80, 150, 1535, 0.93), (30, 16, 109, 0.4), (25, 140, 90, 0.9), (50, 1000, 600, 0.97)]
+    descs = [workload.random_binary(n, d, e, t, workload.instance_seed(43, e + d)) for n, d, e, t in shapes]
+    for per_unit in (True, False):
+        res, _ = Batch(descs).run(30, persistent=not per_unit)
+        for desc, r in zip(descs, res):
+            want = oracle.Oracle(desc).mac(node_limit=30)
+            assert (r.num_positive, r.num_negative) == (want.num_positive, want.num_negative)
+
+
+@pytest.mark.parametrize("n,d,e,t", [(300, 250, 20000, 0.963), (300, 250, 3000, 0.963)])
+def test_tight_root_of_a_search_takes_no_longer_than_the_fixpoint(gpu, n, d, e, t):
+    # the same workgroup fixpoint; without the tight path the search took twice as long
+    desc = workload.random_binary(n, d, e, t, 5)
+    with GModelAdapter.Build(desc) as m:
+        init = m.ReadDomains(0)
+        block, root = [], []
+        for _ in range(3):
+            m.WriteDomains(0, init)
+            block.append(m.EnforceGAC_Block().kernel_ms)
+            m.WriteDomains(0, init)
+            root.append(m.Solve(node_limit=1)[0].gac_time * 1e3)
+    assert min(root) < 1.4 * min(block)
