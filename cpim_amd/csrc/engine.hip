@@ -1015,11 +1015,23 @@ void gac_start(cpim_gmodel* m, unsigned* F, GacCtl* ctl) {
 }
 
 // Lanes of a grid round: one per word of every arc, words rounded up to a
-// power of two.
-long long grid_lanes(const cpim_gmodel* m) {
+// power of two, and a wave per table.  With several words a wave takes fewer
+// arcs than it has lanes for, down to 16 lanes, as long as there is at most one
+// workgroup per CU (`later`: at most the two that a round launches): what a
+// wave's arcs settle together is done one after the other (wave_settle).
+// Against full waves, us: n=60 d=1024 e=60 t=0.995 785 -> 297, n=100 d=1024
+// e=300 t=0.99 345 -> 149, n=300 d=250 e=4000 t=0.96 131 -> 73.  A full round of
+// loose relations pays for a second workgroup per CU (n=500 d=250 e=20000 t=0.25
+// 20 -> 26); a later round, of the changed variables' arcs only, does not (the
+// same at t=0.963 252 -> 235, at t=0.9 after one assignment 330 -> 246).
+long long grid_lanes(const cpim_gmodel* m, bool later) {
+  const long long arcs = (long long)m->im.adj.size();
+  const long long most = (later ? 2ll : 1ll) * std::max(1, m->props.cus) * kRoundThreads;
   long long wp = 1;
   while (wp < m->dm.W) wp *= 2;
-  return (long long)m->im.adj.size() * wp;
+  long long lanes = arcs * wp;
+  for (int used = 32; wp > 1 && used >= 16 && (later ? lanes : 2 * lanes) <= most; used /= 2) lanes *= 2;
+  return std::max(lanes, 64ll * m->dm.ntabs);
 }
 
 // Largest round copy of the persistent fixpoint in LDS: one workgroup per CU.
@@ -1033,10 +1045,10 @@ constexpr long long kPersistentLdsMax = 128 * 1024;
 void persistent_launch(cpim_gmodel* m, int assigned_var, unsigned* F, GacCtl* ctl, GacResult* out,
                        unsigned long long* seq_at, unsigned long long seq) {
   const int L = m->current_level;
-  const long long lanes = grid_lanes(m);
+  const long long lanes = grid_lanes(m, false);
   const long long lds = persistent_lds_bytes(m->dm.n, m->dm.W);
   const bool staged = lds <= std::min<long long>(kPersistentLdsMax, m->props.max_lds - 1024);
-  const long long want = (std::max(lanes, 64ll * m->dm.ntabs) + kPersistentThreads - 1) / kPersistentThreads;
+  const long long want = (lanes + kPersistentThreads - 1) / kPersistentThreads;
   const int grid = (int)std::max<long long>(1, std::min<long long>(want, m->props.cus));
   const long long max_rounds = (long long)m->dm.n * m->dm.max_dom + 2;
   const int mr = (int)std::min<long long>(max_rounds, INT_MAX);
@@ -1086,9 +1098,11 @@ void gac_grid(cpim_gmodel* m, int assigned_var, bool persistent, cpim_gac_stats*
   } else {
     const DevNet net = m->dm.net();
     const long long max_rounds = (long long)m->dm.n * m->dm.max_dom + 2;
-    const long long lanes = std::max(grid_lanes(m), 64ll * m->dm.ntabs);
-    const int grid = (int)std::max<long long>(
-        1, std::min<long long>((lanes + kRoundThreads - 1) / kRoundThreads, 2ll * m->props.cus));
+    auto blocks = [&](bool later) {
+      const long long k = (grid_lanes(m, later) + kRoundThreads - 1) / kRoundThreads;
+      return (int)std::max<long long>(1, std::min<long long>(k, 2ll * m->props.cus));
+    };
+    const int grid[2] = {blocks(false), blocks(true)};
     // each round of a batch answers in a result of its own
     GacResult* answers = reinterpret_cast<GacResult*>(box->data);
     bool over = false;
@@ -1097,7 +1111,7 @@ void gac_grid(cpim_gmodel* m, int assigned_var, bool persistent, cpim_gac_stats*
       for (int i = 0; i < k; ++i) {
         if (r0 + i > 0) seq = m->next_seq();
         answers[i].rounds = 0;  // stays 0 if the fixpoint was over before
-        hipLaunchKernelGGL(k_gac_round, dim3(grid), dim3(kRoundThreads), 0, m->stream, net, m->level_dom(L),
+        hipLaunchKernelGGL(k_gac_round, dim3(grid[r0 + i > 0 ? 1 : 0]), dim3(kRoundThreads), 0, m->stream, net, m->level_dom(L),
                            m->level_size(L), F, m->nvw, ctl, r0 + i, assigned_var,
                            assigned_var >= 0 && !by_variable ? 1 : 0, (int)m->im.adj.size(), &answers[i], &box->seq,
                            seq);

@@ -275,7 +275,7 @@ struct GacCtl {
   int wipe_round;       // lowest round that emptied a domain
   unsigned long long bar_ticket;  // grid barrier arrivals so far (only grows)
   int err;              // set by a block whose barrier wait ran out of time
-  unsigned done;        // blocks that finished
+  unsigned done;        // blocks of the running launch that finished
   unsigned long long start;  // device clock at the start of the launch
   unsigned long long deletions[kStatSlots];
   unsigned long long revisions[kStatSlots];
@@ -481,7 +481,7 @@ __device__ __forceinline__ void grid_finish(GacCtl* ctl, unsigned* F, int nvw, G
     e->tot[1] = 0ull;
     wait_memory_ops();
     const unsigned ticket = atomicAdd(&ctl->done, 1u);
-    e->last = (ticket + 1u) % gridDim.x == 0u ? 1 : 0;
+    e->last = ticket + 1u == gridDim.x ? 1 : 0;
   }
   __syncthreads();
   if (uniform_int(e->last) == 0) return;
@@ -499,9 +499,11 @@ __device__ __forceinline__ void grid_finish(GacCtl* ctl, unsigned* F, int nvw, G
   const int lp = uniform_int(ld_agent(&ctl->last_push_round)), wr = uniform_int(ld_agent(&ctl->wipe_round));
   const int err = uniform_int(ld_agent(&ctl->err));
   __syncthreads();
-  if (tid == 0)
+  if (tid == 0) {
+    ctl->done = 0u;  // (the next round's grid may be another)
     store_result(out, rounds, converged, err, lp, wr, e->tot[1], e->tot[0],
                  wall_clock64() - (start ? start : ld_view<true>((const u64*)&ctl->start)));
+  }
   if (!err && final(lp, wr)) {
     for (int i = tid; i < kStatSlots; i += blockDim.x) {
       ctl->deletions[i] = 0ull;
@@ -512,7 +514,6 @@ __device__ __forceinline__ void grid_finish(GacCtl* ctl, unsigned* F, int nvw, G
       ctl->last_push_round = -1;
       ctl->wipe_round = INT_MAX;
       ctl->bar_ticket = 0ull;
-      ctl->done = 0u;
     }
   }
   box_publish(seq_at, seq);
