@@ -1176,7 +1176,16 @@ __device__ __forceinline__ bool wg_fixpoint(const DevNet& net, const WgMem& mem,
     const bool both = both_dirs_round0 && round == 0;
     int mine = wave;  // this wave's next unit, counted from the block of variables below
     bool stop = false;
+    u64 some = ~0ull;  // words of the frontier with a changed variable, 64 of them from v0 / 32 on
     for (int v0 = 0; v0 < n && !stop; v0 += 64) {
+      // blocks without one are passed over: a path of 2,800 variables, one
+      // changed a round, took 20 us a round with every block counted
+      if (n > 128) {
+        if ((v0 & 2047) == 0) some = __ballot((v0 >> 5) + lane < nvw && cur[(v0 >> 5) + lane] != 0u);
+        const u64 rest = some >> ((v0 >> 5) & 63);
+        v0 = rest ? v0 + ((int)__builtin_ctzll(rest) >> 1) * 64 : v0 | 1984;
+        if (rest == 0ull) continue;
+      }
       const int v = v0 + lane;
       int a0 = 0, deg = 0;
       if (v < n) {

@@ -152,3 +152,21 @@ def test_wide_rounds_on_few_constraints_are_not_slower_than_one_workgroup(gpu):
                 m.WriteDomains(0, init)
                 ms[name] = min(ms.get(name, 1e9), run().kernel_ms)
     assert ms["rounds"] < 0.5 * ms["block"], ms
+
+
+def test_workgroup_rounds_pass_over_unchanged_variables(gpu):
+    # one changed variable a round: a round's cost must not grow with the
+    # variables that did not change (counting every one, 21 us a round of 3,000
+    # variables against 5 us of 700)
+    us = {}
+    for n in (700, 2800):
+        desc = path(n, 64)
+        with GModelAdapter.Build(desc) as m:
+            cut = m.ReadDomains(0)
+            cut[0, 0] = np.uint64(1 << 63)
+            for _ in range(3):
+                m.WriteDomains(0, cut)
+                st = m.EnforceGAC_Block(0)
+                assert st.converged and st.deletions == 63 * (n - 1)
+                us[n] = min(us.get(n, 1e9), st.kernel_ms * 1e3 / n)
+    assert us[2800] < 2.5 * us[700], us
