@@ -725,7 +725,7 @@ struct cpim_gmodel {
   int assigned_size = 0;
   DevAlloc dom;    // [max_depth][n][W]
   DevAlloc size;   // [max_depth][n]
-  DevAlloc front;  // three bitmaps of variables (grid rounds), or one of constraints (asynchronous)
+  DevAlloc front;  // three bitmaps of variables (grid rounds), then one of constraints (asynchronous)
   DevAlloc ctl;    // GacCtl
   bool ctl_ready = false;      // ctl and front are in their first state (k_gac_init, grid_finish)
   mutable HostBox* box_ = nullptr;  // answers of the model's kernels
@@ -927,7 +927,7 @@ int cpim_gmodel_create(const cpim_model_desc* desc, const cpim_gmodel_options* o
     const long long lw = (long long)n * m->im.W;
     const long long dom_bytes = (long long)sizeof(u64) * lw * m->max_depth;
     const long long size_bytes = (long long)sizeof(int) * n * m->max_depth;
-    const long long front_bytes = (long long)sizeof(unsigned) * std::max<long long>(m->nfw, 3ll * m->nvw);
+    const long long front_bytes = (long long)sizeof(unsigned) * (3ll * m->nvw + m->nfw);
     m->arena.reserve(model_arena_bytes(m->im) + Arena::round(dom_bytes) + Arena::round(size_bytes) +
                      Arena::round(front_bytes) + Arena::round((long long)sizeof(GacCtl)));
     build_device_model(m->im, m->dm, m->stream, &m->arena);
@@ -1073,9 +1073,81 @@ void fill_gac_stats(const GacResult& res, int rounds, bool converged, double kms
 // a launch that finds the fixpoint over about 2 us.
 constexpr int kRoundsAhead = 8;
 
+// changed: a bitmap of variables to go on from (NULL: starts from assigned_var).
+void gac_async(cpim_gmodel* m, int assigned_var, cpim_gac_stats* st, const unsigned* changed = nullptr) {
+  const int L = m->current_level;
+  u64* dom = m->level_dom(L);
+  int* size = m->level_size(L);
+  unsigned* F = m->front.as<unsigned>() + 3ll * m->nvw;
+  const int nfw = m->nfw;
+  if (!m->async_ctl.p) m->async_ctl = DevAlloc(sizeof(AsyncCtl));
+  AsyncCtl* ctl = m->async_ctl.as<AsyncCtl>();
+  m->gac_events();
+  HIPC(hipEventRecord(m->gev[0], m->stream));
+  AsyncCtl init{};
+  HIPC(hipMemcpyAsync(ctl, &init, sizeof(init), hipMemcpyHostToDevice, m->stream));
+  HIPC(hipMemsetAsync(F, 0, sizeof(unsigned) * nfw, m->stream));
+  const int seed_blocks = changed ? (m->dm.n + 255) / 256 : (assigned_var < 0 ? (nfw + 255) / 256 : 1);
+  hipLaunchKernelGGL(k_seed_async, dim3(seed_blocks), dim3(256), 0, m->stream, F, nfw, m->dm.num_active,
+                     m->dm.adj_off.as<int>(), m->dm.adj.as<int4>(), assigned_var, changed, m->dm.n, ctl);
+  HIPC(hipGetLastError());
+  // two waves per CU: on the C2 cascade 1024 waves took 5.0-6.0 ms, 512
+  // waves 3.8-4.4 ms and 256 waves 4.4-4.9 ms (more waves, more contention on
+  // the frontier words and the pending count)
+  const int threads = 256;
+  const int waves = std::max(1, std::min(nfw, kAsyncWavesPerCu * m->props.cus));
+  const int blocks = (waves + threads / 64 - 1) / (threads / 64);
+  const unsigned long long max_ticks = fixpoint_budget_ticks(m);
+  DevNet net = m->dm.net();
+  hipLaunchKernelGGL(k_gac_async, dim3(blocks), dim3(threads), 0, m->stream, net, dom, size, F, nfw, ctl, max_ticks);
+  HIPC(hipGetLastError());
+  HIPC(hipEventRecord(m->gev[1], m->stream));
+  AsyncCtl res{};
+  HIPC(hipMemcpyAsync(&res, ctl, sizeof(res), hipMemcpyDeviceToHost, m->stream));
+  m->sync();
+  st->kernel_ms = m->gac_elapsed_ms();
+  if (res.err) fail(CPIM_ERR_RUNTIME, "asynchronous fixpoint exceeded its time budget");
+  st->iterations = 1;
+  st->deletions = (int32_t)slot_sum(res.deletions);
+  st->inconsistent = res.wipe != 0;
+  st->converged = !res.wipe && res.pending == 0;
+  st->revisions = (int64_t)slot_sum(res.revisions);
+}
+
+void gac_block(cpim_gmodel* m, int assigned_var, cpim_gac_stats* st, const unsigned* changed = nullptr) {
+  const int L = m->current_level;
+  DevNet net = m->dm.net();
+  const long long bytes = wg_mem_bytes(m->dm.n, m->dm.W);
+  const int threads = 1024;
+  HostBox* box = m->box();
+  const unsigned long long seq = m->next_seq();
+  if (bytes <= kLdsBudget) {
+    hipLaunchKernelGGL(k_block_gac<true>, dim3(1), dim3(threads), (size_t)bytes, m->stream, net,
+                       m->level_dom(L), m->level_size(L), assigned_var, changed, (char*)nullptr, &box->gac, &box->seq, seq);
+  } else {
+    char* scratch = m->get_scratch(bytes);
+    hipLaunchKernelGGL(k_block_gac<false>, dim3(1), dim3(threads), 0, m->stream, net, m->level_dom(L),
+                       m->level_size(L), assigned_var, changed, scratch, &box->gac, &box->seq, seq);
+  }
+  HIPC(hipGetLastError());
+  m->wait_box(seq);
+  fill_gac_stats(box->gac, 1, box->gac.converged != 0, m->ticks_ms(box->gac.ticks), st);
+}
+
+// What AUTO does with a long, narrow cascade: rounds that look like a chain
+// (kTailRounds of them, the last ones of at most kTailArcWords arc words) go on
+// in one launch.  A round over the grid costs 8 us however little it does, one
+// of the workgroup fixpoint 2.5 to 4 us, one of the asynchronous kernel 5 us:
+// a path of 1,000 variables 7.6 ms by rounds alone and 2.7 with the workgroup
+// fixpoint; of 4,200, seeded, 35 and 23 ms with the asynchronous kernel.
+enum class Tail { kNone, kBlock, kAsync };
+constexpr int kTailRounds = 31;
+constexpr long long kTailArcWords = 1024;  // one turn of a 1024-thread workgroup
+
 // by_variable: a seeded fixpoint keeps a frontier of variables, as the workgroup
 // fixpoint does, instead of one of constraints (host-driven rounds only).
-void gac_grid(cpim_gmodel* m, int assigned_var, bool persistent, cpim_gac_stats* st, bool by_variable = false) {
+void gac_grid(cpim_gmodel* m, int assigned_var, bool persistent, cpim_gac_stats* st, bool by_variable = false,
+              Tail tail = Tail::kNone) {
   const int L = m->current_level;
   unsigned* F = m->front.as<unsigned>();
   GacCtl* ctl = m->ctl.as<GacCtl>();
@@ -1105,14 +1177,14 @@ void gac_grid(cpim_gmodel* m, int assigned_var, bool persistent, cpim_gac_stats*
     const int grid[2] = {blocks(false), blocks(true)};
     // each round of a batch answers in a result of its own
     GacResult* answers = reinterpret_cast<GacResult*>(box->data);
-    bool over = false;
-    for (int r0 = 0, ahead = 1; r0 < max_rounds && !over; r0 += ahead, ahead = std::min(2 * ahead, kRoundsAhead)) {
+    bool over = false, narrow = false;
+    for (int r0 = 0, ahead = 1; r0 < max_rounds && !over && !narrow; r0 += ahead, ahead = std::min(2 * ahead, kRoundsAhead)) {
       const int k = (int)std::min<long long>(ahead, max_rounds - r0);
       for (int i = 0; i < k; ++i) {
         if (r0 + i > 0) seq = m->next_seq();
         answers[i].rounds = 0;  // stays 0 if the fixpoint was over before
-        hipLaunchKernelGGL(k_gac_round, dim3(grid[r0 + i > 0 ? 1 : 0]), dim3(kRoundThreads), 0, m->stream, net, m->level_dom(L),
-                           m->level_size(L), F, m->nvw, ctl, r0 + i, assigned_var,
+        hipLaunchKernelGGL(k_gac_round, dim3(grid[r0 + i > 0 ? 1 : 0]), dim3(kRoundThreads), 0, m->stream, net,
+                           m->level_dom(L), m->level_size(L), F, m->nvw, ctl, r0 + i, assigned_var,
                            assigned_var >= 0 && !by_variable ? 1 : 0, (int)m->im.adj.size(), &answers[i], &box->seq,
                            seq);
         const hipError_t e = hipGetLastError();
@@ -1120,6 +1192,7 @@ void gac_grid(cpim_gmodel* m, int assigned_var, bool persistent, cpim_gac_stats*
         HIPC(e);
       }
       m->wait_box(seq);
+      const unsigned long long revisions = res.revisions;
       for (int i = 0; i < k && !over; ++i) {
         if (answers[i].rounds == 0) continue;
         res = answers[i];
@@ -1128,6 +1201,24 @@ void gac_grid(cpim_gmodel* m, int assigned_var, bool persistent, cpim_gac_stats*
         converged = res.last_push_round < rounds - 1;
         over = converged || res.wipe_round < rounds;
       }
+      narrow = tail != Tail::kNone && !over && rounds >= kTailRounds &&
+               (long long)(res.revisions - revisions) * m->dm.W <= kTailArcWords * k;
+    }
+    if (narrow) {
+      cpim_gac_stats rest{};
+      const unsigned* changed = F + (long long)(rounds % 3) * m->nvw;  // in the last round
+      if (tail == Tail::kBlock) gac_block(m, assigned_var, &rest, changed);
+      else gac_async(m, assigned_var, &rest, changed);
+      gac_start(m, F, ctl);
+      m->ctl_ready = true;
+      fill_gac_stats(res, rounds, false, kms, st);
+      st->iterations += rest.iterations;
+      st->deletions += rest.deletions;
+      st->revisions += rest.revisions;
+      st->inconsistent = rest.inconsistent;
+      st->converged = rest.converged;
+      st->kernel_ms += rest.kernel_ms;
+      return;
     }
     if (!over) {  // rounds bounded by the number of values: not reached
       m->sync();
@@ -1136,66 +1227,6 @@ void gac_grid(cpim_gmodel* m, int assigned_var, bool persistent, cpim_gac_stats*
   }
   m->ctl_ready = true;
   fill_gac_stats(res, rounds, converged, kms, st);
-}
-
-void gac_async(cpim_gmodel* m, int assigned_var, cpim_gac_stats* st) {
-  const int L = m->current_level;
-  u64* dom = m->level_dom(L);
-  int* size = m->level_size(L);
-  unsigned* F = m->front.as<unsigned>();
-  const int nfw = m->nfw;
-  m->ctl_ready = false;  // the frontier of constraints goes where the changed bitmaps lie
-  if (!m->async_ctl.p) m->async_ctl = DevAlloc(sizeof(AsyncCtl));
-  AsyncCtl* ctl = m->async_ctl.as<AsyncCtl>();
-  m->gac_events();
-  HIPC(hipEventRecord(m->gev[0], m->stream));
-  AsyncCtl init{};
-  HIPC(hipMemcpyAsync(ctl, &init, sizeof(init), hipMemcpyHostToDevice, m->stream));
-  HIPC(hipMemsetAsync(F, 0, sizeof(unsigned) * nfw, m->stream));
-  hipLaunchKernelGGL(k_seed_async, dim3(assigned_var < 0 ? (nfw + 255) / 256 : 1), dim3(256), 0, m->stream, F, nfw,
-                     m->dm.num_active, m->dm.adj_off.as<int>(), m->dm.adj.as<int4>(), assigned_var, ctl);
-  HIPC(hipGetLastError());
-  // two waves per CU: on the C2 cascade 1024 waves took 5.0-6.0 ms, 512
-  // waves 3.8-4.4 ms and 256 waves 4.4-4.9 ms (more waves, more contention on
-  // the frontier words and the pending count)
-  const int threads = 256;
-  const int waves = std::max(1, std::min(nfw, kAsyncWavesPerCu * m->props.cus));
-  const int blocks = (waves + threads / 64 - 1) / (threads / 64);
-  const unsigned long long max_ticks = fixpoint_budget_ticks(m);
-  DevNet net = m->dm.net();
-  hipLaunchKernelGGL(k_gac_async, dim3(blocks), dim3(threads), 0, m->stream, net, dom, size, F, nfw, ctl, max_ticks);
-  HIPC(hipGetLastError());
-  HIPC(hipEventRecord(m->gev[1], m->stream));
-  AsyncCtl res{};
-  HIPC(hipMemcpyAsync(&res, ctl, sizeof(res), hipMemcpyDeviceToHost, m->stream));
-  m->sync();
-  st->kernel_ms = m->gac_elapsed_ms();
-  if (res.err) fail(CPIM_ERR_RUNTIME, "asynchronous fixpoint exceeded its time budget");
-  st->iterations = 1;
-  st->deletions = (int32_t)slot_sum(res.deletions);
-  st->inconsistent = res.wipe != 0;
-  st->converged = !res.wipe && res.pending == 0;
-  st->revisions = (int64_t)slot_sum(res.revisions);
-}
-
-void gac_block(cpim_gmodel* m, int assigned_var, cpim_gac_stats* st) {
-  const int L = m->current_level;
-  DevNet net = m->dm.net();
-  const long long bytes = wg_mem_bytes(m->dm.n, m->dm.W);
-  const int threads = 1024;
-  HostBox* box = m->box();
-  const unsigned long long seq = m->next_seq();
-  if (bytes <= kLdsBudget) {
-    hipLaunchKernelGGL(k_block_gac<true>, dim3(1), dim3(threads), (size_t)bytes, m->stream, net,
-                       m->level_dom(L), m->level_size(L), assigned_var, (char*)nullptr, &box->gac, &box->seq, seq);
-  } else {
-    char* scratch = m->get_scratch(bytes);
-    hipLaunchKernelGGL(k_block_gac<false>, dim3(1), dim3(threads), 0, m->stream, net, m->level_dom(L),
-                       m->level_size(L), assigned_var, scratch, &box->gac, &box->seq, seq);
-  }
-  HIPC(hipGetLastError());
-  m->wait_box(seq);
-  fill_gac_stats(box->gac, 1, box->gac.converged != 0, m->ticks_ms(box->gac.ticks), st);
 }
 
 // Constraints times words a domain up to which AUTO takes one workgroup with
@@ -1224,6 +1255,9 @@ int auto_gac_mode(const cpim_gmodel* m) {
 void gac(cpim_gmodel* m, int assigned_var, int mode, cpim_gac_stats* st) {
   std::memset(st, 0, sizeof(*st));
   const bool by_variable = mode == CPIM_GAC_AUTO && fits_lds(m) && m->dm.num_active <= kAutoByVariable;
+  Tail tail = Tail::kNone;
+  if (by_variable) tail = Tail::kBlock;
+  else if (mode == CPIM_GAC_AUTO && assigned_var >= 0) tail = Tail::kAsync;
   if (mode == CPIM_GAC_AUTO) mode = auto_gac_mode(m);
   if (m->dm.num_active == 0) {
     st->converged = 1;
@@ -1232,7 +1266,7 @@ void gac(cpim_gmodel* m, int assigned_var, int mode, cpim_gac_stats* st) {
   const int L = m->current_level, before = m->closure[L];
   m->closure[L] = cpim_gmodel::kOpen;
   switch (mode) {
-    case CPIM_GAC_PLAIN: gac_grid(m, assigned_var, false, st, by_variable); break;
+    case CPIM_GAC_PLAIN: gac_grid(m, assigned_var, false, st, by_variable, tail); break;
     case CPIM_GAC_PERSISTENT: gac_grid(m, assigned_var, true, st); break;
     case CPIM_GAC_BLOCK: gac_block(m, assigned_var, st); break;
     case CPIM_GAC_ASYNC: gac_async(m, assigned_var, st); break;

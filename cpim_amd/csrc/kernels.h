@@ -884,9 +884,21 @@ __global__ void k_gac_async(DevNet net, u64* dom, int* size, unsigned* F, int nf
   }
 }
 
-// Seed the asynchronous frontier: all active constraints, or those of var.
+// Seed the asynchronous frontier: all active constraints, or those of var, or
+// those of the variables in the bitmap `changed` (n variables) if there is one.
 __global__ void k_seed_async(unsigned* F, int nfw, int ncons, const int* adj_off, const int4* adj, int var,
-                             AsyncCtl* ctl) {
+                             const unsigned* changed, int n, AsyncCtl* ctl) {
+  if (changed) {
+    const int v = blockIdx.x * blockDim.x + threadIdx.x;
+    if (v >= n || !((changed[v >> 5] >> (v & 31)) & 1u)) return;
+    int fresh = 0;
+    for (int i = adj_off[v]; i < adj_off[v + 1]; ++i) {
+      const unsigned bit = 1u << (adj[i].x & 31);
+      if (!(atomicOr(&F[adj[i].x >> 5], bit) & bit)) ++fresh;
+    }
+    if (fresh) atomicAdd(&ctl->pending, (unsigned long long)fresh);
+    return;
+  }
   if (var < 0) {
     const long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x;
     if (i < nfw) {
@@ -1103,15 +1115,18 @@ __device__ __forceinline__ void lane_remove(const WgMem& mem, WgCtl* ctl, unsign
 }
 
 // Frontier of a fixpoint's first round: variable `seed`, or every variable
-// (seed < 0); the other two bitmaps and the wipe-out word of `slot` are
-// cleared.  Called by every thread, a __syncthreads() before wg_fixpoint.
-__device__ __forceinline__ void wg_seed(const WgMem& mem, WgCtl* ctl, int n, int slot, int seed) {
+// (seed < 0), or the bitmap `changed` if there is one; the other two bitmaps and
+// the wipe-out word of `slot` are cleared.  Called by every thread, a
+// __syncthreads() before wg_fixpoint.
+__device__ __forceinline__ void wg_seed(const WgMem& mem, WgCtl* ctl, int n, int slot, int seed,
+                                        const unsigned* changed = nullptr) {
   const int nvw = (n + 31) / 32;
   for (int i = threadIdx.x; i < 3 * nvw; i += blockDim.x) {
     unsigned v = 0u;
     if (i < nvw) {
       const int k = n - 32 * i;
-      if (seed < 0) v = k >= 32 ? 0xffffffffu : ((1u << k) - 1u);
+      if (changed) v = changed[i];
+      else if (seed < 0) v = k >= 32 ? 0xffffffffu : ((1u << k) - 1u);
       else if (i == seed >> 5) v = 1u << (seed & 31);
     }
     mem.bm[i] = v;
@@ -1532,10 +1547,11 @@ __device__ __forceinline__ u64 wg_reduce_sum_u64(WgCtl* ctl, u64 v) {
 }
 
 // ---------------------------------------------------------------------------
-// Block-mode GAC on one level (one workgroup).
+// Block-mode GAC on one level (one workgroup).  changed: goes on from these
+// variables, where rounds over the grid left off (NULL: starts from seed_var).
 // ---------------------------------------------------------------------------
 template <bool kLds>
-__global__ void k_block_gac(DevNet net, u64* dom, int* size, int seed_var, char* scratch,
+__global__ void k_block_gac(DevNet net, u64* dom, int* size, int seed_var, const unsigned* changed, char* scratch,
                             GacResult* out, unsigned long long* seq_at, unsigned long long seq) {
   const unsigned long long t0 = wall_clock64();
   extern __shared__ __align__(16) char smem[];
@@ -1547,11 +1563,11 @@ __global__ void k_block_gac(DevNet net, u64* dom, int* size, int seed_var, char*
   wg_copy_words(mem.dom, dom, (long long)n * W);
   for (int v = threadIdx.x; v < n; v += blockDim.x) mem.size[v] = size[v];
   wg_clear_bitmap(mem.asg, (n + 31) / 32);
-  wg_seed(mem, &ctl, n, 0, seed_var);
+  wg_seed(mem, &ctl, n, 0, seed_var, changed);
   __syncthreads();
   long long before = 0;
   for (int v = threadIdx.x; v < n; v += blockDim.x) before += mem.size[v];
-  const bool ok = wg_fixpoint<true>(net, mem, &ctl, 0, seed_var >= 0);
+  const bool ok = wg_fixpoint<true>(net, mem, &ctl, 0, seed_var >= 0 && !changed);
   long long after = 0;
   for (int v = threadIdx.x; v < n; v += blockDim.x) after += mem.size[v];
   const u64 delta = wg_reduce_sum_u64(&ctl, (u64)(before - after));

@@ -1,5 +1,7 @@
 """Automatic choices between kernels, where the wrong one costs several times
 the right one (needs an MI355X)."""
+import time
+
 import numpy as np
 import pytest
 
@@ -170,3 +172,57 @@ def test_workgroup_rounds_pass_over_unchanged_variables(gpu):
                 assert st.converged and st.deletions == 63 * (n - 1)
                 us[n] = min(us.get(n, 1e9), st.kernel_ms * 1e3 / n)
     assert us[2800] < 2.5 * us[700], us
+
+
+@pytest.mark.parametrize("n,d,seed", [(1000, 64, -1), (1000, 64, 0), (4200, 64, 0)])
+def test_auto_does_not_run_a_long_chain_by_rounds_alone(gpu, n, d, seed):
+    # a round over the grid costs 8 us however little it does: 7.6 ms against 2.7
+    # with the workgroup fixpoint at 1,000, 35 against 23 with the asynchronous
+    # kernel at 4,200
+    desc = path(n, d)
+    with GModelAdapter.Build(desc) as m:
+        cut = m.ReadDomains(0)
+        cut[0, 0] = np.uint64(1 << (d - 1))
+        s = {}
+        for _ in range(3):
+            for name, run in (("auto", lambda: m.EnforceGAC_Auto(seed)), ("plain", lambda: m.EnforceGAC(False, seed))):
+                m.WriteDomains(0, cut)
+                t0 = time.perf_counter()
+                st = run()
+                s[name] = min(s.get(name, 1e9), time.perf_counter() - t0)
+                assert st.converged and not st.inconsistent and st.deletions == (d - 1) * (n - 1)
+                dom = m.ReadDomains(0)
+                assert (dom == np.uint64(1 << (d - 1))).all()
+    assert s["auto"] < 0.8 * s["plain"], s
+
+
+@pytest.mark.parametrize("n,d,wipe", [(900, 8, False), (900, 8, True), (4200, 4, False), (4200, 4, True), (850, 70, False)])
+def test_auto_chain_on_an_open_level(gpu, n, d, wipe):
+    """The long chain's second kernel answers what the first one's frontier
+    does: of variables up to 4,096 constraints, of constraints beyond.  Some
+    values are missing along the path; wipe: the chain empties a variable near
+    its end."""
+    from test_gpu_open_levels import seeded_closure
+    desc = path(n, d)
+    rng = np.random.default_rng(n + wipe)
+    sets = [set(np.flatnonzero(rng.random(d) < 0.7).tolist()) | {0, d - 1} for _ in range(n)]
+    sets[0] = {d - 1}
+    if wipe:
+        sets[n - 10] = set(range(d - 1))
+    want = seeded_closure(desc, sets, 0, "constraint" if n - 1 > 4096 else "variable")
+    dom = np.zeros((n, words_for(d)), np.uint64)
+    for v, s in enumerate(sets):
+        for a in s:
+            dom[v, a // 64] |= np.uint64(1 << (a % 64))
+    with GModelAdapter.Build(desc) as m:
+        m.WriteDomains(0, dom)
+        st = m.EnforceGAC_Auto(0)
+        assert st.inconsistent == (want is None)
+        if want is not None:
+            assert [set(g) for g in domains_to_sets(m.ReadDomains(0), desc.dom_size)] == want
+            assert st.deletions == sum(map(len, sets)) - sum(map(len, want))
+        # rounds again, on the control block that the second kernel left
+        m.WriteDomains(0, dom)
+        ok, full, _ = oracle.Oracle(desc.with_init_dom(dom)).root_ac()
+        assert m.EnforceGAC(False).inconsistent == (not ok)
+        assert not ok or (m.ReadDomains(0) == full).all()
