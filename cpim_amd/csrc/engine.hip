@@ -1084,9 +1084,10 @@ void gac_async(cpim_gmodel* m, int assigned_var, cpim_gac_stats* st, const unsig
   AsyncCtl* ctl = m->async_ctl.as<AsyncCtl>();
   m->gac_events();
   HIPC(hipEventRecord(m->gev[0], m->stream));
-  AsyncCtl init{};
-  HIPC(hipMemcpyAsync(ctl, &init, sizeof(init), hipMemcpyHostToDevice, m->stream));
-  HIPC(hipMemsetAsync(F, 0, sizeof(unsigned) * nfw, m->stream));
+  // (cleared by a kernel: a copy from the host right after a call that answered
+  // in the box first waits for the runtime to see that call's kernel end, some
+  // 18 us)
+  hipLaunchKernelGGL(k_async_init, dim3(std::min((nfw + 255) / 256, 1024)), dim3(256), 0, m->stream, F, nfw, ctl);
   const int seed_blocks = changed ? (m->dm.n + 255) / 256 : (assigned_var < 0 ? (nfw + 255) / 256 : 1);
   hipLaunchKernelGGL(k_seed_async, dim3(seed_blocks), dim3(256), 0, m->stream, F, nfw, m->dm.num_active,
                      m->dm.adj_off.as<int>(), m->dm.adj.as<int4>(), assigned_var, changed, m->dm.n, ctl);

@@ -884,6 +884,21 @@ __global__ void k_gac_async(DevNet net, u64* dom, int* size, unsigned* F, int nf
   }
 }
 
+// First state of the asynchronous fixpoint, before k_seed_async.
+__global__ void k_async_init(unsigned* F, int nfw, AsyncCtl* ctl) {
+  const int i0 = blockIdx.x * blockDim.x + threadIdx.x;
+  for (int i = i0; i < nfw; i += gridDim.x * blockDim.x) F[i] = 0u;
+  for (int i = i0; i < kStatSlots; i += gridDim.x * blockDim.x) {
+    ctl->deletions[i] = 0ull;
+    ctl->revisions[i] = 0ull;
+  }
+  if (i0 == 0) {
+    ctl->pending = 0ull;
+    ctl->wipe = 0;
+    ctl->err = 0;
+  }
+}
+
 // Seed the asynchronous frontier: all active constraints, or those of var, or
 // those of the variables in the bitmap `changed` (n variables) if there is one.
 __global__ void k_seed_async(unsigned* F, int nfw, int ncons, const int* adj_off, const int4* adj, int var,
