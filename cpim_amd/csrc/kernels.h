@@ -1600,14 +1600,14 @@ __global__ void k_block_gac(DevNet net, u64* dom, int* size, int seed_var, const
 // ---------------------------------------------------------------------------
 __global__ void k_level_put(const u64* src, u64* dom, int* size, int n, int W, unsigned long long* seq_at,
                             unsigned long long seq) {
+  // the words in order (a thread per variable reads host memory 8 bytes a line:
+  // 64 KB took 36 us so), then the sizes
+  for (int i = threadIdx.x; i < n * W; i += blockDim.x)
+    dom[i] = __hip_atomic_load(const_cast<u64*>(&src[i]), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+  __syncthreads();
   for (int v = threadIdx.x; v < n; v += blockDim.x) {
     int s = 0;
-    for (int w = 0; w < W; ++w) {
-      const u64 d = __hip_atomic_load(const_cast<u64*>(&src[(long long)v * W + w]), __ATOMIC_RELAXED,
-                                      __HIP_MEMORY_SCOPE_SYSTEM);
-      dom[(long long)v * W + w] = d;
-      s += __popcll(d);
-    }
+    for (int w = 0; w < W; ++w) s += __popcll(dom[(long long)v * W + w]);
     size[v] = s;
   }
   box_publish(seq_at, seq);
@@ -1636,16 +1636,17 @@ enum LevelOp {
   kOpAll        // 1: every variable is assigned
 };
 
-__global__ void __launch_bounds__(256) k_level_op(int op, u64* dom, int* size, int n, int W, int max_dom, int var,
+template <int kThreads>
+__global__ void __launch_bounds__(kThreads) k_level_op(int op, u64* dom, int* size, int n, int W, int max_dom, int var,
                                                   int value, int* answer, unsigned long long* seq_at,
                                                   unsigned long long seq) {
-  __shared__ u64 red[4];
+  __shared__ u64 red[kThreads / 64];
   const int tid = threadIdx.x;
   u64* d = dom + (long long)var * W;
   int res = 0;
   if (op == kOpMinVar || op == kOpAll) {
     u64 key = ~0ull;
-    for (int v = tid; v < n; v += 256) {
+    for (int v = tid; v < n; v += kThreads) {
       const int s = size[v];
       const u64 k = op == kOpAll ? (u64)(s == 1) : (s > 1 ? ((u64)(unsigned)s << 32) | (unsigned)v : ~0ull);
       key = k < key ? k : key;
@@ -1653,7 +1654,7 @@ __global__ void __launch_bounds__(256) k_level_op(int op, u64* dom, int* size, i
     key = wave_min64_dpp(key);
     if (lane_id() == 0) red[tid >> 6] = key;
     __syncthreads();
-    for (int i = 0; i < 4; ++i) key = red[i] < key ? red[i] : key;
+    for (int i = 0; i < kThreads / 64; ++i) key = red[i] < key ? red[i] : key;
     res = op == kOpAll ? (int)(key & 1ull) : (key == ~0ull ? -1 : (int)(unsigned)key);
   } else if (tid == 0) {
     if (op == kOpAssign) {

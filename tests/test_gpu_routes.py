@@ -226,3 +226,33 @@ def test_auto_chain_on_an_open_level(gpu, n, d, wipe):
         ok, full, _ = oracle.Oracle(desc.with_init_dom(dom)).root_ac()
         assert m.EnforceGAC(False).inconsistent == (not ok)
         assert not ok or (m.ReadDomains(0) == full).all()
+
+
+@pytest.mark.parametrize("n,d", [(2047, 8), (2048, 8), (2049, 8), (4097, 70), (1024, 1), (300, 70), (1638, 300), (9, 1024)])
+def test_level_calls_on_many_variables(gpu, n, d):
+    # queries by 256 or 1024 threads, levels written in order up to 64 KB through
+    # the host box and by copy beyond, the last words of a domain partly used
+    rng = np.random.default_rng(n)
+    W = words_for(d)
+    desc = ModelDesc(np.full(n, d, np.int32), np.full(1, 2, np.int32), np.array([0, n - 1], np.int32),
+                     np.full((1, d, W), ~np.uint64(0)))
+    dom = rng.integers(0, 1 << 63, (n, W), dtype=np.uint64) | np.uint64(1 << 63) | np.uint64(3)
+    cap = np.array([(1 << min(64, max(0, d - 64 * w))) - 1 for w in range(W)], dtype=object)
+    want = np.array([[int(x) & c for x, c in zip(row, cap)] for row in dom], dtype=np.uint64)
+    sizes = np.bitwise_count(want).sum(axis=1)
+    with GModelAdapter.Build(desc) as m:
+        m.WriteDomains(0, dom)
+        assert (m.ReadDomains(0) == want).all()
+        for v in (0, 1, n // 2, n - 1):
+            assert m.GetDomainSize(v, 0) == sizes[v]
+        open_ = np.flatnonzero(sizes > 1)
+        assert m.GetMinDomainVar(0) == (open_[np.argmin(sizes[open_])] if len(open_) else -1)
+        assert m.IsFullyAssigned(0) == bool((sizes == 1).all())
+        one = np.zeros((n, W), np.uint64)
+        one[:, 0] = 1
+        m.WriteDomains(0, one)
+        assert m.IsFullyAssigned(0) and m.GetMinDomainVar(0) == -1
+        if d > 1:
+            one[n - 1, 0] = 3
+            m.WriteDomains(0, one)
+            assert not m.IsFullyAssigned(0) and m.GetMinDomainVar(0) == n - 1
