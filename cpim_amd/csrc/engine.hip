@@ -714,6 +714,10 @@ void give_box(HostBox* b) {
 // ---------------------------------------------------------------------------
 // GModel
 // ---------------------------------------------------------------------------
+// Words before the asynchronous frontier in `front`: the rounds' three bitmaps,
+// up to the next 256 bytes (its waves read 64 words at a time).
+constexpr long long async_front(int nvw) { return (3ll * nvw + 63) & ~63ll; }
+
 struct cpim_gmodel {
   int device = 0;
   hipStream_t stream = nullptr;
@@ -930,7 +934,7 @@ int cpim_gmodel_create(const cpim_model_desc* desc, const cpim_gmodel_options* o
     const long long lw = (long long)n * m->im.W;
     const long long dom_bytes = (long long)sizeof(u64) * lw * m->max_depth;
     const long long size_bytes = (long long)sizeof(int) * n * m->max_depth;
-    const long long front_bytes = (long long)sizeof(unsigned) * (3ll * m->nvw + m->nfw);
+    const long long front_bytes = (long long)sizeof(unsigned) * (async_front(m->nvw) + m->nfw);
     m->arena.reserve(model_arena_bytes(m->im) + Arena::round(dom_bytes) + Arena::round(size_bytes) +
                      Arena::round(front_bytes) + Arena::round((long long)sizeof(GacCtl)));
     build_device_model(m->im, m->dm, m->stream, &m->arena);
@@ -1081,7 +1085,7 @@ void gac_async(cpim_gmodel* m, int assigned_var, cpim_gac_stats* st, const unsig
   const int L = m->current_level;
   u64* dom = m->level_dom(L);
   int* size = m->level_size(L);
-  unsigned* F = m->front.as<unsigned>() + 3ll * m->nvw;
+  unsigned* F = m->front.as<unsigned>() + async_front(m->nvw);
   const int nfw = m->nfw;
   if (!m->async_ctl.p) m->async_ctl = DevAlloc(sizeof(AsyncCtl));
   AsyncCtl* ctl = m->async_ctl.as<AsyncCtl>();
