@@ -130,6 +130,7 @@ struct ModelImage {
   std::vector<int> tabs;              // active indices of table constraints
   bool simple = true;                 // no two binary constraints have the same scope
   int max_deg = 0;                    // most constraints on one variable
+  int big_tabs = 0;                   // tables of more than 512 tuples or over more than one word
   double reach = 0.0;                 // arcs of a variable and of its neighbours, mean over the values
   double density = 0.0;               // allowed share of the binary tuples (sample_density)
   std::vector<u64> rel_dense;         // owned dense rows when the desc has none
@@ -241,6 +242,7 @@ ModelImage make_image(const cpim_model_desc* d, bool skip_non_binary, bool own_r
       tsup_off += words;
       bin_ordinal_of_active.push_back(-1);
       im.tabs.push_back((int)im.con.size());
+      if (im.W > 1 || m.tw > 8) ++im.big_tabs;
       im.con.push_back(m);
     }
   }
@@ -1022,7 +1024,9 @@ void gac_start(cpim_gmodel* m, unsigned* F, GacCtl* ctl) {
 }
 
 // Lanes of a grid round: one per word of every arc, words rounded up to a
-// power of two, and a wave per table.  With several words a wave takes fewer
+// power of two, and a wave per table; beyond small tables, a workgroup each up to
+// one per CU (30 tables of 20,000 tuples over 200 values, 7.9 ms on two CUs, 5.9
+// spread).  With several words a wave takes fewer
 // arcs than it has lanes for, down to 16 lanes, as long as there is at most one
 // workgroup per CU (`later`: at most the two that a round launches): what a
 // wave's arcs settle together is done one after the other (wave_settle).
@@ -1038,7 +1042,7 @@ long long grid_lanes(const cpim_gmodel* m, bool later) {
   while (wp < m->dm.W) wp *= 2;
   long long lanes = arcs * wp;
   for (int used = 32; wp > 1 && used >= 16 && (later ? lanes : 2 * lanes) <= most; used /= 2) lanes *= 2;
-  return std::max(lanes, 64ll * m->dm.ntabs);
+  return std::max({lanes, 64ll * m->dm.ntabs, std::min<long long>(m->im.big_tabs, m->props.cus) * kRoundThreads});
 }
 
 // Largest round copy of the persistent fixpoint in LDS: one workgroup per CU.

@@ -351,8 +351,9 @@ __device__ __forceinline__ void grid_round(const DevNet& net, const u64* view, u
     revs += __popcll(m);
     grid_arc<kCoherent>(net, view, dom, size, nxt, ctl, r, e, w, act, dels);
   }
-  // tables, one per wave, the last waves of the grid first
-  for (int k = nwaves - 1 - gw; k < net.ntabs; k += nwaves) {
+  // tables, one per wave, over the workgroups in turn, their last waves first
+  const int wib = uniform_int(threadIdx.x >> 6), wpb = (int)(blockDim.x >> 6), nb = (int)gridDim.x;
+  for (int k = (wpb - 1 - wib) * nb + nb - 1 - (int)blockIdx.x; k < net.ntabs; k += nwaves) {
     const int c = uniform_int(net.tabs[k]);
     const ConMeta* mp = net.con + c;
     const int y = lane < mp->arity ? mp->scope[lane] : -1;
