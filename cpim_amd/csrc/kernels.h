@@ -224,11 +224,11 @@ struct GacResult {
 // through to host memory), waits until they have completed, and stores the
 // call's number in `seq`, on which the host waits.
 struct HostBox {
-  unsigned long long seq;     // the last call answered
-  unsigned long long issued;  // the last call numbered (the host's)
+  unsigned long long seq;  // the last call answered
   int scalar;
   int pad;
   GacResult gac;
+  alignas(64) unsigned long long issued;  // the last call numbered: the host's, on a line of its own
   alignas(64) unsigned long long data[1];  // kBoxDataBytes
 };
 
@@ -1603,13 +1603,18 @@ __global__ void k_level_put(const u64* src, u64* dom, int* size, int n, int W, u
                             unsigned long long seq) {
   // the words in order (a thread per variable reads host memory 8 bytes a line:
   // 64 KB took 36 us so), then the sizes
-  for (int i = threadIdx.x; i < n * W; i += blockDim.x)
-    dom[i] = __hip_atomic_load(const_cast<u64*>(&src[i]), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
-  __syncthreads();
-  for (int v = threadIdx.x; v < n; v += blockDim.x) {
-    int s = 0;
-    for (int w = 0; w < W; ++w) s += __popcll(dom[(long long)v * W + w]);
-    size[v] = s;
+  for (int i = threadIdx.x; i < n * W; i += blockDim.x) {
+    const u64 d = __hip_atomic_load(const_cast<u64*>(&src[i]), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+    dom[i] = d;
+    if (W == 1) size[i] = __popcll(d);
+  }
+  if (W > 1) {
+    __syncthreads();
+    for (int v = threadIdx.x; v < n; v += blockDim.x) {
+      int s = 0;
+      for (int w = 0; w < W; ++w) s += __popcll(dom[(long long)v * W + w]);
+      size[v] = s;
+    }
   }
   box_publish(seq_at, seq);
 }
