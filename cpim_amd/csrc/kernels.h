@@ -1151,8 +1151,8 @@ __device__ __forceinline__ void wg_seed(const WgMem& mem, WgCtl* ctl, int n, int
 }
 
 // AC fixpoint from the seed that wg_seed put in mem.bm (a __syncthreads()
-// lies between).  both_dirs_round0: in the first round also revise t <- u for
-// every arc of a seed variable t (constraint seeding, as
+// lies between).  seed_both >= 0: in the first round also revise t <- u for
+// every arc of this seed variable t (constraint seeding, as
 // GModel::EnforceGAC(assigned_var) does).  Returns false on wipe-out.  Must
 // be called by every thread of the workgroup.
 //
@@ -1182,7 +1182,7 @@ __device__ __forceinline__ void wg_seed(const WgMem& mem, WgCtl* ctl, int n, int
 // wg_seed never resets the word a slow wave still reads.
 template <bool kTight>
 __device__ __forceinline__ bool wg_fixpoint(const DevNet& net, const WgMem& mem, WgCtl* ctl, int slot,
-                                            bool both_dirs_round0) {
+                                            int seed_both) {
   const int n = net.n, W = net.W;
   const int nvw = (n + 31) / 32;
   const int tid = threadIdx.x;
@@ -1204,7 +1204,7 @@ __device__ __forceinline__ bool wg_fixpoint(const DevNet& net, const WgMem& mem,
     const unsigned* cur = mem.bm + c0;
     unsigned* nxt = mem.bm + c1;
     for (int i = tid; i < nvw; i += nthreads) mem.bm[c2 + i] = 0u;
-    const bool both = both_dirs_round0 && round == 0;
+    const bool both = seed_both >= 0 && round == 0;
     int mine = wave;  // this wave's next unit, counted from the block of variables below
     bool stop = false;
     u64 some = ~0ull;  // words of the frontier with a changed variable, 64 of them from v0 / 32 on
@@ -1258,25 +1258,28 @@ __device__ __forceinline__ bool wg_fixpoint(const DevNet& net, const WgMem& mem,
                                                   pair + (long long)(1 - pos_t) * W * net.dpad + 64 * w, need);
         if (gone) lane_remove(mem, ctl, nxt, slot, round, u, word, gone);
         revs += cnt;
-        if (both && !bit_of(mem.asg, t)) {
-          // t <- u for the same arcs, one after the other (first round only):
-          // source u, target t, whose words the lanes 0..W-1 hold
-          for (int i = 0; i < cnt; ++i) {
-            const int ui = uniform_int(mem.adj[arc - la + i].y);
-            if (ui < 0) continue;
-            const int pi = 1 - uniform_int(adj_pos(mem.adj[arc - la + i]));
-            u64* tw = mem.dom + (long long)t * W + lane;
-            const u64* pp = net.sup + uniform_int(mem.adj[arc - la + i].w) * pair_words;
-            const int wl = lane < W ? lane : 0;
-            const u64 g = wave_unsupported<kTight>(net, mem.dom, ui, pp + (long long)(pi * W + wl) * net.dpad,
-                                                   pp + (long long)(1 - pi) * W * net.dpad + 64 * wl,
-                                                   lane < W ? ld_wg(tw) : 0ull);
-            if (g) lane_remove(mem, ctl, nxt, slot, round, t, tw, g);
-          }
-          revs += cnt;
-        }
       }
       mine -= total;
+    }
+    if (both && !bit_of(mem.asg, seed_both)) {
+      // t <- u of the seed's arcs, spread over the waves and settled by them, a
+      // lane per value of t (by a lane per arc word, up to 64 values of it one
+      // after the other, 40 arcs of 64 values at t=0.886 cost 110 us)
+      const int a0 = uniform_int(mem.aoff[seed_both]), deg = uniform_int(mem.aoff[seed_both + 1]) - a0;
+      for (int i0 = 0; i0 < deg; i0 += nwaves * per) {
+        const int i = i0 + la * nwaves + nwaves - 1 - wave;
+        int4 e = make_int4(0, -1, 0, 0);
+        if (i < deg) e = mem.adj[a0 + i];
+        const bool act = e.y >= 0 && w < W;
+        u64* word = mem.dom + (long long)seed_both * W + (w < W ? w : 0);
+        const u64 need = act ? ld_wg(word) : 0ull;
+        const u64 todo = __ballot(need != 0ull);
+        if (todo == 0ull) continue;
+        const long long own = act ? e.w * pair_words + (long long)adj_pos(e) * W * net.dpad + 64 * w : 0ll;
+        const u64 gone = wave_settle<false>(net, mem.dom, own, act ? e.y : 0, need, todo);
+        if (gone) lane_remove(mem, ctl, nxt, slot, round, seed_both, word, gone);
+        revs += __popcll(__ballot(act && w == 0));
+      }
     }
     for (int i = itab; i < net.ntabs; i += nwaves) {
       const int c = uniform_int(net.tabs[i]);
@@ -1583,7 +1586,7 @@ __global__ void k_block_gac(DevNet net, u64* dom, int* size, int seed_var, const
   __syncthreads();
   long long before = 0;
   for (int v = threadIdx.x; v < n; v += blockDim.x) before += mem.size[v];
-  const bool ok = wg_fixpoint<true>(net, mem, &ctl, 0, seed_var >= 0 && !changed);
+  const bool ok = wg_fixpoint<true>(net, mem, &ctl, 0, changed ? -1 : seed_var);
   long long after = 0;
   for (int v = threadIdx.x; v < n; v += blockDim.x) after += mem.size[v];
   const u64 delta = wg_reduce_sum_u64(&ctl, (u64)(before - after));
@@ -1728,7 +1731,7 @@ __global__ void k_singleton_tests(DevNet net, const u64* __restrict__ base_dom,
     mem.asg[x >> 5] |= 1u << (x & 31);
   }
   __syncthreads();
-  const bool ok = wg_fixpoint<true>(net, mem, &ctl, 0, false);
+  const bool ok = wg_fixpoint<true>(net, mem, &ctl, 0, -1);
   __syncthreads();  // every wave's revision count
   if (threadIdx.x == 0) {
     fail[unit] = ok ? 0 : 1;
@@ -3375,7 +3378,7 @@ __device__ __forceinline__ void wg_mac_run(const DevNet& net, const WgMem& mem, 
       ok = wg_fixpoint_flat(mem, ctl, flat, seen, phase == ROOT ? -1 : x, phase == POSITIVE ? bit : dx & ~bit,
                             phase == POSITIVE, turn, flat_revs);
     } else {
-      ok = wg_fixpoint<kTight>(net, mem, ctl, slot, false);
+      ok = wg_fixpoint<kTight>(net, mem, ctl, slot, -1);
     }
     if (kWdeg && !ok) {
       // a wipe-out raises the weight of the constraint that AC3's order

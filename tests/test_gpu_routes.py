@@ -315,3 +315,40 @@ def test_large_tables_of_a_round_go_to_workgroups_of_their_own(gpu):
                 m.WriteDomains(0, init)
                 ms[name] = min(ms.get(name, 1e9), run().kernel_ms)
     assert ms["rounds"] < 0.43 * ms["block"], ms  # 0.36 spread, 0.49 on two workgroups
+
+
+@pytest.mark.parametrize("n,d,e,t", [(130, 64, 900, 0.886), (40, 200, 500, 0.95), (20, 1000, 120, 0.985), (70, 3, 1200, 0.05)])
+def test_workgroup_seed_with_many_arcs_equals_oracle(gpu, n, d, e, t):
+    # the seed's own arcs, 1 to 64 of them per wave, by the wave
+    desc = workload.random_binary(n, d, e, t, workload.instance_seed(44, n))
+    ok, dom, _ = oracle.Oracle(desc).root_ac()
+    assert ok
+    deg = np.bincount(desc.con_scope, minlength=n)
+    with GModelAdapter.Build(desc) as m:
+        for v in (int(np.argmax(deg)), int(np.argmin(deg))):
+            vals = domains_to_sets(dom, desc.dom_size)[v]
+            for gone in (vals[:1], vals[:len(vals) * 2 // 3]):
+                cut = dom.copy()
+                for a in gone:
+                    cut[v, a // 64] &= ~np.uint64(1 << (a % 64))
+                m.WriteDomains(0, cut)
+                st = m.EnforceGAC_Block(v)
+                ok2, dom2, _ = oracle.Oracle(desc.with_init_dom(cut)).root_ac()
+                assert st.inconsistent == (not ok2)
+                assert not ok2 or (m.ReadDomains(0) == dom2).all()
+
+
+def test_workgroup_seed_on_a_tight_network_costs_what_it_does_on_a_loose_one(gpu):
+    # one value gone, nothing follows: 16 us either way (142 and 56 with the
+    # seed's arcs settled by a lane each)
+    ms = {}
+    for t in (0.25, 0.886):
+        desc = workload.random_binary(2000, 64, 40000, t, 5, preremove=0.05)
+        with GModelAdapter.Build(desc) as m:
+            assert not m.EnforceGAC(False).inconsistent
+            cut = m.ReadDomains(0)
+            cut[1000, 0] &= cut[1000, 0] - np.uint64(1)
+            for _ in range(3):
+                m.WriteDomains(0, cut)
+                ms[t] = min(ms.get(t, 1e9), m.EnforceGAC_Block(1000).kernel_ms)
+    assert ms[0.886] < 1.8 * ms[0.25], ms
