@@ -47,6 +47,7 @@ struct DevNet {
   int ntabs;
   int cap;          // largest domain
   int simple;       // 1: no two binary constraints have the same scope
+  int big_tabs;     // how many of the tables small_table does not take
 };
 
 // Position of the variable in the constraint's scope, and the variable itself.

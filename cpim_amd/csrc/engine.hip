@@ -130,7 +130,7 @@ struct ModelImage {
   std::vector<int> tabs;              // active indices of table constraints
   bool simple = true;                 // no two binary constraints have the same scope
   int max_deg = 0;                    // most constraints on one variable
-  int big_tabs = 0;                   // tables of more than 512 tuples or over more than one word
+  int big_tabs = 0;                   // tables that small_table (device.h) does not take
   double reach = 0.0;                 // arcs of a variable and of its neighbours, mean over the values
   double density = 0.0;               // allowed share of the binary tuples (sample_density)
   std::vector<u64> rel_dense;         // owned dense rows when the desc has none
@@ -158,6 +158,22 @@ double sample_density(const ModelImage& im) {
     all += (long long)rows * im.cap[m.scope[1]];
   }
   return all ? std::min(1.0, (double)ones / (double)all) : 1.0;
+}
+
+// What tests_by_workgroup asks of a network.
+void measure_network(ModelImage& im) {
+  auto deg = [&](int v) { return im.adj_off[v + 1] - im.adj_off[v]; };
+  double values = 0.0;
+  for (int v = 0; v < im.n; ++v) {
+    long long arcs = deg(v);
+    for (int k = im.adj_off[v]; k < im.adj_off[v + 1]; ++k)
+      if (im.adj[k].y >= 0) arcs += deg(im.adj[k].y);
+    im.max_deg = std::max(im.max_deg, deg(v));
+    im.reach += (double)std::min<long long>(arcs, (long long)im.adj.size()) * im.cap[v];
+    values += im.cap[v];
+  }
+  im.reach /= values;
+  im.density = sample_density(im);
 }
 
 ModelImage make_image(const cpim_model_desc* d, bool skip_non_binary, bool own_rel = false) {
@@ -242,7 +258,7 @@ ModelImage make_image(const cpim_model_desc* d, bool skip_non_binary, bool own_r
       tsup_off += words;
       bin_ordinal_of_active.push_back(-1);
       im.tabs.push_back((int)im.con.size());
-      if (im.W > 1 || m.tw > 8) ++im.big_tabs;
+      if (im.max_dom > 16 || ar > 4 || m.tw > 8) ++im.big_tabs;
       im.con.push_back(m);
     }
   }
@@ -316,17 +332,6 @@ ModelImage make_image(const cpim_model_desc* d, bool skip_non_binary, bool own_r
       }
   }
   im.nbr.insert(im.nbr.end(), im.tabs.begin(), im.tabs.end());
-  double values = 0.0;
-  for (int v = 0; v < im.n; ++v) {
-    long long arcs = deg[v];
-    for (int k = im.adj_off[v]; k < im.adj_off[v + 1]; ++k)
-      if (im.adj[k].y >= 0) arcs += deg[im.adj[k].y];
-    im.max_deg = std::max(im.max_deg, deg[v]);
-    im.reach += (double)std::min<long long>(arcs, (long long)im.adj.size()) * im.cap[v];
-    values += im.cap[v];
-  }
-  im.reach /= values;
-  im.density = sample_density(im);
   // level 0
   im.init_dom.assign(nw, 0ull);
   for (int v = 0; v < im.n; ++v)
@@ -403,7 +408,7 @@ struct Arena {
 struct DevModel {
   int n = 0, W = 0, dpad = 0, max_dom = 0, num_active = 0;
   DevAlloc adj_off, adj, con, sup, tsup, cap, nbr;  // nbr: [n], then the table constraints
-  int ntabs = 0;
+  int ntabs = 0, big_tabs = 0;
   bool simple = false;
   DevAlloc lnet_img;  // the network image for LDS (LdsNet), when small enough
   LdsNet lnet{};
@@ -421,6 +426,7 @@ struct DevModel {
     d.tsup = tsup.as<u64>();
     d.tabs = nbr.as<int>() + n;
     d.ntabs = ntabs;
+    d.big_tabs = big_tabs;
     d.cap = max_dom;
     d.simple = simple ? 1 : 0;
     return d;
@@ -592,6 +598,7 @@ void build_device_model(const ModelImage& im, DevModel& dm, hipStream_t s, Arena
   upload(dm.cap, im.cap, s, dm.bytes, arena);
   upload(dm.nbr, im.nbr, s, dm.bytes, arena);
   dm.ntabs = (int)im.tabs.size();
+  dm.big_tabs = im.big_tabs;
   dm.simple = im.simple;
   dm.sup = dev_array(arena, (long long)sizeof(u64) * im.sup_words);
   dm.bytes += sizeof(u64) * im.sup_words;
@@ -920,6 +927,7 @@ int cpim_gmodel_create(const cpim_model_desc* desc, const cpim_gmodel_options* o
     if (opts) o = *opts;
     // validate the model before touching the device
     ModelImage im = make_image(desc, o.skip_non_binary != 0);
+    measure_network(im);
     int count = 0;
     HIPC(hipGetDeviceCount(&count));
     REQUIRE(o.device_id >= 0 && o.device_id < count, "invalid device id");

@@ -352,3 +352,52 @@ def test_workgroup_seed_on_a_tight_network_costs_what_it_does_on_a_loose_one(gpu
                 m.WriteDomains(0, cut)
                 ms[t] = min(ms.get(t, 1e9), m.EnforceGAC_Block(1000).kernel_ms)
     assert ms[0.886] < 1.8 * ms[0.25], ms
+
+
+@pytest.mark.parametrize("tables", [8, 9, 32, 33, 64, 65, 200])
+def test_tables_in_turn_and_by_changed_variable_equal_oracle(gpu, tables):
+    # up to two tables a wave (4 waves in a singleton test, 16 in the others) are
+    # taken in turn, more of them by their changed variables
+    desc = with_tables(90, 10, 120, 0.35, tables, 3, 200)
+    ok, dom, _ = oracle.Oracle(desc, oracle.AC3).root_ac()
+    assert ok
+    desc = desc.with_init_dom(dom)
+    tests = np.array([(v, a) for v, vals in enumerate(domains_to_sets(dom, desc.dom_size)) for a in vals], np.int32)
+    want, _ = oracle.Oracle(desc, oracle.AC3).singleton_tests(tests)
+    mac = oracle.Oracle(desc, oracle.AC3).mac(node_limit=150, trace_cap=400)
+    with GModelAdapter.Build(desc, GModelOptions(skip_non_binary=False)) as m:
+        got, _ = m.SingletonTests(tests, mode="workgroup")
+        assert (got == want).all()
+        for v in (int(desc.con_scope[-1]), 3):
+            vals = domains_to_sets(dom, desc.dom_size)[v]
+            cut = dom.copy()
+            cut[v] = np.uint64(1 << vals[0])
+            m.WriteDomains(0, cut)
+            st = m.EnforceGAC_Block(v)
+            ok2, dom2, _ = oracle.Oracle(desc.with_init_dom(cut), oracle.AC3).root_ac()
+            assert st.inconsistent == (not ok2)
+            assert not ok2 or (m.ReadDomains(0) == dom2).all()
+        m.WriteDomains(0, dom)
+        st, _, trace = m.Solve(node_limit=150, trace_capacity=400)
+        assert trace == mac.trace
+
+
+def test_workgroup_passes_over_unchanged_tables(gpu):
+    # a value gone from a variable of one table, which loses nothing: one round,
+    # whose cost must not grow with the tables of other variables as if they
+    # were looked at one after the other (16 waves: 56 turns for 900)
+    ms = {}
+    for tables in (30, 900):
+        desc = with_tables(2000, 12, 100, 0.2, tables, 5, 600)
+        count = np.bincount(np.concatenate([s for s in desc.scopes() if len(s) == 5]), minlength=2000)
+        v = int(np.flatnonzero(count == 1)[0])
+        with GModelAdapter.Build(desc, GModelOptions(skip_non_binary=False)) as m:
+            assert not m.EnforceGAC(False).inconsistent
+            cut = m.ReadDomains(0)
+            cut[v, 0] &= cut[v, 0] - np.uint64(1)
+            for _ in range(5):
+                m.WriteDomains(0, cut)
+                st = m.EnforceGAC_Block(v)
+                ms[tables] = min(ms.get(tables, 1e9), st.kernel_ms)
+            assert st.deletions == 0
+    assert ms[900] < 2.0 * ms[30], ms
