@@ -112,9 +112,11 @@ __device__ __forceinline__ u64 wave_settle(const DevNet& net, const u64* dom, lo
 // four tightnesses, so a few such steps settle nearly every value of a loose
 // relation.  Target side: an open value is settled by the W words of its own
 // row, by the lane, four reads a step.  Lanes that tight relations leave with
-// more than 12 steps per four words of a domain (never one-word domains) are
-// settled by the wave, one after the other (wave_settle; kTight: the searches
-// take that path only on networks of wide domains and many constraints).
+// more than 12 steps per four words of a domain are settled by the wave, one
+// after the other (wave_settle; kTight: the searches take that path only on
+// networks of wide domains and many constraints).  One-word domains get there
+// with at least 57 values against 49 open ones; by the lane n=2000 d=64 e=1500
+// t=0.97 takes 131 us persistent, so 122, and n=200 e=150 t=0.985 36 and 33.
 template <bool kCoherent, bool kTight>
 __device__ __forceinline__ u64 arcs_unsupported(const DevNet& net, const u64* dom, long long off, int src, int pos_src,
                                                 int w, u64 need) {

@@ -401,3 +401,60 @@ def test_workgroup_passes_over_unchanged_tables(gpu):
                 ms[tables] = min(ms.get(tables, 1e9), st.kernel_ms)
             assert st.deletions == 0
     assert ms[900] < 2.0 * ms[30], ms
+
+
+@pytest.mark.parametrize("mode", ["plain", "persistent", "block"])
+@pytest.mark.parametrize("n,d,e,t", [
+    # full one-word domains that tight relations leave with many open values:
+    # settled by the wave (57 values and 49 open ones are the least)
+    (2000, 64, 2000, 0.95), (2000, 64, 1500, 0.97), (60, 64, 60, 0.98), (40, 58, 30, 0.975), (30, 64, 15, 0.97),
+])
+def test_full_tight_one_word_domains_equal_oracle(gpu, n, d, e, t, mode):
+    desc = workload.random_binary(n, d, e, t, 5)
+    ok, dom, _ = oracle.Oracle(desc).root_ac()
+    with GModelAdapter.Build(desc) as m:
+        st = {"plain": lambda: m.EnforceGAC(False), "persistent": lambda: m.EnforceGAC_Persistent(False),
+              "block": m.EnforceGAC_Block}[mode]()
+        assert st.inconsistent == (not ok)
+        assert not ok or (m.ReadDomains(0) == dom).all()
+
+
+@pytest.mark.parametrize("mode", ["plain", "persistent"])
+@pytest.mark.parametrize("n,d,e,t,tables", [
+    # the persistent rounds stage up to 128 KB of domains in LDS: 72, 100 and 120
+    # KB, and beyond it, where every lane reads memory, with and without tables
+    (600, 960, 90, 0.992, 0), (800, 1000, 120, 0.992, 0), (960, 1000, 120, 0.99, 0), (1030, 1000, 150, 0.991, 0),
+    (8400, 70, 60, 0.93, 30),
+])
+def test_staged_and_unstaged_rounds_equal_oracle(gpu, n, d, e, t, tables, mode):
+    base = workload.random_binary(n, d, e, t, workload.instance_seed(45, n), preremove=0.1)
+    desc = base
+    if tables:
+        scopes, lists = [list(s) for s in base.scopes()], list(base.tuple_lists())
+        rng = np.random.default_rng(n)
+        for k in range(tables):
+            scopes.append([int(base.con_scope[2 * k]), *map(int, rng.choice(np.arange(n // 2, n), 2, replace=False))])
+            lists.append(workload.random_table(500 * n + k, 3, d, 2500))
+        desc = from_tuples(base.dom_size, scopes, lists, base.init_dom)
+    algo = oracle.AC3 if tables else oracle.AC3BIT
+    ok, dom, _ = oracle.Oracle(desc, algo).root_ac()
+    assert ok
+    with GModelAdapter.Build(desc, GModelOptions(skip_non_binary=False)) as m:
+        run = (lambda v: m.EnforceGAC(False, v)) if mode == "plain" else (lambda v: m.EnforceGAC_Persistent(False, v))
+        st = run(-1)
+        assert not st.inconsistent and st.converged
+        assert (m.ReadDomains(0) == dom).all()
+        removed = 0
+        for v in np.argsort(np.bincount(desc.con_scope, minlength=n))[::-1][:3]:  # the best connected ones
+            vals = domains_to_sets(dom, desc.dom_size)[v]
+            cut = dom.copy()
+            for a in vals[::2]:
+                cut[v, a // 64] &= ~np.uint64(1 << (a % 64))
+            m.WriteDomains(0, cut)
+            st = run(int(v))
+            ok2, dom2, _ = oracle.Oracle(desc.with_init_dom(cut), algo).root_ac()
+            assert st.inconsistent == (not ok2)
+            if ok2:
+                assert (m.ReadDomains(0) == dom2).all()
+                removed += int(np.bitwise_count(cut).sum()) - int(np.bitwise_count(dom2).sum())
+        assert removed > 0, "the seeded half removed nothing"
