@@ -1936,16 +1936,19 @@ void run_singleton_plain(cpim_gmodel* m, const int2* tests, long long count, uns
 // against 33.5 ms).  A variable whose neighbour kept p d values loses a value to
 // it with probability (1 - p)^(p d); 50 values lost to deg neighbours are the
 // line (24 lost at n=300 d=64 e=1000 t=0.80, 965 against 631 us; 73 at t=0.84,
-// 1350 against 4026 us).
+// 1350 against 4026 us); beyond 10 turns one loss a value is asked as well
+// (n=150 d=200 e=300, 14.6 turns: 0.9 lost at t=0.916, 1396 against 947 us; 2.3
+// at t=0.948, 6200 against 11868).
 // A long chain (a path, a lattice) takes about as many rounds as it changes
 // variables, and every turn of workgroups pays for all of them: there a group's
-// variables, times the arcs within reach over a path's six, must outnumber the
-// turns.  Measured, workgroups against bit-sliced, us:
+// variables, times the arcs within reach over a path's six (with cascades arc
+// words over three), must outnumber the turns.  Measured, workgroups against bit-sliced, us:
 //   n=60 d=37 e=500      88 / 173, cascading 330 / 2899
 //   n=120 d=50 e=3570   309 / 761      n=200 d=64 e=4000   379 / 503
 //   n=100 d=100 e=1500  347 / 421      n=500 d=16 e=3000   171 / 342
 //   n=200 d=64 e=800    182 / 157, cascading 1572 / 5611
 //   n=60 d=300 e=300    427 / 341, cascading 6686 / 26152
+//   n=40 d=1000 e=100   cascading 44416 / 119273
 //   n=100 d=128 e=600   215 / 199      n=200 d=128 e=2000  616 / 398
 //   star n=600 d=64     684 / 1309     star n=2000 d=64    6977 / 5211
 //   path n=60 d=37      495 / 355      path n=700 d=64     148098 / 8566
@@ -1962,10 +1965,11 @@ bool tests_by_workgroup(const cpim_gmodel* m, long long tests) {
   const double waves = std::max(1.0, std::ceil((double)tests / (64.0 * M * 2.0 * cus)));
   const double by_wg = turns * (18.0 + m->im.reach * W / 50.0);
   const double sliced = waves * (vars * (1.0 + deg) * (7.5 + 0.5 * W) + 2.5 * (m->im.max_deg - deg));
-  const double p = m->im.density;
-  const bool cascades =
-      (double)tests * m->im.reach * W <= (double)(24ll << 20) && d * deg * std::pow(1.0 - p, p * d) >= 50.0;
-  return (cascades || by_wg <= sliced) && 1.6 * turns <= vars * std::max(1.0, m->im.reach / (cascades ? 3.0 : 6.0));
+  const double p = m->im.density, lost = deg * std::pow(1.0 - p, p * d);  // of a value's chances, by all neighbours
+  const bool cascades = (double)tests * m->im.reach * W <= (double)(24ll << 20) && d * lost >= 50.0 &&
+                        (turns <= 10.0 || lost >= 1.0);
+  const double spread = cascades ? m->im.reach * W / 3.0 : m->im.reach / 6.0;
+  return (cascades || by_wg <= sliced) && 1.6 * turns <= vars * std::max(1.0, spread);
 }
 
 void run_singleton_device(cpim_gmodel* m, int mode, const int2* tests, long long count, unsigned char* fail_out,
