@@ -3525,14 +3525,15 @@ __device__ __forceinline__ void wg_mac_run(const DevNet& net, const WgMem& mem, 
 
 // lnet.bytes > 0 (kLds only): the network image is copied into LDS behind
 // the working memory and the search reads the network from there.  kTight: the
-// network is one for the tight path (tight_search; it has no image).
+// network is one for the tight path (tight_search), whose rows alone are more
+// than 3 MB: it has no image.
 template <bool kLds, bool kWdeg, bool kTight>
 __global__ void k_mac(DevNet net, MacArgs args, char* scratch, LdsNet lnet) {
   extern __shared__ __align__(16) char smem[];
   __shared__ WgCtl ctl;
   int* stamp = nullptr;
   if (kWdeg) stamp = args.stamp_off ? (int*)(smem + args.stamp_off) : args.stamp_tab;
-  if (kLds && lnet.bytes > 0) {
+  if (kLds && !kTight && lnet.bytes > 0) {
     const DevNet ln = wg_load_net(net, lnet, smem + wg_mem_bytes(net.n, net.W));
     WgMem mem = wg_carve(smem, ln);
     mem.stamp = stamp;
