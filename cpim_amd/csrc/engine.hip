@@ -462,7 +462,10 @@ struct LdsLayout {
 };
 
 LdsLayout lds_layout(const ModelImage& im, bool odd = true) {
-  // an even stride only where the odd one alone keeps the image out of LDS
+  // an even stride only where the odd one alone keeps the image out of LDS.
+  // The odd one can make the image too large for a unit's share of a CU; the
+  // rows are then read from memory.  A batch at that line, 512 x n=60 d=8
+  // e=355, takes 1.6 ms all the same.
   const int n = im.n, W = im.W, dc = odd ? im.max_dom | 1 : im.max_dom;
   const long long npairs = (long long)im.bin_cons.size();
   long long tsup_c = 0;
@@ -1253,12 +1256,12 @@ void gac_grid(cpim_gmodel* m, int assigned_var, bool persistent, cpim_gac_stats*
 // the domains in LDS, and beyond which the host-driven rounds, each spread
 // over the grid.  Measured (one workgroup against rounds, us; the root of a
 // network whose revisions all find supports / of one that cascades / after
-// one assignment): 300 constraints of 20 values 16/23/25 against 15/38/28;
-// 1000 of 16 values 23/32/31 against 16/38/33; 1000 of 64 values 24/85/32
-// against 16/58/30; 2500 of 16 values 35/57/38 against 16/58/32; 1000 of 200
-// values (4 words) 43/712/36 against 17/189/35.  The asynchronous kernel takes
-// 200 to 750 us after one assignment where the rounds take 31 to 39 (500 to
-// 2000 variables); the persistent kernel is faster still (21 to 34), but needs
+// one assignment): 300 constraints of 20 values 16/23/17 against 14/36/27;
+// 1000 of 16 values 23/32/19 against 15/38/31; 1000 of 64 values 24/84/19
+// against 15/58/29; 2500 of 16 values 36/57/21 against 16/57/33; 1000 of 200
+// values (4 words) 42/708/24 against 16/133/35.  The asynchronous kernel takes
+// 165 to 700 us after one assignment where the rounds take 31 to 46 (300 to
+// 2000 variables); the persistent kernel is faster still (22 to 34), but needs
 // every workgroup resident at once, which AUTO does not ask of a caller with
 // several streams.
 constexpr long long kAutoBlockWords = 800;
@@ -1991,7 +1994,7 @@ void run_singleton_device(cpim_gmodel* m, int mode, const int2* tests, long long
 }
 
 // One host-driven fixpoint per test on a scratch level: copy the level,
-// reduce x to {a}, seed the constraints of x, rounds with a sync each.
+// reduce x to {a}, seed the constraints of x, rounds as in gac_grid.
 void run_singleton_plain(cpim_gmodel* m, const int2* tests, long long count, unsigned char* fail_host,
                          cpim_sac_stats* st) {
   const int L = m->current_level;

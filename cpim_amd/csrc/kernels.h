@@ -205,9 +205,9 @@ __device__ __forceinline__ u64 arcs_unsupported(const DevNet& net, const u64* do
 // a frontier of constraints, each revised in both directions by a wave that
 // read 64 rows of either side, and every removal marked all constraints of its
 // variable.  Kernel time, before and after (host-driven rounds): n=2000 d=64
-// e=40000, one round without removals 24.8 -> 12.5 us; its cascade at t=0.886
-// (10 rounds, 6,485 removals) 225 -> 151 us, persistent 269 -> 162 us; n=500
-// d=250 e=20000 t=0.963 (5 rounds) 293 -> 188 us, persistent 346 -> 195 us.
+// e=40000, one round without removals 30 -> 7.2 us; its cascade at t=0.886
+// (10 rounds, 6,485 removals) 255 -> 160 us, persistent 318 -> 158 us; n=500
+// d=250 e=20000 t=0.963 (5 rounds) 314 -> 197 us, persistent 372 -> 183 us.
 // ===========================================================================
 // Outcome of a fixpoint (or of one of its host-driven rounds).
 struct GacResult {
@@ -555,8 +555,9 @@ __global__ void __launch_bounds__(kRoundThreads) k_gac_round(DevNet net, u64* do
 
 // ===========================================================================
 // Persistent fixpoint: every round in one launch, rounds separated by a grid
-// barrier.  The grid is sized by the host so that every workgroup is resident
-// at once (occupancy x CUs).
+// barrier.  The host launches at most one workgroup a CU (1024 threads, at most
+// 128 KB of LDS), so that all are resident at once unless other launches hold
+// CUs; the bounded waits below cover that case.
 //
 // The barrier is a ticket count that only grows: thread 0 of each workgroup
 // takes a ticket (an atomic add that returns the count) and waits until the

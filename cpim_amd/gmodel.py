@@ -301,8 +301,8 @@ class GModel:
 
         heuristic: "dom" (smallest domain, MAC.cpp:356-364), "dom/deg"
         (domain size over neighbour count, MAC.cpp:371-384) or "dom/wdeg"
-        (domain size over failure-weighted degree, MAC.cpp:386-411; its
-        fixpoints run in AC3's order on one wave)."""
+        (domain size over failure-weighted degree, MAC.cpp:386-411; a
+        fixpoint that wipes out is repeated in AC3's order on one wave)."""
         stats, sols, trace = self.SolveAll(1, 1, time_limit_ms, node_limit, trace_capacity, heuristic)
         return stats, (sols[0] if len(sols) else None), trace
 

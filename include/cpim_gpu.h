@@ -157,13 +157,20 @@ typedef struct cpim_gac_stats {
                                  barrier between rounds; every barrier wait is bounded by the
                                  fixpoint_budget_us knob (CPIM_ERR_RUNTIME when it runs out) */
 #define CPIM_GAC_BLOCK 2      /* one workgroup, domains in LDS, one launch */
-#define CPIM_GAC_AUTO 3       /* autotuned choice among the modes that run */
+#define CPIM_GAC_AUTO 3       /* BLOCK for small networks, else PLAIN (by constraints and words a
+                                 domain); a long narrow cascade goes on in one launch */
 #define CPIM_GAC_ASYNC 4      /* one launch, whole GPU, asynchronous work queue,
                                  no grid barrier */
 
 /* GModel::EnforceGAC / EnforceGAC_Persistent (include/GModel.cuh:191-197,
  * src/GModel.cu:1110-1391) on the current level.  assigned_var < 0 seeds all
- * constraints; assigned_var >= 0 seeds the constraints of that variable.
+ * constraints; assigned_var >= 0 seeds the constraints of that variable.  The
+ * result is the closure if only that variable changed since the level was at
+ * its closure.  On any other level a seeded fixpoint reaches as far as its
+ * frontier does: PLAIN, PERSISTENT and ASYNC, and AUTO above 4,096 constraints
+ * or where the domains don't fit in LDS, revise every constraint of a changed
+ * variable in both directions; BLOCK, and AUTO otherwise, revise the other
+ * variables of its constraints.
  * Never fails on inconsistency: that is reported in stats->inconsistent. */
 int cpim_gmodel_enforce_gac(cpim_gmodel* model, int32_t assigned_var, int32_t mode,
                             cpim_gac_stats* stats);
@@ -171,10 +178,11 @@ int cpim_gmodel_enforce_gac(cpim_gmodel* model, int32_t assigned_var, int32_t mo
 /* No counterpart in the reference.  The persistent mode of
  * cpim_gmodel_enforce_gac for callers that cannot allocate (code under HIP
  * graph capture, tight serving loops, harnesses that forbid hipMalloc): it
- * allocates nothing.  Its scratch (control block and frontier bitmaps) is a
- * file-scope device array of 776 KiB per GPU, held until the process ends, so
- * it takes networks of at most 2,097,152 propagated constraints
- * (CPIM_ERR_INVALID_ARGUMENT above that).  Calls that overlap on one GPU race
+ * allocates nothing.  Its scratch (control block and bitmaps of
+ * the changed variables) is a file-scope device array of 776 KiB per GPU, held
+ * until the process ends.  It takes networks of at most 2,097,152 variables
+ * (what the scratch holds) and 2,097,152 propagated constraints
+ * (CPIM_ERR_INVALID_ARGUMENT above either).  Calls that overlap on one GPU race
  * on that array.  stats->kernel_ms is 0 (no events are created). */
 int cpim_gmodel_enforce_gac_noalloc(cpim_gmodel* model, int32_t assigned_var, cpim_gac_stats* stats);
 
@@ -240,8 +248,9 @@ typedef struct cpim_sac_stats {
 int cpim_tune_set(const char* name, int64_t value);
 int cpim_tune_get(const char* name, int64_t* value);
 
-#define CPIM_SAC_BATCHED 0   /* every singleton test of a pass on the device: SLICED for large passes
-                                over binary networks, else WORKGROUP */
+#define CPIM_SAC_BATCHED 0   /* every singleton test of a pass on the device: WORKGROUP for networks
+                                with tables and, on a level at its closure, for passes that an
+                                estimate of both finds shorter that way; else SLICED */
 #define CPIM_SAC_PLAIN 1     /* one host-driven fixpoint per singleton test */
 #define CPIM_SAC_WORKGROUP 2 /* one workgroup per singleton test, domain copy in LDS */
 #define CPIM_SAC_SLICED 3    /* 64 singleton tests per workgroup, bit-sliced; CPIM_ERR_UNSUPPORTED
@@ -275,9 +284,9 @@ int cpim_gmodel_singleton_tests(cpim_gmodel* model, const int32_t* tests, int64_
  *             start at 1 with the model, persist across solves (read and
  *             reset them with cpim_gmodel_weights) and grow by one on the
  *             constraint that empties a domain first in AC3's order
- *             (src/AC3.cpp:122-126);
- *             with this ordering every fixpoint of the search runs in that
- *             order, on one wave, so it is slower than the other two.
+ *             (src/AC3.cpp:122-126).  A fixpoint that ends in a wipe-out is
+ *             therefore run a second time in that order, on one wave, so this
+ *             ordering is slower than the other two.
  * Neighbours are the distinct other variables of the constraints on x
  * (Network::get_neighbor, src/Network.cpp:467-474), counted over the
  * constraints the model propagates. */
