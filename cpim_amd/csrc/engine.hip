@@ -542,19 +542,25 @@ void build_lds_image(const ModelImage& im, DevModel& dm, hipStream_t s, std::vec
   }
 }
 
-// Whether a search on this network settles tight relations by the wave
-// (wave_settle): domains of three words and more, and at least 12 turns of a
+// Whether a search takes the whole workgroup fixpoint (wg_fixpoint's kFull) when
+// it has no network image.
+//
+// For the tables, more than kTableTurns a wave: 300 of arity 5 and 3,000 tuples,
+// 60 nodes, 34 ms against 43; 900 of arity 3, 7.4 against 15.3 ms.
+//
+// For tight relations settled by the wave (wave_settle), domains of three words and more, and at least 12 turns of a
 // 1024-lane workgroup over the arc words.  Where that is so, a lane's serial
 // work is what a round waits for.  With it against without it, ms: n=300 d=250
 // e=20000 t=0.963, 30 nodes 13.8 / 25.5, t=0.95 6.3 / 10.1; n=300 d=250 e=2000
 // t=0.97 2.7 / 3.7; n=50 d=1000 e=600 t=0.97 2.7 / 3.2, t=0.5 2.24 / 2.17.
 // Below that line, and for two words, the choice between the two sides costs
 // more than it saves: n=30 d=1000 e=131 3.7 / 2.4; n=100 d=250 e=1000 t=0.9 5.9
-// / 5.1; n=300 d=100 e=6000 t=0.84 1.66 / 1.39.
-bool tight_search(const ModelImage& im) {
+// / 5.1; n=300 d=100 e=6000 t=0.84 1.66 / 1.39.  (Such a network's rows alone
+// are more than 3 MB, far beyond an image.)
+bool full_search(const ModelImage& im, int waves) {
   long long wp = 1;
   while (wp < im.W) wp *= 2;
-  return im.W >= 3 && (long long)im.adj.size() * wp >= 12 * 1024;
+  return (int)im.tabs.size() > kTableTurns * waves || (im.W >= 3 && (long long)im.adj.size() * wp >= 12 * 1024);
 }
 
 // Device bytes build_device_model takes from an arena for im (the same
@@ -2221,7 +2227,7 @@ int cpim_gmodel_solve(cpim_gmodel* m, const cpim_solve_opts* opts, cpim_search_s
       char* scratch = lds ? nullptr : m->get_scratch(bytes);
       auto* kernel = lds ? (A.weight ? k_mac<true, true, false> : k_mac<true, false, false>)
                          : (A.weight ? k_mac<false, true, false> : k_mac<false, false, false>);
-      if (tight_search(m->im))
+      if ((!lds || lnet.bytes == 0) && full_search(m->im, threads / 64))
         kernel = lds ? (A.weight ? k_mac<true, true, true> : k_mac<true, false, true>)
                      : (A.weight ? k_mac<false, true, true> : k_mac<false, false, true>);
       hipLaunchKernelGGL(kernel, dim3(1), dim3(threads), (size_t)dyn, m->stream, net, A, scratch, lds ? lnet : LdsNet{});

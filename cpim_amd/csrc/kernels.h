@@ -1183,7 +1183,16 @@ __device__ __forceinline__ void wg_seed(const WgMem& mem, WgCtl* ctl, int n, int
 // that still decides round r is not misled by one already in round r + 1.
 // slot: two wipe-out words used in turn by successive fixpoints, so that
 // wg_seed never resets the word a slow wave still reads.
-template <bool kTight>
+//
+// kFull: tight relations are settled by the wave (wave_unsupported), and of many
+// tables only those with a changed variable are taken up.  Both only cost
+// registers on the other networks, where a search waits for every instruction of
+// its chain (n=23 d=23 e=253 and dom/wdeg on n=100 d=50 take 3 % longer with the
+// look at the tables in their kernels): searches take the whole fixpoint where
+// the host's full_search says so.
+constexpr int kTableTurns = 4;  // tables a wave takes up in turn at most
+
+template <bool kFull>
 __device__ __forceinline__ bool wg_fixpoint(const DevNet& net, const WgMem& mem, WgCtl* ctl, int slot,
                                             int seed_both) {
   const int n = net.n, W = net.W;
@@ -1201,7 +1210,7 @@ __device__ __forceinline__ bool wg_fixpoint(const DevNet& net, const WgMem& mem,
   int c0 = 0, c1 = nvw, c2 = 2 * nvw;
   // this wave's first table, its lanes' part kept over the rounds
   const int itab = nwaves - 1 - wave;
-  const bool many_tabs = net.ntabs > 2 * nwaves;
+  const bool many_tabs = kFull && net.ntabs > kTableTurns * nwaves;
   SmallTable tab0{};
   if (itab < net.ntabs) tab0 = load_small_table(net, uniform_int(net.tabs[itab]));
   for (int round = 0;; ++round) {
@@ -1258,7 +1267,7 @@ __device__ __forceinline__ bool wg_fixpoint(const DevNet& net, const WgMem& mem,
           stop = true;
           break;
         }
-        const u64 gone = wave_unsupported<kTight>(net, mem.dom, t, pair + (long long)(pos_t * W + w) * net.dpad,
+        const u64 gone = wave_unsupported<kFull>(net, mem.dom, t, pair + (long long)(pos_t * W + w) * net.dpad,
                                                   pair + (long long)(1 - pos_t) * W * net.dpad + 64 * w, need);
         if (gone) lane_remove(mem, ctl, nxt, slot, round, u, word, gone);
         revs += cnt;
@@ -1285,8 +1294,8 @@ __device__ __forceinline__ bool wg_fixpoint(const DevNet& net, const WgMem& mem,
         revs += __popcll(__ballot(act && w == 0));
       }
     }
-    // Tables in turn, one a wave; where they are more than two a wave, its lanes
-    // first look which ones have a changed variable.  Small tables: each wave
+    // Tables in turn, one a wave; where they are more than kTableTurns a wave, its
+    // lanes first look which ones have a changed variable.  Small tables: each wave
     // looks at its own (every nwaves-th, so that a variable's tables, often
     // neighbours, are not left to one wave).  Larger ones cost more than the
     // look, so that every wave looks at all of them and takes every nwaves-th
@@ -1294,70 +1303,68 @@ __device__ __forceinline__ bool wg_fixpoint(const DevNet& net, const WgMem& mem,
     // tuples after one assignment 201 / 190 / 142, the tests of that network 1208
     // / 1013 / 774; 900 small ones 174 / 86 / 131, tests 2410 / 1273 / 1385.
     const int look = net.big_tabs ? 1 : nwaves;  // tables between two lanes'
-    u64 found = 0ull;
-    int base = -64 * look, turn = look == 1 ? itab : 0;
-    for (int i = itab;; i += nwaves) {
-      if (many_tabs) {
-        while (turn >= __popcll(found) && base + 64 * look < net.ntabs) {
-          turn -= __popcll(found);
-          base += 64 * look;
-          const int k = base + lane * look + (look == 1 ? 0 : itab);
-          bool ch = false;
-          if (k < net.ntabs) {
-            const ConMeta* mp = net.con + net.tabs[k];
-            const int arity = mp->arity;
-            unsigned bits = 0u;
+    int seen = 0;                                // changed tables before this turn's
+    for (int base = many_tabs && look == 1 ? 0 : itab; base < net.ntabs; base += many_tabs ? 64 * look : nwaves) {
+      u64 found = 1ull;  // bit k: table base + k * look is this wave's
+      if (kFull && many_tabs) {
+        const int k = base + lane * look;
+        bool ch = false;
+        if (k < net.ntabs) {
+          const ConMeta* mp = net.con + net.tabs[k];
+          const int arity = mp->arity;
+          unsigned bits = 0u;
 #pragma unroll
-            for (int p = 0; p < CPIM_MAX_ARITY; ++p) {  // (unused positions hold variable 0)
-              const int y = mp->scope[p];
-              bits |= p < arity ? cur[y >> 5] >> (y & 31) : 0u;
-            }
-            ch = bits & 1u;
+          for (int p = 0; p < CPIM_MAX_ARITY; ++p) {  // (unused positions hold variable 0)
+            const int y = mp->scope[p];
+            bits |= p < arity ? cur[y >> 5] >> (y & 31) : 0u;
           }
-          found = __ballot(ch);
+          ch = bits & 1u;
         }
-        if (turn >= __popcll(found)) break;
-        for (; turn > 0; --turn) found &= found - 1ull;
-        i = uniform_int(base + (int)__builtin_ctzll(found) * look + (look == 1 ? 0 : itab));
-        found &= found - 1ull;
-        turn = look == 1 ? nwaves - 1 : 0;
+        found = __ballot(ch);
+        if (look == 1) {
+          const int rank = seen + __popcll(found & ((1ull << lane) - 1ull));
+          seen += __popcll(found);
+          found = __ballot(ch && rank % nwaves == itab);
+        }
       }
-      if (i >= net.ntabs) break;
-      const int c = uniform_int(net.tabs[i]);
-      SmallTable tab = tab0;
-      if (i != itab) tab = load_small_table(net, c);
-      const bool small = uniform_int(small_table(net, net.con[c].arity, tab.tw)) != 0;
-      int y = tab.y;
-      if (!small) y = lane < net.con[c].arity ? net.con[c].scope[lane] : -1;
-      const int yy = y >= 0 ? y : 0;
-      const bool mine_changed = y >= 0 && bit_of(cur, yy);
-      const bool assigned = bit_of(mem.asg, yy);
-      const u64 dp = small ? ld_wg(&mem.dom[yy]) : 0ull;
-      const u64 changed = __ballot(mine_changed);
-      if (changed == 0ull) continue;
-      ++revs;
-      if (small) {
-        // lane 8 p removes for position p, but not for the only changed one
-        u64 rows[8];
-        small_table_rows(tab, rows);
-        const unsigned gone = (unsigned)dp & ~small_table_keep(tab.y, tab.tw, rows, (unsigned)dp);
-        const unsigned pos = (unsigned)changed & 0x01010101u;
-        const u64 stays = both || (pos & (pos - 1u)) ? 0ull : pos;
-        if (gone && y >= 0 && !assigned && lane < 32 && (lane & 7) == 0 && !((stays >> lane) & 1ull))
-          lane_remove(mem, ctl, nxt, slot, round, y, &mem.dom[y], (u64)gone);
-        continue;
+      for (; found != 0ull; found &= found - 1ull) {
+        const int i = uniform_int(base + (int)__builtin_ctzll(found) * look);
+        const int c = uniform_int(net.tabs[i]);
+        SmallTable tab = tab0;
+        if (i != itab) tab = load_small_table(net, c);
+        const bool small = uniform_int(small_table(net, net.con[c].arity, tab.tw)) != 0;
+        int y = tab.y;
+        if (!small) y = lane < net.con[c].arity ? net.con[c].scope[lane] : -1;
+        const int yy = y >= 0 ? y : 0;
+        const bool mine_changed = y >= 0 && bit_of(cur, yy);
+        const bool assigned = bit_of(mem.asg, yy);
+        const u64 dp = small ? ld_wg(&mem.dom[yy]) : 0ull;
+        const u64 changed = __ballot(mine_changed);
+        if (changed == 0ull) continue;
+        ++revs;
+        if (small) {
+          // lane 8 p removes for position p, but not for the only changed one
+          u64 rows[8];
+          small_table_rows(tab, rows);
+          const unsigned gone = (unsigned)dp & ~small_table_keep(tab.y, tab.tw, rows, (unsigned)dp);
+          const unsigned pos = (unsigned)changed & 0x01010101u;
+          const u64 stays = both || (pos & (pos - 1u)) ? 0ull : pos;
+          if (gone && y >= 0 && !assigned && lane < 32 && (lane & 7) == 0 && !((stays >> lane) & 1ull))
+            lane_remove(mem, ctl, nxt, slot, round, y, &mem.dom[y], (u64)gone);
+          continue;
+        }
+        // one changed variable: its own position is not revised (AC3 does not
+        // either, src/AC3.cpp:106-118; at a closure its values keep their supports)
+        int skip = -1;
+        if (!both && (changed & (changed - 1ull)) == 0ull) skip = __builtin_amdgcn_readlane(y, (int)__builtin_ctzll(changed));
+        bool wiped = false;
+        revise_table(net, mem.dom, mem.size, c, skip, mem.asg,
+                     [&](int v, int) {
+                       if (lane == 0) atomicOr(&nxt[v >> 5], 1u << (v & 31));
+                     },
+                     &wiped);
+        if (wiped && lane == 0) atomicMin(&ctl->wipe_round[slot], round);
       }
-      // one changed variable: its own position is not revised (AC3 does not
-      // either, src/AC3.cpp:106-118; at a closure its values keep their supports)
-      int skip = -1;
-      if (!both && (changed & (changed - 1ull)) == 0ull) skip = __builtin_amdgcn_readlane(y, (int)__builtin_ctzll(changed));
-      bool wiped = false;
-      revise_table(net, mem.dom, mem.size, c, skip, mem.asg,
-                   [&](int v, int) {
-                     if (lane == 0) atomicOr(&nxt[v >> 5], 1u << (v & 31));
-                   },
-                   &wiped);
-      if (wiped && lane == 0) atomicMin(&ctl->wipe_round[slot], round);
     }
     __syncthreads();
     const int wr = ld_wg_int(&ctl->wipe_round[slot]);
@@ -3268,8 +3275,8 @@ __device__ __forceinline__ void wg_load_level(const WgMem& mem, const u64* level
 // one, beside the fixpoint's own.  kWdeg: dom/wdeg ordering, wipe-outs
 // repeated in AC3's order.  kFlat: wg_fixpoint_flat propagates, and a
 // refutation that follows its decision takes the domains from registers (dom
-// and dom/deg only).  kTight: tight relations are settled by the wave.
-template <bool kWdeg, bool kFlat, bool kTight>
+// and dom/deg only).  kFull: as wg_fixpoint's.
+template <bool kWdeg, bool kFlat, bool kFull>
 __device__ __forceinline__ void wg_mac_run(const DevNet& net, const WgMem& mem, WgCtl* ctl, const MacArgs& A) {
   enum { ROOT, POSITIVE, NEGATIVE };
   const int n = net.n, W = net.W;
@@ -3419,7 +3426,7 @@ __device__ __forceinline__ void wg_mac_run(const DevNet& net, const WgMem& mem, 
       ok = wg_fixpoint_flat(mem, ctl, flat, seen, phase == ROOT ? -1 : x, phase == POSITIVE ? bit : dx & ~bit,
                             phase == POSITIVE, turn, flat_revs);
     } else {
-      ok = wg_fixpoint<kTight>(net, mem, ctl, slot, -1);
+      ok = wg_fixpoint<kFull>(net, mem, ctl, slot, -1);
     }
     if (kWdeg && !ok) {
       // a wipe-out raises the weight of the constraint that AC3's order
@@ -3525,16 +3532,15 @@ __device__ __forceinline__ void wg_mac_run(const DevNet& net, const WgMem& mem, 
 }
 
 // lnet.bytes > 0 (kLds only): the network image is copied into LDS behind
-// the working memory and the search reads the network from there.  kTight: the
-// network is one for the tight path (tight_search), whose rows alone are more
-// than 3 MB: it has no image.
-template <bool kLds, bool kWdeg, bool kTight>
+// the working memory and the search reads the network from there.  kFull: a
+// network for the whole fixpoint (full_search), which has no image.
+template <bool kLds, bool kWdeg, bool kFull>
 __global__ void k_mac(DevNet net, MacArgs args, char* scratch, LdsNet lnet) {
   extern __shared__ __align__(16) char smem[];
   __shared__ WgCtl ctl;
   int* stamp = nullptr;
   if (kWdeg) stamp = args.stamp_off ? (int*)(smem + args.stamp_off) : args.stamp_tab;
-  if (kLds && !kTight && lnet.bytes > 0) {
+  if (kLds && !kFull && lnet.bytes > 0) {
     const DevNet ln = wg_load_net(net, lnet, smem + wg_mem_bytes(net.n, net.W));
     WgMem mem = wg_carve(smem, ln);
     mem.stamp = stamp;
@@ -3543,7 +3549,7 @@ __global__ void k_mac(DevNet net, MacArgs args, char* scratch, LdsNet lnet) {
   } else {
     WgMem mem = wg_carve(kLds ? smem : scratch, net);
     mem.stamp = stamp;
-    wg_mac_run<kWdeg, false, kTight>(net, mem, &ctl, args);
+    wg_mac_run<kWdeg, false, kFull>(net, mem, &ctl, args);
   }
 }
 
@@ -3558,15 +3564,15 @@ struct UnitDesc {
   long long scratch_off;  // per-unit global scratch when the domain does not fit in LDS
   int use_lds;            // 1: working memory in LDS; 2: network image in LDS as well
   int reset;              // 1: start the search over: level 0 = init, state = MAC_INIT
-  int tight;              // 1: the fixpoints keep the tight path (k_mac_units<true>)
+  int full;               // 1: the search takes the whole fixpoint (k_mac_units<true>)
   const u64* init;        // the unit's initial domains, [n][W]
   LdsNet lnet;
 };
 
 // states_out[u] receives a copy of unit u's state when its launch ends, so
-// the host reads every unit's outcome with one copy.  kTight: launches with a
-// unit for the tight path (the others of it still leave it out).
-template <bool kTight>
+// the host reads every unit's outcome with one copy.  kFull: launches with a
+// unit that takes the whole fixpoint (the others of it still don't).
+template <bool kFull>
 __global__ void k_mac_units(const UnitDesc* __restrict__ units, int count, unsigned* counter,
                             int only, char* scratch, MacState* states_out) {
   extern __shared__ __align__(16) char smem[];
@@ -3603,11 +3609,11 @@ __global__ void k_mac_units(const UnitDesc* __restrict__ units, int count, unsig
       else
         wg_mac_run<false, false, false>(ln, wg_carve(smem, ln), &ctl, d.args);
     } else if (where == 1) {
-      if (kTight && uniform_int(d.tight)) wg_mac_run<false, false, kTight>(d.net, wg_carve(smem, d.net), &ctl, d.args);
+      if (kFull && uniform_int(d.full)) wg_mac_run<false, false, kFull>(d.net, wg_carve(smem, d.net), &ctl, d.args);
       else wg_mac_run<false, false, false>(d.net, wg_carve(smem, d.net), &ctl, d.args);
     } else {
       const WgMem mem = wg_carve(scratch + d.scratch_off, d.net);
-      if (kTight && uniform_int(d.tight)) wg_mac_run<false, false, kTight>(d.net, mem, &ctl, d.args);
+      if (kFull && uniform_int(d.full)) wg_mac_run<false, false, kFull>(d.net, mem, &ctl, d.args);
       else wg_mac_run<false, false, false>(d.net, mem, &ctl, d.args);
     }
     if (threadIdx.x == 0) states_out[u] = *d.args.state;

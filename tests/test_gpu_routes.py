@@ -7,6 +7,7 @@ import pytest
 
 import oracle
 from cpim_amd import Batch, GModelAdapter, GModelOptions, workload
+from cpim_amd import _native as N
 from cpim_amd.model import ModelDesc, domains_to_sets, from_tuples, words_for
 
 pytestmark = pytest.mark.gpu
@@ -354,9 +355,9 @@ def test_workgroup_seed_on_a_tight_network_costs_what_it_does_on_a_loose_one(gpu
     assert ms[0.886] < 1.8 * ms[0.25], ms
 
 
-@pytest.mark.parametrize("tables", [8, 9, 32, 33, 64, 65, 200])
+@pytest.mark.parametrize("tables", [8, 16, 17, 32, 33, 64, 65, 200])
 def test_tables_in_turn_and_by_changed_variable_equal_oracle(gpu, tables):
-    # up to two tables a wave (4 waves in a singleton test, 16 in the others) are
+    # up to four tables a wave (4 waves in a singleton test, 16 in the others) are
     # taken in turn, more of them by their changed variables
     desc = with_tables(90, 10, 120, 0.35, tables, 3, 200)
     ok, dom, _ = oracle.Oracle(desc, oracle.AC3).root_ac()
@@ -380,6 +381,43 @@ def test_tables_in_turn_and_by_changed_variable_equal_oracle(gpu, tables):
         m.WriteDomains(0, dom)
         st, _, trace = m.Solve(node_limit=150, trace_capacity=400)
         assert trace == mac.trace
+
+
+@pytest.mark.parametrize("heuristic", ["dom", "dom/wdeg"])
+@pytest.mark.parametrize("tables", [64, 65, 200])
+@pytest.mark.parametrize("d,arity,tuples,keep", [(12, 3, 700, 0.8), (70, 3, 4000, 0.5)])
+def test_searches_over_many_tables_equal_oracle(gpu, d, arity, tuples, keep, tables, heuristic):
+    # the search looks at the tables in turn up to four a wave (64), and at the
+    # changed ones beyond; small and larger tables
+    desc = with_tables(60, d, 50, 0.25, tables, arity, tuples)
+    rng = np.random.default_rng(11)
+    init = desc.full_domains()
+    for v in range(60):
+        for a in range(d):
+            if rng.random() > keep and a != v % d:
+                init[v, a // 64] &= ~np.uint64(1 << (a % 64))
+    desc = desc.with_init_dom(init)
+    with oracle.var_heuristic(2 if heuristic == "dom/wdeg" else 0):
+        want = oracle.Oracle(desc, oracle.AC3).mac(node_limit=60, trace_cap=200)
+    with GModelAdapter.Build(desc, GModelOptions(skip_non_binary=False)) as m:
+        _, _, trace = m.Solve(node_limit=60, trace_capacity=200, heuristic=heuristic)
+    assert trace == want.trace
+
+
+def test_units_over_many_tables_equal_oracle(gpu):
+    # units of 16 tables and of more in one launch, at four waves and at sixteen
+    descs = [with_tables(60, 12, 50, 0.25, k, 3, 700) for k in (0, 16, 17, 64, 65, 150)]
+    want = [oracle.Oracle(desc, oracle.AC3).mac(node_limit=40) for desc in descs]
+    try:
+        N.tune_set("mac_lds_net", 1)  # (with an image the tables are taken up in turn)
+        for threads in (256, 1024):
+            N.tune_set("unit_threads", threads)
+            res, _ = Batch(descs, GModelOptions(skip_non_binary=False)).run(40)
+            for w, r in zip(want, res):
+                assert (r.num_positive, r.num_negative) == (w.num_positive, w.num_negative)
+    finally:
+        N.tune_set("unit_threads", 0)
+        N.tune_set("mac_lds_net", 0)
 
 
 def test_workgroup_passes_over_unchanged_tables(gpu):
