@@ -542,8 +542,13 @@ void build_lds_image(const ModelImage& im, DevModel& dm, hipStream_t s, std::vec
   }
 }
 
-// Whether a search takes the whole workgroup fixpoint (wg_fixpoint's kFull) when
-// it has no network image.
+// Whether the workgroup fixpoint looks at the tables first (wg_fixpoint's kTabs).
+bool many_tables(const ModelImage& im, int threads) {
+  return (int)im.tabs.size() > kTableTurns * (threads / 64);
+}
+
+// Whether a search takes the whole workgroup fixpoint (kTight and kTabs) when it
+// has no network image.
 //
 // For the tables, more than kTableTurns a wave: 300 of arity 5 and 3,000 tuples,
 // 60 nodes, 34 ms against 43; 900 of arity 3, 7.4 against 15.3 ms.
@@ -557,10 +562,10 @@ void build_lds_image(const ModelImage& im, DevModel& dm, hipStream_t s, std::vec
 // more than it saves: n=30 d=1000 e=131 3.7 / 2.4; n=100 d=250 e=1000 t=0.9 5.9
 // / 5.1; n=300 d=100 e=6000 t=0.84 1.66 / 1.39.  (Such a network's rows alone
 // are more than 3 MB, far beyond an image.)
-bool full_search(const ModelImage& im, int waves) {
+bool full_search(const ModelImage& im, int threads) {
   long long wp = 1;
   while (wp < im.W) wp *= 2;
-  return (int)im.tabs.size() > kTableTurns * waves || (im.W >= 3 && (long long)im.adj.size() * wp >= 12 * 1024);
+  return many_tables(im, threads) || (im.W >= 3 && (long long)im.adj.size() * wp >= 12 * 1024);
 }
 
 // Device bytes build_device_model takes from an arena for im (the same
@@ -1148,15 +1153,18 @@ void gac_block(cpim_gmodel* m, int assigned_var, cpim_gac_stats* st, const unsig
   DevNet net = m->dm.net();
   const long long bytes = wg_mem_bytes(m->dm.n, m->dm.W);
   const int threads = 1024;
+  const bool tabs = many_tables(m->im, threads);
   HostBox* box = m->box();
   const unsigned long long seq = m->next_seq();
   if (bytes <= kLdsBudget) {
-    hipLaunchKernelGGL(k_block_gac<true>, dim3(1), dim3(threads), (size_t)bytes, m->stream, net,
-                       m->level_dom(L), m->level_size(L), assigned_var, changed, (char*)nullptr, &box->gac, &box->seq, seq);
+    hipLaunchKernelGGL((tabs ? k_block_gac<true, true> : k_block_gac<true, false>), dim3(1), dim3(threads),
+                       (size_t)bytes, m->stream, net, m->level_dom(L), m->level_size(L), assigned_var, changed,
+                       (char*)nullptr, &box->gac, &box->seq, seq);
   } else {
     char* scratch = m->get_scratch(bytes);
-    hipLaunchKernelGGL(k_block_gac<false>, dim3(1), dim3(threads), 0, m->stream, net, m->level_dom(L),
-                       m->level_size(L), assigned_var, changed, scratch, &box->gac, &box->seq, seq);
+    hipLaunchKernelGGL((tabs ? k_block_gac<false, true> : k_block_gac<false, false>), dim3(1), dim3(threads), 0,
+                       m->stream, net, m->level_dom(L), m->level_size(L), assigned_var, changed, scratch,
+                       &box->gac, &box->seq, seq);
   }
   HIPC(hipGetLastError());
   m->wait_box(seq);
@@ -1590,13 +1598,15 @@ void run_singleton_batched(cpim_gmodel* m, const int2* tests_host, long long cou
   DevNet net = m->dm.net();
   const long long bytes = wg_mem_bytes(m->dm.n, m->dm.W);
   const int threads = 256;
+  const bool tabs = many_tables(m->im, threads);
   S.events();
   HIPC(hipEventRecord(S.ev[0], m->stream));
   if (bytes <= kLdsBudget) {
     for (long long first = 0; first < count; first += INT_MAX) {
       const long long blocks = std::min<long long>(count - first, INT_MAX);
-      hipLaunchKernelGGL(k_singleton_tests<true>, dim3((unsigned)blocks), dim3(threads), (size_t)bytes,
-                         m->stream, net, m->level_dom(L), m->level_size(L), S.tests.as<int2>(), count, first,
+      hipLaunchKernelGGL((tabs ? k_singleton_tests<true, true> : k_singleton_tests<true, false>),
+                         dim3((unsigned)blocks), dim3(threads), (size_t)bytes, m->stream, net, m->level_dom(L),
+                         m->level_size(L), S.tests.as<int2>(), count, first,
                          S.fails.as<unsigned char>(), S.revs.as<unsigned long long>(), (char*)nullptr, 0ll);
       HIPC(hipGetLastError());
     }
@@ -1604,7 +1614,8 @@ void run_singleton_batched(cpim_gmodel* m, const int2* tests_host, long long cou
     char* scratch = m->get_scratch(bytes * kScratchBlocks);
     for (long long first = 0; first < count; first += kScratchBlocks) {
       const long long blocks = std::min<long long>(count - first, kScratchBlocks);
-      hipLaunchKernelGGL(k_singleton_tests<false>, dim3((unsigned)blocks), dim3(threads), 0, m->stream, net,
+      hipLaunchKernelGGL((tabs ? k_singleton_tests<false, true> : k_singleton_tests<false, false>),
+                         dim3((unsigned)blocks), dim3(threads), 0, m->stream, net,
                          m->level_dom(L), m->level_size(L), S.tests.as<int2>(), count, first,
                          S.fails.as<unsigned char>(), S.revs.as<unsigned long long>(), scratch, bytes);
       HIPC(hipGetLastError());
@@ -2227,7 +2238,7 @@ int cpim_gmodel_solve(cpim_gmodel* m, const cpim_solve_opts* opts, cpim_search_s
       char* scratch = lds ? nullptr : m->get_scratch(bytes);
       auto* kernel = lds ? (A.weight ? k_mac<true, true, false> : k_mac<true, false, false>)
                          : (A.weight ? k_mac<false, true, false> : k_mac<false, false, false>);
-      if ((!lds || lnet.bytes == 0) && full_search(m->im, threads / 64))
+      if ((!lds || lnet.bytes == 0) && full_search(m->im, threads))
         kernel = lds ? (A.weight ? k_mac<true, true, true> : k_mac<true, false, true>)
                      : (A.weight ? k_mac<false, true, true> : k_mac<false, false, true>);
       hipLaunchKernelGGL(kernel, dim3(1), dim3(threads), (size_t)dyn, m->stream, net, A, scratch, lds ? lnet : LdsNet{});

@@ -1184,15 +1184,16 @@ __device__ __forceinline__ void wg_seed(const WgMem& mem, WgCtl* ctl, int n, int
 // slot: two wipe-out words used in turn by successive fixpoints, so that
 // wg_seed never resets the word a slow wave still reads.
 //
-// kFull: tight relations are settled by the wave (wave_unsupported), and of many
-// tables only those with a changed variable are taken up.  Both only cost
-// registers on the other networks, where a search waits for every instruction of
-// its chain (n=23 d=23 e=253 and dom/wdeg on n=100 d=50 take 3 % longer with the
-// look at the tables in their kernels): searches take the whole fixpoint where
-// the host's full_search says so.
-constexpr int kTableTurns = 4;  // tables a wave takes up in turn at most
+// kTight: tight relations are settled by the wave (wave_unsupported).  kTabs: of
+// many tables only those with a changed variable are taken up.  Each only costs
+// registers on the other networks (with the look at the tables in the kernel,
+// searches on n=23 d=23 e=253 and under dom/wdeg on n=100 d=50 take 3 % longer,
+// the tests of n=60 d=37 e=500 3.5 %, a fixpoint of n=40 d=16 e=195 7.9 instead
+// of 7.4 us): kTabs is for networks of more than kTableTurns tables a wave, and
+// searches take both (kFull) where the host's full_search says so.
+constexpr int kTableTurns = 4;
 
-template <bool kFull>
+template <bool kTight, bool kTabs>
 __device__ __forceinline__ bool wg_fixpoint(const DevNet& net, const WgMem& mem, WgCtl* ctl, int slot,
                                             int seed_both) {
   const int n = net.n, W = net.W;
@@ -1210,7 +1211,7 @@ __device__ __forceinline__ bool wg_fixpoint(const DevNet& net, const WgMem& mem,
   int c0 = 0, c1 = nvw, c2 = 2 * nvw;
   // this wave's first table, its lanes' part kept over the rounds
   const int itab = nwaves - 1 - wave;
-  const bool many_tabs = kFull && net.ntabs > kTableTurns * nwaves;
+  const bool many_tabs = kTabs && net.ntabs > kTableTurns * nwaves;
   SmallTable tab0{};
   if (itab < net.ntabs) tab0 = load_small_table(net, uniform_int(net.tabs[itab]));
   for (int round = 0;; ++round) {
@@ -1267,7 +1268,7 @@ __device__ __forceinline__ bool wg_fixpoint(const DevNet& net, const WgMem& mem,
           stop = true;
           break;
         }
-        const u64 gone = wave_unsupported<kFull>(net, mem.dom, t, pair + (long long)(pos_t * W + w) * net.dpad,
+        const u64 gone = wave_unsupported<kTight>(net, mem.dom, t, pair + (long long)(pos_t * W + w) * net.dpad,
                                                   pair + (long long)(1 - pos_t) * W * net.dpad + 64 * w, need);
         if (gone) lane_remove(mem, ctl, nxt, slot, round, u, word, gone);
         revs += cnt;
@@ -1306,7 +1307,7 @@ __device__ __forceinline__ bool wg_fixpoint(const DevNet& net, const WgMem& mem,
     int seen = 0;                                // changed tables before this turn's
     for (int base = many_tabs && look == 1 ? 0 : itab; base < net.ntabs; base += many_tabs ? 64 * look : nwaves) {
       u64 found = 1ull;  // bit k: table base + k * look is this wave's
-      if (kFull && many_tabs) {
+      if (kTabs && many_tabs) {
         const int k = base + lane * look;
         bool ch = false;
         if (k < net.ntabs) {
@@ -1617,7 +1618,7 @@ __device__ __forceinline__ u64 wg_reduce_sum_u64(WgCtl* ctl, u64 v) {
 // Block-mode GAC on one level (one workgroup).  changed: goes on from these
 // variables, where rounds over the grid left off (NULL: starts from seed_var).
 // ---------------------------------------------------------------------------
-template <bool kLds>
+template <bool kLds, bool kTabs>
 __global__ void k_block_gac(DevNet net, u64* dom, int* size, int seed_var, const unsigned* changed, char* scratch,
                             GacResult* out, unsigned long long* seq_at, unsigned long long seq) {
   const unsigned long long t0 = wall_clock64();
@@ -1634,7 +1635,7 @@ __global__ void k_block_gac(DevNet net, u64* dom, int* size, int seed_var, const
   __syncthreads();
   long long before = 0;
   for (int v = threadIdx.x; v < n; v += blockDim.x) before += mem.size[v];
-  const bool ok = wg_fixpoint<true>(net, mem, &ctl, 0, changed ? -1 : seed_var);
+  const bool ok = wg_fixpoint<true, kTabs>(net, mem, &ctl, 0, changed ? -1 : seed_var);
   long long after = 0;
   for (int v = threadIdx.x; v < n; v += blockDim.x) after += mem.size[v];
   const u64 delta = wg_reduce_sum_u64(&ctl, (u64)(before - after));
@@ -1752,7 +1753,7 @@ __global__ void __launch_bounds__(kThreads) k_level_op(int op, u64* dom, int* si
 // kernel has no loop around its barriers, and the hardware dispatcher keeps
 // every CU busy as workgroups finish at different times.
 // ---------------------------------------------------------------------------
-template <bool kLds>
+template <bool kLds, bool kTabs>
 __global__ void k_singleton_tests(DevNet net, const u64* __restrict__ base_dom,
                                   const int* __restrict__ base_size, const int2* __restrict__ tests,
                                   long long ntests, long long first, unsigned char* fail,
@@ -1779,7 +1780,7 @@ __global__ void k_singleton_tests(DevNet net, const u64* __restrict__ base_dom,
     mem.asg[x >> 5] |= 1u << (x & 31);
   }
   __syncthreads();
-  const bool ok = wg_fixpoint<true>(net, mem, &ctl, 0, -1);
+  const bool ok = wg_fixpoint<true, kTabs>(net, mem, &ctl, 0, -1);
   __syncthreads();  // every wave's revision count
   if (threadIdx.x == 0) {
     fail[unit] = ok ? 0 : 1;
@@ -3275,7 +3276,7 @@ __device__ __forceinline__ void wg_load_level(const WgMem& mem, const u64* level
 // one, beside the fixpoint's own.  kWdeg: dom/wdeg ordering, wipe-outs
 // repeated in AC3's order.  kFlat: wg_fixpoint_flat propagates, and a
 // refutation that follows its decision takes the domains from registers (dom
-// and dom/deg only).  kFull: as wg_fixpoint's.
+// and dom/deg only).  kFull: wg_fixpoint's kTight and kTabs.
 template <bool kWdeg, bool kFlat, bool kFull>
 __device__ __forceinline__ void wg_mac_run(const DevNet& net, const WgMem& mem, WgCtl* ctl, const MacArgs& A) {
   enum { ROOT, POSITIVE, NEGATIVE };
@@ -3426,7 +3427,7 @@ __device__ __forceinline__ void wg_mac_run(const DevNet& net, const WgMem& mem, 
       ok = wg_fixpoint_flat(mem, ctl, flat, seen, phase == ROOT ? -1 : x, phase == POSITIVE ? bit : dx & ~bit,
                             phase == POSITIVE, turn, flat_revs);
     } else {
-      ok = wg_fixpoint<kFull>(net, mem, ctl, slot, -1);
+      ok = wg_fixpoint<kFull, kFull>(net, mem, ctl, slot, -1);
     }
     if (kWdeg && !ok) {
       // a wipe-out raises the weight of the constraint that AC3's order
