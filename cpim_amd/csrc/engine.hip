@@ -241,7 +241,7 @@ ModelImage make_image(const cpim_model_desc* d, bool skip_non_binary, bool own_r
       ConMeta m{};
       m.kind = 1;
       m.arity = ar;
-      for (int i = 0; i < ar; ++i) m.scope[i] = sc[i];
+      for (int i = 0; i < CPIM_MAX_ARITY; ++i) m.scope[i] = sc[i < ar ? i : 0];  // (wg_fixpoint reads all)
       m.tw = std::max<int>(1, (int)((T + 63) / 64));
       m.off = tsup_off;
       const long long words = (long long)ar * im.dpad * m.tw;
@@ -551,7 +551,7 @@ bool many_tables(const ModelImage& im, int threads) {
 // has no network image.
 //
 // For the tables, more than kTableTurns a wave: 300 of arity 5 and 3,000 tuples,
-// 60 nodes, 34 ms against 43; 900 of arity 3, 7.4 against 15.3 ms.
+// 60 nodes, 33 ms against 43; 900 of arity 3, 7.3 against 15.3 ms.
 //
 // For tight relations settled by the wave (wave_settle), domains of three words and more, and at least 12 turns of a
 // 1024-lane workgroup over the arc words.  Where that is so, a lane's serial

@@ -1311,14 +1311,11 @@ __device__ __forceinline__ bool wg_fixpoint(const DevNet& net, const WgMem& mem,
         const int k = base + lane * look;
         bool ch = false;
         if (k < net.ntabs) {
+          // (unused positions of a table hold its first variable: no arity to read)
           const ConMeta* mp = net.con + net.tabs[k];
-          const int arity = mp->arity;
           unsigned bits = 0u;
 #pragma unroll
-          for (int p = 0; p < CPIM_MAX_ARITY; ++p) {  // (unused positions hold variable 0)
-            const int y = mp->scope[p];
-            bits |= p < arity ? cur[y >> 5] >> (y & 31) : 0u;
-          }
+          for (int p = 0; p < CPIM_MAX_ARITY; ++p) bits |= cur[mp->scope[p] >> 5] >> (mp->scope[p] & 31);
           ch = bits & 1u;
         }
         found = __ballot(ch);
